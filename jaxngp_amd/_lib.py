@@ -31,6 +31,7 @@ TARGETS = (
     "integrate_rays_backward",
     "integrate_rays_inference",
     "hashgrid_encode",
+    "hashgrid_encode_staged",
     "hashgrid_encode_backward",
     "tcnn_hashgrid_encode",
     "tcnn_hashgrid_encode_backward",

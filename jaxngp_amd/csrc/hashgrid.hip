@@ -6,10 +6,8 @@
 // registers: normalise, scale, floor, 8 vertex indices (dense x + y res + z res^2
 // below first_hash_level, else x ^ y*2654435761 ^ z*805459861, both mod T, plus the
 // level's row offset), trilinear weights, weighted sum of the gathered rows.
-// Point-major output: threads are laid out level-fastest, so the L*F outputs of a
-// point are written by L consecutive lanes as one contiguous run.  Level-major
-// output: workgroups are level-affine per XCD (see level_block) so each level's
-// gathers hit one L2.
+// Workgroups are level-affine per XCD (see level_block), so a level's gathers hit one
+// L2, whichever layout the output has.
 //
 // Backward is the VJP of the gather (encoders.py:226) and of the weighted sum
 // (encoders.py:231): dtable[idx] += w * g, computed by a counting sort of the
@@ -28,52 +26,28 @@ namespace {
 
 constexpr int kBlock = 256;
 
-template <int F, typename TT>
-__global__ void __launch_bounds__(kBlock)
-    hashgrid_fwd_kernel(HashGridDescriptor d, const float *__restrict__ pos, const TT *__restrict__ table,
-                        float *__restrict__ enc) {
-    __shared__ LevelTables lt;
-    if (threadIdx.x < d.L) {
-        lt.scale[threadIdx.x] = d.scales[threadIdx.x];
-        lt.res[threadIdx.x] = d.resolutions[threadIdx.x];
-        lt.offset[threadIdx.x] = d.offsets[threadIdx.x];
-    }
-    __syncthreads();
-    const uint64_t gid = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (gid >= (uint64_t)d.n_points * d.L) return;
-    const uint32_t n = (uint32_t)(gid / d.L);
-    const uint32_t l = (uint32_t)(gid - (uint64_t)n * d.L);
-    const Divisor two_b = make_divisor(2.0f * d.bound);
-    const float px = divide(two_b, pos[3 * (size_t)n + 0] + d.bound);
-    const float py = divide(two_b, pos[3 * (size_t)n + 1] + d.bound);
-    const float pz = divide(two_b, pos[3 * (size_t)n + 2] + d.bound);
-    uint32_t idx[8];
-    float w[8];
-    level_vertices(px, py, pz, lt.scale[l], lt.res[l], l < d.first_hash_level, d.T, (d.T & (d.T - 1u)) == 0,
-                   lt.offset[l], d.n_rows - 1u, idx, w);
-    float acc[F];
-#pragma unroll
-    for (int f = 0; f < F; ++f) acc[f] = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const TT *row = table + (size_t)idx[c] * F;
-#pragma unroll
-        for (int f = 0; f < F; ++f) acc[f] = acc[f] + to_f32<TT>(row[f]) * w[c];
-    }
-    float *out = enc + gid * F;
-#pragma unroll
-    for (int f = 0; f < F; ++f) out[f] = acc[f];
-}
-
 // Workgroups are dispatched round-robin over the 8 XCDs of the chip (block b runs
-// on XCD b % 8), each with its own 4 MiB L2.  Level-affine kernels therefore give
-// block b the level 8 * phase + b % 8: all blocks of one XCD work on the same level
-// in a phase, so that level's rows (at most T * F * 4 B = 4 MiB for T = 2^19, F = 2)
-// stay resident in that XCD's L2 for the gathers / atomics, instead of every L2
-// streaming the whole 46.5 MiB table.
+// on XCD b % 8), each with its own 4 MiB L2.  An XCD therefore works on one level at a
+// time, so that level's rows (at most T * F * 4 B = 4 MiB for T = 2^19, F = 2) stay in
+// its L2 for the gathers, instead of every L2 streaming the whole 46.5 MiB table.
+// Levels cost differently (2^18 ray samples, one level on every XCD: 16 us for a dense
+// or coarse one, whose cells a ray's samples share, 54 us for the finest, f32), so two
+// whole levels per XCD left the ones with the finest levels working alone (71 us
+// against a mean of 57).  Four pairs of XCDs instead deal the levels in snake order
+// from the finest down, each XCD of a pair taking every second group of points: the
+// sums of the four sets are within 6% of the mean for ray samples, and random points,
+// where all hashed levels cost alike, get 2 or 3 of the 11 per pair.
 constexpr uint32_t kXcds = 8;
 constexpr int kLmPointsPerThread = 2;
 constexpr int kPointsPerBlock = kBlock * kLmPointsPerThread;
+
+constexpr uint32_t kLevelSets = kXcds / 2;
+
+// Point groups of one XCD and level: every second group of kPointsPerBlock points.
+__host__ __device__ inline uint32_t half_groups(uint32_t n_points) {
+    const uint64_t n_pg = ((uint64_t)n_points + kPointsPerBlock - 1) / kPointsPerBlock;
+    return (uint32_t)((n_pg + 1) / 2);
+}
 
 struct LevelBlock {
     uint32_t level, point0;
@@ -81,65 +55,109 @@ struct LevelBlock {
 };
 
 __device__ __forceinline__ LevelBlock level_block(uint32_t n_points, uint32_t L) {
-    const uint32_t n_pg = (n_points + kPointsPerBlock - 1) / kPointsPerBlock;
+    const uint32_t n_half = half_groups(n_points);
     const uint32_t b = blockIdx.x;
     const uint32_t x = b % kXcds, rest = b / kXcds;
-    const uint32_t pg = rest % n_pg, phase = rest / n_pg;
+    const uint32_t i = rest % n_half, phase = rest / n_half;
+    const uint32_t s = x % kLevelSets;
+    const uint32_t k = phase * kLevelSets + ((phase & 1u) ? kLevelSets - 1u - s : s);
     LevelBlock lb;
-    lb.level = phase * kXcds + x;
-    lb.point0 = pg * kPointsPerBlock;
-    lb.live = lb.level < L;
+    lb.level = L - 1u - k;
+    lb.point0 = (2u * i + x / kLevelSets) * kPointsPerBlock;
+    lb.live = k < L && lb.point0 < n_points;
     return lb;
 }
 
 inline uint32_t level_grid(uint32_t n_points, uint32_t L) {
-    const uint32_t n_pg = div_up(n_points, kPointsPerBlock);
-    return kXcds * n_pg * div_up(L, kXcds);
+    return kXcds * half_groups(n_points) * div_up(L, kLevelSets);
 }
 
-// Level-major forward: each thread takes kLmPointsPerThread points of the block's
-// level, kBlock apart, so the gathers of both are in flight together; output
-// enc[(l * N + n) * F + f] written as one contiguous run per wavefront.  Points past
-// the end load the last point and store nothing.
-template <int F, typename TT>
+// Forward: each thread takes kLmPointsPerThread points of the block's level, kBlock
+// apart, so the gathers of both are in flight together; points past the end load the
+// last point and store nothing.  Level-major output is one contiguous run per
+// wavefront; point-major output is 8 bytes per point, 128 apart, which costs less than
+// giving up the level's residency in L2 did (a wavefront of 4 points x 16 levels).
+// kGroups: see GroupedGather.  Measured, 2^18 ray samples: f32 level-major 92 -> 55 us
+// (68 with the levels two to an XCD), point-major 109 -> 93; f16 82 -> 46 and 97 -> 76.
+template <int F, typename TT, bool kGroups>
 __global__ void __launch_bounds__(kBlock)
-    hashgrid_fwd_lm_kernel(HashGridDescriptor d, const float *__restrict__ pos, const TT *__restrict__ table,
+    hashgrid_fwd_kernel(HashGridDescriptor d, const float *__restrict__ pos, const TT *__restrict__ table,
                            float *__restrict__ enc) {
     constexpr int P = kLmPointsPerThread;
     const LevelBlock lb = level_block(d.n_points, d.L);
     if (!lb.live) return;
     const uint32_t l = lb.level;
-    const Divisor two_b = make_divisor(2.0f * d.bound);
-    uint32_t idx[P][8];
-    float w[P][8];
+    const bool level_major = d.enc_layout == NGP_ENC_LEVEL_MAJOR;
+    const size_t point_stride = level_major ? F : (size_t)d.L * F;
+    float *const level_out = enc + (size_t)l * (level_major ? (size_t)d.n_points * F : F);
+    float at[P][3], q[P][3];
 #pragma unroll
     for (int j = 0; j < P; ++j) {
         const uint32_t n = lb.point0 + j * kBlock + threadIdx.x;
         const uint32_t np = n < d.n_points ? n : d.n_points - 1;
-        const float px = divide(two_b, pos[3 * (size_t)np + 0] + d.bound);
-        const float py = divide(two_b, pos[3 * (size_t)np + 1] + d.bound);
-        const float pz = divide(two_b, pos[3 * (size_t)np + 2] + d.bound);
-        level_vertices(px, py, pz, d.scales[l], d.resolutions[l], l < d.first_hash_level, d.T,
-                       (d.T & (d.T - 1u)) == 0, d.offsets[l], d.n_rows - 1u, idx[j], w[j]);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) at[j][a] = pos[3 * (size_t)np + a];
     }
+    const Divisor two_b = make_divisor(2.0f * d.bound);
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
-        float acc[F];
+    for (int j = 0; j < P; ++j) normalise(two_b, d.bound, at[j], q[j]);
+    with_rule(l < d.first_hash_level, (d.T & (d.T - 1u)) == 0, [&](auto rule, auto pow2) {
+        uint32_t idx[P][8];
+        float w[P][8];
 #pragma unroll
-        for (int f = 0; f < F; ++f) acc[f] = 0.0f;
+        for (int j = 0; j < P; ++j)
+            level_vertices_t<decltype(rule)::value, decltype(pow2)::value>(
+                q[j][0], q[j][1], q[j][2], d.scales[l], d.resolutions[l], l < d.first_hash_level, d.T, d.offsets[l],
+                d.n_rows - 1u, idx[j], w[j]);
+        if constexpr (kGroups) {
+            static_assert(F == 2, "grouped rows hold two features");
+            GroupedGather<TT> gg[P];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const TT *row = table + (size_t)idx[j][c] * F;
+            for (int j = 0; j < P; ++j) gg[j].load(table_buffer(d, table), idx[j]);
 #pragma unroll
-            for (int f = 0; f < F; ++f) acc[f] = acc[f] + to_f32<TT>(row[f]) * w[j][c];
+            for (int j = 0; j < P; ++j) {
+                const float2 v = gg[j].sum(idx[j], w[j]);
+                const uint32_t n = lb.point0 + j * kBlock + threadIdx.x;
+                if (n < d.n_points) *reinterpret_cast<float2 *>(level_out + n * point_stride) = v;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < P; ++j) {
+                float acc[F];
+#pragma unroll
+                for (int f = 0; f < F; ++f) acc[f] = 0.0f;
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    const TT *row = table + (size_t)idx[j][c] * F;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) acc[f] = acc[f] + to_f32<TT>(row[f]) * w[j][c];
+                }
+                const uint32_t n = lb.point0 + j * kBlock + threadIdx.x;
+                if (n < d.n_points) {
+                    float *out = level_out + n * point_stride;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) out[f] = acc[f];
+                }
+            }
         }
-        const uint32_t n = lb.point0 + j * kBlock + threadIdx.x;
-        if (n < d.n_points) {
-            float *out = enc + ((size_t)l * d.n_points + n) * F;
-#pragma unroll
-            for (int f = 0; f < F; ++f) out[f] = acc[f];
-        }
+    });
+}
+
+// [L, n, F] encodings -> [n, L * F], for F = 2: a workgroup takes kTransposePoints
+// points, reads each level's run (512 bytes) and writes the points' rows, both coalesced,
+// through LDS.
+constexpr int kTransposePoints = 64;
+__global__ void __launch_bounds__(kBlock)
+    encodings_to_points_kernel(uint32_t n_points, uint32_t L, const float2 *__restrict__ lm, float2 *__restrict__ pm) {
+    __shared__ float2 tile[kTransposePoints * (NGP_HASHGRID_MAX_LEVELS + 1)];
+    const uint32_t p0 = blockIdx.x * kTransposePoints;
+    const uint32_t n = min((uint32_t)kTransposePoints, n_points - p0), row = L + 1;
+    for (uint32_t t = threadIdx.x; t < L * kTransposePoints; t += kBlock) {
+        const uint32_t l = t / kTransposePoints, i = t % kTransposePoints;
+        if (i < n) tile[i * row + l] = lm[(size_t)l * n_points + p0 + i];
     }
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < n * L; t += kBlock) pm[(size_t)p0 * L + t] = tile[t / L * row + t % L];
 }
 
 // Backward without global atomics.  Device-scope atomics on this chip (float or
@@ -331,13 +349,14 @@ __device__ __forceinline__ void point_runs(const HashGridDescriptor &d, uint32_t
                                            bool dense, bool pow2, const float *xyz, const float *gin, bool active,
                                            Emit emit) {
     const int lane = lane_id();
-    const Divisor two_b = make_divisor(2.0f * d.bound);
-    const float px = divide(two_b, xyz[0] + d.bound);
-    const float py = divide(two_b, xyz[1] + d.bound);
-    const float pz = divide(two_b, xyz[2] + d.bound);
+    float p[3];
+    normalise(make_divisor(2.0f * d.bound), d.bound, xyz, p);
     uint32_t idx[8];
     float w[8];
-    level_vertices(px, py, pz, scale, res, dense, d.T, pow2, d.offsets[l], d.n_rows - 1u, idx, w);
+    with_rule(dense, pow2, [&](auto rule, auto p2) {
+        level_vertices_t<decltype(rule)::value, decltype(p2)::value>(p[0], p[1], p[2], scale, res, dense, d.T,
+                                                                     d.offsets[l], d.n_rows - 1u, idx, w);
+    });
     float g[F];
 #pragma unroll
     for (int f = 0; f < F; ++f) g[f] = kValues && active ? gin[f] : 0.0f;
@@ -1079,22 +1098,17 @@ bool validate(const HashGridDescriptor &d, const char *target) {
 template <typename TT>
 void launch_fwd(const HashGridDescriptor &d, hipStream_t s, const float *pos, const void *table, float *enc) {
     const TT *t = static_cast<const TT *>(table);
-    if (d.enc_layout == NGP_ENC_LEVEL_MAJOR) {
-        const uint32_t g = level_grid(d.n_points, d.L);
-        switch (d.F) {
-            case 1: hipLaunchKernelGGL((hashgrid_fwd_lm_kernel<1, TT>), dim3(g), dim3(kBlock), 0, s, d, pos, t, enc); break;
-            case 2: hipLaunchKernelGGL((hashgrid_fwd_lm_kernel<2, TT>), dim3(g), dim3(kBlock), 0, s, d, pos, t, enc); break;
-            case 4: hipLaunchKernelGGL((hashgrid_fwd_lm_kernel<4, TT>), dim3(g), dim3(kBlock), 0, s, d, pos, t, enc); break;
-            default: hipLaunchKernelGGL((hashgrid_fwd_lm_kernel<8, TT>), dim3(g), dim3(kBlock), 0, s, d, pos, t, enc); break;
-        }
-        return;
-    }
-    const uint32_t grid = div_up((uint64_t)d.n_points * d.L, kBlock);
+    // the grouped gather writes a row's two features as one 8-byte vector
+    const bool groups = grouped_rows_ok(d, table) && (reinterpret_cast<uintptr_t>(enc) & 7u) == 0;
+    const dim3 g(level_grid(d.n_points, d.L)), b(kBlock);
     switch (d.F) {
-        case 1: hipLaunchKernelGGL((hashgrid_fwd_kernel<1, TT>), dim3(grid), dim3(kBlock), 0, s, d, pos, t, enc); break;
-        case 2: hipLaunchKernelGGL((hashgrid_fwd_kernel<2, TT>), dim3(grid), dim3(kBlock), 0, s, d, pos, t, enc); break;
-        case 4: hipLaunchKernelGGL((hashgrid_fwd_kernel<4, TT>), dim3(grid), dim3(kBlock), 0, s, d, pos, t, enc); break;
-        default: hipLaunchKernelGGL((hashgrid_fwd_kernel<8, TT>), dim3(grid), dim3(kBlock), 0, s, d, pos, t, enc); break;
+        case 1: hipLaunchKernelGGL((hashgrid_fwd_kernel<1, TT, false>), g, b, 0, s, d, pos, t, enc); break;
+        case 2:
+            if (groups) hipLaunchKernelGGL((hashgrid_fwd_kernel<2, TT, true>), g, b, 0, s, d, pos, t, enc);
+            else hipLaunchKernelGGL((hashgrid_fwd_kernel<2, TT, false>), g, b, 0, s, d, pos, t, enc);
+            break;
+        case 4: hipLaunchKernelGGL((hashgrid_fwd_kernel<4, TT, false>), g, b, 0, s, d, pos, t, enc); break;
+        default: hipLaunchKernelGGL((hashgrid_fwd_kernel<8, TT, false>), g, b, 0, s, d, pos, t, enc); break;
     }
 }
 
@@ -1115,6 +1129,34 @@ extern "C" void hashgrid_encode(ngp_stream_t stream_, void **buffers, const char
     float *enc = (float *)buffers[2];
     if (d.table_dtype == NGP_DTYPE_F32) launch_fwd<float>(d, stream, pos, buffers[1], enc);
     else launch_fwd<__half>(d, stream, pos, buffers[1], enc);
+    check_launch(target);
+}
+
+extern "C" void hashgrid_encode_staged(ngp_stream_t stream_, void **buffers, const char *opaque, size_t opaque_len) {
+    const char *target = "hashgrid_encode_staged";
+    HashGridDescriptor d;
+    if (!read_descriptor(opaque, opaque_len, &d, target)) return;
+    if (!validate(d, target)) return;
+    if (d.F != 2 || d.enc_layout != NGP_ENC_POINT_MAJOR) {
+        set_error(kBadDescriptor, "%s: F must be 2 and enc_layout 0 (point-major)", target);
+        return;
+    }
+    if (d.n_points == 0) return;
+    if (!check_buffers(buffers, 4, target)) return;
+    if (((reinterpret_cast<uintptr_t>(buffers[2]) | reinterpret_cast<uintptr_t>(buffers[3])) & 7u) != 0) {
+        set_error(kBadArgument, "%s: encodings and the workspace must be 8-byte aligned", target);
+        return;
+    }
+    hipStream_t stream = (hipStream_t)stream_;
+    const float *pos = (const float *)buffers[0];
+    float *lm = (float *)buffers[3];
+    HashGridDescriptor dl = d;
+    dl.enc_layout = NGP_ENC_LEVEL_MAJOR;
+    if (d.table_dtype == NGP_DTYPE_F32) launch_fwd<float>(dl, stream, pos, buffers[1], lm);
+    else launch_fwd<__half>(dl, stream, pos, buffers[1], lm);
+    if (!check_launch(target)) return;
+    hipLaunchKernelGGL(encodings_to_points_kernel, dim3(div_up(d.n_points, kTransposePoints)), dim3(kBlock), 0, stream,
+                       d.n_points, d.L, (const float2 *)lm, (float2 *)buffers[2]);
     check_launch(target);
 }
 

@@ -823,22 +823,29 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 // arithmetic, so the result equals hashgrid_encode followed by nerf_mlp_forward.
 // ---------------------------------------------------------------------------
 
+// Levels l and l + 1 of a normalised position, as four features.  Row by row: the
+// grouped gather of the encoder needs 24 more registers here and cost a wave per SIMD.
 template <typename TT>
-__device__ __forceinline__ float2 encode_level(const HashGridDescriptor &d, const LevelTables &lt,
-                                               const TT *__restrict__ table, float px, float py, float pz,
-                                               uint32_t l) {
-    uint32_t idx[8];
-    float w[8];
-    level_vertices(px, py, pz, lt.scale[l], lt.res[l], l < d.first_hash_level, d.T, (d.T & (d.T - 1u)) == 0,
-                   lt.offset[l], d.n_rows - 1u, idx, w);
-    float a0 = 0.0f, a1 = 0.0f;
+__device__ __forceinline__ v4f encode_two_levels(const HashGridDescriptor &d, const LevelTables &lt,
+                                                 const TT *__restrict__ table, const float p[3], uint32_t l) {
+    v4f out;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const TT *row = table + (size_t)idx[c] * 2;
-        a0 = a0 + to_f32<TT>(row[0]) * w[c];
-        a1 = a1 + to_f32<TT>(row[1]) * w[c];
+    for (int k = 0; k < 2; ++k) {
+        uint32_t idx[8];
+        float w[8];
+        level_vertices(p[0], p[1], p[2], lt.scale[l + k], lt.res[l + k], l + k < d.first_hash_level, d.T,
+                       (d.T & (d.T - 1u)) == 0, lt.offset[l + k], d.n_rows - 1u, idx, w);
+        float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const TT *row = table + (size_t)idx[c] * 2;
+            a0 = a0 + to_f32<TT>(row[0]) * w[c];
+            a1 = a1 + to_f32<TT>(row[1]) * w[c];
+        }
+        out[2 * k] = a0;
+        out[2 * k + 1] = a1;
     }
-    return make_float2(a0, a1);
+    return out;
 }
 
 template <typename TT, bool kHalf>
@@ -882,25 +889,17 @@ __global__ void __launch_bounds__(kThreads)
             if (g == 0 && e < n_entries) *reinterpret_cast<v4f *>(drgbs + 4 * e) = zero;
             continue;
         }
-        float px = 0.0f, py = 0.0f, pz = 0.0f, dx = 0.0f, dy = 0.0f, dz = 0.0f;
+        float dx = 0.0f, dy = 0.0f, dz = 0.0f;
+        v4f x[2] = {zero, zero};
         if (live) {
-            px = divide(two_b, xyzs[3 * e + 0] + d.bound);
-            py = divide(two_b, xyzs[3 * e + 1] + d.bound);
-            pz = divide(two_b, xyzs[3 * e + 2] + d.bound);
+            const float at[3] = {xyzs[3 * e + 0], xyzs[3 * e + 1], xyzs[3 * e + 2]};
             dx = rays_d[3 * (size_t)ray + 0];
             dy = rays_d[3 * (size_t)ray + 1];
             dz = rays_d[3 * (size_t)ray + 2];
-        }
-        v4f x[2];
-        if (live) {
+            float p[3];
+            normalise(two_b, d.bound, at, p);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const float2 lo = encode_level(d, lt, table, px, py, pz, 8 * b + 2 * g);
-                const float2 hi = encode_level(d, lt, table, px, py, pz, 8 * b + 2 * g + 1);
-                x[b] = v4f{lo.x, lo.y, hi.x, hi.y};
-            }
-        } else {
-            x[0] = x[1] = zero;
+            for (int b = 0; b < 2; ++b) x[b] = encode_two_levels(d, lt, table, p, 8 * b + 2 * g);
         }
         v4f out = zero;
         float o0;
@@ -1044,16 +1043,11 @@ __global__ void __launch_bounds__(kThreads)
             live = m < G3;  // an alive index past the cascade is dropped, as JAX drops it
         }
         if (live) {
-            float wx, wy, wz;
-            ogrid_point(a, m, j, wx, wy, wz);
-            const float px = divide(two_b, wx + a.bound), py = divide(two_b, wy + a.bound),
-                        pz = divide(two_b, wz + a.bound);
+            float at[3], p[3];
+            ogrid_point(a, m, j, at[0], at[1], at[2]);
+            normalise(two_b, a.bound, at, p);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const float2 lo = encode_level(d, lt, table, px, py, pz, 8 * b + 2 * g);
-                const float2 hi = encode_level(d, lt, table, px, py, pz, 8 * b + 2 * g + 1);
-                x[b] = v4f{lo.x, lo.y, hi.x, hi.y};
-            }
+            for (int b = 0; b < 2; ++b) x[b] = encode_two_levels(d, lt, table, p, 8 * b + 2 * g);
         }
         float o0;
         if (kHalf) {
@@ -1263,6 +1257,20 @@ extern "C" void nerf_mlp_backward_no_alloc(ngp_stream_t stream_, void **buffers,
 }
 
 namespace {
+template <typename T>
+struct TypeTag {
+    using type = T;
+};
+
+// Calls f(table type, f16 weights) with both as compile-time values.
+template <typename Fn>
+void with_field_types(bool t16, bool w16, Fn f) {
+    if (t16 && w16) f(TypeTag<_Float16>{}, std::true_type{});
+    else if (t16) f(TypeTag<_Float16>{}, std::false_type{});
+    else if (w16) f(TypeTag<float>{}, std::true_type{});
+    else f(TypeTag<float>{}, std::false_type{});
+}
+
 // The NeRF position encoder's descriptor: L = 16, F = 2, a consistent level table.
 bool check_nerf_grid(const HashGridDescriptor &g, uint32_t param_dtype, const char *target) {
     if (g.L != 16 || g.F != 2 || g.T == 0 || g.n_rows == 0 || g.first_hash_level > g.L || g.offsets[0] != 0 ||
@@ -1308,18 +1316,12 @@ extern "C" void nerf_field_chunks(ngp_stream_t stream, void **buffers, const cha
     const float *rd = (const float *)buffers[3];
     const void *params = buffers[5];
     float *out = (float *)buffers[6];
-    if (t16 && w16)
-        hipLaunchKernelGGL((field_chunks_kernel<_Float16, true>), dim3(grid), dim3(kThreads), 0, s, g, d.n_slots, d.cap,
-                           d.n_total_rays, xyzs, ns, idx, rd, (const _Float16 *)buffers[4], params, out);
-    else if (t16)
-        hipLaunchKernelGGL((field_chunks_kernel<_Float16, false>), dim3(grid), dim3(kThreads), 0, s, g, d.n_slots,
-                           d.cap, d.n_total_rays, xyzs, ns, idx, rd, (const _Float16 *)buffers[4], params, out);
-    else if (w16)
-        hipLaunchKernelGGL((field_chunks_kernel<float, true>), dim3(grid), dim3(kThreads), 0, s, g, d.n_slots, d.cap,
-                           d.n_total_rays, xyzs, ns, idx, rd, (const float *)buffers[4], params, out);
-    else
-        hipLaunchKernelGGL((field_chunks_kernel<float, false>), dim3(grid), dim3(kThreads), 0, s, g, d.n_slots, d.cap,
-                           d.n_total_rays, xyzs, ns, idx, rd, (const float *)buffers[4], params, out);
+    with_field_types(t16, w16, [&](auto tt, auto half) {
+        using TT = typename decltype(tt)::type;
+        hipLaunchKernelGGL((field_chunks_kernel<TT, decltype(half)::value>), dim3(grid),
+                           dim3(kThreads), 0, s, g, d.n_slots, d.cap, d.n_total_rays, xyzs, ns, idx, rd,
+                           (const TT *)buffers[4], params, out);
+    });
     check_launch(target);
 }
 
@@ -1378,17 +1380,10 @@ extern "C" void occupancy_grid_update(ngp_stream_t stream, void **buffers, const
     const uint32_t grid = std::max<uint32_t>(1, std::min<uint32_t>(div_up(tiles, kWaves), 2048));
     const void *params = buffers[3];
     const bool t16 = g.table_dtype == NGP_DTYPE_F16, w16 = d.param_dtype == NGP_DTYPE_F16;
-    if (t16 && w16)
-        hipLaunchKernelGGL((ogrid_update_kernel<_Float16, true>), dim3(grid), dim3(kThreads), 0, s, g, a, alive,
-                           prefix, words, (const _Float16 *)buffers[2], params, density);
-    else if (t16)
-        hipLaunchKernelGGL((ogrid_update_kernel<_Float16, false>), dim3(grid), dim3(kThreads), 0, s, g, a, alive,
-                           prefix, words, (const _Float16 *)buffers[2], params, density);
-    else if (w16)
-        hipLaunchKernelGGL((ogrid_update_kernel<float, true>), dim3(grid), dim3(kThreads), 0, s, g, a, alive, prefix,
-                           words, (const float *)buffers[2], params, density);
-    else
-        hipLaunchKernelGGL((ogrid_update_kernel<float, false>), dim3(grid), dim3(kThreads), 0, s, g, a, alive, prefix,
-                           words, (const float *)buffers[2], params, density);
+    with_field_types(t16, w16, [&](auto tt, auto half) {
+        using TT = typename decltype(tt)::type;
+        hipLaunchKernelGGL((ogrid_update_kernel<TT, decltype(half)::value>), dim3(grid),
+                           dim3(kThreads), 0, s, g, a, alive, prefix, words, (const TT *)buffers[2], params, density);
+    });
     check_launch(target);
 }

@@ -63,12 +63,22 @@ def level_table(L: int, T: int, N_min: int, N_max: int, dim: int = 3) -> LevelTa
     return LevelTable(b, tuple(scales), tuple(res), tuple(offsets), first)
 
 
+# From this many points on, point-major encodings go through a level-major workspace:
+# written point by point, 8 bytes at a stride of 128, every cache line reaches memory in
+# pieces.  2^18 points, f32, a new output each call: 130 us point by point, 115 with a
+# wavefront of 4 points x 16 levels (whole lines, but every level in every L2), 78 staged;
+# below the line the pieces cost less than the second launch and the workspace.
+STAGED_POINTS = 1 << 15
+
+
 class _HashGridFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, pos, table, desc_fn, n_out):
+    def forward(ctx, pos, table, desc_fn, n_out, n_features):
         N = pos.shape[0]
         enc = torch.empty(N, n_out, dtype=torch.float32, device=pos.device)
-        if N:
+        if n_features == 2 and N >= STAGED_POINTS:
+            _lib.call("hashgrid_encode_staged", [pos, table.contiguous(), enc, torch.empty_like(enc)], desc_fn(N))
+        elif N:
             _lib.call("hashgrid_encode", [pos, table.contiguous(), enc], desc_fn(N))
         ctx.save_for_backward(pos)
         ctx.desc_fn = desc_fn
@@ -83,7 +93,7 @@ class _HashGridFn(torch.autograd.Function):
         desc = ctx.desc_fn(pos.shape[0])
         ws = torch.empty(_lib.hashgrid_backward_workspace_bytes(desc), dtype=torch.uint8, device=pos.device)
         _lib.call("hashgrid_encode_backward", [pos, g.float().contiguous(), dtable, ws], desc)
-        return None, dtable.to(ctx.table_dtype), None, None
+        return None, dtable.to(ctx.table_dtype), None, None, None
 
 
 class HashGridEncoder(torch.nn.Module):
@@ -136,5 +146,5 @@ class HashGridEncoder(torch.nn.Module):
         if self.tv_scale > 0:
             raise NotImplementedError("total-variation regularisation (tv_scale > 0) is not implemented")
         desc = lambda n, _b=float(bound): self.descriptor(n, _b)
-        enc = _HashGridFn.apply(pos.contiguous(), self.table, desc, self.L * self.F)
+        enc = _HashGridFn.apply(pos.contiguous(), self.table, desc, self.L * self.F, self.F)
         return enc, 0.0

@@ -158,6 +158,36 @@ def test_level_major_layout_matches_point_major(dev):
         assert (np.abs(dt - want) <= 1e-5 * absw + 1e-30).all()
 
 
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("T,N", [(2 ** 19, 1), (2 ** 14, 513), (1000, 1025), (999, 511), (2 ** 19, 32769)])
+def test_grouped_rows_match_row_by_row_and_staged(dev, T, N, half):
+    """The grouped gather (16-byte aligned tables of whole groups), the row-by-row gather
+    (the same table a row past alignment, and T = 999, whose row count is odd) and the
+    staged point-major output are bit-exact against the oracle."""
+    from jaxngp_amd import _lib
+    rng = np.random.default_rng(T + N)
+    enc = HashGridEncoder(L=16, T=T, F=2, N_min=16, N_max=2048, param_dtype=torch.float16 if half else torch.float32,
+                          generator=torch.Generator().manual_seed(1)).to(dev)
+    n_rows = enc.levels.n_rows
+    buf = torch.empty(n_rows + 1, 2, dtype=enc.table.dtype, device=dev).uniform_(-1, 1)
+    shifted = buf[1:]
+    table = shifted.clone()
+    assert table.data_ptr() % 16 == 0 and shifted.data_ptr() % 16 != 0
+    pos_np = rng.uniform(-1, 1, (N, 3)).astype(np.float32)
+    pos_np[0] = 1.0  # the upper corner: dense vertices past their level
+    pos = torch.from_numpy(pos_np).to(dev)
+    want = _c_forward(enc, pos_np, table.float().cpu().numpy())
+    for t in (table, shifted):
+        for layout in (_lib.ENC_POINT_MAJOR, _lib.ENC_LEVEL_MAJOR):
+            out = torch.empty(16, N, 2, device=dev)
+            _lib.call("hashgrid_encode", [pos, t, out], enc.descriptor(N, 1.0, layout))
+            got = out.permute(1, 0, 2).reshape(N, 32) if layout == _lib.ENC_LEVEL_MAJOR else out.reshape(N, 32)
+            np.testing.assert_array_equal(got.cpu().numpy(), want)
+        out, ws = torch.empty(N, 32, device=dev), torch.empty(N, 32, device=dev)
+        _lib.call("hashgrid_encode_staged", [pos, t, out, ws], enc.descriptor(N, 1.0))
+        np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
 def _backward_raw(enc, pos_t, g_t):
     from jaxngp_amd import _lib
     N = pos_t.shape[0]
