@@ -182,6 +182,8 @@ constexpr int kReduceThreads = 1024;
 constexpr uint32_t kPart = 65536;    // entries one reduce workgroup sums
 constexpr uint32_t kMaxSlices = 8192;
 constexpr uint32_t kSliceBytes = 131072;
+constexpr uint32_t kRunSliceBytes = 65536;  // one-pass form: two reduce workgroups per CU
+constexpr int kRunThreads = 512;
 constexpr int kScanThreads = 1024;
 constexpr int kScanPer = 4;  // elements per thread in the scan kernels
 
@@ -237,12 +239,42 @@ __host__ __device__ inline uint32_t level_last_row(const HashGridDescriptor &d, 
 }
 
 // The one-pass table gradient (F <= 2, every level's rows within kStageSlices
-// slices): work item = (level, kBucketPoints consecutive points).
+// slices): work item = (level, bucket_points consecutive points).  Its entries are kept
+// in two arrays, the F values (f32, or one half2 for an f16 table with F = 2) and the
+// 16-bit row within the slice: 10 or 6 bytes instead of 12 or 8.
 constexpr int kBucketThreads = 512;
-constexpr int kBucketPhases = 2;
-constexpr uint32_t kBucketPoints = kBucketThreads * kBucketPhases;
-constexpr uint32_t kBucketEntries = kBucketPoints * 8;  // entries one item may write
+// f32 entries: items of 1024 points (two per thread) leave the reducer half as many runs
+// (reduce 64 against 67 us at 2^18 points); the smaller f16 entries gain more from the
+// lighter kernel of one point per thread (bucket 50 against 60 us).
+constexpr int bucket_phases(bool half_values) { return half_values ? 1 : 2; }
+constexpr uint32_t bucket_points(bool half_values) { return kBucketThreads * bucket_phases(half_values); }
+constexpr uint32_t bucket_entries(bool half_values) { return bucket_points(half_values) * 8; }  // one item's at most
 constexpr uint32_t kStageSlices = 1024;                 // slices one level may span
+
+constexpr uint32_t kStageEntries = 4096;                // entries staged in LDS at a time
+
+template <int F, bool kHalf>
+struct EntryValue {
+    uint32_t w[kHalf && F == 2 ? 1 : F];
+    __device__ __forceinline__ void pack(const float *v) {
+        if constexpr (kHalf && F == 2) {
+            w[0] = __builtin_bit_cast(uint32_t, __floats2half2_rn(v[0], v[1]));
+        } else {
+#pragma unroll
+            for (int f = 0; f < F; ++f) w[f] = __float_as_uint(v[f]);
+        }
+    }
+    __device__ __forceinline__ float get(int f) const {
+        if constexpr (kHalf && F == 2) {
+            const __half2 h = __builtin_bit_cast(__half2, w[0]);
+            return f ? __high2float(h) : __low2float(h);
+        } else {
+            return __uint_as_float(w[f]);
+        }
+    }
+};
+
+inline uint32_t value_bytes(uint32_t F, bool half) { return half && F == 2 ? 4 : 4 * F; }
 
 struct BwdPlan {
     uint32_t R, n_slices, n_chunks, n_items;
@@ -250,12 +282,13 @@ struct BwdPlan {
     uint64_t scan_blocks;   // blocks of the counter scan
     uint32_t max_parts;     // upper bound of the reduce grid
     uint64_t counts_off, sums_off, meta_off, parts_off, part_slice_off, partials_off, entries_off, bytes;
-    // one-pass path: items of kBucketPoints points, each level's slices
+    // one-pass path: items of bucket_points points, each level's slices
     // [s_lo[l], s_hi[l]], per item and slice of its level the run's start and length
     bool bucket;
     uint32_t n_bchunks, n_bitems, span_stride;
+    uint32_t run_part;  // entries one workgroup of the reducer sums
     uint32_t s_lo[NGP_HASHGRID_MAX_LEVELS], s_hi[NGP_HASHGRID_MAX_LEVELS];
-    uint64_t run_cnt_off, run_off_off, slice_np_off;
+    uint64_t runs_off, slice_np_off, rows_off;
 };
 
 // Rows of one slice: R rows of F f64 accumulators fill kSliceBytes of LDS.  A power
@@ -266,36 +299,49 @@ constexpr uint32_t slice_rows() {
     return kSliceBytes / (8 * F);
 }
 
-inline BwdPlan make_plan(const HashGridDescriptor &d) {
-    auto align = [](uint64_t x) { return (x + 255) / 256 * 256; };
-    BwdPlan p{};
-    p.R = kSliceBytes / (8 * d.F);  // slice_rows<F>()
+// Slices of kRunSliceBytes for the one-pass form where every level then spans at most
+// kStageSlices slices, else of kSliceBytes; whether either fits.
+inline bool plan_slices(const HashGridDescriptor &d, uint32_t slice_bytes, BwdPlan &p) {
+    p.R = slice_bytes / (8 * d.F);
     p.n_slices = div_up(d.n_rows, p.R);
-    const int ew = entry_words_host(d.F, d.table_dtype == NGP_DTYPE_F16);
-    p.bucket = d.F <= 2;
     p.span_stride = 1;
     for (uint32_t l = 0; l < d.L; ++l) {
         p.s_lo[l] = d.offsets[l] / p.R;
         p.s_hi[l] = level_last_row(d, l) / p.R;
-        const uint32_t span = p.s_hi[l] - p.s_lo[l] + 1u;
-        if (span > kStageSlices) p.bucket = false;
-        p.span_stride = std::max(p.span_stride, span);
+        p.span_stride = std::max(p.span_stride, p.s_hi[l] - p.s_lo[l] + 1u);
     }
+    return d.F <= 2 && p.span_stride <= kStageSlices;
+}
+
+inline BwdPlan make_plan(const HashGridDescriptor &d) {
+    auto align = [](uint64_t x) { return (x + 255) / 256 * 256; };
+    BwdPlan p{};
+    const int ew = entry_words_host(d.F, d.table_dtype == NGP_DTYPE_F16);
+    const bool half_values = d.F == 2 && d.table_dtype == NGP_DTYPE_F16;
+    p.n_bchunks = std::max<uint32_t>(1, div_up(d.n_points, bucket_points(half_values)));
+    // (entry indexes within a level are 32 bits)
+    p.bucket = (plan_slices(d, kRunSliceBytes, p) || plan_slices(d, kSliceBytes, p)) &&
+               (uint64_t)p.n_bchunks * bucket_entries(half_values) <= 0xffffffffull;
     if (p.bucket) {
-        p.n_bchunks = std::max<uint32_t>(1, div_up(d.n_points, kBucketPoints));
         p.n_bitems = d.L * p.n_bchunks;
         const uint64_t runs = (uint64_t)p.n_bitems * p.span_stride;
-        const uint64_t max_entries = (uint64_t)p.n_bitems * kBucketEntries;
-        p.max_parts = (uint32_t)(p.n_slices + max_entries / kPart);
-        p.run_cnt_off = 0;
-        p.run_off_off = align(p.run_cnt_off + 4 * runs);
-        p.slice_np_off = align(p.run_off_off + 4 * runs);
+        const uint64_t max_entries = (uint64_t)p.n_bitems * bucket_entries(half_values);
+        // A hashed level spreads 8 contributions a point evenly over its slices; a part holds
+        // a quarter more than one such slice, so these stay whole and the fuller slices of
+        // coarse levels, whose entries also collide more in the LDS atomics, are cut to the
+        // same length (77,777 points: reducer 32 us; with parts of 32,768 entries, 44).
+        const uint64_t mean = (uint64_t)d.n_points * 8 * p.R / d.T;
+        p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 4 + 1023) / 1024 * 1024));
+        p.max_parts = (uint32_t)(p.n_slices + max_entries / p.run_part);
+        p.runs_off = 0;
+        p.slice_np_off = align(p.runs_off + 4 * runs);
         p.meta_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
         p.parts_off = align(p.meta_off + 8);
         p.part_slice_off = align(p.parts_off + 4 * ((uint64_t)p.n_slices + 1));
         p.partials_off = align(p.part_slice_off + 4 * (uint64_t)p.max_parts);
         p.entries_off = align(p.partials_off + (uint64_t)p.max_parts * p.R * d.F * 4);
-        p.bytes = p.entries_off + max_entries * 4 * ew;
+        p.rows_off = align(p.entries_off + max_entries * value_bytes(d.F, d.table_dtype == NGP_DTYPE_F16));
+        p.bytes = p.rows_off + max_entries * sizeof(uint16_t);
         return p;
     }
     p.n_chunks = std::max<uint32_t>(1, div_up(d.n_points, kChunk));
@@ -564,35 +610,104 @@ __global__ void __launch_bounds__(kItemThreads)
 }
 
 
-// One-pass table gradient, part 1 (F <= 2).  Block = item (level l, kBucketPoints
-// consecutive points, one per thread and phase).  The item's run-merged
-// contributions are computed once and kept in registers; their count per slice of
-// the level goes to LDS, an exclusive scan of the counts places each slice's run
-// in the item's own region of the entry buffer (kBucketEntries entries), and the
-// run's start and length are stored for the reducers.  Within a run, entries are in
+// Item (l, k)'s run of the sl-th slice of level l: start within the item's region and
+// length (both at most bucket_entries, 2^13) in one word.  Slice-major, so a reducer
+// reads the runs of one slice side by side.
+static_assert(bucket_entries(false) < 0x10000u, "run starts and lengths fit 16 bits");
+__device__ __forceinline__ uint32_t pack_run(uint32_t start, uint32_t n) { return start | n << 16; }
+__device__ __forceinline__ uint32_t run_start(uint32_t r) { return r & 0xffffu; }
+__device__ __forceinline__ uint32_t run_length(uint32_t r) { return r >> 16; }
+__device__ __forceinline__ size_t run_index(const BwdPlan &p, uint32_t l, uint32_t sl, uint32_t k) {
+    return ((size_t)l * p.span_stride + sl) * p.n_bchunks + k;
+}
+
+// The wavefront's runs of consecutive points in one cell, as lane masks: `head` bit i is
+// set where lane i starts a run, `keep[s]` where lane i takes nothing in step s of the
+// segmented sum (its own run starts within the lanes step s would add).  Computed on the
+// scalar unit once per point, for all corners and features.
+struct CellRuns {
+    uint64_t head, keep[6];
+};
+
+__device__ __forceinline__ CellRuns cell_runs(uint64_t head) {
+    constexpr uint64_t kRow1 = 0x0001000100010001ull, kRow2 = 0x0003000300030003ull, kRow4 = 0x000f000f000f000full,
+                       kRow8 = 0x00ff00ff00ff00ffull, kRows13 = 0xffff0000ffff0000ull, kRows23 = 0xffffffff00000000ull;
+    CellRuns r;
+    r.head = head;
+    uint64_t f = head;  // lane i: a run starts within the lanes summed so far
+    r.keep[0] = f;
+    f |= (f << 1) & ~kRow1;
+    r.keep[1] = f;
+    f |= (f << 2) & ~kRow2;
+    r.keep[2] = f;
+    f |= (f << 4) & ~kRow4;
+    r.keep[3] = f;
+    f |= (f << 8) & ~kRow8;
+    r.keep[4] = f | ~kRows13;
+    f |= ((f >> 15) & 1ull) * 0x00000000ffff0000ull | ((f >> 47) & 1ull) * 0xffff000000000000ull;
+    r.keep[5] = f | ~kRows23;
+    return r;
+}
+
+template <int kCtrl, int N>
+__device__ __forceinline__ void run_step(float *v, uint64_t keep) {
+    if (~keep == 0ull) return;  // uniform: no lane has anything to take in this step
+    const bool k = __builtin_amdgcn_inverse_ballot_w64(keep);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float in = v[i] + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), kCtrl, 0xf, 0xf, true));
+        v[i] = k ? v[i] : in;
+    }
+}
+
+// Sums N values over each run; a run's last lane ends with its total.  Shifts within
+// 16-lane rows, then row 15 -> rows 1 and 3, lane 31 -> rows 2 and 3.  Steps that no
+// run reaches are skipped, so the finest levels, where consecutive samples lie in
+// different cells, do none.
+template <int N>
+__device__ __forceinline__ void sum_runs(float *v, const CellRuns &r) {
+    run_step<kRowShr1, N>(v, r.keep[0]);
+    run_step<kRowShr2, N>(v, r.keep[1]);
+    run_step<kRowShr4, N>(v, r.keep[2]);
+    run_step<kRowShr8, N>(v, r.keep[3]);
+    run_step<kRowBcast15, N>(v, r.keep[4]);
+    run_step<kRowBcast31, N>(v, r.keep[5]);
+}
+
+// One-pass table gradient, part 1 (F <= 2).  Block = item (level l, bucket_points
+// consecutive points, one per thread and phase).  The item's contributions are computed
+// once and kept in registers: a wavefront's 64 lanes hold 64 consecutive points, and
+// runs of points in the same cell (all eight corners alike) are summed into the run's
+// last lane, which takes each corner's rank within its slice from an LDS counter.  An
+// exclusive scan of the counters places each slice's run in the item's own region of
+// the entry buffer (bucket_entries), the entries go to run start + rank, and
+// the run's start and length are stored for the reducers.  Within a run, entries are in
 // LDS-atomic order; the reducer's sums do not depend on it beyond f64 rounding.
-template <int F, bool kHalf>
+// 2^18 ray samples: f32 110 -> 68 us, f16 90 -> 50 us.  It was bound by the run merge
+// (each corner found its own runs: 626 vector instructions a wavefront and level) and,
+// once that was cheaper (86 us), by 17 M scattered 12-byte stores.
+template <int F, bool kHalf, uint32_t R>
 __global__ void __launch_bounds__(kBucketThreads)
     bwd_bucket_kernel(HashGridDescriptor d, BwdPlan p, const float *__restrict__ pos,
-                      const float *__restrict__ dL_denc, uint32_t *__restrict__ run_cnt,
-                      uint32_t *__restrict__ run_off, uint32_t *__restrict__ entries) {
-    constexpr int EW = entry_words<F, kHalf>();
-    constexpr uint32_t R = slice_rows<F>();
-    static_assert(kStageSlices == 2 * kBucketThreads, "two slice counters per thread");
+                      const float *__restrict__ dL_denc, uint32_t *__restrict__ runs_out,
+                      EntryValue<F, kHalf> *__restrict__ values, uint16_t *__restrict__ rows_out) {
+    typedef EntryValue<F, kHalf> Value;
+    constexpr int kBucketPhases = bucket_phases(kHalf);
+    constexpr uint32_t kBucketPoints = bucket_points(kHalf), kBucketEntries = bucket_entries(kHalf);
+    static_assert(R <= 0x10000u, "rows within a slice fit 16 bits");
+    constexpr int kPer = kStageSlices / kBucketThreads;
+    static_assert(kPer * kBucketThreads == kStageSlices, "whole slice counters per thread");
     __shared__ uint32_t cnt[kStageSlices];
-    __shared__ uint32_t cur[kStageSlices];
+    __shared__ __align__(16) Value stage_v[kStageEntries];
+    __shared__ __align__(16) uint16_t stage_r[kStageEntries];
     const uint32_t item = blockIdx.x;
     const uint32_t l = item / p.n_bchunks, k = item % p.n_bchunks;
     const uint32_t s_lo = p.s_lo[l];
     const uint32_t span = p.s_hi[l] - s_lo + 1u;  // <= kStageSlices (host check)
-    cnt[2 * threadIdx.x] = 0u;
-    cnt[2 * threadIdx.x + 1] = 0u;
     const bool pow2 = (d.T & (d.T - 1u)) == 0;
     const bool level_major = d.enc_layout == NGP_ENC_LEVEL_MAJOR;
     const float scale = d.scales[l];
-    const uint32_t res = d.resolutions[l];
-    const bool dense = l < d.first_hash_level;
-    // both phases' inputs are loaded up front, so only the first phase waits on memory
+    // all phases' inputs are loaded up front, so only the first phase waits on memory
     float xyz_all[kBucketPhases][3], gin_all[kBucketPhases][F];
 #pragma unroll
     for (int ph = 0; ph < kBucketPhases; ++ph) {
@@ -604,71 +719,108 @@ __global__ void __launch_bounds__(kBucketThreads)
 #pragma unroll
         for (int f = 0; f < F; ++f) gin_all[ph][f] = dL_denc[gb + f];
     }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) cnt[kPer * threadIdx.x + q] = 0u;
     __syncthreads();  // counters cleared
-    uint32_t rows[kBucketPhases][8];
-    float vals[kBucketPhases][8][F];
-    uint32_t mask[kBucketPhases];
+    uint32_t rows[kBucketPhases][8], rank[kBucketPhases][8];
+    float vals[kBucketPhases][8 * F];
+    uint64_t emits[kBucketPhases];
+    const Divisor two_b = make_divisor(2.0f * d.bound);
 #pragma unroll
     for (int ph = 0; ph < kBucketPhases; ++ph) {
         const uint32_t n = k * kBucketPoints + ph * kBucketThreads + threadIdx.x;
-        uint32_t m = 0;
-        point_runs<F, true>(d, l, scale, res, dense, pow2, xyz_all[ph], gin_all[ph], n < d.n_points,
-                            [&](uint32_t row, const float *v, int c) {
-                                rows[ph][c] = row;
+        const uint64_t active = __ballot(n < d.n_points);
+        float q[3], w[8];
+        normalise(two_b, d.bound, xyz_all[ph], q);
+        with_rule(l < d.first_hash_level, pow2, [&](auto rule, auto p2) {
+            level_vertices_t<decltype(rule)::value, decltype(p2)::value>(
+                q[0], q[1], q[2], scale, d.resolutions[l], l < d.first_hash_level, d.T, d.offsets[l], d.n_rows - 1u,
+                rows[ph], w);
+        });
+        // a lane continues the previous lane's run if both points lie in one cell (a NaN
+        // position is in none); points past the end are runs of their own.  The lane shifts
+        // come before any comparison: a shift reads nothing from a lane that is masked off.
+        float cell[3], before[3];
 #pragma unroll
-                                for (int f = 0; f < F; ++f) vals[ph][c][f] = v[f];
-                                m |= 1u << c;
-                            });
-        mask[ph] = m;
+        for (int a = 0; a < 3; ++a) {
+            cell[a] = floorf(q[a] * scale + 0.5f);
+            before[a] = __uint_as_float(dpp_u32<kWaveShr1, 0xf>(__float_as_uint(cell[a]), 0x7fc00000u));
+        }
+        const bool same = (n < d.n_points) & (cell[0] == before[0]) & (cell[1] == before[1]) & (cell[2] == before[2]);
 #pragma unroll
         for (int c = 0; c < 8; ++c)
-            if ((m >> c) & 1u) atomicAdd(&cnt[rows[ph][c] / R - s_lo], 1u);
+#pragma unroll
+            for (int f = 0; f < F; ++f) vals[ph][c * F + f] = w[c] * gin_all[ph][f];
+        const CellRuns runs = cell_runs(~__ballot(same));
+        sum_runs<8 * F>(vals[ph], runs);
+        emits[ph] = (runs.head >> 1 | 1ull << 63) & active;
+        // the last active lane's run ends there even if it is not the last lane: lane i + 1
+        // is then past the end, a head
+        if (__builtin_amdgcn_inverse_ballot_w64(emits[ph])) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) rank[ph][c] = atomicAdd(&cnt[rows[ph][c] / R - s_lo], 1u);
+        }
     }
     __syncthreads();
-    const uint32_t c0 = cnt[2 * threadIdx.x], c1 = cnt[2 * threadIdx.x + 1];
+    uint32_t mine[kPer], sum = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        mine[q] = cnt[kPer * threadIdx.x + q];
+        sum += mine[q];
+    }
     uint32_t total;
-    const uint32_t ex = block_exclusive_scan<kBucketThreads>(c0 + c1, &total);
-    cur[2 * threadIdx.x] = ex;
-    cur[2 * threadIdx.x + 1] = ex + c0;
-    const size_t rb = (size_t)item * p.span_stride;
-    if (2 * threadIdx.x < span) {
-        run_cnt[rb + 2 * threadIdx.x] = c0;
-        run_off[rb + 2 * threadIdx.x] = ex;
-    }
-    if (2 * threadIdx.x + 1 < span) {
-        run_cnt[rb + 2 * threadIdx.x + 1] = c1;
-        run_off[rb + 2 * threadIdx.x + 1] = ex + c0;
+    uint32_t ex = block_exclusive_scan<kBucketThreads>(sum, &total);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const uint32_t sl = kPer * threadIdx.x + q;
+        cnt[sl] = ex;  // from here on, the start of slice sl's run
+        if (sl < span) runs_out[run_index(p, l, sl, k)] = pack_run(ex, mine[q]);
+        ex += mine[q];
     }
     __syncthreads();
-    uint32_t *region = entries + (size_t)item * kBucketEntries * EW;
+    // rank becomes the entry's place in the item's region
 #pragma unroll
     for (int ph = 0; ph < kBucketPhases; ++ph) {
+        const bool emit = __builtin_amdgcn_inverse_ballot_w64(emits[ph]);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if ((mask[ph] >> c) & 1u) {
-                const uint32_t sl = rows[ph][c] / R;
-                const uint32_t at = atomicAdd(&cur[sl - s_lo], 1u);
-                uint32_t w[EW];
+        for (int c = 0; c < 8; ++c) rank[ph][c] = emit ? rank[ph][c] + cnt[rows[ph][c] / R - s_lo] : 0xffffffffu;
+    }
+    // the region, kStageEntries at a time through LDS: each 64-byte request to the L2
+    // carries whole neighbouring entries (scattered entry by entry, 17 M requests of 12
+    // bytes took the L2 channels longer than everything else here)
+    const size_t region = (size_t)item * kBucketEntries;
+    for (uint32_t e0 = 0; e0 < total; e0 += kStageEntries) {
+        if (e0 > 0) __syncthreads();  // the stage is read out
 #pragma unroll
-                for (int q = 0; q < EW; ++q) w[q] = 0u;
-                w[0] = rows[ph][c] - sl * R;
-                pack_values<F, kHalf>(w, vals[ph][c]);
-                uint32_t *dst = region + (size_t)at * EW;
-                if constexpr (EW == 2) {
-                    *reinterpret_cast<uint2 *>(dst) = make_uint2(w[0], w[1]);
-                } else {
-                    static_assert(EW == 3, "one-pass entries are 2 or 3 words");
-                    *reinterpret_cast<uint3 *>(dst) = make_uint3(w[0], w[1], w[2]);
+        for (int ph = 0; ph < kBucketPhases; ++ph) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const uint32_t at = rank[ph][c] - e0;
+                if (at < kStageEntries) {
+                    Value v;
+                    v.pack(vals[ph] + c * F);
+                    stage_v[at] = v;
+                    stage_r[at] = (uint16_t)(rows[ph][c] % R);
                 }
             }
         }
+        __syncthreads();
+        const uint32_t n = min(total - e0, kStageEntries);
+        // whole 16-byte vectors; the last may reach past n, within the item's region
+        constexpr uint32_t kV = 16 / sizeof(Value), kR = 16 / sizeof(uint16_t);
+        uint4 *const gv = reinterpret_cast<uint4 *>(values + region + e0);
+        uint4 *const gr = reinterpret_cast<uint4 *>(rows_out + region + e0);
+        for (uint32_t t = threadIdx.x; t < (n + kV - 1) / kV; t += kBucketThreads)
+            gv[t] = reinterpret_cast<const uint4 *>(stage_v)[t];
+        for (uint32_t t = threadIdx.x; t < (n + kR - 1) / kR; t += kBucketThreads)
+            gr[t] = reinterpret_cast<const uint4 *>(stage_r)[t];
     }
 }
 
-// One-pass table gradient, part 2: parts of slice s (kPart entries each, at least
+// One-pass table gradient, part 2: parts of slice s (run_part entries each, at least
 // one), from the run lengths of every item whose level reaches s.
 __global__ void __launch_bounds__(256)
-    bwd_slice_parts_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ run_cnt,
+    bwd_slice_parts_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ runs,
                            uint32_t *__restrict__ slice_np) {
     const uint32_t s = blockIdx.x;
     uint32_t tot = 0;
@@ -676,7 +828,7 @@ __global__ void __launch_bounds__(256)
         if (s < p.s_lo[l] || s > p.s_hi[l]) continue;
         const uint32_t sl = s - p.s_lo[l];
         for (uint32_t k = threadIdx.x; k < p.n_bchunks; k += 256)
-            tot += run_cnt[(size_t)(l * p.n_bchunks + k) * p.span_stride + sl];
+            tot += run_length(runs[run_index(p, l, sl, k)]);
     }
     __shared__ uint32_t ws[256 / kWave];
     tot = wave_sum(tot);
@@ -685,7 +837,7 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x == 0) {
         uint32_t t = 0;
         for (int w = 0; w < 256 / kWave; ++w) t += ws[w];
-        slice_np[s] = t == 0 ? 1u : (t + kPart - 1) / kPart;
+        slice_np[s] = t == 0 ? 1u : (t + p.run_part - 1) / p.run_part;
     }
 }
 
@@ -790,102 +942,160 @@ __global__ void __launch_bounds__(kReduceThreads)
 }
 
 // One-pass table gradient, part 4: workgroup b sums part b of slice s, as
-// bwd_reduce_kernel does, from the runs of the items whose level reaches s.  The
-// items are visited in (level, chunk) order and a part takes those whose exclusive
-// prefix of run lengths falls in [part * kPart, (part + 1) * kPart).  A wavefront
-// reads kRunsPerWave runs side by side, two loads per lane and run in flight (a
-// hashed level's run holds about 128 entries; longer runs loop), so eight entry
-// loads per lane are in flight as in bwd_reduce_kernel.
+// bwd_reduce_kernel does, from the runs of the items whose level reaches s.  The LDS
+// atomics set the time (about 31 cycles of a CU per 64-lane f64 add, however many of its
+// lanes are masked off), so a wavefront reads its runs as one sequence with every lane
+// filled: lane i of wavefront w loads the run of item w + i * kWaves, a prefix sum of the
+// lengths places the runs in the sequence, and 64 entries at a time find their runs by
+// pushing each run's lane number to the lane of its first entry and a running maximum
+// (RunSequence).  kSteps such groups are loaded before the previous ones are added.  A
+// slice of one part (nearly all of them) needs no barrier between its runs; a slice of
+// several parts first cuts the items, in (level, chunk) order, by the prefix of their
+// run lengths: a part takes those whose exclusive prefix falls in
+// [part * run_part, (part + 1) * run_part).
 // With kAdam, a slice summed in one part is not stored: its rows take the optimizer
 // step in place (params, m, v), and bwd_combine does the same for the others.
-template <int F, bool kHalf, bool kAdam = false>
-__global__ void __launch_bounds__(kReduceThreads)
+// 2^18 ray samples, f32: 82 -> 62 us, of which the atomics themselves need 27 (34 M f64
+// adds at 1.27 T/s); slices of 64 KiB, two workgroups to a CU, so that one clears or
+// stores its rows while the other adds (128 KiB slices: 80 us); 1,024 points: 29 -> 18.
+struct RunSequence {
+    uint32_t *marks;        // 64 words of LDS of the wavefront's own, tags below `tag`
+    uint32_t tag;           // of the latest group of 64 places
+    uint32_t start, total;  // this lane's run: first place in the sequence; places in all
+    uint32_t shift;         // entry index of a place of this lane's run, less the place
+    uint32_t last;          // lane number + 1 of the run the previous group ended in
+    bool any;               // this lane's run is not empty
+
+    // `entry0`: index of the run's first entry
+    __device__ __forceinline__ void init(uint32_t len, uint32_t entry0) {
+        const uint32_t incl = wave_inclusive_scan(len);
+        start = incl - len;
+        total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        shift = entry0 - start;
+        any = len > 0;
+        last = 0;
+    }
+    // The entry at place t0 + lane (the last one past the end), for t0 = 0, 64, ...
+    __device__ __forceinline__ uint32_t entry(uint32_t t0) {
+        const uint32_t lane = lane_id(), to = start - t0;
+        ++tag;
+        if (any && to < (uint32_t)kWave) marks[to] = tag << 8 | (lane + 1u);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const uint32_t m = marks[lane];
+        uint32_t r = m >> 8 == tag ? m & 0xffu : 0u;  // a run of this group starts here
+        r = max(r, dpp_u32<kRowShr1, 0xf>(r, 0u));
+        r = max(r, dpp_u32<kRowShr2, 0xf>(r, 0u));
+        r = max(r, dpp_u32<kRowShr4, 0xf>(r, 0u));
+        r = max(r, dpp_u32<kRowShr8, 0xf>(r, 0u));
+        r = max(r, dpp_u32<kRowBcast15, 0xf>(r, 0u));
+        r = max(r, dpp_u32<kRowBcast31, 0xf>(r, 0u));
+        r = max(r, last);
+        last = (uint32_t)__builtin_amdgcn_readlane((int)r, kWave - 1);
+        const uint32_t sh = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((r - 1u) * 4u), (int)shift);
+        return sh + min(t0 + lane, total - 1u);
+    }
+};
+
+constexpr int kSteps = 6;  // groups of 64 entries in flight
+
+template <int F, bool kHalf>
+struct EntryGroup {
+    EntryValue<F, kHalf> v[kSteps];
+    uint32_t row[kSteps];
+
+    __device__ __forceinline__ void load(RunSequence &seq, uint32_t t0, const EntryValue<F, kHalf> *__restrict__ values,
+                                         const uint16_t *__restrict__ rows) {
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) {
+            if (t0 + q * kWave < seq.total) {  // the same for the whole wavefront
+                const uint32_t e = seq.entry(t0 + q * kWave);
+                v[q] = values[e];
+                row[q] = rows[e];
+            }
+        }
+    }
+    template <uint32_t R>
+    __device__ __forceinline__ void add(double *acc, uint32_t t0, uint32_t total) const {
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) {
+            const bool in = t0 + q * kWave + lane_id() < total;
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const float x = v[q].get(f);
+                if (in && x != 0.0f) atomicAdd(&acc[f * R + row[q]], (double)x);
+            }
+        }
+    }
+};
+
+template <int F, bool kHalf, uint32_t R, bool kAdam = false>
+__global__ void __launch_bounds__(kRunThreads)
     bwd_reduce_runs_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ meta,
                            const uint32_t *__restrict__ parts, const uint32_t *__restrict__ part_slice,
-                           const uint32_t *__restrict__ run_cnt, const uint32_t *__restrict__ run_off,
-                           const uint32_t *__restrict__ entries, float *__restrict__ partials,
+                           const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
+                           const uint16_t *__restrict__ entry_rows, float *__restrict__ partials,
                            float *__restrict__ dtable, AdamStep adam = {}, float *__restrict__ adam_p = nullptr,
                            float *__restrict__ adam_m = nullptr, float *__restrict__ adam_v = nullptr) {
-    constexpr int EW = entry_words<F, kHalf>();
-    constexpr uint32_t R = slice_rows<F>();
-    constexpr uint32_t kWaves = kReduceThreads / kWave;
-    constexpr int kRunsPerWave = 4, kPerRun = 2;
+    typedef EntryGroup<F, kHalf> Group;
+    constexpr uint32_t kBucketEntries = bucket_entries(kHalf);
+    constexpr uint32_t kWaves = kRunThreads / kWave;
     extern __shared__ double acc[];
-    // selected runs: entry base (item region + run offset) and length
-    __shared__ uint64_t sel_base[kReduceThreads];
-    __shared__ uint32_t sel_cnt[kReduceThreads];
+    __shared__ uint32_t chosen[kRunThreads];
+    __shared__ uint32_t marks[kWaves][kWave];
     const uint32_t b = blockIdx.x;
     if (b >= meta[1]) return;
     const uint32_t s = part_slice[b];
     const uint32_t part = b - parts[s];
     const uint32_t n_parts = parts[s + 1] - parts[s];
     const uint32_t rows = min(d.n_rows - s * R, R);
-    for (uint32_t t = threadIdx.x; t < R * F; t += kReduceThreads) acc[t] = 0.0;
+    for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) reinterpret_cast<double2 *>(acc)[t] = double2{0.0, 0.0};
     __syncthreads();
-    const uint32_t wave = threadIdx.x / kWave;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t lane = lane_id();
+    RunSequence seq;
+    seq.marks = marks[wave];
+    seq.tag = 0;
+    seq.marks[lane] = 0u;
     uint32_t carry = 0;  // entries of the items visited before
     for (uint32_t l = 0; l < d.L; ++l) {
         if (s < p.s_lo[l] || s > p.s_hi[l]) continue;
-        const uint32_t sl = s - p.s_lo[l];
-        for (uint32_t k0 = 0; k0 < p.n_bchunks; k0 += kReduceThreads) {
-            const uint32_t k = k0 + threadIdx.x;
-            const uint32_t item = l * p.n_bchunks + k;
-            uint32_t c = 0, off = 0;
-            if (k < p.n_bchunks) {
-                c = run_cnt[(size_t)item * p.span_stride + sl];
-                off = run_off[(size_t)item * p.span_stride + sl];
+        const uint32_t *level_runs = runs + run_index(p, l, s - p.s_lo[l], 0);
+        for (uint32_t k0 = 0; k0 < p.n_bchunks; k0 += kRunThreads) {
+            const uint32_t n_k = min(p.n_bchunks - k0, (uint32_t)kRunThreads);
+            const uint32_t k = wave + lane * kWaves;  // this lane's run of the tile
+            uint32_t my_run = 0;
+            if (n_parts == 1) {
+                if (k < n_k) my_run = level_runs[k0 + k];
+            } else {
+                const uint32_t r = threadIdx.x < n_k ? level_runs[k0 + threadIdx.x] : 0u;
+                uint32_t tot;
+                const uint32_t ex = block_exclusive_scan<kRunThreads>(run_length(r), &tot);
+                chosen[threadIdx.x] = (carry + ex) / p.run_part == part ? r : 0u;
+                carry += tot;
+                __syncthreads();
+                my_run = chosen[k];
+                __syncthreads();  // rewritten by the next tile
             }
-            uint32_t tot, n_sel;
-            const uint32_t ex = block_exclusive_scan<kReduceThreads>(c, &tot);
-            const bool sel = c > 0 && (carry + ex) / kPart == part;
-            const uint32_t at = block_exclusive_scan<kReduceThreads>(sel ? 1u : 0u, &n_sel);
-            if (sel) {
-                sel_base[at] = (uint64_t)item * kBucketEntries + off;
-                sel_cnt[at] = c;
+            seq.init(run_length(my_run), (k0 + k) * kBucketEntries + run_start(my_run));
+            const auto *v = values + (size_t)l * p.n_bchunks * kBucketEntries;
+            const uint16_t *r = entry_rows + (size_t)l * p.n_bchunks * kBucketEntries;
+            Group cur, next;
+            cur.load(seq, 0, v, r);
+            for (uint32_t t0 = 0; t0 < seq.total; t0 += kSteps * kWave) {
+                next.load(seq, t0 + kSteps * kWave, v, r);
+                cur.template add<R>(acc, t0, seq.total);
+                cur = next;
             }
-            carry += tot;
-            __syncthreads();
-            for (uint32_t j0 = wave; j0 < n_sel; j0 += kWaves * kRunsPerWave) {
-                uint64_t base[kRunsPerWave];
-                uint32_t cnt[kRunsPerWave], longest = 0;
-#pragma unroll
-                for (int q = 0; q < kRunsPerWave; ++q) {
-                    const uint32_t j = j0 + q * kWaves;
-                    cnt[q] = j < n_sel ? sel_cnt[j] : 0u;
-                    base[q] = j < n_sel ? sel_base[j] : 0ull;
-                    longest = max(longest, cnt[q]);
-                }
-                for (uint32_t e0 = 0; e0 < longest; e0 += kPerRun * kWave) {
-                    uint32_t w[kRunsPerWave][kPerRun][EW];
-#pragma unroll
-                    for (int q = 0; q < kRunsPerWave; ++q)
-#pragma unroll
-                        for (int h = 0; h < kPerRun; ++h) {
-                            const uint32_t e = cnt[q] ? min(e0 + h * kWave + lane, cnt[q] - 1u) : 0u;
-                            load_entry<EW>(entries + (base[q] + e) * EW, w[q][h]);
-                        }
-#pragma unroll
-                    for (int q = 0; q < kRunsPerWave; ++q)
-#pragma unroll
-                        for (int h = 0; h < kPerRun; ++h) {
-                            const bool in = e0 + h * kWave + lane < cnt[q];
-#pragma unroll
-                            for (int f = 0; f < F; ++f) {
-                                const float v = entry_value<F, kHalf>(w[q][h], f);
-                                if (in && v != 0.0f) atomicAdd(&acc[f * R + w[q][h][0]], (double)v);
-                            }
-                        }
-                }
-            }
-            __syncthreads();  // the selection is rewritten by the next tile
         }
     }
+    __syncthreads();
+    const size_t o = (size_t)s * R * F;
     if (kAdam && n_parts == 1) {
-        const size_t o = (size_t)s * R * F;
         // unrolled so that several rows' params, m and v loads are in flight at once
 #pragma unroll 8
-        for (uint32_t t = threadIdx.x; t < rows * F; t += kReduceThreads) {
+        for (uint32_t t = threadIdx.x; t < rows * F; t += kRunThreads) {
             float mk = adam_m[o + t], vk = adam_v[o + t];
             adam_p[o + t] = adam_step(adam, adam_p[o + t], (float)acc[(t % F) * R + t / F], mk, vk);
             adam_m[o + t] = mk;
@@ -893,8 +1103,14 @@ __global__ void __launch_bounds__(kReduceThreads)
         }
         return;
     }
-    float *out = n_parts == 1 ? dtable + (size_t)s * R * F : partials + (size_t)b * R * F;
-    for (uint32_t t = threadIdx.x; t < rows * F; t += kReduceThreads) out[t] = (float)acc[(t % F) * R + t / F];
+    float *out = n_parts == 1 ? dtable + o : partials + (size_t)b * R * F;
+    for (uint32_t t = threadIdx.x; t < rows; t += kRunThreads) {
+        if constexpr (F == 2) {
+            reinterpret_cast<float2 *>(out)[t] = make_float2((float)acc[t], (float)acc[R + t]);
+        } else {
+            out[t] = (float)acc[t];
+        }
+    }
 }
 
 // 5. slices of several parts: rows = sum of the parts' partial rows, in part
@@ -977,6 +1193,53 @@ struct FusedAdam {
     float *p, *m, *v;
 };
 
+template <typename K>
+bool reserve_lds(K kernel, size_t lds, const char *target) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess)
+        set_error(kLaunchFailed, "%s: cannot reserve %zu bytes of LDS: %s", target, lds, hipGetErrorString(e));
+    return e == hipSuccess;
+}
+
+// The one-pass form on slices of R rows.
+template <int F, bool kHalf, uint32_t R>
+bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStream_t stream, const float *pos,
+                          const float *g, float *dtable, uint8_t *ws, const char *target, const FusedAdam *fused) {
+    uint32_t *runs = reinterpret_cast<uint32_t *>(ws + p.runs_off);
+    uint32_t *slice_np = reinterpret_cast<uint32_t *>(ws + p.slice_np_off);
+    uint32_t *meta = reinterpret_cast<uint32_t *>(ws + p.meta_off);
+    uint32_t *parts = reinterpret_cast<uint32_t *>(ws + p.parts_off);
+    uint32_t *part_slice = reinterpret_cast<uint32_t *>(ws + p.part_slice_off);
+    float *partials = reinterpret_cast<float *>(ws + p.partials_off);
+    auto *values = reinterpret_cast<EntryValue<F, kHalf> *>(ws + p.entries_off);
+    uint16_t *entry_rows = reinterpret_cast<uint16_t *>(ws + p.rows_off);
+    const size_t lds = (size_t)R * F * sizeof(double);
+    const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, false>;
+    const auto reduce_adam = bwd_reduce_runs_kernel<F, false, R, true>;
+    if (fused == nullptr ? !reserve_lds(reduce, lds, target) : !reserve_lds(reduce_adam, lds, target)) return false;
+    hipLaunchKernelGGL((bwd_bucket_kernel<F, kHalf, R>), dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, d, p, pos, g,
+                       runs, values, entry_rows);
+    hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, runs, slice_np);
+    hipLaunchKernelGGL(bwd_bucket_plan_kernel, dim3(1), dim3(kScanThreads), 0, stream, p, slice_np, meta, parts,
+                       part_slice);
+    if constexpr (!kHalf) {
+        if (fused != nullptr) {
+            hipLaunchKernelGGL(reduce_adam, dim3(p.max_parts), dim3(kRunThreads), lds, stream, d, p, meta, parts,
+                               part_slice, runs, values, entry_rows, partials, dtable, fused->step, fused->p, fused->m,
+                               fused->v);
+            hipLaunchKernelGGL((bwd_combine_kernel<F, true>), dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d, p,
+                               parts, partials, dtable, fused->step, fused->p, fused->m, fused->v);
+            return true;
+        }
+    }
+    hipLaunchKernelGGL(reduce, dim3(p.max_parts), dim3(kRunThreads), lds, stream, d, p, meta, parts, part_slice, runs,
+                       values, entry_rows, partials, dtable, AdamStep{}, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((bwd_combine_kernel<F>), dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d, p, parts,
+                       partials, dtable, AdamStep{}, nullptr, nullptr, nullptr);
+    return true;
+}
+
 template <int F, bool kHalf>
 bool launch_backward(const HashGridDescriptor &d, hipStream_t stream, const float *pos, const float *g, float *dtable,
                      uint8_t *ws, const char *target, const FusedAdam *fused = nullptr) {
@@ -989,43 +1252,9 @@ bool launch_backward(const HashGridDescriptor &d, hipStream_t stream, const floa
     const size_t lds = (size_t)p.R * F * sizeof(double);
     if constexpr (F <= 2) {
         if (p.bucket) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&bwd_reduce_runs_kernel<F, kHalf>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) {
-                set_error(kLaunchFailed, "%s: cannot reserve %zu bytes of LDS: %s", target, lds, hipGetErrorString(e));
-                return false;
-            }
-            uint32_t *run_cnt = reinterpret_cast<uint32_t *>(ws + p.run_cnt_off);
-            uint32_t *run_off = reinterpret_cast<uint32_t *>(ws + p.run_off_off);
-            uint32_t *slice_np = reinterpret_cast<uint32_t *>(ws + p.slice_np_off);
-            hipLaunchKernelGGL((bwd_bucket_kernel<F, kHalf>), dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, d, p,
-                               pos, g, run_cnt, run_off, entries);
-            hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, run_cnt, slice_np);
-            hipLaunchKernelGGL(bwd_bucket_plan_kernel, dim3(1), dim3(kScanThreads), 0, stream, p, slice_np, meta, parts,
-                               part_slice);
-            if constexpr (!kHalf) {
-                if (fused != nullptr) {
-                    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&bwd_reduce_runs_kernel<F, false, true>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                    if (e != hipSuccess) {
-                        set_error(kLaunchFailed, "%s: cannot reserve %zu bytes of LDS: %s", target, lds,
-                                  hipGetErrorString(e));
-                        return false;
-                    }
-                    hipLaunchKernelGGL((bwd_reduce_runs_kernel<F, false, true>), dim3(p.max_parts),
-                                       dim3(kReduceThreads), lds, stream, d, p, meta, parts, part_slice, run_cnt,
-                                       run_off, entries, partials, dtable, fused->step, fused->p, fused->m, fused->v);
-                    hipLaunchKernelGGL((bwd_combine_kernel<F, true>), dim3(p.n_slices, kCombineSplit), dim3(256), 0,
-                                       stream, d, p, parts, partials, dtable, fused->step, fused->p, fused->m,
-                                       fused->v);
-                    return true;
-                }
-            }
-            hipLaunchKernelGGL((bwd_reduce_runs_kernel<F, kHalf>), dim3(p.max_parts), dim3(kReduceThreads), lds, stream,
-                               d, p, meta, parts, part_slice, run_cnt, run_off, entries, partials, dtable);
-            hipLaunchKernelGGL(bwd_combine_kernel<F>, dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d, p,
-                               parts, partials, dtable);
-            return true;
+            constexpr uint32_t kSmall = kRunSliceBytes / (8 * F), kLarge = kSliceBytes / (8 * F);
+            return p.R == kSmall ? launch_backward_runs<F, kHalf, kSmall>(d, p, stream, pos, g, dtable, ws, target, fused)
+                                 : launch_backward_runs<F, kHalf, kLarge>(d, p, stream, pos, g, dtable, ws, target, fused);
         }
     }
     if (fused != nullptr) {

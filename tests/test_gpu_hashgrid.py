@@ -198,6 +198,29 @@ def _backward_raw(enc, pos_t, g_t):
     return d
 
 
+@pytest.mark.parametrize("kind,N", [("random", 1), ("ray", 63), ("one_cell", 64), ("ray", 65), ("ray", 513),
+                                    ("random", 1025), ("one_cell", 5000), ("random", 30000)])
+def test_backward_item_and_run_edges(dev, kind, N):
+    """Sizes around a wavefront, a phase and an item of the one-pass table gradient; all
+    points in one cell (runs as long as the wavefront, few rows, several parts a slice)
+    and none sharing a cell.  The bound of test_hashgrid_forward_backward."""
+    rng = np.random.default_rng(N)
+    enc = HashGridEncoder(**CONFIGS["l16_t2e19"], generator=torch.Generator().manual_seed(1)).to(dev)
+    if kind == "random":
+        pos = rng.uniform(-1, 1, (N, 3))
+    elif kind == "ray":
+        d = np.array([0.48, -0.6, 0.64])
+        pos = (np.arange(N)[:, None] - N / 2) * (2 * 3 ** 0.5 / 1024) * d
+    else:
+        pos = 0.3 + rng.uniform(0, 2e-4, (N, 3))
+    pos = pos.astype(np.float32)
+    g = rng.normal(size=(N, 32)).astype(np.float32)
+    got = _backward_raw(enc, torch.from_numpy(pos).to(dev), torch.from_numpy(g).to(dev)).cpu().numpy().astype(np.float64)
+    want, absw = _c_backward(enc, pos, g), _c_backward(enc, pos, np.abs(g))
+    assert (got[absw == 0] == 0).all()
+    assert (np.abs(got - want) <= 1e-5 * absw + 1e-30).all()
+
+
 def test_backward_scale_free(dev):
     """The table gradient's sums keep relative precision at any magnitude:
     cotangents scaled by 2^-60 or 2^+60 give the gradient scaled by the same power
