@@ -286,9 +286,10 @@ struct BwdPlan {
     // [s_lo[l], s_hi[l]], per item and slice of its level the run's start and length
     bool bucket;
     uint32_t n_bchunks, n_bitems, span_stride;
-    uint32_t run_part;  // entries one workgroup of the reducer sums
+    uint32_t run_part;     // entries one workgroup of the reducer sums
+    uint32_t group_shift;  // log2 of the slices in kSliceBytes
     uint32_t s_lo[NGP_HASHGRID_MAX_LEVELS], s_hi[NGP_HASHGRID_MAX_LEVELS];
-    uint64_t runs_off, slice_np_off, rows_off;
+    uint64_t runs_off, slice_np_off, rows_off, part_group_off;
 };
 
 // Rows of one slice: R rows of F f64 accumulators fill kSliceBytes of LDS.  A power
@@ -332,14 +333,16 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         // same length (77,777 points: reducer 32 us; with parts of 32,768 entries, 44).
         const uint64_t mean = (uint64_t)d.n_points * 8 * p.R / d.T;
         p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 4 + 1023) / 1024 * 1024));
-        p.max_parts = (uint32_t)(p.n_slices + max_entries / p.run_part);
+        p.group_shift = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
+        p.max_parts = (uint32_t)(p.n_slices + max_entries / p.run_part + (max_entries << p.group_shift) / kPart);
         p.runs_off = 0;
         p.slice_np_off = align(p.runs_off + 4 * runs);
         p.meta_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
         p.parts_off = align(p.meta_off + 8);
         p.part_slice_off = align(p.parts_off + 4 * ((uint64_t)p.n_slices + 1));
         p.partials_off = align(p.part_slice_off + 4 * (uint64_t)p.max_parts);
-        p.entries_off = align(p.partials_off + (uint64_t)p.max_parts * p.R * d.F * 4);
+        p.part_group_off = align(p.partials_off + (uint64_t)p.max_parts * p.R * d.F * 8);
+        p.entries_off = align(p.part_group_off + 4 * (uint64_t)p.max_parts);
         p.rows_off = align(p.entries_off + max_entries * value_bytes(d.F, d.table_dtype == NGP_DTYPE_F16));
         p.bytes = p.rows_off + max_entries * sizeof(uint16_t);
         return p;
@@ -649,6 +652,12 @@ __device__ __forceinline__ CellRuns cell_runs(uint64_t head) {
     return r;
 }
 
+// The last lane of each run (a lane past the last point starts a run of its own, so the
+// last point's lane ends one).
+__device__ __forceinline__ uint64_t run_ends(const CellRuns &r) { return r.head >> 1 | 1ull << 63; }
+
+constexpr uint32_t kNoEntry = 0xffffffffu;
+
 template <int kCtrl, int N>
 __device__ __forceinline__ void run_step(float *v, uint64_t keep) {
     if (~keep == 0ull) return;  // uniform: no lane has anything to take in this step
@@ -724,7 +733,6 @@ __global__ void __launch_bounds__(kBucketThreads)
     __syncthreads();  // counters cleared
     uint32_t rows[kBucketPhases][8], rank[kBucketPhases][8];
     float vals[kBucketPhases][8 * F];
-    uint64_t emits[kBucketPhases];
     const Divisor two_b = make_divisor(2.0f * d.bound);
 #pragma unroll
     for (int ph = 0; ph < kBucketPhases; ++ph) {
@@ -751,14 +759,34 @@ __global__ void __launch_bounds__(kBucketThreads)
         for (int c = 0; c < 8; ++c)
 #pragma unroll
             for (int f = 0; f < F; ++f) vals[ph][c * F + f] = w[c] * gin_all[ph][f];
-        const CellRuns runs = cell_runs(~__ballot(same));
-        sum_runs<8 * F>(vals[ph], runs);
-        emits[ph] = (runs.head >> 1 | 1ull << 63) & active;
-        // the last active lane's run ends there even if it is not the last lane: lane i + 1
-        // is then past the end, a head
-        if (__builtin_amdgcn_inverse_ballot_w64(emits[ph])) {
+        // f16 values are rounded once per entry, so there a row that neighbouring points of
+        // different cells share by a hash collision is one entry too: its wavefront (rare)
+        // finds the runs of each corner
+        bool clash = false;
+        if constexpr (kHalf) {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) rank[ph][c] = atomicAdd(&cnt[rows[ph][c] / R - s_lo], 1u);
+            for (int c = 0; c < 8; ++c) clash |= rows[ph][c] == dpp_u32<kWaveShr1, 0xf>(rows[ph][c], ~rows[ph][c]);
+            clash = clash & !same & (n < d.n_points);
+        }
+        if (kHalf && __ballot(clash) != 0ull) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const bool eq = rows[ph][c] == dpp_u32<kWaveShr1, 0xf>(rows[ph][c], ~rows[ph][c]);
+                const CellRuns runs = cell_runs(~__ballot(eq & (n < d.n_points)));
+                sum_runs<F>(vals[ph] + c * F, runs);
+                rank[ph][c] = kNoEntry;
+                if (__builtin_amdgcn_inverse_ballot_w64(run_ends(runs) & active))
+                    rank[ph][c] = atomicAdd(&cnt[rows[ph][c] / R - s_lo], 1u);
+            }
+        } else {
+            const CellRuns runs = cell_runs(~__ballot(same));
+            sum_runs<8 * F>(vals[ph], runs);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) rank[ph][c] = kNoEntry;
+            if (__builtin_amdgcn_inverse_ballot_w64(run_ends(runs) & active)) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) rank[ph][c] = atomicAdd(&cnt[rows[ph][c] / R - s_lo], 1u);
+            }
         }
     }
     __syncthreads();
@@ -781,9 +809,9 @@ __global__ void __launch_bounds__(kBucketThreads)
     // rank becomes the entry's place in the item's region
 #pragma unroll
     for (int ph = 0; ph < kBucketPhases; ++ph) {
-        const bool emit = __builtin_amdgcn_inverse_ballot_w64(emits[ph]);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) rank[ph][c] = emit ? rank[ph][c] + cnt[rows[ph][c] / R - s_lo] : 0xffffffffu;
+        for (int c = 0; c < 8; ++c)
+            if (rank[ph][c] != kNoEntry) rank[ph][c] += cnt[rows[ph][c] / R - s_lo];
     }
     // the region, kStageEntries at a time through LDS: each 64-byte request to the L2
     // carries whole neighbouring entries (scattered entry by entry, 17 M requests of 12
@@ -817,27 +845,57 @@ __global__ void __launch_bounds__(kBucketThreads)
     }
 }
 
-// One-pass table gradient, part 2: parts of slice s (run_part entries each, at least
-// one), from the run lengths of every item whose level reaches s.
+// How a slice's entries are summed.  Its items, in (level, chunk) order, are cut in two
+// ways by exclusive prefixes of run lengths: into work, of run_part entries of the slice
+// (one workgroup's), and into groups, of kPart entries of the kSliceBytes of rows the
+// slice lies in (with all their runs, and whole items of kGroupPoints points).  Each
+// group's sum is rounded to f32 once and the groups are added in f32; within a group the
+// parts' sums stay f64, so the result does not depend on run_part.  Both cuts only move
+// forward over the items, so work + group numbers the parts.
+constexpr uint32_t kGroupPoints = 1024;
+
+__device__ __forceinline__ uint32_t n_cuts(uint64_t entries, uint32_t per) {
+    return entries == 0 ? 1u : (uint32_t)((entries + per - 1) / per);
+}
+
+// Run length of item (l, k) in slice s; 0 if level l does not reach it.
+__device__ __forceinline__ uint32_t slice_run_length(const BwdPlan &p, const uint32_t *__restrict__ runs, uint32_t l,
+                                                     uint32_t s, uint32_t k) {
+    return s < p.s_lo[l] || s > p.s_hi[l] ? 0u : run_length(runs[run_index(p, l, s - p.s_lo[l], k)]);
+}
+
+// One-pass table gradient, part 2: parts of slice s, from the run lengths of every item
+// whose level reaches s or the other slice of its group.
 __global__ void __launch_bounds__(256)
     bwd_slice_parts_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ runs,
                            uint32_t *__restrict__ slice_np) {
-    const uint32_t s = blockIdx.x;
-    uint32_t tot = 0;
+    const uint32_t s = blockIdx.x, other = p.group_shift ? s ^ 1u : s;
+    uint32_t own = 0, both = 0;
     for (uint32_t l = 0; l < d.L; ++l) {
-        if (s < p.s_lo[l] || s > p.s_hi[l]) continue;
-        const uint32_t sl = s - p.s_lo[l];
-        for (uint32_t k = threadIdx.x; k < p.n_bchunks; k += 256)
-            tot += run_length(runs[run_index(p, l, sl, k)]);
+        const bool here = s >= p.s_lo[l] && s <= p.s_hi[l], there = other >= p.s_lo[l] && other <= p.s_hi[l];
+        if (!here && !there) continue;
+        for (uint32_t k = threadIdx.x; k < p.n_bchunks; k += 256) {
+            const uint32_t n = here ? run_length(runs[run_index(p, l, s - p.s_lo[l], k)]) : 0u;
+            own += n;
+            both += n;
+            if (p.group_shift && there) both += run_length(runs[run_index(p, l, other - p.s_lo[l], k)]);
+        }
     }
-    __shared__ uint32_t ws[256 / kWave];
-    tot = wave_sum(tot);
-    if (lane_id() == 0) ws[threadIdx.x / kWave] = tot;
+    __shared__ uint32_t ws[2][256 / kWave];
+    own = wave_sum(own);
+    both = wave_sum(both);
+    if (lane_id() == 0) {
+        ws[0][threadIdx.x / kWave] = own;
+        ws[1][threadIdx.x / kWave] = both;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int w = 0; w < 256 / kWave; ++w) t += ws[w];
-        slice_np[s] = t == 0 ? 1u : (t + p.run_part - 1) / p.run_part;
+        uint64_t t = 0, g = 0;
+        for (int w = 0; w < 256 / kWave; ++w) {
+            t += ws[0][w];
+            g += ws[1][w];
+        }
+        slice_np[s] = n_cuts(t, p.run_part) + n_cuts(g, kPart) - 1u;
     }
 }
 
@@ -950,11 +1008,9 @@ __global__ void __launch_bounds__(kReduceThreads)
 // pushing each run's lane number to the lane of its first entry and a running maximum
 // (RunSequence).  kSteps such groups are loaded before the previous ones are added.  A
 // slice of one part (nearly all of them) needs no barrier between its runs; a slice of
-// several parts first cuts the items, in (level, chunk) order, by the prefix of their
-// run lengths: a part takes those whose exclusive prefix falls in
-// [part * run_part, (part + 1) * run_part).
+// several parts first finds its items by the prefixes of their run lengths (see n_cuts).
 // With kAdam, a slice summed in one part is not stored: its rows take the optimizer
-// step in place (params, m, v), and bwd_combine does the same for the others.
+// step in place (params, m, v), and bwd_combine_runs does the same for the others.
 // 2^18 ray samples, f32: 82 -> 62 us, of which the atomics themselves need 27 (34 M f64
 // adds at 1.27 T/s); slices of 64 KiB, two workgroups to a CU, so that one clears or
 // stores its rows while the other adds (128 KiB slices: 80 us); 1,024 points: 29 -> 18.
@@ -1035,14 +1091,16 @@ __global__ void __launch_bounds__(kRunThreads)
     bwd_reduce_runs_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ meta,
                            const uint32_t *__restrict__ parts, const uint32_t *__restrict__ part_slice,
                            const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
-                           const uint16_t *__restrict__ entry_rows, float *__restrict__ partials,
-                           float *__restrict__ dtable, AdamStep adam = {}, float *__restrict__ adam_p = nullptr,
-                           float *__restrict__ adam_m = nullptr, float *__restrict__ adam_v = nullptr) {
+                           const uint16_t *__restrict__ entry_rows, double *__restrict__ partials,
+                           uint32_t *__restrict__ part_group, float *__restrict__ dtable, AdamStep adam = {},
+                           float *__restrict__ adam_p = nullptr, float *__restrict__ adam_m = nullptr,
+                           float *__restrict__ adam_v = nullptr) {
     typedef EntryGroup<F, kHalf> Group;
     constexpr uint32_t kBucketEntries = bucket_entries(kHalf);
     constexpr uint32_t kWaves = kRunThreads / kWave;
     extern __shared__ double acc[];
     __shared__ uint32_t chosen[kRunThreads];
+    __shared__ uint32_t my_group;
     __shared__ uint32_t marks[kWaves][kWave];
     const uint32_t b = blockIdx.x;
     if (b >= meta[1]) return;
@@ -1058,10 +1116,13 @@ __global__ void __launch_bounds__(kRunThreads)
     seq.marks = marks[wave];
     seq.tag = 0;
     seq.marks[lane] = 0u;
-    uint32_t carry = 0;  // entries of the items visited before
+    if (threadIdx.x == 0) my_group = 0xffffffffu;
+    uint32_t carry = 0, carry_group = 0;  // entries of the items visited before
+    const uint32_t other = p.group_shift ? s ^ 1u : s;
     for (uint32_t l = 0; l < d.L; ++l) {
-        if (s < p.s_lo[l] || s > p.s_hi[l]) continue;
-        const uint32_t *level_runs = runs + run_index(p, l, s - p.s_lo[l], 0);
+        const bool here = s >= p.s_lo[l] && s <= p.s_hi[l];
+        if (!here && (n_parts == 1 || other < p.s_lo[l] || other > p.s_hi[l])) continue;
+        const uint32_t *level_runs = runs + (here ? run_index(p, l, s - p.s_lo[l], 0) : 0);
         for (uint32_t k0 = 0; k0 < p.n_bchunks; k0 += kRunThreads) {
             const uint32_t n_k = min(p.n_bchunks - k0, (uint32_t)kRunThreads);
             const uint32_t k = wave + lane * kWaves;  // this lane's run of the tile
@@ -1069,11 +1130,23 @@ __global__ void __launch_bounds__(kRunThreads)
             if (n_parts == 1) {
                 if (k < n_k) my_run = level_runs[k0 + k];
             } else {
-                const uint32_t r = threadIdx.x < n_k ? level_runs[k0 + threadIdx.x] : 0u;
-                uint32_t tot;
+                const uint32_t r = here && threadIdx.x < n_k ? level_runs[k0 + threadIdx.x] : 0u;
+                uint32_t g = run_length(r), tot, tot_group;
+                if (p.group_shift && threadIdx.x < n_k) g += slice_run_length(p, runs, l, other, k0 + threadIdx.x);
                 const uint32_t ex = block_exclusive_scan<kRunThreads>(run_length(r), &tot);
-                chosen[threadIdx.x] = (carry + ex) / p.run_part == part ? r : 0u;
+                uint32_t ex_group = block_exclusive_scan<kRunThreads>(g, &tot_group);
+                if constexpr (bucket_points(kHalf) < kGroupPoints) {
+                    // the second item of a group's kGroupPoints goes with the first
+                    static_assert(2 * bucket_points(kHalf) == kGroupPoints, "two items");
+                    const uint32_t before = __shfl_up(g, 1, kWave);
+                    if (threadIdx.x & 1u) ex_group -= before;
+                }
+                const uint32_t group = (carry_group + ex_group) / kPart;
+                const bool mine = r >> 16 != 0u && (carry + ex) / p.run_part + group == part;
+                chosen[threadIdx.x] = mine ? r : 0u;
+                if (mine) my_group = group;  // the same for all of the part's items
                 carry += tot;
+                carry_group += tot_group;
                 __syncthreads();
                 my_run = chosen[k];
                 __syncthreads();  // rewritten by the next tile
@@ -1103,7 +1176,13 @@ __global__ void __launch_bounds__(kRunThreads)
         }
         return;
     }
-    float *out = n_parts == 1 ? dtable + o : partials + (size_t)b * R * F;
+    if (n_parts > 1) {
+        if (threadIdx.x == 0) part_group[b] = my_group;
+        double2 *out = reinterpret_cast<double2 *>(partials + (size_t)b * R * F);
+        for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) out[t] = reinterpret_cast<const double2 *>(acc)[t];
+        return;
+    }
+    float *out = dtable + o;
     for (uint32_t t = threadIdx.x; t < rows; t += kRunThreads) {
         if constexpr (F == 2) {
             reinterpret_cast<float2 *>(out)[t] = make_float2((float)acc[t], (float)acc[R + t]);
@@ -1113,16 +1192,53 @@ __global__ void __launch_bounds__(kRunThreads)
     }
 }
 
+// One-pass table gradient, part 5: slices of several parts.  Block (s, c) covers
+// 1 / kCombineSplit of slice s's rows.  With kAdam the sums are not stored: the rows take
+// the optimizer step in place.
+constexpr uint32_t kCombineSplit = 16;
+template <int F, uint32_t R, bool kAdam>
+__global__ void __launch_bounds__(256)
+    bwd_combine_runs_kernel(HashGridDescriptor d, const uint32_t *__restrict__ parts,
+                            const double *__restrict__ partials, const uint32_t *__restrict__ part_group,
+                            float *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
+                            float *__restrict__ adam_m, float *__restrict__ adam_v) {
+    const uint32_t s = blockIdx.x;
+    const uint32_t p0 = parts[s], n_parts = parts[s + 1] - p0;
+    if (n_parts <= 1) return;
+    const uint32_t rows = min(d.n_rows - s * R, R);
+    constexpr uint32_t kPer = R * F / kCombineSplit;
+    // feature f of row r is value f * R + r of a part
+    for (uint32_t t = blockIdx.y * kPer + threadIdx.x; t < (blockIdx.y + 1) * kPer; t += 256) {
+        const uint32_t f = t / R, r = t % R;
+        if (r >= rows) continue;
+        float sum = 0.0f;
+        double in_group = 0.0;
+        uint32_t group = 0xffffffffu;
+        for (uint32_t q = 0; q < n_parts; ++q) {
+            const uint32_t g = part_group[p0 + q];
+            if (g == 0xffffffffu) continue;  // no item: both cuts moved on together
+            if (g != group) sum += (float)in_group, in_group = 0.0, group = g;
+            in_group += partials[(size_t)(p0 + q) * R * F + t];
+        }
+        sum += (float)in_group;
+        const size_t o = ((size_t)s * R + r) * F + f;
+        if constexpr (kAdam) {
+            float mk = adam_m[o], vk = adam_v[o];
+            adam_p[o] = adam_step(adam, adam_p[o], sum, mk, vk);
+            adam_m[o] = mk;
+            adam_v[o] = vk;
+        } else {
+            dtable[o] = sum;
+        }
+    }
+}
+
 // 5. slices of several parts: rows = sum of the parts' partial rows, in part
 // order.  Block (s, c) covers 1/kCombineSplit of slice s.
-constexpr uint32_t kCombineSplit = 16;
-// With kAdam the sums are not stored: the rows take the optimizer step in place.
-template <int F, bool kAdam = false>
+template <int F>
 __global__ void __launch_bounds__(256)
     bwd_combine_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ parts,
-                       const float *__restrict__ partials, float *__restrict__ dtable, AdamStep adam = {},
-                       float *__restrict__ adam_p = nullptr, float *__restrict__ adam_m = nullptr,
-                       float *__restrict__ adam_v = nullptr) {
+                       const float *__restrict__ partials, float *__restrict__ dtable) {
     const uint32_t s = blockIdx.x;
     const uint32_t p0 = parts[s], n_parts = parts[s + 1] - p0;
     if (n_parts <= 1) return;
@@ -1142,32 +1258,12 @@ __global__ void __launch_bounds__(256)
                 a.z += v.z;
                 a.w += v.w;
             }
-            if constexpr (kAdam) {
-                float4 p4 = *reinterpret_cast<const float4 *>(adam_p + o + t);
-                float4 m4 = *reinterpret_cast<const float4 *>(adam_m + o + t);
-                float4 v4 = *reinterpret_cast<const float4 *>(adam_v + o + t);
-                p4.x = adam_step(adam, p4.x, a.x, m4.x, v4.x);
-                p4.y = adam_step(adam, p4.y, a.y, m4.y, v4.y);
-                p4.z = adam_step(adam, p4.z, a.z, m4.z, v4.z);
-                p4.w = adam_step(adam, p4.w, a.w, m4.w, v4.w);
-                *reinterpret_cast<float4 *>(adam_m + o + t) = m4;
-                *reinterpret_cast<float4 *>(adam_v + o + t) = v4;
-                *reinterpret_cast<float4 *>(adam_p + o + t) = p4;
-            } else {
-                *reinterpret_cast<float4 *>(dtable + o + t) = a;
-            }
+            *reinterpret_cast<float4 *>(dtable + o + t) = a;
         } else {
             for (uint32_t u = t; u < hi; ++u) {
                 float a = 0.0f;
                 for (uint32_t q = 0; q < n_parts; ++q) a += src[q * pstride + u];
-                if constexpr (kAdam) {
-                    float mk = adam_m[o + u], vk = adam_v[o + u];
-                    adam_p[o + u] = adam_step(adam, adam_p[o + u], a, mk, vk);
-                    adam_m[o + u] = mk;
-                    adam_v[o + u] = vk;
-                } else {
-                    dtable[o + u] = a;
-                }
+                dtable[o + u] = a;
             }
         }
     }
@@ -1211,7 +1307,8 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
     uint32_t *meta = reinterpret_cast<uint32_t *>(ws + p.meta_off);
     uint32_t *parts = reinterpret_cast<uint32_t *>(ws + p.parts_off);
     uint32_t *part_slice = reinterpret_cast<uint32_t *>(ws + p.part_slice_off);
-    float *partials = reinterpret_cast<float *>(ws + p.partials_off);
+    double *partials = reinterpret_cast<double *>(ws + p.partials_off);
+    uint32_t *part_group = reinterpret_cast<uint32_t *>(ws + p.part_group_off);
     auto *values = reinterpret_cast<EntryValue<F, kHalf> *>(ws + p.entries_off);
     uint16_t *entry_rows = reinterpret_cast<uint16_t *>(ws + p.rows_off);
     const size_t lds = (size_t)R * F * sizeof(double);
@@ -1226,17 +1323,18 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
     if constexpr (!kHalf) {
         if (fused != nullptr) {
             hipLaunchKernelGGL(reduce_adam, dim3(p.max_parts), dim3(kRunThreads), lds, stream, d, p, meta, parts,
-                               part_slice, runs, values, entry_rows, partials, dtable, fused->step, fused->p, fused->m,
+                               part_slice, runs, values, entry_rows, partials, part_group, dtable, fused->step,
+                               fused->p, fused->m, fused->v);
+            hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, true>), dim3(p.n_slices, kCombineSplit), dim3(256), 0,
+                               stream, d, parts, partials, part_group, dtable, fused->step, fused->p, fused->m,
                                fused->v);
-            hipLaunchKernelGGL((bwd_combine_kernel<F, true>), dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d, p,
-                               parts, partials, dtable, fused->step, fused->p, fused->m, fused->v);
             return true;
         }
     }
     hipLaunchKernelGGL(reduce, dim3(p.max_parts), dim3(kRunThreads), lds, stream, d, p, meta, parts, part_slice, runs,
-                       values, entry_rows, partials, dtable, AdamStep{}, nullptr, nullptr, nullptr);
-    hipLaunchKernelGGL((bwd_combine_kernel<F>), dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d, p, parts,
-                       partials, dtable, AdamStep{}, nullptr, nullptr, nullptr);
+                       values, entry_rows, partials, part_group, dtable, AdamStep{}, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, false>), dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d,
+                       parts, partials, part_group, dtable, AdamStep{}, nullptr, nullptr, nullptr);
     return true;
 }
 

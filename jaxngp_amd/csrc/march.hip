@@ -7,25 +7,20 @@
 // atomicAdd in scheduling order and marches every ray twice.  Here the ranges are
 // an exclusive prefix sum of the per-ray counts in ray order, which makes the
 // output deterministic and equal to processing rays one after another:
-//   1. march_count:  one wavefront per ray counts its samples; the block total is
-//                    parked in rays_sample_startidx[first ray of the block] (slot
-//                    owned by the block, so no scratch memory).  Rays are counted
-//                    in ray-ordered launches (2048 rays, up to 16384, up to
-//                    131072, the rest); a later launch's workgroups first add the
-//                    parked totals of the earlier launches, and a launch that finds
-//                    the sample buffer already full skips marching, which changes
-//                    no output (its rays are invalid regardless of their counts).
-//                    The first launch's rays also record their samples' t in the
-//                    sample outputs, which are not written yet (a "t record" of up
-//                    to `slot` floats per ray);
-//   2. march_scan:   one workgroup scans the block totals, finds the ray where the
-//                    sample buffer fills up and writes the two helper counters;
-//   3. march_emit:   one wavefront per valid ray writes its samples' t to z_vals at
-//                    its offset: copied from its t record (the first launch's rays,
-//                    in training the whole batch), else marched again;
-//   4. march_fill:   one wavefront per valid ray writes the outputs that follow from
+//   1. march_begin:  marks every ray's count and start as "past the filled buffer";
+//   2. march_count:  workgroups take blocks of rays in rounds, count their samples and add
+//                    them to the round's counter.  A workgroup that finds the earlier
+//                    rounds' counters at total_samples stops: all of them are of earlier
+//                    rays, so the rays left are invalid whatever their counts and keep their
+//                    marks.  Each ray leaves a record of its samples (see RayRecord) in
+//                    the xyzs output, which nothing has written yet;
+//   3. march_scan:   one workgroup scans the counts, finds the ray where the sample buffer
+//                    fills up and writes the two helper counters;
+//   4. march_emit:   one wavefront per valid ray writes its samples' t to z_vals at its
+//                    offset: from its record, or marched again where it has none;
+//   5. march_fill:   one wavefront per valid ray writes the outputs that follow from
 //                    t (index, position, direction, step size);
-//   5. march_finish: validity, final counts and offsets, zeros in the unused tail.
+//   6. march_finish: validity, final counts and offsets, zeros in the unused tail.
 // A ray is valid iff the samples of the rays before it leave room (prefix <
 // total_samples), t_end > t_start, and its own samples fit; rays after the buffer
 // fills are invalid, as the reference's early exit at marching.cu:135 makes them.
@@ -34,9 +29,9 @@
 // lies on the sequence c_0 = t_start, c_{k+1} = c_k + step_size(c_k): an occupied
 // step moves to the next element, an empty-cell skip to the first later element
 // at or past the cell's exit.  So a wavefront generates 64 consecutive elements
-// (one per lane, a serial chain of adds), looks up all 64 cells and exit distances
-// at once, and walks the visited elements with ballots: runs of occupied lanes
-// are emitted together, a skip is a search for the first lane past the exit.
+// (one per lane), looks up all 64 cells and exit distances at once, and walks the
+// visited elements with ballots: runs of occupied lanes are emitted together, a skip is
+// a search for the first lane past the exit.
 // Samples go to their slots by lane prefix counts.  The walk visits exactly the
 // reference's t values in its order; where the chain stops growing (t + ds == t)
 // the ray finishes on one lane with the serial loop, which handles that case.
@@ -49,7 +44,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kRaysPerBlock = kBlock / kWave;  // one wavefront per ray
 constexpr int kScanThreads = 1024;
-// parked total of a block whose launch found the sample buffer already full
+// count of a ray that was not marched: the sample buffer was already full
 constexpr uint32_t kPastFill = 0xffffffffu;
 
 struct Ray {
@@ -72,34 +67,23 @@ __device__ __forceinline__ Ray load_ray(const float *__restrict__ rays_o, const 
     return r;
 }
 
-// Where a marching wavefront records its samples: the t of sample k goes to ts[k]
-// for k < cap (the other outputs follow from t, see march_fill_kernel).
+// Where a marching wavefront writes its samples: the t of sample k goes to ts[k]
+// (the other outputs follow from t, see march_fill_kernel).
 struct RaySamples {
     float *ts;
-    uint32_t cap;
 };
 
-__device__ __forceinline__ void put_t(const RaySamples &o, uint32_t k, float t) {
-    if (k < o.cap) o.ts[k] = t;
-}
-
-// The t records of the first count launch's rays, kept in the sample outputs before
-// they are written (xyzs, dirs, dss, then idcs, 8 floats per sample slot in all):
-// ray i of that launch owns `slot` floats of the region q with
-// first[q] <= i < first[q + 1].  A ray with more than `slot` samples, or past
-// first[4], is marched again by the emit pass.
-struct TStore {
-    float *region[4];
-    uint32_t first[5];
-    uint32_t slot;
+// A ray's record: for every window of 64 chain elements (see Window) that holds samples,
+// the window's first element and the mask of the elements that are samples, three words;
+// word 0 holds the number of windows, or kNoRecord for a ray with more than the record
+// takes or one that left the windows.  52 words a ray at bound 1 instead of its up to
+// 1,024 t values, at a place that does not depend on its count, and no LDS: the marcher
+// runs beside the MLP backward, whose two workgroups take a CU's whole LDS.
+struct RayRecord {
+    uint32_t *words;  // null: none is kept
+    uint32_t max_windows;
 };
-
-__device__ __forceinline__ float *t_record(const TStore &st, uint32_t i) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        if (i >= st.first[q] && i < st.first[q + 1]) return st.region[q] + (size_t)(i - st.first[q]) * st.slot;
-    return nullptr;
-}
+constexpr uint32_t kNoRecord = 0xffffffffu;
 
 // The reference's loop (marching.cu:162-192) from position t with n samples taken,
 // on one lane.
@@ -111,7 +95,7 @@ __device__ uint32_t march_serial(const MarchParams &p, const uint8_t *__restrict
         const float ds = step_size(p, t);
         float gx, gy, gz, mb;
         if (lookup_cell(p, bits, cache, px, py, pz, ds, gx, gy, gz, mb)) {
-            if (kWrite) put_t(o, n, t);
+            if (kWrite) o.ts[n] = t;
             ++n;
             t = t + ds;
         } else {
@@ -121,6 +105,19 @@ __device__ uint32_t march_serial(const MarchParams &p, const uint8_t *__restrict
     }
     return n;
 }
+
+// 64 consecutive elements of the chain c_0 = base, c_{j+1} = c_j + step_size(c_j), one
+// per lane, with what the walk needs of each.
+struct Window {
+    float w;        // c_lane
+    float exit;     // exit distance of its cell
+    uint64_t word;  // the occupancy word (or byte) of its cell
+    uint32_t bit;   // its bit there
+    bool live;      // w < t_end
+    // the same in all lanes
+    float base, next;  // c_0, c_64
+    bool stall;        // the chain stops growing
+};
 
 // Lane j's element of the chain c_0 = base, c_{j+1} = c_j + k (k > 0 constant).
 // While the chain stays in base's binade, where every float is a multiple of the
@@ -135,7 +132,9 @@ __device__ __forceinline__ bool chain_in_binade(float base, float k, int lane, f
     const uint32_t e8 = __float_as_uint(base) >> 23;  // sign bit included: negative base fails
     if (e8 < 24u || e8 >= 255u) return false;
     const float u = __uint_as_float((e8 - 23u) << 23);
-    const float m = rintf(k / u);  // division by a power of two: exact
+    // k / u is a scaling by a power of two: exact, also as a product with 1 / u (normal
+    // for the exponents that pass the test above and leave m in range)
+    const float m = e8 <= 253u ? rintf(k * __uint_as_float((277u - e8) << 23)) : 0.0f;
     if (!(m >= 1.0f && m <= 65536.0f)) return false;
     const float x = base + ((float)lane * m) * u;
     const float nx = x + k;
@@ -150,163 +149,81 @@ __device__ __forceinline__ bool chain_in_binade(float base, float k, int lane, f
     return true;
 }
 
-// Lane j's element of the window starting at `base` (c_j of the chain from base) and
-// the element after the window (c_64); `stall` where the chain stops growing.
-__device__ __forceinline__ void chain_window(const MarchParams &p, bool const_step, float k_step, float base, int lane,
-                                             float &w, float &next, bool &stall) {
-    w = base;
-    next = base;
+// The 64 elements from `base` on: lane j's in w, c_64 in next; `stall` where the chain
+// stops growing.
+__device__ __forceinline__ void chain_window(const MarchParams &p, bool const_step, float k_step, float base, float &w,
+                                             float &next, bool &stall) {
+    const int lane = lane_id();
     stall = false;
-    if (const_step && chain_in_binade(base, k_step, lane, w, next)) return;  // 64 elements at once
+    if (const_step && chain_in_binade(base, k_step, lane, w, next)) return;
     float c = base;
-    if (const_step) {
-#pragma unroll
-        for (int q = 0; q < kWave; ++q) {
-            if (lane == q) w = c;
-            const float nx = c + k_step;
-            stall |= nx == c;
-            c = nx;
-        }
-    } else {
-#pragma unroll 8
-        for (int q = 0; q < kWave; ++q) {
-            if (lane == q) w = c;
-            const float nx = c + step_size(p, c);
-            stall |= nx == c;
-            c = nx;
-        }
+    w = base;
+    bool stops = false;
+#pragma unroll 4
+    for (int q = 0; q < kWave; ++q) {
+        if (lane == q) w = c;
+        const float nx = c + (const_step ? k_step : step_size(p, c));
+        stops |= nx == c;
+        c = nx;
     }
     next = c;
+    stall = __ballot(stops) != 0ull;
 }
 
-// Windows of 64 chain elements a marching wavefront looks up together: their
-// bitfield loads are all in flight before the first window is walked.
-constexpr int kMarchWindows = 4;
+// The window starting at `base`, its occupancy load issued.  Call with all lanes active.
+__device__ __forceinline__ Window make_window(const MarchParams &p, const uint8_t *__restrict__ bits, bool word_ok,
+                                              const Ray &r, bool const_step, float k_step, float base) {
+    Window v;
+    v.base = base;
+    chain_window(p, const_step, k_step, base, v.w, v.next, v.stall);
+    v.live = v.w < r.t1;
+    const float px = r.ox + v.w * r.dx, py = r.oy + v.w * r.dy, pz = r.oz + v.w * r.dz;
+    float gx, gy, gz, mb;
+    const uint32_t idx = cell_index(p, px, py, pz, step_size(p, v.w), gx, gy, gz, mb);
+    v.word = 0ull;
+    if (word_ok) {
+        v.bit = idx & 63u;
+        if (v.live) v.word = reinterpret_cast<const uint64_t *>(bits)[idx >> 6];
+    } else {
+        v.bit = idx & 7u;
+        if (v.live) v.word = bits[idx >> 3];
+    }
+    v.exit = cell_exit_t(p, v.w, px, py, pz, gx, gy, gz, mb, r.dx, r.dy, r.dz, r.idx, r.idy, r.idz);
+    return v;
+}
+
+__device__ __forceinline__ float lane_float(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
 
 // Counts the samples of one ray with the whole wavefront, starting at t_start,
-// taking at most cap samples (kWrite: also records their t).  Call with all 64
-// lanes active.
+// taking at most cap samples (kWrite: also writes their t; with a record: also keeps
+// it).  Call with all 64 lanes active.  The next window is made, its occupancy load in flight, before this
+// one is walked.
 template <bool kWrite>
 __device__ uint32_t march_ray_wave(const MarchParams &p, const uint8_t *__restrict__ bits, bool word_ok, const Ray &r,
-                                   float t_start, uint32_t cap, const RaySamples &o) {
+                                   float t_start, uint32_t cap, const RaySamples &o, const RayRecord &rec) {
     const int lane = lane_id();
+    uint32_t windows = 0;  // in the record
     const uint64_t below = (1ull << lane) - 1ull;
     // with stepsize_portion 0 every step is the same constant, for every t
     const bool const_step = p.portion == 0.0f;
     const float k_step = step_size(p, 0.0f);
-    const uint64_t *__restrict__ words = reinterpret_cast<const uint64_t *>(bits);
     uint32_t n = 0;
-    float base = t_start;  // sequence element of lane 0 of the next window
     bool pending = false;  // a skip is searching for the first element >= thr
     float thr = 0.0f;
-    while (n < cap) {
-        // up to kMarchWindows windows: stop after a window that reaches t_end, and
-        // before one whose chain stalls (finished on one lane below)
-        float w[kMarchWindows];
-        int nw = 0;
-        bool stall = false;
-#pragma unroll
-        for (int q = 0; q < kMarchWindows; ++q) {
-            if (nw == q && !stall) {
-                float wq, next;
-                bool st;
-                chain_window(p, const_step, k_step, base, lane, wq, next, st);
-                if (__ballot(st) != 0ull) {
-                    stall = true;
-                } else {
-                    w[q] = wq;
-                    nw = q + 1;
-                    base = next;
-                    // the window's last element at or past t_end: later windows are dead
-                    if (!(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(wq), kWave - 1)) < r.t1)) break;
-                }
-            }
-        }
-        // cells of every window, the bitfield loads issued together
-        uint32_t idx[kMarchWindows];
-        float gx[kMarchWindows], gy[kMarchWindows], gz[kMarchWindows], mb[kMarchWindows];
-        bool live[kMarchWindows], occ[kMarchWindows];
-#pragma unroll
-        for (int q = 0; q < kMarchWindows; ++q) {
-            live[q] = q < nw && w[q] < r.t1;
-            idx[q] = 0u;
-            if (live[q]) {
-                const float px = r.ox + w[q] * r.dx, py = r.oy + w[q] * r.dy, pz = r.oz + w[q] * r.dz;
-                idx[q] = cell_index(p, px, py, pz, step_size(p, w[q]), gx[q], gy[q], gz[q], mb[q]);
-            }
-        }
-        if (word_ok) {
-            uint64_t wd[kMarchWindows];
-#pragma unroll
-            for (int q = 0; q < kMarchWindows; ++q) wd[q] = live[q] ? words[idx[q] >> 6] : 0ull;
-#pragma unroll
-            for (int q = 0; q < kMarchWindows; ++q) occ[q] = live[q] && ((wd[q] >> (idx[q] & 63u)) & 1ull);
-        } else {
-            uint32_t by[kMarchWindows];
-#pragma unroll
-            for (int q = 0; q < kMarchWindows; ++q) by[q] = live[q] ? bits[idx[q] >> 3] : 0u;
-#pragma unroll
-            for (int q = 0; q < kMarchWindows; ++q) occ[q] = live[q] && ((by[q] >> (idx[q] & 7u)) & 1u);
-        }
-        bool done = false;
-#pragma unroll
-        for (int q = 0; q < kMarchWindows; ++q) {
-            if (q < nw && !done) {
-                float ex = 0.0f;
-                if (live[q] && !occ[q]) {
-                    const float px = r.ox + w[q] * r.dx, py = r.oy + w[q] * r.dy, pz = r.oz + w[q] * r.dz;
-                    ex = cell_exit_t(p, w[q], px, py, pz, gx[q], gy[q], gz[q], mb[q], r.dx, r.dy, r.dz, r.idx, r.idy,
-                                     r.idz);
-                }
-                const uint64_t live_m = __ballot(live[q]);
-                const uint64_t occ_m = __ballot(occ[q]);
-                const uint32_t n0 = n;
-                uint64_t emit = 0ull;
-                int cur = 0;
-                while (cur < kWave) {
-                    if (pending) {
-                        // skip_to stops at the first element with !(t < thr)
-                        const uint64_t m = __ballot(!(w[q] < thr)) & (~0ull << cur);
-                        if (m == 0ull) {
-                            // the target lies past this window; if the window already
-                            // reached t_end, so does the target and the ray is done
-                            done = ((live_m >> (kWave - 1)) & 1ull) == 0ull;
-                            break;
-                        }
-                        cur = __builtin_ctzll(m);
-                        pending = false;
-                    }
-                    if (((live_m >> cur) & 1ull) == 0ull) {
-                        done = true;
-                        break;
-                    }
-                    if ((occ_m >> cur) & 1ull) {
-                        const uint64_t from = occ_m >> cur;
-                        const int run = ~from == 0ull ? kWave - cur : __builtin_ctzll(~from);
-                        const uint32_t take = min((uint32_t)run, cap - n);
-                        emit |= (take >= 64u ? ~0ull : ((1ull << take) - 1ull)) << cur;
-                        n += take;
-                        if (n >= cap) {
-                            done = true;
-                            break;
-                        }
-                        cur += run;
-                    } else {
-                        thr = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ex), cur));
-                        pending = true;
-                        cur += 1;
-                    }
-                }
-                if (kWrite && ((emit >> lane) & 1ull)) put_t(o, n0 + (uint32_t)__popcll(emit & below), w[q]);
-            }
-        }
-        if (done) break;
-        if (stall) {
+    if (cap == 0) {
+        if (rec.words != nullptr && lane == 0) rec.words[0] = 0u;
+        return 0;
+    }
+    Window v = make_window(p, bits, word_ok, r, const_step, k_step, t_start);
+    for (;;) {
+        if (v.stall) {
             // the chain stops growing at or after `base`: the serial loop on one lane
             uint32_t nn = n;
             if (lane == 0) {
                 BitCache cache = make_bit_cache(bits, word_ok);
-                float t = base;
+                float t = v.base;
                 if (pending) {
                     // rest of skip_to: t is the first step past the skipped element
                     while (t < thr) {
@@ -319,101 +236,134 @@ __device__ uint32_t march_ray_wave(const MarchParams &p, const uint8_t *__restri
                     }
                 }
                 nn = march_serial<kWrite>(p, bits, cache, r, t, n, cap, o);
+                if (rec.words != nullptr) rec.words[0] = kNoRecord;
             }
             return (uint32_t)__builtin_amdgcn_readlane((int)nn, 0);
         }
+        const uint64_t live_m = __ballot(v.live);
+        const bool last = (live_m >> (kWave - 1)) == 0ull;  // the chain reaches t_end here
+        Window next;
+        if (!last) next = make_window(p, bits, word_ok, r, const_step, k_step, v.next);
+        const uint64_t occ_m = __ballot(v.live && ((v.word >> v.bit) & 1ull));
+        const uint32_t n0 = n;
+        uint64_t emit = 0ull;
+        int cur = 0;
+        while (cur < kWave) {
+            if (pending) {
+                // skip_to stops at the first element with !(t < thr)
+                const uint64_t m = __ballot(!(v.w < thr)) & (~0ull << cur);
+                if (m == 0ull) break;  // the target lies past this window
+                cur = __builtin_ctzll(m);
+                pending = false;
+            }
+            if (((live_m >> cur) & 1ull) == 0ull) break;  // at or past t_end: `last` holds
+            if ((occ_m >> cur) & 1ull) {
+                const uint64_t from = occ_m >> cur;
+                const int run = ~from == 0ull ? kWave - cur : __builtin_ctzll(~from);
+                const uint32_t take = min((uint32_t)run, cap - n);
+                emit |= (take >= 64u ? ~0ull : ((1ull << take) - 1ull)) << cur;
+                n += take;
+                if (n >= cap) break;
+                cur += run;
+            } else {
+                thr = lane_float(v.exit, cur);
+                pending = true;
+                cur += 1;
+            }
+        }
+        if (kWrite && ((emit >> lane) & 1ull)) o.ts[n0 + (uint32_t)__popcll(emit & below)] = v.w;
+        if (rec.words != nullptr && emit != 0ull) {
+            if (windows < rec.max_windows && lane < 3)
+                rec.words[1 + 3 * windows + lane] =
+                    lane == 0 ? __float_as_uint(v.base) : (uint32_t)(emit >> (lane == 1 ? 0 : 32));
+            ++windows;
+        }
+        if (last || n >= cap) {
+            if (rec.words != nullptr && lane == 0) rec.words[0] = windows <= rec.max_windows ? windows : kNoRecord;
+            return n;
+        }
+        v = next;
     }
-    return n;
 }
 
 __device__ __forceinline__ float start_t(const MarchParams &p, float t0, float noise) {
     return t0 + step_size(p, t0) * noise;  // marching.cu:159-160
 }
 
-// Whether the blocks before `block_begin` (earlier launches, finished) already took
-// total_samples samples: the workgroup adds their parked totals 1024 at a time and
-// stops as soon as the sum reaches total_samples or meets a block an earlier
-// launch marked kPastFill (that launch saw the buffer full).  Once the batch fills
-// in the first launch, as in training, that is one chunk per workgroup.
-__device__ bool filled_before(uint32_t block_begin, uint32_t total_samples,
-                              const uint32_t *__restrict__ block_totals) {
-    constexpr int kPer = 4;
-    __shared__ uint64_t part[kBlock / kWave];
-    __shared__ int verdict;
-    const int wave = (int)threadIdx.x / kWave;
-    uint64_t run = 0;
-    for (uint32_t c0 = 0; c0 < block_begin; c0 += kBlock * kPer) {
-        uint64_t sum = 0;
-        bool past = false;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const uint32_t b = c0 + k * kBlock + threadIdx.x;
-            if (b < block_begin) {
-                const uint32_t v = block_totals[(size_t)b * kRaysPerBlock];
-                if (v == kPastFill) past = true;
-                else sum += v;
-            }
-        }
-        sum = wave_sum64(sum);
-        const bool wave_past = __ballot(past) != 0ull;
-        if (lane_id() == 0) part[wave] = wave_past ? ~0ull : sum;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            bool full = false;
-            for (int w = 0; w < kBlock / kWave; ++w) {
-                if (part[w] == ~0ull) full = true;
-                else run += part[w];
-            }
-            verdict = full || run >= total_samples;
-        }
-        __syncthreads();
-        if (verdict) return true;
+// Marks every ray as not marched.  Of a block's start slots the first takes its sample
+// prefix (march_scan_kernel); the second of block c is counter c of the count rounds.
+__global__ void __launch_bounds__(kBlock)
+    march_begin_kernel(uint32_t n_rays, uint32_t *__restrict__ rays_n_samples, uint32_t *__restrict__ startidx) {
+    const size_t stride = (size_t)gridDim.x * kBlock;
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n_rays; i += stride) {
+        rays_n_samples[i] = kPastFill;
+        startidx[i] = i % kRaysPerBlock == 0 ? kPastFill : 0u;
     }
-    return false;
 }
 
-// Counts the rays of blocks [block_begin, block_end) (grid-stride).  A launch whose
-// predecessors already took total_samples samples marks its blocks kPastFill
-// without marching.  kRecord (the first launch): rays with a t record also record
-// their samples' t there.
-template <bool kRecord>
+// The records of rays [0, n): `words` words each, in the xyzs output.
+struct RecordStore {
+    uint32_t *base;
+    uint32_t n, words;
+};
+
+__device__ __forceinline__ RayRecord record_of(const RecordStore &st, uint32_t i) {
+    return i < st.n ? RayRecord{st.base + (size_t)i * st.words, (st.words - 1u) / 3u} : RayRecord{nullptr, 0u};
+}
+
+// Counts the rays of blocks [block_begin, block_end), one block a workgroup and round,
+// one ray a wavefront.  Round r of the launch has counter first_counter + r, and a
+// workgroup goes into it only while the counters before it, all of rays before its own,
+// are short of total_samples; what it reads too early costs a block marched in vain, no
+// more.  (Drawing rays from one shared counter instead cost a device atomic on one
+// address per ray, about 10 ns each one after another: 4096 rays took 114 us.)
+// The march is bound by one ray's latency, a chain of windows of about 350
+// instructions: few wavefronts in flight lose little and march few rays past the fill.
+// 2^18 rays, total_samples 2^18 filled by the first 3300: MARCH_NOTE.
 __global__ void __launch_bounds__(kBlock)
     march_count_kernel(MarchParams p, bool word_ok, uint32_t n_rays, uint32_t total_samples, uint32_t block_begin,
-                       uint32_t block_end, const float *__restrict__ rays_o, const float *__restrict__ rays_d,
-                       const float *__restrict__ t_starts, const float *__restrict__ t_ends,
-                       const float *__restrict__ noises, const uint8_t *__restrict__ bits, TStore store,
-                       uint32_t *__restrict__ rays_n_samples,
-                       uint32_t *__restrict__ block_totals /* = rays_sample_startidx */) {
-    if (block_begin > 0 && filled_before(block_begin, total_samples, block_totals)) {
-        for (uint32_t b = block_begin + blockIdx.x * kBlock + threadIdx.x; b < block_end; b += gridDim.x * kBlock)
-            block_totals[(size_t)b * kRaysPerBlock] = kPastFill;
-        return;
-    }
+                       uint32_t block_end, uint32_t first_counter, const float *__restrict__ rays_o,
+                       const float *__restrict__ rays_d, const float *__restrict__ t_starts,
+                       const float *__restrict__ t_ends, const float *__restrict__ noises,
+                       const uint8_t *__restrict__ bits, RecordStore records, uint32_t *__restrict__ rays_n_samples,
+                       uint32_t *__restrict__ counters /* = rays_sample_startidx */) {
     __shared__ uint32_t wave_n[kRaysPerBlock];
-    const int wave = (int)threadIdx.x / kWave;
-    for (uint32_t blk = block_begin + blockIdx.x; blk < block_end; blk += gridDim.x) {
-        const uint32_t i = blk * kRaysPerBlock + wave;
+    __shared__ uint64_t before;
+    const int lane = lane_id(), wave = (int)threadIdx.x / kWave;
+    uint32_t c = first_counter;
+    for (uint32_t blk = block_begin + blockIdx.x; blk < block_end; blk += gridDim.x, ++c) {
+        if (c > 0) {
+            if (wave == 0) {
+                uint64_t sum = 0;
+                for (uint32_t j = lane; j < c; j += kWave)
+                    sum += __hip_atomic_load(counters + (size_t)j * kRaysPerBlock + 1, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+                sum = wave_sum64(sum);
+                if (lane == 0) before = sum;
+            }
+            __syncthreads();
+            if (before >= total_samples) return;
+        }
+        const uint32_t i = __builtin_amdgcn_readfirstlane(blk * kRaysPerBlock + wave);
         uint32_t n = 0;
         if (i < n_rays) {
             const float t0 = t_starts[i], t1 = t_ends[i];
             if (t1 > t0) {
                 const Ray r = load_ray(rays_o, rays_d, i, t1);
-                const float ts = start_t(p, t0, noises[i]);
-                float *rec = kRecord ? t_record(store, i) : nullptr;
-                if (rec != nullptr) n = march_ray_wave<true>(p, bits, word_ok, r, ts, p.n_cap, RaySamples{rec, store.slot});
-                else n = march_ray_wave<false>(p, bits, word_ok, r, ts, p.n_cap, RaySamples{});
+                n = march_ray_wave<false>(p, bits, word_ok, r, start_t(p, t0, noises[i]), p.n_cap, RaySamples{},
+                                          record_of(records, i));
             }
-            if (lane_id() == 0) rays_n_samples[i] = n;
+            if (lane == 0) rays_n_samples[i] = min(n, kPastFill - 1u);
         }
-        if (lane_id() == 0) wave_n[wave] = n;
+        if (lane == 0) wave_n[wave] = n;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            uint64_t s = 0;
+        // (clamped so that a counter cannot wrap: counting less only stops later)
+        if (threadIdx.x == 0 && (uint64_t)c * kRaysPerBlock + 1 < n_rays) {
+            uint32_t s = 0;
 #pragma unroll
-            for (int w = 0; w < kRaysPerBlock; ++w) s += wave_n[w];
-            block_totals[(size_t)blk * kRaysPerBlock] = (uint32_t)min(s, (uint64_t)kPastFill - 1);
+            for (int w = 0; w < kRaysPerBlock; ++w) s += min(wave_n[w], 1u << 17);
+            if (s > 0) atomicAdd(counters + (size_t)c * kRaysPerBlock + 1, s);
         }
-        __syncthreads();
     }
 }
 
@@ -422,12 +372,13 @@ __device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b) {
     return c < a ? 0xffffffffu : c;
 }
 
-// Single workgroup.  Replaces each parked block total with the block's exclusive
-// prefix (saturated: only its comparison with total_samples matters) and writes
+// Single workgroup.  Writes each block's exclusive sample prefix (a block is
+// kRaysPerBlock consecutive rays; saturated: only its comparison with total_samples
+// matters) to the first of its rays_sample_startidx slots, and
 // next_sample_write_location / number_of_exceeded_samples.  Blocks are read in
-// tiles of 4096 with all loads of a tile in flight; the scan stops at the first
-// block of a skipped launch (every later block was skipped too, and their
-// kPastFill slots already mark their rays as past the filled buffer).
+// tiles of 4096 with all loads of a tile in flight; the scan stops after the first
+// block with a ray that was not marched (the rays before it already fill the buffer,
+// and the marks of later blocks are prefixes past it).
 constexpr int kScanPerThread = 4;
 __global__ void __launch_bounds__(kScanThreads)
     march_scan_kernel(uint32_t n_rays, uint32_t n_blocks, uint32_t total_samples,
@@ -444,24 +395,37 @@ __global__ void __launch_bounds__(kScanThreads)
     uint32_t scanned = 0;
     for (uint32_t t0 = 0; t0 < n_blocks; t0 += kTile) {
         if (tid == 0) first_past = 0xffffffffu;
-        uint32_t v[kScanPerThread];
+        uint32_t v[kScanPerThread], my_first = 0xffffffffu;
+        {
+            uint32_t cnt[kScanPerThread][kRaysPerBlock];
 #pragma unroll
-        for (int k = 0; k < kScanPerThread; ++k) {
-            const uint32_t b = t0 + tid * kScanPerThread + k;
-            v[k] = b < n_blocks ? block_slots[(size_t)b * kRaysPerBlock] : kPastFill;
+            for (int k = 0; k < kScanPerThread; ++k)
+#pragma unroll
+                for (int j = 0; j < kRaysPerBlock; ++j) {
+                    const uint64_t r = (uint64_t)(t0 + tid * kScanPerThread + k) * kRaysPerBlock + j;
+                    cnt[k][j] = r < n_rays ? rays_n_samples[r] : 0u;
+                }
+            // the samples of the block's rays before its first unmarched one
+#pragma unroll
+            for (int k = kScanPerThread - 1; k >= 0; --k) {
+                bool past = false;
+                v[k] = 0u;
+#pragma unroll
+                for (int j = 0; j < kRaysPerBlock; ++j) {
+                    past = past || cnt[k][j] == kPastFill;
+                    if (!past) v[k] = sat_add(v[k], cnt[k][j]);
+                }
+                if (past) my_first = t0 + tid * kScanPerThread + k;
+            }
         }
         __syncthreads();
-        // first skipped block of the tile: block indices grow with the thread and slot,
+        // first such block of the tile: block indices grow with the thread and slot,
         // so the lowest lane holding one has the wave's first; one LDS atomic per wave
-        // (not one per skipped block, which serialised on the one address)
-        uint32_t my_first = 0xffffffffu;
-#pragma unroll
-        for (int k = kScanPerThread - 1; k >= 0; --k)
-            if (v[k] == kPastFill) my_first = t0 + tid * kScanPerThread + k;
+        // (not one per block, which serialised on the one address)
         const uint64_t has = __ballot(my_first != 0xffffffffu);
         if (has != 0ull && lane == __ffsll((unsigned long long)has) - 1) atomicMin(&first_past, my_first);
         __syncthreads();
-        const uint32_t stop = first_past;
+        const uint32_t stop = first_past == 0xffffffffu ? first_past : first_past + 1u;
         uint32_t mine = 0;
 #pragma unroll
         for (int k = 0; k < kScanPerThread; ++k) {
@@ -512,10 +476,14 @@ __global__ void __launch_bounds__(kScanThreads)
             // walk the fill block's rays: first ray whose inclusive prefix passes total_samples
             const uint32_t b = fill_block < scanned ? fill_block : scanned - 1;  // set whenever grand > S
             uint64_t pre = block_slots[(size_t)b * kRaysPerBlock];
-            const uint32_t first = b * kRaysPerBlock, last = min(n_rays, first + kRaysPerBlock);
+            const uint32_t first = b * kRaysPerBlock, last = min(n_rays - first, (uint32_t)kRaysPerBlock);
+            uint32_t cnt[kRaysPerBlock];
+#pragma unroll
+            for (uint32_t j = 0; j < kRaysPerBlock; ++j) cnt[j] = j < last ? rays_n_samples[first + j] : 0u;
             uint32_t measured = (uint32_t)pre, over = 0;
-            for (uint32_t r = first; r < last; ++r) {
-                const uint32_t n = rays_n_samples[r];
+#pragma unroll
+            for (uint32_t j = 0; j < kRaysPerBlock; ++j) {
+                const uint32_t n = cnt[j];
                 if (pre + n > total_samples) {
                     measured = (uint32_t)pre;
                     over = pre < total_samples ? n : 0;
@@ -540,7 +508,7 @@ __device__ __forceinline__ uint64_t ray_start(const uint32_t *__restrict__ rays_
 }
 
 // Wavefront per ray, grid-stride over rays: writes the t of every valid ray's
-// samples to z_vals at the ray's range, copied from its t record, or marched again
+// samples to z_vals at the ray's range, made from its record, or marched again
 // where it has none.  Stops at the first ray whose block prefix reaches
 // total_samples (every later ray is past the filled buffer).  Runs before
 // march_finish_kernel overwrites the block slots.
@@ -548,8 +516,8 @@ __global__ void __launch_bounds__(kBlock)
     march_emit_kernel(MarchParams p, bool word_ok, uint32_t n_rays, uint32_t total_samples,
                       const float *__restrict__ rays_o, const float *__restrict__ rays_d,
                       const float *__restrict__ t_starts, const float *__restrict__ t_ends,
-                      const float *__restrict__ noises, const uint8_t *__restrict__ bits, TStore store,
-                      uint32_t n_recorded, const uint32_t *__restrict__ rays_n_samples,
+                      const float *__restrict__ noises, const uint8_t *__restrict__ bits, RecordStore records,
+                      const uint32_t *__restrict__ rays_n_samples,
                       const uint32_t *__restrict__ block_slots, float *__restrict__ zs) {
     const uint32_t n_waves = gridDim.x * kRaysPerBlock;
     for (uint32_t i = blockIdx.x * kRaysPerBlock + threadIdx.x / kWave; i < n_rays; i += n_waves) {
@@ -559,13 +527,24 @@ __global__ void __launch_bounds__(kBlock)
         const float t0 = t_starts[i], t1 = t_ends[i];
         if (start < total_samples && t1 > t0 && start + n <= total_samples && n > 0) {
             const uint32_t s = (uint32_t)start;
-            const float *rec = i < n_recorded && n <= store.slot ? t_record(store, i) : nullptr;
-            if (rec != nullptr) {
-                for (uint32_t k = lane_id(); k < n; k += kWave) zs[s + k] = rec[k];
+            const RayRecord rec = record_of(records, i);
+            const uint32_t windows = rec.words != nullptr ? rec.words[0] : kNoRecord;
+            if (windows != kNoRecord) {
+                uint32_t k = s;
+                for (uint32_t j = 0; j < windows; ++j) {
+                    const uint32_t *e = rec.words + 1 + 3 * j;
+                    const uint64_t mask = (uint64_t)e[2] << 32 | e[1];
+                    float w, next;
+                    bool stall;
+                    chain_window(p, p.portion == 0.0f, step_size(p, 0.0f), __uint_as_float(e[0]), w, next, stall);
+                    const int lane = lane_id();
+                    if ((mask >> lane) & 1ull) zs[k + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = w;
+                    k += (uint32_t)__popcll(mask);
+                }
             } else {
                 const Ray r = load_ray(rays_o, rays_d, i, t1);
                 march_ray_wave<true>(p, bits, word_ok, r, start_t(p, t0, noises[i]), min(p.n_cap, n),
-                                     RaySamples{zs + s, 0xffffffffu});
+                                     RaySamples{zs + s}, RayRecord{nullptr, 0u});
             }
         }
     }
@@ -863,47 +842,35 @@ extern "C" void march_rays(ngp_stream_t stream_, void **buffers, const char *opa
         return;
     }
     const uint32_t n_blocks = div_up(d.n_rays, kRaysPerBlock);
-    // count in ray-ordered launches of 2048, 16384, 131072 and all rays; grids
-    // of at most kMaxCountBlocks blocks (8192 resident wavefronts) stride over them
     constexpr uint32_t kMaxCountBlocks = 2048;
-    const uint32_t bounds[5] = {0, std::min(n_blocks, 2048u / kRaysPerBlock),
-                                std::min(n_blocks, 16384u / kRaysPerBlock), std::min(n_blocks, 131072u / kRaysPerBlock),
-                                n_blocks};
-    // t records of the first launch's rays in the sample outputs (8 floats per slot)
-    const uint32_t n_first = std::min(d.n_rays, bounds[1] * kRaysPerBlock);
-    TStore store{};
-    store.slot = (uint32_t)std::min<uint64_t>(p.n_cap, 8ull * d.total_samples / n_first);
-    {
-        float *region[4] = {xyzs, dirs, dss, (float *)idcs};
-        const uint64_t floats[4] = {3ull * d.total_samples, 3ull * d.total_samples, d.total_samples, d.total_samples};
-        uint32_t first = 0;
-        for (int q = 0; q < 4; ++q) {
-            store.region[q] = region[q];
-            store.first[q] = first;
-            const uint64_t fit = store.slot ? floats[q] / store.slot : 0;
-            first = (uint32_t)std::min<uint64_t>(n_first, first + fit);
-        }
-        store.first[4] = first;
-    }
-    for (int c = 0; c < 4; ++c) {
-        if (bounds[c + 1] <= bounds[c]) continue;
-        const dim3 grid(std::min(bounds[c + 1] - bounds[c], kMaxCountBlocks));
-        if (c == 0)
-            hipLaunchKernelGGL(march_count_kernel<true>, grid, dim3(kBlock), 0, stream, p, word_ok, d.n_rays,
-                               d.total_samples, bounds[c], bounds[c + 1], rays_o, rays_d, t_starts, t_ends, noises,
-                               bits, store, n_samples, startidx);
-        else
-            hipLaunchKernelGGL(march_count_kernel<false>, grid, dim3(kBlock), 0, stream, p, word_ok, d.n_rays,
-                               d.total_samples, bounds[c], bounds[c + 1], rays_o, rays_d, t_starts, t_ends, noises,
-                               bits, store, n_samples, startidx);
+    hipLaunchKernelGGL(march_begin_kernel, dim3(std::min(div_up(d.n_rays, kBlock), 2048u)), dim3(kBlock), 0, stream,
+                       d.n_rays, n_samples, startidx);
+    if (!check_launch(target)) return;
+    // records of the first rays in xyzs: a ray across the bound's diagonal, one that starts
+    // and ends inside a window, has at most n_cap / 64 + 2 windows
+    RecordStore rec;
+    rec.base = (uint32_t *)xyzs;
+    rec.words = 1u + 3u * (std::min(p.n_cap, 1u << 16) / kWave + 2u);
+    rec.n = (uint32_t)std::min<uint64_t>(d.n_rays, 3ull * d.total_samples / rec.words);
+    // the first rays, which fill a training batch, in rounds of 2048, the rest in rounds of
+    // 8192 (every ray of a sparse field is marched: more wavefronts, more throughput)
+    constexpr uint32_t kFirstBlocks = 512, kFirstRounds = 8;
+    const uint32_t first_end = std::min(n_blocks, kFirstBlocks * kFirstRounds);
+    for (int c = 0; c < 2; ++c) {
+        const uint32_t begin = c == 0 ? 0 : first_end, end = c == 0 ? first_end : n_blocks;
+        if (end <= begin) continue;
+        hipLaunchKernelGGL(march_count_kernel, dim3(std::min(end - begin, c == 0 ? kFirstBlocks : kMaxCountBlocks)),
+                           dim3(kBlock), 0, stream, p, word_ok, d.n_rays, d.total_samples, begin, end,
+                           c == 0 ? 0 : kFirstRounds, rays_o, rays_d, t_starts, t_ends, noises, bits, rec, n_samples,
+                           startidx);
         if (!check_launch(target)) return;
     }
     hipLaunchKernelGGL(march_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, d.n_rays, n_blocks, d.total_samples,
                        n_samples, startidx, next_loc, exceeded);
     if (!check_launch(target)) return;
     hipLaunchKernelGGL(march_emit_kernel, dim3(std::min(n_blocks, kMaxCountBlocks)), dim3(kBlock), 0, stream, p, word_ok,
-                       d.n_rays, d.total_samples, rays_o, rays_d, t_starts, t_ends, noises, bits, store,
-                       store.first[4], n_samples, startidx, zs);
+                       d.n_rays, d.total_samples, rays_o, rays_d, t_starts, t_ends, noises, bits, rec,
+                       n_samples, startidx, zs);
     if (!check_launch(target)) return;
     hipLaunchKernelGGL(march_fill_kernel, dim3(std::min(n_blocks, kMaxCountBlocks)), dim3(kBlock), 0, stream, p,
                        d.n_rays, d.total_samples, rays_o, rays_d, t_starts, t_ends, n_samples, startidx, zs, idcs, xyzs,

@@ -24,6 +24,15 @@ __device__ __forceinline__ uint32_t morton_spread(uint32_t v) {
 __device__ __forceinline__ uint32_t morton3(uint32_t x, uint32_t y, uint32_t z) {
     return morton_spread(x) | (morton_spread(y) << 1) | (morton_spread(z) << 2);
 }
+// The same for coordinates below 1024, where the products never carry and are
+// v | v << k: one full-rate instruction instead of a multiply at a quarter of the rate.
+__device__ __forceinline__ uint32_t morton_spread10(uint32_t v) {
+    v = (v | v << 16) & 0xFF0000FFu;
+    v = (v | v << 8) & 0x0F00F00Fu;
+    v = (v | v << 4) & 0xC30C30C3u;
+    v = (v | v << 2) & 0x49249249u;
+    return v;
+}
 // Keep every third bit and compact (marching.cu:70-77).
 __device__ __forceinline__ uint32_t morton_compact(uint32_t x) {
     x = x & 0x49249249u;
@@ -145,7 +154,8 @@ __device__ __forceinline__ uint32_t cell_index(const MarchParams &p, float px, f
     uint32_t ix = (uint32_t)fminf(fmaxf(floorf(gx), 0.0f), gmax);
     uint32_t iy = (uint32_t)fminf(fmaxf(floorf(gy), 0.0f), gmax);
     uint32_t iz = (uint32_t)fminf(fmaxf(floorf(gz), 0.0f), gmax);
-    return cascade * p.G3 + morton3(ix, iy, iz);
+    // (coordinates below G <= 1024)
+    return cascade * p.G3 + (morton_spread10(ix) | (morton_spread10(iy) << 1) | (morton_spread10(iz) << 2));
 }
 
 // Occupancy lookup of one position through the ray's bit cache.

@@ -113,7 +113,8 @@ def march_rays(
          dss, z_vals],
         _lib.marching_descriptor(n_rays, S, diagonal_n_steps, K, G, float(bound), float(stepsize_portion)),
     )
-    measured = (_u32_to_i64(next_loc) - _u32_to_i64(exceeded))[0].to(torch.int32).view(u32)
+    # modulo 2^32 the 32-bit difference is the unsigned one: one launch
+    measured = (next_loc.view(torch.int32) - exceeded.view(torch.int32))[0].view(u32)
     return measured, valid, n_samples, startidx, idcs, xyzs, dirs, dss, z_vals
 
 
