@@ -128,20 +128,31 @@ def _check() -> None:
 
 
 def current_stream(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw handle of the current stream of `device` (None: the current device).
+    Read without building a torch Stream object, which cost 2 us of a 20 us call."""
+    index = None if device is None else device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+_ptr_arrays: dict = {}  # n -> the ctypes type of an array of n pointers
 
 
 def call(name: str, tensors: Sequence[torch.Tensor], opaque: bytes, stream: int | None = None) -> None:
     """Calls target `name` with device tensors (operands then results)."""
-    for i, t in enumerate(tensors):
+    ptrs = []
+    for t in tensors:
         if not t.is_cuda:
-            raise ValueError(f"{name}: buffer {i} is not a device tensor")
+            raise ValueError(f"{name}: buffer {len(ptrs)} is not a device tensor")
         if not t.is_contiguous():
-            raise ValueError(f"{name}: buffer {i} is not contiguous")
-    ptrs = (ctypes.c_void_p * max(1, len(tensors)))(*[t.data_ptr() for t in tensors])
+            raise ValueError(f"{name}: buffer {len(ptrs)} is not contiguous")
+        ptrs.append(t.data_ptr())
+    n = len(ptrs) or 1
+    array = _ptr_arrays.get(n)
+    if array is None:
+        array = _ptr_arrays[n] = ctypes.c_void_p * n
     if stream is None:
-        stream = current_stream(tensors[0].device if tensors else None)
-    target(name)(ctypes.c_void_p(stream), ptrs, opaque, len(opaque))
+        stream = current_stream(tensors[0].device if ptrs else None)
+    (_targets.get(name) or target(name))(stream, array(*ptrs), opaque, len(opaque))
     _check()
 
 

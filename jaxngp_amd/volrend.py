@@ -209,6 +209,7 @@ class _IntegrateRays(torch.autograd.Function):
         ctx.save_for_backward(*ins, rgbds, opac)
         ctx.near_distance = float(near_distance)
         ctx.mark_non_differentiable(measured)
+        ctx.set_materialize_grads(False)  # no zeros launched for outputs without a gradient
         return measured, rgbds, opac
 
     @staticmethod
