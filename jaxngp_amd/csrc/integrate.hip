@@ -21,17 +21,6 @@ constexpr int kBlock = 256;
 
 __global__ void zero_u32_kernel(uint32_t *p) { *p = 0u; }
 
-__global__ void fill_zero_kernel(float *__restrict__ a, size_t n) {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) a[j] = 0.0f;
-}
-
-__global__ void fill_zero4_kernel(float4 *__restrict__ a, size_t n4) {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < n4; j += stride)
-        a[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-}
-
 // Samples of a ray that lie inside the sample arrays.  Ranges produced by
 // march_rays always do; a range running past total_samples is cut there instead of
 // reading out of bounds.
@@ -390,39 +379,39 @@ inline uint32_t wave_grid(uint32_t n_rays) {
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-void zero_floats(float *p, size_t n, hipStream_t stream) {
-    if (n == 0) return;
-    if (aligned16(p) && (n & 3u) == 0) {
-        size_t n4 = n / 4;
-        uint32_t grid = (uint32_t)std::min<size_t>((n4 + 255) / 256, 8192);
-        hipLaunchKernelGGL(fill_zero4_kernel, dim3(grid), dim3(256), 0, stream, reinterpret_cast<float4 *>(p), n4);
-    } else {
-        uint32_t grid = (uint32_t)std::min<size_t>((n + 255) / 256, 8192);
-        hipLaunchKernelGGL(fill_zero_kernel, dim3(grid), dim3(256), 0, stream, p, n);
-    }
+// Clears two 4-byte aligned buffers with one launch (a launch and its gap cost more than
+// the few MB cleared): whole float4s of each from its first 16-byte boundary on, and the
+// up to three floats before and after them.
+struct ZeroRange {
+    float *p;
+    size_t n;
+    uint32_t head;  // floats before the first 16-byte boundary
+};
+
+__device__ __forceinline__ void zero_range(const ZeroRange &r, size_t first, size_t stride) {
+    const size_t n4 = (r.n - r.head) / 4, tail = r.head + 4 * n4;
+    float4 *const v = reinterpret_cast<float4 *>(r.p + r.head);
+    for (size_t j = first; j < n4; j += stride) v[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (first < r.head) r.p[first] = 0.0f;
+    if (first < r.n - tail) r.p[tail + first] = 0.0f;
 }
 
-// Clears two buffers with one launch when both are float4-aligned (a launch and
-// its gap cost more than the few MB cleared), else one launch each.
-__global__ void fill_zero4x2_kernel(float4 *__restrict__ a, size_t na4, float4 *__restrict__ b, size_t nb4) {
+__global__ void fill_zero2_kernel(ZeroRange a, ZeroRange b) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < na4 + nb4; j += stride) {
-        if (j < na4) a[j] = z;
-        else b[j - na4] = z;
-    }
+    const size_t first = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    zero_range(a, first, stride);
+    zero_range(b, first, stride);
+}
+
+ZeroRange zero_range_of(float *p, size_t n) {
+    const uint32_t head = (uint32_t)((16u - (reinterpret_cast<uintptr_t>(p) & 15u)) & 15u) / 4u;
+    return ZeroRange{p, n, (uint32_t)std::min<size_t>(head, n)};
 }
 
 void zero_floats2(float *a, size_t na, float *b, size_t nb, hipStream_t stream) {
-    if (aligned16(a) && aligned16(b) && (na & 3u) == 0 && (nb & 3u) == 0 && na + nb > 0) {
-        const size_t n4 = (na + nb) / 4;
-        const uint32_t grid = (uint32_t)std::min<size_t>((n4 + 255) / 256, 8192);
-        hipLaunchKernelGGL(fill_zero4x2_kernel, dim3(grid), dim3(256), 0, stream, reinterpret_cast<float4 *>(a),
-                           na / 4, reinterpret_cast<float4 *>(b), nb / 4);
-    } else {
-        zero_floats(a, na, stream);
-        zero_floats(b, nb, stream);
-    }
+    if (na + nb == 0) return;
+    const uint32_t grid = (uint32_t)std::max<size_t>(1, std::min<size_t>((std::max(na, nb) / 4 + 255) / 256, 8192));
+    hipLaunchKernelGGL(fill_zero2_kernel, dim3(grid), dim3(256), 0, stream, zero_range_of(a, na), zero_range_of(b, nb));
 }
 
 }  // namespace
