@@ -289,7 +289,8 @@ struct BwdPlan {
     uint32_t run_part;     // entries one workgroup of the reducer sums
     uint32_t group_shift;  // log2 of the slices in kSliceBytes
     uint32_t s_lo[NGP_HASHGRID_MAX_LEVELS], s_hi[NGP_HASHGRID_MAX_LEVELS];
-    uint64_t runs_off, slice_np_off, rows_off, part_group_off;
+    uint64_t runs_off, slice_np_off, first_part_off, split_off, rows_off, part_group_off;
+    bool whole;  // no slice can be cut into parts
 };
 
 // Rows of one slice: R rows of F f64 accumulators fill kSliceBytes of LDS.  A power
@@ -334,12 +335,30 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         const uint64_t mean = (uint64_t)d.n_points * 8 * p.R / d.T;
         p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 4 + 1023) / 1024 * 1024));
         p.group_shift = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
-        p.max_parts = (uint32_t)(p.n_slices + max_entries / p.run_part + (max_entries << p.group_shift) / kPart);
+        // Few points: even all contributions of all levels that share a group of slices
+        // make one part, so nothing is counted, cut or combined: two launches, not four
+        // (2000 ray samples f32: 35 -> 26 us; the line is where a group could be cut, and
+        // with every point in a fifth of the box 4000 points take 73 us on either side).
+        uint32_t sharing = 0;
+        for (uint32_t l = 0; l < d.L; ++l) {
+            uint32_t n = 0;
+            for (uint32_t k = 0; k < d.L; ++k)
+                n += (p.s_lo[k] >> p.group_shift) <= (p.s_lo[l] >> p.group_shift) &&
+                     (p.s_hi[k] >> p.group_shift) >= (p.s_lo[l] >> p.group_shift);
+            sharing = std::max(sharing, n);
+        }
+        p.whole = (uint64_t)d.n_points * 8 * sharing <= kPart;
+        // parts of cut slices: a slice is cut where it holds more than run_part entries or
+        // its group more than kPart, so its parts are fewer than twice the quotients, and
+        // at most one more than they are
+        const uint64_t cuts = max_entries / p.run_part + (max_entries << p.group_shift) / kPart + 2;
+        p.max_parts = p.whole ? 0 : (uint32_t)(cuts + std::min<uint64_t>(cuts, p.n_slices));
         p.runs_off = 0;
         p.slice_np_off = align(p.runs_off + 4 * runs);
-        p.meta_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
-        p.parts_off = align(p.meta_off + 8);
-        p.part_slice_off = align(p.parts_off + 4 * ((uint64_t)p.n_slices + 1));
+        p.first_part_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
+        p.split_off = align(p.first_part_off + 4 * (uint64_t)p.n_slices);
+        p.meta_off = align(p.split_off + 4 * (uint64_t)p.n_slices);  // [0] parts, [1] cut slices
+        p.part_slice_off = align(p.meta_off + 8);
         p.partials_off = align(p.part_slice_off + 4 * (uint64_t)p.max_parts);
         p.part_group_off = align(p.partials_off + (uint64_t)p.max_parts * p.R * d.F * 8);
         p.entries_off = align(p.part_group_off + 4 * (uint64_t)p.max_parts);
@@ -699,7 +718,8 @@ template <int F, bool kHalf, uint32_t R>
 __global__ void __launch_bounds__(kBucketThreads)
     bwd_bucket_kernel(HashGridDescriptor d, BwdPlan p, const float *__restrict__ pos,
                       const float *__restrict__ dL_denc, uint32_t *__restrict__ runs_out,
-                      EntryValue<F, kHalf> *__restrict__ values, uint16_t *__restrict__ rows_out) {
+                      EntryValue<F, kHalf> *__restrict__ values, uint16_t *__restrict__ rows_out,
+                      uint32_t *__restrict__ meta) {
     typedef EntryValue<F, kHalf> Value;
     constexpr int kBucketPhases = bucket_phases(kHalf);
     constexpr uint32_t kBucketPoints = bucket_points(kHalf), kBucketEntries = bucket_entries(kHalf);
@@ -710,6 +730,7 @@ __global__ void __launch_bounds__(kBucketThreads)
     __shared__ __align__(16) Value stage_v[kStageEntries];
     __shared__ __align__(16) uint16_t stage_r[kStageEntries];
     const uint32_t item = blockIdx.x;
+    if (item == 0 && threadIdx.x < 2) meta[threadIdx.x] = 0u;  // for bwd_slice_parts_kernel
     const uint32_t l = item / p.n_bchunks, k = item % p.n_bchunks;
     const uint32_t s_lo = p.s_lo[l];
     const uint32_t span = p.s_hi[l] - s_lo + 1u;  // <= kStageSlices (host check)
@@ -864,11 +885,14 @@ __device__ __forceinline__ uint32_t slice_run_length(const BwdPlan &p, const uin
     return s < p.s_lo[l] || s > p.s_hi[l] ? 0u : run_length(runs[run_index(p, l, s - p.s_lo[l], k)]);
 }
 
-// One-pass table gradient, part 2: parts of slice s, from the run lengths of every item
-// whose level reaches s or the other slice of its group.
+// One-pass table gradient, part 2: the number of parts of slice s, from the run lengths of
+// every item whose level reaches s or the other slice of its group, and for a slice of
+// several a slot for each and its place in the list of cut slices.
 __global__ void __launch_bounds__(256)
     bwd_slice_parts_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ runs,
-                           uint32_t *__restrict__ slice_np) {
+                           uint32_t *__restrict__ meta, uint32_t *__restrict__ slice_np,
+                           uint32_t *__restrict__ first_part, uint32_t *__restrict__ part_slice,
+                           uint32_t *__restrict__ split) {
     const uint32_t s = blockIdx.x, other = p.group_shift ? s ^ 1u : s;
     uint32_t own = 0, both = 0;
     for (uint32_t l = 0; l < d.L; ++l) {
@@ -895,31 +919,14 @@ __global__ void __launch_bounds__(256)
             t += ws[0][w];
             g += ws[1][w];
         }
-        slice_np[s] = n_cuts(t, p.run_part) + n_cuts(g, kPart) - 1u;
-    }
-}
-
-// One-pass table gradient, part 3 (one workgroup): prefix of the parts per slice and
-// the slice of every part; parts[n_slices] and meta[1] hold the total.
-__global__ void __launch_bounds__(kScanThreads) bwd_bucket_plan_kernel(BwdPlan p, const uint32_t *__restrict__ slice_np,
-                                                                       uint32_t *__restrict__ meta,
-                                                                       uint32_t *__restrict__ parts,
-                                                                       uint32_t *__restrict__ part_slice) {
-    uint32_t carry = 0;
-    for (uint32_t c = 0; c < p.n_slices; c += kScanThreads) {
-        const uint32_t s = c + threadIdx.x;
-        const uint32_t k = s < p.n_slices ? slice_np[s] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_exclusive_scan<kScanThreads>(k, &tot);
-        if (s < p.n_slices) {
-            parts[s] = carry + ex;
-            for (uint32_t j = 0; j < k; ++j) part_slice[carry + ex + j] = s;
+        const uint32_t n = n_cuts(t, p.run_part) + n_cuts(g, kPart) - 1u;
+        slice_np[s] = n;
+        if (n > 1) {  // which slot a part gets does not matter to its sums
+            const uint32_t at = atomicAdd(meta, n);
+            first_part[s] = at;
+            for (uint32_t j = 0; j < n; ++j) part_slice[at + j] = s;
+            split[atomicAdd(meta + 1, 1u)] = s;
         }
-        carry += tot;
-    }
-    if (threadIdx.x == 0) {
-        parts[p.n_slices] = carry;
-        meta[1] = carry;
     }
 }
 
@@ -999,21 +1006,23 @@ __global__ void __launch_bounds__(kReduceThreads)
     for (uint32_t t = threadIdx.x; t < rows * F; t += kReduceThreads) out[t] = (float)acc[(t % F) * p.R + t / F];
 }
 
-// One-pass table gradient, part 4: workgroup b sums part b of slice s, as
-// bwd_reduce_kernel does, from the runs of the items whose level reaches s.  The LDS
-// atomics set the time (about 31 cycles of a CU per 64-lane f64 add, however many of its
-// lanes are masked off), so a wavefront reads its runs as one sequence with every lane
-// filled: lane i of wavefront w loads the run of item w + i * kWaves, a prefix sum of the
-// lengths places the runs in the sequence, and 64 entries at a time find their runs by
+// One-pass table gradient, part 3: a workgroup sums one part of slice s, as
+// bwd_reduce_kernel does, from the runs of the items whose level reaches s.  The first
+// kSplitBlocks workgroups take the parts of cut slices, the others a whole slice each.
+// The LDS atomics set the time (about 31 cycles of a CU per 64-lane f64 add, however many
+// of its lanes are masked off), so a wavefront reads its runs as one sequence with every
+// lane filled: lane i of wavefront w loads the run of item w + i * kWaves, a prefix sum of
+// the lengths places the runs in the sequence, and 64 entries at a time find their runs by
 // pushing each run's lane number to the lane of its first entry and a running maximum
 // (RunSequence).  kSteps such groups are loaded before the previous ones are added.  A
-// slice of one part (nearly all of them) needs no barrier between its runs; a slice of
-// several parts first finds its items by the prefixes of their run lengths (see n_cuts).
+// whole slice (nearly all of them) needs no barrier between its runs; a part of a cut
+// slice first finds its items by the prefixes of their run lengths (see n_cuts).
 // With kAdam, a slice summed in one part is not stored: its rows take the optimizer
 // step in place (params, m, v), and bwd_combine_runs does the same for the others.
-// 2^18 ray samples, f32: 82 -> 62 us, of which the atomics themselves need 27 (34 M f64
+// 2^18 ray samples, f32: 82 -> 65 us, of which the atomics themselves need 27 (34 M f64
 // adds at 1.27 T/s); slices of 64 KiB, two workgroups to a CU, so that one clears or
-// stores its rows while the other adds (128 KiB slices: 80 us); 1,024 points: 29 -> 18.
+// stores its rows while the other adds (128 KiB slices: 80 us); 1,024 points: 29 -> 17.
+// All four parts: f32 190 -> 147 us, f16 176 -> 129; 1,024 points, two parts: 44 -> 28.
 struct RunSequence {
     uint32_t *marks;        // 64 words of LDS of the wavefront's own, tags below `tag`
     uint32_t tag;           // of the latest group of 64 places
@@ -1086,15 +1095,15 @@ struct EntryGroup {
     }
 };
 
-template <int F, bool kHalf, uint32_t R, bool kAdam = false>
-__global__ void __launch_bounds__(kRunThreads)
-    bwd_reduce_runs_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ meta,
-                           const uint32_t *__restrict__ parts, const uint32_t *__restrict__ part_slice,
-                           const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
-                           const uint16_t *__restrict__ entry_rows, double *__restrict__ partials,
-                           uint32_t *__restrict__ part_group, float *__restrict__ dtable, AdamStep adam = {},
-                           float *__restrict__ adam_p = nullptr, float *__restrict__ adam_m = nullptr,
-                           float *__restrict__ adam_v = nullptr) {
+constexpr uint32_t kSplitBlocks = 512;  // two to a CU
+
+template <int F, bool kHalf, uint32_t R, bool kAdam>
+__device__ __forceinline__ void
+reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t part, uint32_t n_parts, uint32_t slot,
+            const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
+            const uint16_t *__restrict__ entry_rows, double *__restrict__ partials, uint32_t *__restrict__ part_group,
+            float *__restrict__ dtable, const AdamStep &adam, float *__restrict__ adam_p, float *__restrict__ adam_m,
+            float *__restrict__ adam_v) {
     typedef EntryGroup<F, kHalf> Group;
     constexpr uint32_t kBucketEntries = bucket_entries(kHalf);
     constexpr uint32_t kWaves = kRunThreads / kWave;
@@ -1102,11 +1111,6 @@ __global__ void __launch_bounds__(kRunThreads)
     __shared__ uint32_t chosen[kRunThreads];
     __shared__ uint32_t my_group;
     __shared__ uint32_t marks[kWaves][kWave];
-    const uint32_t b = blockIdx.x;
-    if (b >= meta[1]) return;
-    const uint32_t s = part_slice[b];
-    const uint32_t part = b - parts[s];
-    const uint32_t n_parts = parts[s + 1] - parts[s];
     const uint32_t rows = min(d.n_rows - s * R, R);
     for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) reinterpret_cast<double2 *>(acc)[t] = double2{0.0, 0.0};
     __syncthreads();
@@ -1177,8 +1181,8 @@ __global__ void __launch_bounds__(kRunThreads)
         return;
     }
     if (n_parts > 1) {
-        if (threadIdx.x == 0) part_group[b] = my_group;
-        double2 *out = reinterpret_cast<double2 *>(partials + (size_t)b * R * F);
+        if (threadIdx.x == 0) part_group[slot] = my_group;
+        double2 *out = reinterpret_cast<double2 *>(partials + (size_t)slot * R * F);
         for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) out[t] = reinterpret_cast<const double2 *>(acc)[t];
         return;
     }
@@ -1192,43 +1196,90 @@ __global__ void __launch_bounds__(kRunThreads)
     }
 }
 
-// One-pass table gradient, part 5: slices of several parts.  Block (s, c) covers
-// 1 / kCombineSplit of slice s's rows.  With kAdam the sums are not stored: the rows take
+template <int F, bool kHalf, uint32_t R, bool kAdam>
+__global__ void __launch_bounds__(kRunThreads)
+    bwd_reduce_runs_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ meta,
+                           const uint32_t *__restrict__ slice_np, const uint32_t *__restrict__ first_part,
+                           const uint32_t *__restrict__ part_slice, const uint32_t *__restrict__ runs,
+                           const EntryValue<F, kHalf> *__restrict__ values, const uint16_t *__restrict__ entry_rows,
+                           double *__restrict__ partials, uint32_t *__restrict__ part_group,
+                           float *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
+                           float *__restrict__ adam_m, float *__restrict__ adam_v) {
+    uint32_t s = blockIdx.x;
+    if (!p.whole) {
+        if (blockIdx.x < kSplitBlocks) {
+            const uint32_t n = meta[0];
+            for (uint32_t i = blockIdx.x; i < n; i += kSplitBlocks) {
+                const uint32_t cut = part_slice[i];
+                reduce_part<F, kHalf, R, kAdam>(d, p, cut, i - first_part[cut], slice_np[cut], i, runs, values, entry_rows,
+                                                partials, part_group, dtable, adam, adam_p, adam_m, adam_v);
+                __syncthreads();  // the sums are read out
+            }
+            return;
+        }
+        s -= kSplitBlocks;
+        if (slice_np[s] != 1) return;
+    }
+    reduce_part<F, kHalf, R, kAdam>(d, p, s, 0, 1, 0, runs, values, entry_rows, partials, part_group, dtable, adam,
+                                    adam_p, adam_m, adam_v);
+}
+
+// One-pass table gradient, part 4: slices of several parts, in pieces of
+// 1 / kCombineSplit of a slice's rows.  With kAdam the sums are not stored: the rows take
 // the optimizer step in place.
 constexpr uint32_t kCombineSplit = 16;
 template <int F, uint32_t R, bool kAdam>
 __global__ void __launch_bounds__(256)
-    bwd_combine_runs_kernel(HashGridDescriptor d, const uint32_t *__restrict__ parts,
-                            const double *__restrict__ partials, const uint32_t *__restrict__ part_group,
-                            float *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
-                            float *__restrict__ adam_m, float *__restrict__ adam_v) {
-    const uint32_t s = blockIdx.x;
-    const uint32_t p0 = parts[s], n_parts = parts[s + 1] - p0;
-    if (n_parts <= 1) return;
-    const uint32_t rows = min(d.n_rows - s * R, R);
+    bwd_combine_runs_kernel(HashGridDescriptor d, const uint32_t *__restrict__ meta,
+                            const uint32_t *__restrict__ slice_np, const uint32_t *__restrict__ first_part,
+                            const uint32_t *__restrict__ split, const double *__restrict__ partials,
+                            const uint32_t *__restrict__ part_group, float *__restrict__ dtable, AdamStep adam,
+                            float *__restrict__ adam_p, float *__restrict__ adam_m, float *__restrict__ adam_v) {
     constexpr uint32_t kPer = R * F / kCombineSplit;
-    // feature f of row r is value f * R + r of a part
-    for (uint32_t t = blockIdx.y * kPer + threadIdx.x; t < (blockIdx.y + 1) * kPer; t += 256) {
-        const uint32_t f = t / R, r = t % R;
-        if (r >= rows) continue;
-        float sum = 0.0f;
-        double in_group = 0.0;
-        uint32_t group = 0xffffffffu;
-        for (uint32_t q = 0; q < n_parts; ++q) {
-            const uint32_t g = part_group[p0 + q];
-            if (g == 0xffffffffu) continue;  // no item: both cuts moved on together
-            if (g != group) sum += (float)in_group, in_group = 0.0, group = g;
-            in_group += partials[(size_t)(p0 + q) * R * F + t];
-        }
-        sum += (float)in_group;
-        const size_t o = ((size_t)s * R + r) * F + f;
-        if constexpr (kAdam) {
-            float mk = adam_m[o], vk = adam_v[o];
-            adam_p[o] = adam_step(adam, adam_p[o], sum, mk, vk);
-            adam_m[o] = mk;
-            adam_v[o] = vk;
-        } else {
-            dtable[o] = sum;
+    constexpr uint32_t kBatch = 8;  // partial rows in flight per thread
+    const uint32_t n_tasks = meta[1] * kCombineSplit;
+    for (uint32_t task = blockIdx.x; task < n_tasks; task += gridDim.x) {
+        const uint32_t s = split[task / kCombineSplit], piece = task % kCombineSplit;
+        const uint32_t p0 = first_part[s], n_parts = slice_np[s];
+        const uint32_t rows = min(d.n_rows - s * R, R);
+        // feature f of row r is value f * R + r of a part
+        for (uint32_t t = piece * kPer + threadIdx.x; t < (piece + 1) * kPer; t += 256) {
+            const uint32_t f = t / R, r = t % R;
+            if (r >= rows) continue;
+            float sum = 0.0f;
+            double in_group = 0.0;
+            uint32_t group = 0xffffffffu;
+            for (uint32_t q0 = 0; q0 < n_parts; q0 += kBatch) {
+                double v[kBatch];
+                uint32_t g[kBatch];
+#pragma unroll
+                for (uint32_t j = 0; j < kBatch; ++j) {
+                    const uint32_t q = p0 + min(q0 + j, n_parts - 1u);
+                    g[j] = part_group[q];
+                    v[j] = partials[(size_t)q * R * F + t];
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < kBatch; ++j) {
+                    // 0xffffffff: a part without items (both cuts moved on together)
+                    if (q0 + j >= n_parts || g[j] == 0xffffffffu) continue;
+                    if (g[j] != group) {
+                        sum += (float)in_group;
+                        in_group = 0.0;
+                        group = g[j];
+                    }
+                    in_group += v[j];
+                }
+            }
+            sum += (float)in_group;
+            const size_t o = ((size_t)s * R + r) * F + f;
+            if constexpr (kAdam) {
+                float mk = adam_m[o], vk = adam_v[o];
+                adam_p[o] = adam_step(adam, adam_p[o], sum, mk, vk);
+                adam_m[o] = mk;
+                adam_v[o] = vk;
+            } else {
+                dtable[o] = sum;
+            }
         }
     }
 }
@@ -1302,40 +1353,36 @@ bool reserve_lds(K kernel, size_t lds, const char *target) {
 template <int F, bool kHalf, uint32_t R>
 bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStream_t stream, const float *pos,
                           const float *g, float *dtable, uint8_t *ws, const char *target, const FusedAdam *fused) {
-    uint32_t *runs = reinterpret_cast<uint32_t *>(ws + p.runs_off);
-    uint32_t *slice_np = reinterpret_cast<uint32_t *>(ws + p.slice_np_off);
-    uint32_t *meta = reinterpret_cast<uint32_t *>(ws + p.meta_off);
-    uint32_t *parts = reinterpret_cast<uint32_t *>(ws + p.parts_off);
-    uint32_t *part_slice = reinterpret_cast<uint32_t *>(ws + p.part_slice_off);
+    auto word = [&](uint64_t off) { return reinterpret_cast<uint32_t *>(ws + off); };
+    uint32_t *runs = word(p.runs_off), *meta = word(p.meta_off), *slice_np = word(p.slice_np_off);
+    uint32_t *first_part = word(p.first_part_off), *split = word(p.split_off), *part_slice = word(p.part_slice_off);
+    uint32_t *part_group = word(p.part_group_off);
     double *partials = reinterpret_cast<double *>(ws + p.partials_off);
-    uint32_t *part_group = reinterpret_cast<uint32_t *>(ws + p.part_group_off);
     auto *values = reinterpret_cast<EntryValue<F, kHalf> *>(ws + p.entries_off);
     uint16_t *entry_rows = reinterpret_cast<uint16_t *>(ws + p.rows_off);
     const size_t lds = (size_t)R * F * sizeof(double);
-    const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, false>;
-    const auto reduce_adam = bwd_reduce_runs_kernel<F, false, R, true>;
-    if (fused == nullptr ? !reserve_lds(reduce, lds, target) : !reserve_lds(reduce_adam, lds, target)) return false;
+    constexpr uint32_t kCombineBlocks = 512;
     hipLaunchKernelGGL((bwd_bucket_kernel<F, kHalf, R>), dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, d, p, pos, g,
-                       runs, values, entry_rows);
-    hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, runs, slice_np);
-    hipLaunchKernelGGL(bwd_bucket_plan_kernel, dim3(1), dim3(kScanThreads), 0, stream, p, slice_np, meta, parts,
-                       part_slice);
+                       runs, values, entry_rows, meta);
+    if (!p.whole)
+        hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, runs, meta, slice_np,
+                           first_part, part_slice, split);
+    const dim3 reduce_grid(p.n_slices + (p.whole ? 0 : kSplitBlocks));
+    auto finish = [&](auto adam, const AdamStep &step, float *ap, float *am, float *av) {
+        constexpr bool kAdam = decltype(adam)::value;
+        const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, kAdam>;
+        if (!reserve_lds(reduce, lds, target)) return false;
+        hipLaunchKernelGGL(reduce, reduce_grid, dim3(kRunThreads), lds, stream, d, p, meta, slice_np, first_part,
+                           part_slice, runs, values, entry_rows, partials, part_group, dtable, step, ap, am, av);
+        if (!p.whole)
+            hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, kAdam>), dim3(kCombineBlocks), dim3(256), 0, stream, d, meta,
+                               slice_np, first_part, split, partials, part_group, dtable, step, ap, am, av);
+        return true;
+    };
     if constexpr (!kHalf) {
-        if (fused != nullptr) {
-            hipLaunchKernelGGL(reduce_adam, dim3(p.max_parts), dim3(kRunThreads), lds, stream, d, p, meta, parts,
-                               part_slice, runs, values, entry_rows, partials, part_group, dtable, fused->step,
-                               fused->p, fused->m, fused->v);
-            hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, true>), dim3(p.n_slices, kCombineSplit), dim3(256), 0,
-                               stream, d, parts, partials, part_group, dtable, fused->step, fused->p, fused->m,
-                               fused->v);
-            return true;
-        }
+        if (fused != nullptr) return finish(std::true_type{}, fused->step, fused->p, fused->m, fused->v);
     }
-    hipLaunchKernelGGL(reduce, dim3(p.max_parts), dim3(kRunThreads), lds, stream, d, p, meta, parts, part_slice, runs,
-                       values, entry_rows, partials, part_group, dtable, AdamStep{}, nullptr, nullptr, nullptr);
-    hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, false>), dim3(p.n_slices, kCombineSplit), dim3(256), 0, stream, d,
-                       parts, partials, part_group, dtable, AdamStep{}, nullptr, nullptr, nullptr);
-    return true;
+    return finish(std::false_type{}, AdamStep{}, nullptr, nullptr, nullptr);
 }
 
 template <int F, bool kHalf>
