@@ -705,6 +705,120 @@ __global__ void __launch_bounds__(kAssignBlock)
     if (j < n_rays) indices_out[j] = t ? before + (uint32_t)__popcll(m & below) : indices_in[j];
 }
 
+// One ray's march in a cascade of one grid over [-1, 1]^3 with a constant step k (K = 1,
+// bound >= 1, stepsize_portion = 0), on one lane.  The lanes of a wavefront are rays, each
+// as long as its slowest (a slot's new ray crosses empty space, the others take their next
+// samples), and issuing instructions bounds it: the general loop spends 150 on a cell and
+// 30 on steps that a skip adds one by one.  A round of 2^18 slots, 800 x 800 rays through
+// G = 128: 182 -> 78 us.  Here:
+//   * a skip is one multiplication.  Inside a binade of t every addition of k adds the same
+//     `inc`, k rounded to the ulp (ties, where that depends on t, take the loop), so the
+//     n-th step is t + n inc, exactly.
+//   * an occupancy word holds a 4x4x4 block.  If it is zero the skip goes to the first step
+//     past the block.  The loop gets there too: every step it visits inside the block is
+//     empty, and each visit's exit distance lies before the block's up to rounding, so only
+//     a step within the rounding error of the block's exit could be judged differently; if
+//     there is one between the bounds lo and hi below, the cell's own exit is taken.
+struct PlainMarch {
+    float half_G, inv_G, gmax, k;
+    float sx, sy, sz, hx, hy, hz;  // towards the exit: half a cell, a block or none
+    float ex, ey, ez, slack;       // bounds of the rounding error of exit distances
+    float limit, inc, per_inc;     // of the binade t is in (limit: its end)
+
+    __device__ __forceinline__ PlainMarch(const MarchParams &p, const Ray &r) {
+        half_G = 0.5f * (float)p.G;
+        inv_G = p.inv_G;
+        gmax = (float)(p.G - 1);
+        k = step_size(p, 0.0f);
+        sx = copysignf(0.5f, r.dx);
+        sy = copysignf(0.5f, r.dy);
+        sz = copysignf(0.5f, r.dz);
+        hx = sx > 0.0f ? 4.0f : 0.0f;
+        hy = sy > 0.0f ? 4.0f : 0.0f;
+        hz = sz > 0.0f ? 4.0f : 0.0f;
+        ex = error_bound(r.ox, r.dx, r.idx, r.t1);
+        ey = error_bound(r.oy, r.dy, r.idy, r.t1);
+        ez = error_bound(r.oz, r.dz, r.idz, r.t1);
+        const float inf = __builtin_huge_valf();
+        // 1 / d overflows for a tiny d: exit distances say nothing then
+        const bool tiny = (r.dx != 0.0f && fabsf(r.idx) == inf) || (r.dy != 0.0f && fabsf(r.idy) == inf) ||
+                          (r.dz != 0.0f && fabsf(r.idz) == inf);
+        slack = tiny ? inf : 2.3841858e-7f * fabsf(r.t1);  // 2^-22: t + exit
+        limit = 0.0f;
+        inc = per_inc = 0.0f;
+    }
+
+    // A position carries up to 2^-24 (|o| + 2 t|d| + 3), a plane 2^-24, and the exit distance
+    // has two positions' errors over d: 2^-21 (|o| + t|d| + 1.5) is more than twice that.
+    static __device__ __forceinline__ float error_bound(float o, float d, float id, float t1) {
+        return d == 0.0f ? 0.0f : 4.7683716e-7f * (fabsf(o) + fabsf(t1 * d) + 1.5f) * fabsf(id);
+    }
+
+    __device__ __forceinline__ void enter_binade(float t) {
+        const uint32_t e8 = __float_as_uint(t) >> 23;  // sign bit included: a negative t has no inc
+        inc = per_inc = 0.0f;
+        limit = 0.0f;
+        if (e8 < 24u || e8 > 253u) return;
+        limit = __uint_as_float((e8 + 1u) << 23);
+        const float q = k * __uint_as_float((277u - e8) << 23);  // k in ulps of t, exact
+        const float m = rintf(q);
+        if (m >= 1.0f && m <= 65536.0f && fabsf(q - m) != 0.5f) {
+            inc = m * __uint_as_float((e8 - 23u) << 23);
+            per_inc = 1.0f / inc;
+        }
+    }
+
+    // First step after t at or past thr; false where it is not inside t's binade.
+    __device__ __forceinline__ bool step_to(float t, float thr, float &nt) const {
+        const float n = fmaxf(1.0f, ceilf((thr - t) * per_inc));
+        nt = fmaf(n, inc, t);
+        if (!(nt < limit)) return false;  // a sum past the binade is rounded
+        if (n > 1.0f && nt - inc >= thr) nt -= inc;
+        if (nt < thr) nt += inc;
+        return inc > 0.0f && nt < limit;
+    }
+
+    // t of the next visited step after the empty cell at t, position (px, py, pz) and grid
+    // coordinates (gx, gy, gz).
+    __device__ __forceinline__ float skip(const MarchParams &p, const Ray &r, bool empty_block, float t, float px, float py,
+                                          float pz, float gx, float gy, float gz) {
+        if (!(t < limit)) enter_binade(t);
+        float nt;
+        if (empty_block) {
+            const float bx = exit_plane(fmaf(4.0f, floorf(gx * 0.25f), hx), px) * r.idx;
+            const float by = exit_plane(fmaf(4.0f, floorf(gy * 0.25f), hy), py) * r.idy;
+            const float bz = exit_plane(fmaf(4.0f, floorf(gz * 0.25f), hz), pz) * r.idz;
+            const float lo = t + (fminf(bx - ex, fminf(by - ey, bz - ez)) - slack);
+            const float hi = t + (fminf(bx + ex, fminf(by + ey, bz + ez)) + slack);
+            if (step_to(t, hi, nt) && nt - inc < lo && nt < r.t1) return nt;
+        }
+        const float cx = exit_plane(floorf((gx + 0.5f) + sx), px) * r.idx;
+        const float cy = exit_plane(floorf((gy + 0.5f) + sy), py) * r.idy;
+        const float cz = exit_plane(floorf((gz + 0.5f) + sz), pz) * r.idz;
+        const float thr = t + fmaxf(0.0f, fminf(cx, fminf(cy, cz)));
+        return step_to(t, thr, nt) ? nt : skip_to(p, t, k, thr);
+    }
+
+    // distance from x to the plane at grid coordinate n: the products are exact, so this
+    // rounds as ((n * inv_G) - 0.5) * 2 - x does
+    __device__ __forceinline__ float exit_plane(float n, float x) const {
+        return fmaf(2.0f, fmaf(n, inv_G, -0.5f), -x);
+    }
+};
+
+// PlainMarch's case of lookup_cell.
+__device__ __forceinline__ bool lookup_plain(const PlainMarch &m, BitCache &cache, float px, float py, float pz, float &gx,
+                                             float &gy, float &gz) {
+    gx = (px + 1.0f) * m.half_G;  // the factor is a power of two: exact
+    gy = (py + 1.0f) * m.half_G;
+    gz = (pz + 1.0f) * m.half_G;
+    const uint32_t ix = (uint32_t)fminf(fmaxf(gx, 0.0f), m.gmax);
+    const uint32_t iy = (uint32_t)fminf(fmaxf(gy, 0.0f), m.gmax);
+    const uint32_t iz = (uint32_t)fminf(fmaxf(gz, 0.0f), m.gmax);
+    return occupied(cache, nullptr, morton_spread10(ix) | (morton_spread10(iy) << 1) | (morton_spread10(iz) << 2));
+}
+
+template <bool kPlain>
 __global__ void __launch_bounds__(kBlock)
     march_inference_kernel(MarchParams p, bool word_ok, uint32_t n_total_rays, uint32_t n_rays, uint32_t cap,
                            const float *__restrict__ rays_o, const float *__restrict__ rays_d,
@@ -723,32 +837,48 @@ __global__ void __launch_bounds__(kBlock)
     if (r < n_total_rays) {
         const float t0 = t_starts[r], t1 = t_ends[r];
         if (!(t1 < t0)) {
-            const float ox = rays_o[3 * (size_t)r], oy = rays_o[3 * (size_t)r + 1], oz = rays_o[3 * (size_t)r + 2];
-            const float dx = rays_d[3 * (size_t)r], dy = rays_d[3 * (size_t)r + 1], dz = rays_d[3 * (size_t)r + 2];
-            const float idx_ = 1.0f / dx, idy = 1.0f / dy, idz = 1.0f / dz;
-            BitCache cache = make_bit_cache(bits, word_ok);
+            const Ray ray = load_ray(rays_o, rays_d, r, t1);
+            BitCache cache = make_bit_cache(bits, kPlain || word_ok);
             t = t0;
-            while (steps < cap && t < t1) {
-                const float px = ox + t * dx, py = oy + t * dy, pz = oz + t * dz;
-                const float ds = step_size(p, t);
-                float gx, gy, gz, mb;
-                float nt;
-                if (lookup_cell(p, bits, cache, px, py, pz, ds, gx, gy, gz, mb)) {
-                    rx[3 * steps + 0] = px;
-                    rx[3 * steps + 1] = py;
-                    rx[3 * steps + 2] = pz;
-                    rds[steps] = ds;
-                    rz[steps] = t;
-                    ++steps;
-                    nt = t + ds;
-                } else {
-                    nt = skip_to(p, t, ds, cell_exit_t(p, t, px, py, pz, gx, gy, gz, mb, dx, dy, dz, idx_, idy, idz));
+            if constexpr (kPlain) {
+                PlainMarch m(p, ray);
+                while (steps < cap && t < t1) {
+                    const float px = ray.ox + t * ray.dx, py = ray.oy + t * ray.dy, pz = ray.oz + t * ray.dz;
+                    float gx, gy, gz;
+                    if (lookup_plain(m, cache, px, py, pz, gx, gy, gz)) {
+                        rx[3 * steps + 0] = px;
+                        rx[3 * steps + 1] = py;
+                        rx[3 * steps + 2] = pz;
+                        rds[steps] = m.k;
+                        rz[steps] = t;
+                        ++steps;
+                        t = t + m.k;
+                    } else {
+                        t = m.skip(p, ray, cache.word == 0ull, t, px, py, pz, gx, gy, gz);
+                    }
                 }
-                t = nt;
+            } else {
+                while (steps < cap && t < t1) {
+                    const float px = ray.ox + t * ray.dx, py = ray.oy + t * ray.dy, pz = ray.oz + t * ray.dz;
+                    const float ds = step_size(p, t);
+                    float gx, gy, gz, mb;
+                    if (lookup_cell(p, bits, cache, px, py, pz, ds, gx, gy, gz, mb)) {
+                        rx[3 * steps + 0] = px;
+                        rx[3 * steps + 1] = py;
+                        rx[3 * steps + 2] = pz;
+                        rds[steps] = ds;
+                        rz[steps] = t;
+                        ++steps;
+                        t = t + ds;
+                    } else {
+                        t = skip_to(p, t, ds, cell_exit_t(p, t, px, py, pz, gx, gy, gz, mb, ray.dx, ray.dy, ray.dz,
+                                                          ray.idx, ray.idy, ray.idz));
+                    }
+                }
             }
             // far-plane sample (marching.cu:367-394)
             if (t >= t1) {
-                const float px = ox + t1 * dx, py = oy + t1 * dy, pz = oz + t1 * dz;
+                const float px = ray.ox + t1 * ray.dx, py = ray.oy + t1 * ray.dy, pz = ray.oz + t1 * ray.dz;
                 const float ds = step_size(p, t1);
                 float gx, gy, gz, mb;
                 if (lookup_cell(p, bits, cache, px, py, pz, ds, gx, gy, gz, mb)) {
@@ -920,8 +1050,11 @@ extern "C" void march_rays_inference(ngp_stream_t stream_, void **buffers, const
     hipLaunchKernelGGL(assign_write_kernel, dim3(n_assign), dim3(kAssignBlock), 0, stream, d.n_rays, terminated,
                        indices_in, indices_out);
     if (!check_launch(target)) return;
-    hipLaunchKernelGGL(march_inference_kernel, dim3(div_up(d.n_rays, kBlock)), dim3(kBlock), 0, stream, p,
-                       bitfield_words_ok(bits, d.K, d.G), d.n_total_rays, d.n_rays, d.march_steps_cap, rays_o, rays_d, t_starts, t_ends, bits,
-                       indices_out, n_samples, t_out, xyzs, dss, zs);
+    const bool word_ok = bitfield_words_ok(bits, d.K, d.G);
+    const auto kernel = word_ok && d.K == 1 && d.bound >= 1.0f && d.stepsize_portion == 0.0f ? march_inference_kernel<true>
+                                                                                             : march_inference_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(div_up(d.n_rays, kBlock)), dim3(kBlock), 0, stream, p, word_ok, d.n_total_rays,
+                       d.n_rays, d.march_steps_cap, rays_o, rays_d, t_starts, t_ends, bits, indices_out, n_samples, t_out,
+                       xyzs, dss, zs);
     check_launch(target);
 }

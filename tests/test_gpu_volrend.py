@@ -199,6 +199,49 @@ def test_march_rays_inference_bit_exact(dev):
         ts_dev, nri_dev, idx_dev, term_dev = gts, nxt, gidx, T(term, dev)
 
 
+def _crossing_rays(rng, n, G, kind):
+    """Rays towards [-1, 1]^3, through grid planes (`axis`: along an axis on a plane, with zeros of
+    either sign; `graze`: nearly so), from inside it, or long ones that cross t = 4."""
+    d = rng.normal(size=(n, 3))
+    o = rng.uniform(-0.95, 0.95, (n, 3))
+    if kind in ("axis", "graze"):
+        d = np.where(rng.random((n, 3)) < 0.5, -0.0, 0.0) if kind == "axis" else rng.normal(size=(n, 3)) * 1e-4
+        d[np.arange(n), rng.integers(0, 3, n)] = np.where(rng.random(n) < 0.5, -1.0, 1.0)
+        o = rng.integers(0, G + 1, (n, 3)) * (2.0 / G) - 1.0 - 2.0 * d
+    elif kind == "far":
+        o = o * 0.7 - 4.0 * d / np.linalg.norm(d, axis=1, keepdims=True)
+    d = d / np.linalg.norm(d, axis=1, keepdims=True)
+    return o.astype(np.float32), d.astype(np.float32)
+
+
+@pytest.mark.parametrize("G, diag, bound", [(4, 64, 1.0), (64, 1024, 1.0), (128, 333, 2.0)])
+@pytest.mark.parametrize("kind", ["axis", "graze", "inside", "far"])
+def test_march_rays_inference_constant_step_one_cascade(dev, kind, G, diag, bound):
+    """The one-cascade constant-step march (whole empty blocks skipped, skips in one step)
+    against the step-by-step oracle, every output bit for bit: blocks partly filled, blocks
+    of one cell, empty space between them."""
+    rng = np.random.default_rng([G, len(kind)])
+    n, cap = 1500, 8
+    o, d = _crossing_rays(rng, n, G, kind)
+    t0 = rng.uniform(0.0, 1.0, n).astype(np.float32)
+    t1 = (t0 + rng.uniform(0.0, 5.5, n)).astype(np.float32)
+    filled = rng.random(G ** 3 // 64) < 0.3  # blocks: 64 cells in Morton order
+    filled[0] = True
+    bits = np.packbits(np.repeat(filled, 64) & (rng.random(G ** 3) < 0.7), bitorder="little")
+    term, idx, nri, ts = np.ones(n, bool), np.zeros(n, np.uint32), np.zeros(1, np.uint32), t0.copy()
+    for it in range(3):
+        want = oracle.march_rays_inference(diag, 1, G, cap, bound, 0.0, o, d, ts, t1, bits, nri, term, idx)
+        got = volrend.march_rays_inference(diag, 1, G, cap, bound, 0.0, T(o, dev), T(d, dev), T(ts, dev), T(t1, dev),
+                                           T(bits, dev), U(nri, dev), T(term, dev), U(idx, dev))
+        _, _, gns, gts, gx, gds, gz = got
+        keep = want["indices"] < n
+        ts[want["indices"][keep]] = want["t_starts_out"][keep]
+        for g, w in ((gns, want["n_samples"]), (gx, want["xyzs"]), (gds, want["dss"]), (gz, want["z_vals"]), (gts, ts)):
+            np.testing.assert_array_equal(N(g), w)
+        assert it > 0 or want["n_samples"].any()
+        nri, idx, term = np.array([want["next_ray_index"]], np.uint32), want["indices"], np.zeros(n, bool)
+
+
 def test_integrate_rays_bit_exact_and_backward(dev):
     rng = np.random.default_rng(5)
     start, ns, bgs, dss, z, drgbs = integrate_inputs(rng, 4096, 200)
