@@ -72,14 +72,37 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Four floats with the alignment of one.
+struct Quad {
+    float v[4];
+};
+
+// Copies a weight matrix [ROWS][COLS] into its LDS rows, sixteen bytes at a time.
+template <int ROWS, int COLS, int STRIDE>
+__device__ __forceinline__ void stage_matrix(float *lds, const float *__restrict__ w) {
+    static_assert(COLS % 4 == 0 && STRIDE % 4 == 0 && ROWS * COLS % (4 * kThreads) == 0, "whole quads per thread");
+    constexpr int kPer = ROWS * COLS / (4 * kThreads);
+    Quad q[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) q[k] = *reinterpret_cast<const Quad *>(w + 4 * (threadIdx.x + k * kThreads));
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int t = 4 * (threadIdx.x + k * kThreads);
+        *reinterpret_cast<v4f *>(lds + t / COLS * STRIDE + t % COLS) = v4f{q[k].v[0], q[k].v[1], q[k].v[2], q[k].v[3]};
+    }
+}
+
 __device__ void stage_weights(float *lds, const float *__restrict__ params) {
-    for (int t = threadIdx.x; t < L_END; t += kThreads) lds[t] = 0.0f;
-    __syncthreads();
-    for (int t = threadIdx.x; t < 32 * 64; t += kThreads) lds[L_W1 + (t / 64) * S_W1 + t % 64] = params[P_W1 + t];
-    for (int t = threadIdx.x; t < 64 * 16; t += kThreads) lds[L_W2 + (t / 16) * S_W2 + t % 16] = params[P_W2 + t];
-    for (int t = threadIdx.x; t < 32 * 64; t += kThreads) lds[L_W3 + (t / 64) * S_W3 + t % 64] = params[P_W3 + t];
-    for (int t = threadIdx.x; t < 64 * 64; t += kThreads) lds[L_W4 + (t / 64) * S_W4 + t % 64] = params[P_W4 + t];
-    for (int t = threadIdx.x; t < 64 * 3; t += kThreads) lds[L_W5 + (t / 3) * S_W5 + t % 3] = params[P_W5 + t];
+    stage_matrix<32, 64, S_W1>(lds + L_W1, params + P_W1);
+    stage_matrix<64, 16, S_W2>(lds + L_W2, params + P_W2);
+    stage_matrix<32, 64, S_W3>(lds + L_W3, params + P_W3);
+    stage_matrix<64, 64, S_W4>(lds + L_W4, params + P_W4);
+    // W5 has 3 of 16 columns, the others are zero
+    static_assert(64 * 16 == 4 * kThreads, "one quad of W5 per thread");
+    const int row = threadIdx.x / 4;
+    v4f w5 = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (threadIdx.x % 4 == 0) w5 = v4f{params[P_W5 + 3 * row], params[P_W5 + 3 * row + 1], params[P_W5 + 3 * row + 2], 0.0f};
+    *reinterpret_cast<v4f *>(lds + L_W5 + row * S_W5 + 4 * (threadIdx.x % 4)) = w5;
     __syncthreads();
 }
 
@@ -93,6 +116,64 @@ __device__ __forceinline__ void layer_fwd(const float *W, const v4f *in, v4f *ou
         for (int b = 0; b < IN / 16; ++b) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc = mfma(W[(16 * b + 4 * g + r) * STRIDE + 16 * ob + i], in[b][r], acc);
+        }
+        out[ob] = acc;
+    }
+}
+
+// The weights of kernels that only run forward: W^T, so that the four inputs 4q..4q+3 of
+// an output, which a lane feeds to four MFMAs in turn, are one 16-byte read, without
+// padding, so that four workgroups fit a CU.  Quad q of a row stands at q ^ (row & 15), or
+// for rows of 8 quads, two to a line of banks, at q ^ ((row >> 1) & 7): the rows of 16
+// lanes then cover every bank once.  W5's outputs past the third are all the zeros of row 3.
+constexpr int F_W1 = 0, F_W2 = 2048, F_W3 = 3072, F_W4 = 5120, F_W5 = 9216, F_END = F_W5 + 4 * 64;
+
+template <int IN>
+__device__ __forceinline__ int quad_at(int row, int q) {
+    return IN * row + 4 * (IN == 64 ? q ^ (row & 15) : q ^ ((row >> 1) & 7));
+}
+
+// Copies a weight matrix [IN][OUT] to its rows W^T; rows past the last are zero.
+template <int IN, int OUT, int ROWS>
+__device__ __forceinline__ void stage_transposed(float *lds, const float *__restrict__ w) {
+    constexpr int kQuads = ROWS * IN / 4, kPer = (kQuads + kThreads - 1) / kThreads;
+    static_assert(kQuads % kThreads == 0 || kPer == 1, "whole quads per thread");
+    v4f v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int t = min((int)threadIdx.x + k * kThreads, kQuads - 1), row = t % ROWS, q = t / ROWS;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[k][r] = w[(4 * q + r) * OUT + min(row, OUT - 1)];
+        if (ROWS != OUT && row >= OUT) v[k] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int t = min((int)threadIdx.x + k * kThreads, kQuads - 1);
+        *reinterpret_cast<v4f *>(lds + quad_at<IN>(t % ROWS, t / ROWS)) = v[k];
+    }
+}
+
+__device__ void stage_forward(float *lds, const float *__restrict__ params) {
+    stage_transposed<32, 64, 64>(lds + F_W1, params + P_W1);
+    stage_transposed<64, 16, 16>(lds + F_W2, params + P_W2);
+    stage_transposed<32, 64, 64>(lds + F_W3, params + P_W3);
+    stage_transposed<64, 64, 64>(lds + F_W4, params + P_W4);
+    stage_transposed<64, 3, 4>(lds + F_W5, params + P_W5);
+    __syncthreads();
+}
+
+// layer_fwd from W^T rows of which there are ROWS (the last one stands for the rest).
+template <int IN, int OUT, int ROWS = OUT>
+__device__ __forceinline__ void layer_fwd_t(const float *W, const v4f *in, v4f *out, int i, int g) {
+#pragma unroll
+    for (int ob = 0; ob < OUT / 16; ++ob) {
+        const int row = ROWS == OUT ? 16 * ob + i : min(i, ROWS - 1);
+        v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int b = 0; b < IN / 16; ++b) {
+            const v4f a = *reinterpret_cast<const v4f *>(W + quad_at<IN>(row, 4 * b + g));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc = mfma(a[r], in[b][r], acc);
         }
         out[ob] = acc;
     }
@@ -113,12 +194,16 @@ __device__ __forceinline__ void layer_bwd(const float *W, const v4f *dout, v4f *
     }
 }
 
+// max(z, 0) in one instruction: fmaxf quiets its operand first, and so does a median that
+// the compiler knows to be a maximum.  A NaN gives 0 here as there.
 template <int N>
 __device__ __forceinline__ void relu(v4f *z) {
+    float inf = __builtin_huge_valf();
+    asm("" : "+v"(inf));
 #pragma unroll
     for (int b = 0; b < N; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z[b][r] = fmaxf(z[b][r], 0.0f);
+        for (int r = 0; r < 4; ++r) z[b][r] = __builtin_amdgcn_fmed3f(z[b][r], 0.0f, inf);
 }
 
 // gradient through relu: keep where the forward output was positive
@@ -150,6 +235,17 @@ __device__ __forceinline__ v4f sh4_part(float x, float y, float z, int g) {
 }
 
 __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + det_expf(-x)); }
+
+// The outputs of 16 samples: density from o0 and colour from rr[0..2] of lane (i, 0).
+// Lane (i, g) takes value g of sample i, one exponential each instead of four on a
+// quarter of the lanes.  Call with all lanes active; s is sample i's place.
+__device__ __forceinline__ void store_drgbs(float *__restrict__ drgbs, size_t s, bool live, float o0, const v4f &rr, int i,
+                                            int g) {
+    const float a = __shfl(o0, i), b = __shfl(rr[0], i), c = __shfl(rr[1], i), d = __shfl(rr[2], i);
+    const float x = g == 0 ? a : g == 1 ? b : g == 2 ? c : d;
+    const float e = det_expf(g == 0 ? x : -x);
+    if (live) drgbs[4 * s + g] = g == 0 ? e : 1.0f / (1.0f + e);
+}
 
 struct Fwd {
     v4f x[2], h1[4], c[2], h2[4], h3[4], rr;  // c[0] = o (density MLP output), c[1] = SH
@@ -227,15 +323,34 @@ __device__ __forceinline__ void forward_from_x(const float *lds, float dx, float
 }
 
 
-__global__ void __launch_bounds__(kThreads)
+// forward_from_x with the weights of stage_forward.
+__device__ __forceinline__ void forward_only(const float *lds, float dx, float dy, float dz, int i, int g, Fwd &f) {
+    layer_fwd_t<32, 64>(lds + F_W1, f.x, f.h1, i, g);
+    relu<4>(f.h1);
+    layer_fwd_t<64, 16>(lds + F_W2, f.h1, &f.c[0], i, g);
+    f.c[1] = sh4_part(dx, dy, dz, g);
+    layer_fwd_t<32, 64>(lds + F_W3, f.c, f.h2, i, g);
+    relu<4>(f.h2);
+    layer_fwd_t<64, 64>(lds + F_W4, f.h2, f.h3, i, g);
+    relu<4>(f.h3);
+    layer_fwd_t<64, 16, 4>(lds + F_W5, f.h3, &f.rr, i, g);
+}
+
+// Bounded by the f32 matrix unit (2^18 samples: 36 us of MFMA at the clock it holds), in
+// whose way stood three things: the weights' copy to LDS float by float (10 us a workgroup,
+// two rounds of them), one exponential after the other on a quarter of the lanes, and two
+// wavefronts per SIMD, since the compiler kept the 160 weights of a lane in registers.  Now
+// 16-byte reads from LDS and 88 registers, four wavefronts.  2^18 samples: 70 -> 52 us,
+// 2^20: 230 -> 192, 1,000: 9.9 -> 6.0.
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
     mlp_forward_kernel(uint32_t n, bool level_major, const float *__restrict__ enc, const float *__restrict__ dirs,
                        const float *__restrict__ params, float *__restrict__ drgbs) {
-    __shared__ float lds[L_END];
-    stage_weights(lds, params);
+    __shared__ __align__(16) float lds[F_END];
+    stage_forward(lds, params);
     const int lane = lane_id();
     const int i = lane & 15, g = lane >> 4;
     const uint32_t n_tiles = (n + kTile - 1) / kTile;
-    const uint32_t wave = blockIdx.x * kWaves + threadIdx.x / kWave;
+    const uint32_t wave = blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t n_waves = gridDim.x * kWaves;
     TileIn next = load_tile(enc, level_major, dirs, nullptr, n, (size_t)min(wave, n_tiles - 1) * kTile, i, g);
     for (uint32_t t = wave; t < n_tiles; t += n_waves) {
@@ -245,13 +360,9 @@ __global__ void __launch_bounds__(kThreads)
         Fwd f;
         f.x[0] = in.x[0];
         f.x[1] = in.x[1];
-        forward_from_x(lds, in.dx, in.dy, in.dz, i, g, f);
-        const size_t s = s0 + i;
-        if (g == 0 && s < n) {
-            const float sigma = det_expf(f.c[0][0]);
-            v4f out = {sigma, sigmoidf(f.rr[0]), sigmoidf(f.rr[1]), sigmoidf(f.rr[2])};
-            *reinterpret_cast<v4f *>(drgbs + 4 * s) = out;
-        }
+        asm volatile("" ::: "memory");  // the weights are not kept in registers over the tiles
+        forward_only(lds, in.dx, in.dy, in.dz, i, g, f);
+        store_drgbs(drgbs, s0 + i, s0 + i < n, f.c[0][0], f.rr, i, g);
     }
 }
 
@@ -343,7 +454,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     mlp_backward_kernel(uint32_t n, bool level_major, const float *__restrict__ enc, const float *__restrict__ dirs,
                         const float *__restrict__ params, const float *__restrict__ dL_ddrgbs,
                         float *__restrict__ dL_denc, float *__restrict__ workspace) {
-    __shared__ float lds[L_END];
+    __shared__ __align__(16) float lds[L_END];
     __shared__ float scratch[kWaves * 2 * T_FLOATS];
     stage_weights(lds, params);
     const int lane = lane_id();
@@ -625,7 +736,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
     const int lane = lane_id();
     const int i = lane & 15, g = lane >> 4;
     const uint32_t n_tiles = (n + kTile - 1) / kTile;
-    const uint32_t wave = blockIdx.x * kWaves + threadIdx.x / kWave;
+    const uint32_t wave = blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t n_waves = gridDim.x * kWaves;
     TileIn next = load_tile(enc, level_major, dirs, nullptr, n, (size_t)min(wave, n_tiles - 1) * kTile, i, g);
     for (uint32_t t = wave; t < n_tiles; t += n_waves) {
@@ -636,12 +747,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
         f.x[0] = in.x[0];
         f.x[1] = in.x[1];
         forward_from_x_h(lds, in.dx, in.dy, in.dz, i, g, f);
-        const size_t s = s0 + i;
-        if (g == 0 && s < n) {
-            const float sigma = det_expf(f.c[0][0]);
-            v4f out = {sigma, sigmoidf(f.rr[0]), sigmoidf(f.rr[1]), sigmoidf(f.rr[2])};
-            *reinterpret_cast<v4f *>(drgbs + 4 * s) = out;
-        }
+        store_drgbs(drgbs, s0 + i, s0 + i < n, f.c[0][0], f.rr, i, g);
     }
 }
 
