@@ -954,17 +954,36 @@ __device__ __forceinline__ v4f encode_two_levels(const HashGridDescriptor &d, co
     return out;
 }
 
+// A pool round's samples stand in a third of the entries, a whole slot or nothing, so a
+// wavefront packs them: it looks at 64 entries at a time, writes the dead ones' zeros,
+// appends the live ones to a queue of its own in LDS and takes tiles of 16 from that.
+// Bounded by the gathers' misses in L2 (every XCD reads every level of the table, unlike in
+// the encoder): 753,000 samples of 2^21 entries 292 -> 260 us; batches of 64 samples level
+// by level with two rows to a load (270), four wavefronts per SIMD (268) and contiguous
+// entries per wavefront (274) end at the same rate.  A round without samples 46 -> 20 us
+// (the zeros, and the 64-bit division per entry that went).
+constexpr int kQueue = kWave + kTile;
+// Workgroups in a launch, four times what the chip holds: the wavefronts' entries hold
+// different numbers of samples (768 workgroups, one round of them: 303 us, 12,288: 271).
+constexpr uint32_t kChunkBlocks = 3072;
+struct ChunkQueue {
+    float p[3][kQueue];    // normalised positions
+    uint32_t tag[kQueue];  // 64 * (the wavefront's group) + lane
+    uint32_t ray[kQueue];
+};
+
 template <typename TT, bool kHalf>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
     field_chunks_kernel(HashGridDescriptor d, uint32_t n_slots, uint32_t cap, uint32_t n_total,
                         const float *__restrict__ xyzs, const uint32_t *__restrict__ n_samples,
                         const uint32_t *__restrict__ indices, const float *__restrict__ rays_d,
                         const TT *__restrict__ table, const void *__restrict__ params, float *__restrict__ drgbs) {
-    __shared__ __align__(16) float lds_f[kHalf ? 1 : L_END];
-    __shared__ __align__(16) _Float16 lds_h[kHalf ? H_FEND : 1];
+    __shared__ __align__(16) float lds_f[kHalf ? 4 : F_END];
+    __shared__ __align__(16) _Float16 lds_h[kHalf ? H_FEND : 8];
     __shared__ LevelTables lt;
+    __shared__ ChunkQueue queues[kWaves];
     if (kHalf) stage_weights_h<false>(lds_h, static_cast<const _Float16 *>(params));
-    else stage_weights(lds_f, static_cast<const float *>(params));
+    else stage_forward(lds_f, static_cast<const float *>(params));
     if (threadIdx.x < 16) {
         lt.scale[threadIdx.x] = d.scales[threadIdx.x];
         lt.res[threadIdx.x] = d.resolutions[threadIdx.x];
@@ -973,41 +992,81 @@ __global__ void __launch_bounds__(kThreads)
     __syncthreads();
     const int lane = lane_id();
     const int i = lane & 15, g = lane >> 4;
+    ChunkQueue &queue = queues[threadIdx.x / kWave];
     const uint64_t n_entries = (uint64_t)n_slots * cap;
-    const uint64_t n_tiles = (n_entries + kTile - 1) / kTile;
     const uint32_t wave = blockIdx.x * kWaves + threadIdx.x / kWave;
-    const uint32_t n_waves = gridDim.x * kWaves;
+    const uint64_t stride = (uint64_t)gridDim.x * kWaves * kWave;
     const Divisor two_b = make_divisor(2.0f * d.bound);
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint64_t t = wave; t < n_tiles; t += n_waves) {
-        const uint64_t e = t * kTile + i;
-        bool live = false;
-        uint32_t ray = 0;
-        if (e < n_entries) {
-            const uint32_t slot = (uint32_t)(e / cap), k = (uint32_t)(e % cap);
-            live = k < n_samples[slot];
+    // lane's entry of the next group: its number, slot and place in it
+    uint64_t e = (uint64_t)wave * kWave + lane;
+    uint64_t group_e = (uint64_t)wave * kWave;
+    uint32_t slot = (uint32_t)(e / cap), k = (uint32_t)(e % cap);
+    const uint32_t slot_step = (uint32_t)(stride / cap), k_step = (uint32_t)(stride % cap);
+    uint32_t group = 0, queued = 0, head = 0;
+    uint32_t n_next = e < n_entries ? n_samples[slot] : 0u, ray_next = e < n_entries ? indices[slot] : 0u;
+    for (;;) {
+        if (queued < kTile && group_e < n_entries) {
+            const bool live = k < n_next && ray_next < n_total;  // (n_next is 0 past the end)
+            const uint32_t ray = ray_next;
+            float p[3] = {0.0f, 0.0f, 0.0f};
             if (live) {
-                ray = indices[slot];
-                live = ray < n_total;
+                const float at[3] = {xyzs[3 * e + 0], xyzs[3 * e + 1], xyzs[3 * e + 2]};
+                normalise(two_b, d.bound, at, p);
+            } else if (e < n_entries) {
+                *reinterpret_cast<v4f *>(drgbs + 4 * e) = zero;
             }
-        }
-        if (__ballot(live) == 0ull) {
-            if (g == 0 && e < n_entries) *reinterpret_cast<v4f *>(drgbs + 4 * e) = zero;
+            const uint64_t live_m = __ballot(live);
+            // what is left of the last group moves to the front
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (head != 0 && (uint32_t)lane < queued) {
+                const float q0 = queue.p[0][head + lane], q1 = queue.p[1][head + lane], q2 = queue.p[2][head + lane];
+                const uint32_t q3 = queue.tag[head + lane], q4 = queue.ray[head + lane];
+                queue.p[0][lane] = q0;
+                queue.p[1][lane] = q1;
+                queue.p[2][lane] = q2;
+                queue.tag[lane] = q3;
+                queue.ray[lane] = q4;
+            }
+            if (live) {
+                const uint32_t at = queued + (uint32_t)__popcll(live_m & ((1ull << lane) - 1ull));
+                queue.p[0][at] = p[0];
+                queue.p[1][at] = p[1];
+                queue.p[2][at] = p[2];
+                queue.tag[at] = 64u * group + (uint32_t)lane;
+                queue.ray[at] = ray;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            head = 0;
+            queued += (uint32_t)__popcll(live_m);
+            ++group;
+            e += stride;
+            group_e += stride;
+            slot += slot_step;
+            k += k_step;
+            if (k >= cap) {
+                k -= cap;
+                ++slot;
+            }
+            n_next = e < n_entries ? n_samples[slot] : 0u;
+            ray_next = e < n_entries ? indices[slot] : 0u;
             continue;
         }
+        if (queued == 0) break;
+        const bool live = (uint32_t)i < queued;
         float dx = 0.0f, dy = 0.0f, dz = 0.0f;
         v4f x[2] = {zero, zero};
+        uint32_t tag = 0;
         if (live) {
-            const float at[3] = {xyzs[3 * e + 0], xyzs[3 * e + 1], xyzs[3 * e + 2]};
-            dx = rays_d[3 * (size_t)ray + 0];
-            dy = rays_d[3 * (size_t)ray + 1];
-            dz = rays_d[3 * (size_t)ray + 2];
-            float p[3];
-            normalise(two_b, d.bound, at, p);
+            const size_t ray = queue.ray[head + i];
+            tag = queue.tag[head + i];
+            dx = rays_d[3 * ray + 0];
+            dy = rays_d[3 * ray + 1];
+            dz = rays_d[3 * ray + 2];
+            const float p[3] = {queue.p[0][head + i], queue.p[1][head + i], queue.p[2][head + i]};
 #pragma unroll
             for (int b = 0; b < 2; ++b) x[b] = encode_two_levels(d, lt, table, p, 8 * b + 2 * g);
         }
-        v4f out = zero;
         float o0;
         v4f rr;
         if (kHalf) {
@@ -1021,12 +1080,15 @@ __global__ void __launch_bounds__(kThreads)
             Fwd f;
             f.x[0] = x[0];
             f.x[1] = x[1];
-            forward_from_x(lds_f, dx, dy, dz, i, g, f);
+            asm volatile("" ::: "memory");  // as in mlp_forward_kernel
+            forward_only(lds_f, dx, dy, dz, i, g, f);
             o0 = f.c[0][0];
             rr = f.rr;
         }
-        if (live) out = v4f{det_expf(o0), sigmoidf(rr[0]), sigmoidf(rr[1]), sigmoidf(rr[2])};
-        if (g == 0 && e < n_entries) *reinterpret_cast<v4f *>(drgbs + 4 * e) = out;
+        store_drgbs(drgbs, (uint64_t)(tag / kWave) * stride + (uint64_t)wave * kWave + tag % kWave, live, o0, rr, i, g);
+        const uint32_t taken = min(queued, (uint32_t)kTile);
+        head += taken;
+        queued -= taken;
     }
 }
 
@@ -1412,8 +1474,8 @@ extern "C" void nerf_field_chunks(ngp_stream_t stream, void **buffers, const cha
         set_error(kBadArgument, "%s: drgbs must be 16-byte aligned", target);
         return;
     }
-    const uint64_t tiles = ((uint64_t)d.n_slots * d.cap + kTile - 1) / kTile;
-    const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((tiles + kWaves - 1) / kWaves, 2048));
+    const uint64_t groups = ((uint64_t)d.n_slots * d.cap + kWave - 1) / kWave;
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((groups + kWaves - 1) / kWaves, kChunkBlocks);
     const bool t16 = g.table_dtype == NGP_DTYPE_F16, w16 = d.param_dtype == NGP_DTYPE_F16;
     hipStream_t s = (hipStream_t)stream;
     const float *xyzs = (const float *)buffers[0];

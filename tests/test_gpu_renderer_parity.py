@@ -18,7 +18,9 @@ import pytest
 import torch
 
 import oracle
+from jaxngp_amd import _lib
 from jaxngp_amd import scene as sc
+from jaxngp_amd.nerfs import NeRF
 from jaxngp_amd.renderer import make_near_far_from_bound, make_rays_worldspace, render_rays_inference, render_rays_train
 from jaxngp_amd.train import TrainConfig, Trainer
 from tests.test_gpu_hashgrid import _c_forward
@@ -159,3 +161,36 @@ def test_render_rays_train_matches_oracle_chain(dev, trained):
     absT = oracle.hashgrid_backward64(xyz, np.abs(dX), model.bound, lv, 1 << 19, 2)
     assert (np.abs(dtable - dT) <= 2e-3 * absT + 1e-3 * np.abs(dT).max()).all()
     assert np.abs(dT).max() > 0
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n_slots, cap", [(1, 1), (5, 3), (700, 8), (3001, 70)])
+def test_field_chunks_pack_live_entries(dev, n_slots, cap, half):
+    """nerf_field_chunks on rounds of every kind of slot (empty, part, full, without a ray):
+    the field's own outputs on the live entries, bit for bit (the same operations), and zeros
+    on the others; up to several tiles a wavefront and a partial one at the end."""
+    model = NeRF(bound=1.0, device=dev, table_dtype=torch.float16 if half else torch.float32)
+    g = torch.Generator(device=dev).manual_seed(n_slots)
+    with torch.no_grad():
+        model.position_encoder.table.uniform_(-0.5, 0.5, generator=g)
+    n_total = 2 * n_slots
+    xyzs = torch.rand(n_slots, cap, 3, generator=g, device=dev) * 2 - 1
+    rays_d = torch.nn.functional.normalize(torch.randn(n_total, 3, generator=g, device=dev), dim=-1)
+    ray = torch.randint(0, n_total + n_total // 2, (n_slots,), generator=g, device=dev)
+    n = torch.randint(0, cap + 1, (n_slots,), generator=g, device=dev)
+    n = torch.where(torch.rand(n_slots, generator=g, device=dev) < 0.5, n, torch.where(n > cap // 2, cap, 0))
+    half_mlp = getattr(model, "mlp_half", None) is not None
+    params = model.mlp_half if half_mlp else model.mlp_params.detach()
+    out = torch.full((n_slots, cap, 4), 7.0, device=dev)
+    u32 = lambda t: t.to(torch.int32).view(torch.uint32)
+    desc = _lib.field_chunks_descriptor(model.position_encoder.descriptor(0, model.bound), n_slots, cap, n_total,
+                                        _lib.DTYPE_F16 if half_mlp else _lib.DTYPE_F32)
+    _lib.call("nerf_field_chunks", [xyzs, u32(n), u32(ray), rays_d, model.position_encoder.table.detach(), params, out],
+              desc)
+    live = (torch.arange(cap, device=dev)[None] < n[:, None]) & (ray < n_total)[:, None]
+    slot = live.nonzero()[:, 0]
+    want = torch.zeros(n_slots, cap, 4, device=dev)
+    if slot.numel():
+        with torch.no_grad():
+            want[live] = model(xyzs[live].contiguous(), rays_d[ray[slot]].contiguous(), None)[0]
+    assert torch.equal(out, want)
