@@ -329,11 +329,12 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         const uint64_t runs = (uint64_t)p.n_bitems * p.span_stride;
         const uint64_t max_entries = (uint64_t)p.n_bitems * bucket_entries(half_values);
         // A hashed level spreads 8 contributions a point evenly over its slices; a part holds
-        // a quarter more than one such slice, so these stay whole and the fuller slices of
-        // coarse levels, whose entries also collide more in the LDS atomics, are cut to the
-        // same length (77,777 points: reducer 32 us; with parts of 32,768 entries, 44).
+        // two and a half such slices, so these stay whole and the fuller slices of coarse
+        // levels, whose entries also collide more in the LDS atomics, are cut (2^18 points
+        // f32: 145 us, with parts of four slices 170, of one and a quarter 142; those take
+        // a fifth more workspace, for parts that may be full of one slice's entries).
         const uint64_t mean = (uint64_t)d.n_points * 8 * p.R / d.T;
-        p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 4 + 1023) / 1024 * 1024));
+        p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 2 + 1023) / 1024 * 1024));
         p.group_shift = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
         // Few points: even all contributions of all levels that share a group of slices
         // make one part, so nothing is counted, cut or combined: two launches, not four
@@ -348,11 +349,14 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
             sharing = std::max(sharing, n);
         }
         p.whole = (uint64_t)d.n_points * 8 * sharing <= kPart;
-        // parts of cut slices: a slice is cut where it holds more than run_part entries or
-        // its group more than kPart, so its parts are fewer than twice the quotients, and
-        // at most one more than they are
-        const uint64_t cuts = max_entries / p.run_part + (max_entries << p.group_shift) / kPart + 2;
-        p.max_parts = p.whole ? 0 : (uint32_t)(cuts + std::min<uint64_t>(cuts, p.n_slices));
+        // Parts of cut slices: a slice is cut where it holds more than run_part entries or
+        // its group more than kPart.  A group of g <= kPart entries then has at most
+        // 2 (g - 1) / run_part parts, a larger one, of two slices, at most
+        // 2 + (g - 1) / run_part + 2 (g - 1) / kPart, so at most (1 / run_part + 4 / kPart) g.
+        const uint64_t A = (max_entries + p.run_part - 1) / p.run_part, B = (max_entries + kPart - 1) / kPart;
+        const uint32_t shared = 1u << p.group_shift;  // slices of a group
+        const uint64_t dense = std::max<uint64_t>(2 * A, A + 2 * shared * B), sparse = p.n_slices + A + shared * B;
+        p.max_parts = p.whole ? 0 : (uint32_t)std::min(dense, sparse);
         p.runs_off = 0;
         p.slice_np_off = align(p.runs_off + 4 * runs);
         p.first_part_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
