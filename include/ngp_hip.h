@@ -381,6 +381,15 @@ typedef struct OccupancyGridUpdateDescriptor {
  *      be NULL, when update_all) */
 void occupancy_grid_update(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
+/* occupancy_grid_update by way of a workspace: the same densities, bit for bit, chosen,
+ * encoded and evaluated by kernels of their own over up to NGP_OGRID_STAGE_POINTS cells.
+ * in, inout, out: as occupancy_grid_update
+ * scratch: workspace u8[min(n, NGP_OGRID_STAGE_POINTS) rounded up to 64, times
+ *      NGP_OGRID_STAGE_BYTES], 16-byte aligned, for n = max(n_alive, 2) */
+#define NGP_OGRID_STAGE_POINTS (1u << 20)
+#define NGP_OGRID_STAGE_BYTES 144u
+void occupancy_grid_update_staged(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
 typedef struct NgpPoolScatterDescriptor {
     uint32_t n;       /* pool slots */
     uint32_t n_total; /* rows of dst */

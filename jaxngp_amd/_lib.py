@@ -49,6 +49,7 @@ TARGETS = (
     "loss_scale_update",
     "nerf_field_chunks",
     "occupancy_grid_update",
+    "occupancy_grid_update_staged",
     "pool_scatter",
     "proposal_points",
     "proposal_mlp_forward",
@@ -376,6 +377,16 @@ def pool_scatter_descriptor(n, n_total, width) -> bytes:
 def field_chunks_descriptor(grid_desc: bytes, n_slots, cap, n_total_rays, param_dtype=DTYPE_F32) -> bytes:
     """NerfFieldChunksDescriptor: a HashGridDescriptor followed by four u32."""
     return grid_desc + struct.pack("<4I", n_slots, cap, n_total_rays, param_dtype)
+
+
+OGRID_STAGE_POINTS = 1 << 20
+OGRID_STAGE_BYTES = 144
+
+
+def occupancy_update_workspace_bytes(n_alive: int) -> int:
+    """Workspace of occupancy_grid_update_staged."""
+    n = min(max(n_alive, 2), OGRID_STAGE_POINTS)
+    return (n + 63) // 64 * 64 * OGRID_STAGE_BYTES
 
 
 def occupancy_update_descriptor(grid_desc: bytes, G, K, cascade, n_alive, update_all, param_dtype, seed, step) -> bytes:

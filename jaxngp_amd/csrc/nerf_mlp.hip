@@ -234,8 +234,6 @@ __device__ __forceinline__ v4f sh4_part(float x, float y, float z, int g) {
     return v;
 }
 
-__device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + det_expf(-x)); }
-
 // The outputs of 16 samples: density from o0 and colour from rr[0..2] of lane (i, 0).
 // Lane (i, g) takes value g of sample i, one exponential each instead of four on a
 // quarter of the lanes.  Call with all lanes active; s is sample i's place.
@@ -246,6 +244,8 @@ __device__ __forceinline__ void store_drgbs(float *__restrict__ drgbs, size_t s,
     const float e = det_expf(g == 0 ? x : -x);
     if (live) drgbs[4 * s + g] = g == 0 ? e : 1.0f / (1.0f + e);
 }
+
+__device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + det_expf(-x)); }
 
 struct Fwd {
     v4f x[2], h1[4], c[2], h2[4], h3[4], rr;  // c[0] = o (density MLP output), c[1] = SH
@@ -844,7 +844,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         f.x[1] = in.x[1];
         forward_from_x_h(lds, in.dx, in.dy, in.dz, i, g, f);
         const v4f gin = in.gin;
-        v4f dr = zero;
+        v4f dr = {0.0f, 0.0f, 0.0f, 0.0f};
         float dsig = 0.0f;
         if (g == 0) {
 #pragma unroll
@@ -1176,6 +1176,21 @@ __device__ __forceinline__ void ogrid_point(const OgridArgs &a, uint32_t m, uint
     z = p[2];
 }
 
+// Cell m's new density sigma.
+__device__ __forceinline__ void ogrid_apply(const OgridArgs &a, uint32_t m, float sigma, float *__restrict__ density) {
+    const uint32_t G3 = a.G * a.G * a.G;
+    if (m >= G3) return;
+    float *dens = density + (size_t)a.cascade * G3;
+    if (a.update_all) {
+        // each alive cell is in exactly one slot: decay and max in place
+        dens[m] = max_nan(dens[m] * __uint_as_float(kDecayBits), sigma);
+    } else {
+        // decayed by ogrid_decay_kernel; densities of alive cells are >= +0 (or
+        // NaN), so the unsigned order of their bits is the float order, NaN on top
+        atomicMax(reinterpret_cast<unsigned int *>(dens + m), __float_as_uint(sigma));
+    }
+}
+
 template <typename TT, bool kHalf>
 __global__ void __launch_bounds__(kThreads)
     ogrid_update_kernel(HashGridDescriptor d, OgridArgs a, const uint32_t *__restrict__ alive,
@@ -1200,7 +1215,6 @@ __global__ void __launch_bounds__(kThreads)
     const Divisor two_b = make_divisor(2.0f * a.bound);
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t G3 = a.G * a.G * a.G;
-    float *dens = density + (size_t)a.cascade * G3;
     for (uint32_t t = wave; t < n_tiles; t += n_waves) {
         const uint32_t j = t * kTile + i;
         bool live = j < a.n_update;
@@ -1233,17 +1247,7 @@ __global__ void __launch_bounds__(kThreads)
             layer_fwd<64, 16, S_W2>(lds_f + L_W2, f.h1, &f.c[0], i, g);
             o0 = f.c[0][0];
         }
-        if (g == 0 && live) {
-            const float sigma = det_expf(o0);
-            if (a.update_all) {
-                // each alive cell is in exactly one slot: decay and max in place
-                dens[m] = max_nan(dens[m] * __uint_as_float(kDecayBits), sigma);
-            } else {
-                // decayed by ogrid_decay_kernel; densities of alive cells are >= +0 (or
-                // NaN), so the unsigned order of their bits is the float order, NaN on top
-                atomicMax(reinterpret_cast<unsigned int *>(dens + m), __float_as_uint(sigma));
-            }
-        }
+        if (g == 0 && live) ogrid_apply(a, m, det_expf(o0), density);
     }
 }
 
@@ -1255,22 +1259,93 @@ __global__ void __launch_bounds__(256) ogrid_decay_kernel(uint32_t n_alive, uint
     if (m < G3) dens[m] = dens[m] * __uint_as_float(kDecayBits);
 }
 
-// prefix[w] = occupied cells in the cascade's 64-cell words [0, w), w = 0..W
-// (one workgroup; each thread counts a run of consecutive words).
+// prefix[w] = occupied cells in the cascade's 64-cell words [0, w), w = 0..W.  A workgroup
+// counts the words before its run by itself, which is less than waiting for the others
+// (one workgroup, a run of words per thread: 60 us for G = 128; 32 of them: 17).
 constexpr int kPrefixThreads = 1024;
+constexpr uint32_t kPrefixBlocks = 64;
 __global__ void __launch_bounds__(kPrefixThreads)
     ogrid_prefix_kernel(uint32_t W, const uint64_t *__restrict__ words, uint32_t *__restrict__ prefix) {
-    const uint32_t per = (W + kPrefixThreads - 1) / kPrefixThreads;
-    const uint32_t w0 = min(W, threadIdx.x * per), w1 = min(W, w0 + per);
-    uint32_t own = 0;
-    for (uint32_t w = w0; w < w1; ++w) own += (uint32_t)__popcll(words[w]);
-    uint32_t total = 0;
-    uint32_t run = block_exclusive_scan<kPrefixThreads>(own, &total);
-    for (uint32_t w = w0; w < w1; ++w) {
-        prefix[w] = run;
-        run += (uint32_t)__popcll(words[w]);
+    const uint32_t per = (W + gridDim.x - 1) / gridDim.x;
+    const uint32_t w0 = min(W, blockIdx.x * per), w1 = min(W, w0 + per);
+    if (w0 == w1) return;
+    uint32_t own = 0, carry = 0;
+    for (uint32_t w = threadIdx.x; w < w0; w += kPrefixThreads) own += (uint32_t)__popcll(words[w]);
+    block_exclusive_scan<kPrefixThreads>(own, &carry);
+    for (uint32_t base = w0; base < w1; base += kPrefixThreads) {
+        const uint32_t w = base + threadIdx.x;
+        uint32_t total = 0;
+        const uint32_t before =
+            block_exclusive_scan<kPrefixThreads>(w < w1 ? (uint32_t)__popcll(words[w]) : 0u, &total);
+        if (w < w1) prefix[w] = carry + before;
+        carry += total;
     }
-    if (threadIdx.x == 0) prefix[W] = total;
+    if (w1 == W && threadIdx.x == 0) prefix[W] = carry;
+}
+
+// The staged update, in three kernels over up to NGP_OGRID_STAGE_POINTS slots: a thread per
+// slot chooses its cell and point, hashgrid_encode gathers level by level, and the density
+// MLP runs on its encodings.  The points are random, so the gathers miss: the fused kernel
+// waits for them with two wavefronts per SIMD on all levels' rows at once, and its four
+// lanes of a sample each search the occupied cells.  2^20 cells, T = 2^19: f32 1087 -> 420 us,
+// f16 881 -> 370.
+__global__ void __launch_bounds__(256)
+    ogrid_points_kernel(OgridArgs a, uint32_t j0, uint32_t n, const uint32_t *__restrict__ alive,
+                        const uint32_t *__restrict__ prefix, const uint64_t *__restrict__ words,
+                        uint32_t *__restrict__ cells, float *__restrict__ pos) {
+    const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+    if (k >= n) return;
+    const uint32_t m = ogrid_cell(a, j0 + k, alive, prefix, words);
+    float at[3] = {0.0f, 0.0f, 0.0f};
+    if (m < a.G * a.G * a.G) ogrid_point(a, m, j0 + k, at[0], at[1], at[2]);
+    cells[k] = m;  // past the cascade: dropped, as JAX drops it
+    pos[3 * (size_t)k + 0] = at[0];
+    pos[3 * (size_t)k + 1] = at[1];
+    pos[3 * (size_t)k + 2] = at[2];
+}
+
+template <bool kHalf>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+    ogrid_density_kernel(OgridArgs a, uint32_t n, const uint32_t *__restrict__ cells, const float *__restrict__ enc,
+                         const void *__restrict__ params, float *__restrict__ density) {
+    __shared__ __align__(16) float lds_f[kHalf ? 4 : F_W3];
+    __shared__ __align__(16) _Float16 lds_h[kHalf ? H_FEND : 8];
+    if (kHalf) {
+        stage_weights_h<false>(lds_h, static_cast<const _Float16 *>(params));
+    } else {
+        const float *w = static_cast<const float *>(params);
+        stage_transposed<32, 64, 64>(lds_f + F_W1, w + P_W1);
+        stage_transposed<64, 16, 16>(lds_f + F_W2, w + P_W2);
+        __syncthreads();
+    }
+    const int lane = lane_id();
+    const int i = lane & 15, g = lane >> 4;
+    const uint32_t n_tiles = (n + kTile - 1) / kTile;
+    const uint32_t wave = blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    for (uint32_t t = wave; t < n_tiles; t += gridDim.x * kWaves) {
+        const uint32_t k = t * kTile + i, kc = min(k, n - 1u);
+        v4f x[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) x[b] = load_enc4(enc, true, n, kc, b, g);
+        const uint32_t m = cells[kc];
+        float o0;
+        if (kHalf) {
+            FwdH f;
+            const h8 xin = pack_h8(x[0], x[1]);
+            layer_fwd_h<1, 4, FT1>(lds_h + H_F1, &xin, f.h1, i, g);
+            relu<4>(f.h1);
+            const h8 h1in[2] = {pack_h8(f.h1[0], f.h1[1]), pack_h8(f.h1[2], f.h1[3])};
+            layer_fwd_h<2, 1, FT2>(lds_h + H_F2, h1in, &f.c[0], i, g);
+            o0 = f.c[0][0];
+        } else {
+            Fwd f;
+            layer_fwd_t<32, 64>(lds_f + F_W1, x, f.h1, i, g);
+            relu<4>(f.h1);
+            layer_fwd_t<64, 16>(lds_f + F_W2, f.h1, &f.c[0], i, g);
+            o0 = f.c[0][0];
+        }
+        if (g == 0 && k < n) ogrid_apply(a, m, det_expf(o0), density);
+    }
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1493,27 +1568,32 @@ extern "C" void nerf_field_chunks(ngp_stream_t stream, void **buffers, const cha
     check_launch(target);
 }
 
-extern "C" void occupancy_grid_update(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
-    const char *target = "occupancy_grid_update";
-    OccupancyGridUpdateDescriptor d;
-    if (!read_descriptor(opaque, opaque_len, &d, target)) return;
+namespace ngp {
+namespace {
+
+// The checks of both occupancy-grid updates, and the decay and prefix launches: false if
+// there is nothing (more) to do.
+bool begin_ogrid_update(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len, const char *target,
+                        OccupancyGridUpdateDescriptor *out, OgridArgs *args) {
+    OccupancyGridUpdateDescriptor &d = *out;
+    OgridArgs &a = *args;
+    if (!read_descriptor(opaque, opaque_len, &d, target)) return false;
     const HashGridDescriptor &g = d.grid;
-    if (!check_nerf_grid(g, d.param_dtype, target)) return;
+    if (!check_nerf_grid(g, d.param_dtype, target)) return false;
     if (d.G < 4 || d.G > 1024 || (d.G & (d.G - 1u)) != 0 || d.K == 0 || d.cascade >= d.K || d.update_all > 1 ||
         (uint64_t)d.n_alive > (uint64_t)d.G * d.G * d.G) {
         set_error(kBadDescriptor, "%s: G must be a power of two in [4, 1024], cascade < K, update_all 0 or 1, "
                   "n_alive <= G^3", target);
-        return;
+        return false;
     }
-    if (d.n_alive == 0) return;  // no alive cell: nothing to decay or update
-    if (!check_buffers(buffers, 5, target)) return;
-    if (!d.update_all && !check_buffer_list(buffers, {5}, target)) return;
+    if (d.n_alive == 0) return false;  // no alive cell: nothing to decay or update
+    if (!check_buffers(buffers, 5, target)) return false;
+    if (!d.update_all && !check_buffer_list(buffers, {5}, target)) return false;
     if ((reinterpret_cast<uintptr_t>(buffers[1]) & 7u) != 0) {
         set_error(kBadArgument, "%s: the occupancy bitfield must be 8-byte aligned", target);
-        return;
+        return false;
     }
     hipStream_t s = (hipStream_t)stream;
-    OgridArgs a;
     a.G = d.G;
     a.cascade = d.cascade;
     a.n_alive = d.n_alive;
@@ -1523,35 +1603,77 @@ extern "C" void occupancy_grid_update(ngp_stream_t stream, void **buffers, const
     a.bound = g.bound;
     a.mip = std::fmin(g.bound, std::ldexp(1.0f, (int)std::min<uint32_t>(d.cascade, 126u)));
     a.hcw = a.mip / (float)d.G;
-    const uint32_t *alive = (const uint32_t *)buffers[0];
-    const uint64_t *words = (const uint64_t *)buffers[1];
-    float *density = (float *)buffers[4];
-    uint32_t *prefix = (uint32_t *)buffers[5];
-    const uint32_t W = d.G * d.G * d.G / 64u;  // 64-cell words per cascade
     if (a.update_all) {
         a.n_update = d.n_alive;
         a.half = 0;
-        prefix = nullptr;
-    } else {
-        const uint32_t M = std::max<uint32_t>(1, d.n_alive / 2), h = std::max<uint32_t>(1, M / 2);
-        a.n_update = 2 * h;
-        a.half = h;
-        float *dens = density + (size_t)d.cascade * d.G * d.G * d.G;
-        hipLaunchKernelGGL(ogrid_decay_kernel, dim3(div_up(d.n_alive, 256)), dim3(256), 0, s, d.n_alive,
-                           d.G * d.G * d.G, alive, dens);
-        if (!check_launch(target)) return;
-        hipLaunchKernelGGL(ogrid_prefix_kernel, dim3(1), dim3(kPrefixThreads), 0, s, W, words + (size_t)d.cascade * W,
-                           prefix);
-        if (!check_launch(target)) return;
+        return true;
     }
+    const uint32_t *alive = (const uint32_t *)buffers[0];
+    const uint32_t W = d.G * d.G * d.G / 64u;  // 64-cell words per cascade
+    const uint64_t *words = (const uint64_t *)buffers[1] + (size_t)d.cascade * W;
+    const uint32_t M = std::max<uint32_t>(1, d.n_alive / 2), h = std::max<uint32_t>(1, M / 2);
+    a.n_update = 2 * h;
+    a.half = h;
+    float *dens = (float *)buffers[4] + (size_t)d.cascade * d.G * d.G * d.G;
+    hipLaunchKernelGGL(ogrid_decay_kernel, dim3(div_up(d.n_alive, 256)), dim3(256), 0, s, d.n_alive,
+                       d.G * d.G * d.G, alive, dens);
+    if (!check_launch(target)) return false;
+    hipLaunchKernelGGL(ogrid_prefix_kernel, dim3(std::min(div_up(W, kPrefixThreads), kPrefixBlocks)),
+                       dim3(kPrefixThreads), 0, s, W, words, (uint32_t *)buffers[5]);
+    return check_launch(target);
+}
+
+}  // namespace
+}  // namespace ngp
+
+extern "C" void occupancy_grid_update(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
+    const char *target = "occupancy_grid_update";
+    OccupancyGridUpdateDescriptor d;
+    OgridArgs a;
+    if (!begin_ogrid_update(stream, buffers, opaque, opaque_len, target, &d, &a)) return;
+    const HashGridDescriptor &g = d.grid;
     const uint32_t tiles = div_up(a.n_update, kTile);
     const uint32_t grid = std::max<uint32_t>(1, std::min<uint32_t>(div_up(tiles, kWaves), 2048));
-    const void *params = buffers[3];
     const bool t16 = g.table_dtype == NGP_DTYPE_F16, w16 = d.param_dtype == NGP_DTYPE_F16;
     with_field_types(t16, w16, [&](auto tt, auto half) {
         using TT = typename decltype(tt)::type;
-        hipLaunchKernelGGL((ogrid_update_kernel<TT, decltype(half)::value>), dim3(grid),
-                           dim3(kThreads), 0, s, g, a, alive, prefix, words, (const TT *)buffers[2], params, density);
+        hipLaunchKernelGGL((ogrid_update_kernel<TT, decltype(half)::value>), dim3(grid), dim3(kThreads), 0,
+                           (hipStream_t)stream, g, a, (const uint32_t *)buffers[0],
+                           a.update_all ? nullptr : (const uint32_t *)buffers[5], (const uint64_t *)buffers[1],
+                           (const TT *)buffers[2], buffers[3], (float *)buffers[4]);
     });
     check_launch(target);
+}
+
+extern "C" void occupancy_grid_update_staged(ngp_stream_t stream, void **buffers, const char *opaque,
+                                             size_t opaque_len) {
+    const char *target = "occupancy_grid_update_staged";
+    OccupancyGridUpdateDescriptor d;
+    OgridArgs a;
+    if (!begin_ogrid_update(stream, buffers, opaque, opaque_len, target, &d, &a)) return;
+    if (!check_buffer_list(buffers, {6}, target)) return;
+    if (!aligned16(buffers[6])) {
+        set_error(kBadArgument, "%s: the workspace must be 16-byte aligned", target);
+        return;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    const uint32_t most = std::min<uint32_t>(a.n_update, NGP_OGRID_STAGE_POINTS), room = (most + 63u) / 64u * 64u;
+    float *enc = (float *)buffers[6], *pos = enc + 32 * (size_t)room;
+    uint32_t *cells = (uint32_t *)(pos + 3 * (size_t)room);
+    for (uint32_t j0 = 0; j0 < a.n_update; j0 += most) {
+        const uint32_t n = std::min(most, a.n_update - j0);
+        hipLaunchKernelGGL(ogrid_points_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, a, j0, n,
+                           (const uint32_t *)buffers[0], a.update_all ? nullptr : (const uint32_t *)buffers[5],
+                           (const uint64_t *)buffers[1], cells, pos);
+        if (!check_launch(target)) return;
+        HashGridDescriptor g = d.grid;
+        g.n_points = n;
+        g.enc_layout = NGP_ENC_LEVEL_MAJOR;
+        void *encode[3] = {pos, buffers[2], enc};
+        hashgrid_encode(stream, encode, reinterpret_cast<const char *>(&g), sizeof g);
+        const uint32_t grid = std::min<uint32_t>(div_up(div_up(n, kTile), kWaves), 2048);
+        const auto kernel = d.param_dtype == NGP_DTYPE_F16 ? ogrid_density_kernel<true> : ogrid_density_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, s, a, n, cells, enc, buffers[3], (float *)buffers[4]);
+        if (!check_launch(target)) return;
+    }
 }

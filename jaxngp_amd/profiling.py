@@ -43,8 +43,8 @@ TARGET_KERNELS = {
     "nerf_mlp_backward": (["mlp_backward_kernel", "mlp_backward_h_kernel", "sum_rows_kernel"], "sum_rows_kernel"),
     "integrate_rays": (["integrate_kernel"], "integrate_kernel"),
     "integrate_rays_backward": (["integrate_backward_kernel", "fill_zero2_kernel"], "integrate_backward_kernel"),
-    "occupancy_grid_update": (["ogrid_update_kernel", "ogrid_decay_kernel", "ogrid_prefix_kernel"],
-                              "ogrid_update_kernel"),
+    "occupancy_grid_update": (["ogrid_update_kernel", "ogrid_decay_kernel", "ogrid_prefix_kernel",
+                               "ogrid_points_kernel", "ogrid_density_kernel"], "ogrid_decay_kernel"),
     "proposal_train_samples": (["proposal_train_kernel", "proposal_train_scan_kernel", "proposal_train_write_kernel",
                                 "proposal_train_tail_kernel"], "proposal_train_scan_kernel"),
 }

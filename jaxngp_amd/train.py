@@ -354,13 +354,13 @@ class Trainer:
                        for c in range(K)]
 
     def update_ogrid_density(self, cas: int, update_all: bool, max_inference: int | None = None):
-        """types.py:1149-1225 for cascade `cas`, in one fused launch
-        (occupancy_grid_update): decay the alive cells by 0.95, then max each chosen
+        """types.py:1149-1225 for cascade `cas`
+        (occupancy_grid_update_staged): decay the alive cells by 0.95, then max each chosen
         cell's density with the field's density at a random point of the cell (every
         alive cell when `update_all`, else half uniform over the alive cells and half
         uniform over the occupied ones).  `max_inference` (the reference's chunk size
-        for its field evaluations) is accepted and not needed: the kernel evaluates
-        every chosen cell in one launch."""
+        for its field evaluations) is accepted and not needed: the target evaluates
+        2^20 cells at a time in a workspace that holds them."""
         g = self.grid
         alive = g.alive_cas[cas]
         if alive.numel() == 0:
@@ -372,7 +372,9 @@ class Trainer:
         desc = _lib.occupancy_update_descriptor(
             enc.descriptor(0, self.bound), g.G, g.K, cas, alive.numel(), update_all,
             _lib.DTYPE_F16 if w16 else _lib.DTYPE_F32, self.cfg.seed ^ OGRID_SEED_TAG, self.step_count)
-        _lib.call("occupancy_grid_update", [alive, g.bitfield, enc.table.detach(), params, g.density, g.prefix], desc)
+        ws = torch.empty(_lib.occupancy_update_workspace_bytes(alive.numel()), dtype=torch.uint8, device=alive.device)
+        _lib.call("occupancy_grid_update_staged",
+                  [alive, g.bitfield, enc.table.detach(), params, g.density, g.prefix, ws], desc)
 
     def threshold_ogrid(self):
         """types.py:1227-1239."""

@@ -180,3 +180,36 @@ def test_full_grid_equals_unfused_chain(dev):
         dirs = torch.zeros(G3, 3, device=dev)
         sig = nerf_mlp(e, dirs, params_dev)[:, 0].cpu().numpy()
     np.testing.assert_array_equal(got[cells], np.maximum(np.float32(0), sig))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("G, K, cas, n_alive, update_all", [(4, 1, 0, 1, 0), (16, 2, 1, 37, 0), (32, 1, 0, 20000, 1),
+                                                            (128, 1, 0, 1 << 21, 1), (128, 1, 0, 1 << 21, 0)])
+def test_staged_update_equals_the_fused_one(dev, G, K, cas, n_alive, update_all, f16):
+    """occupancy_grid_update_staged against occupancy_grid_update, bit for bit (the same draws,
+    encoder and products): fewer cells than a tile, a partial tile, one chunk, several chunks."""
+    rng = np.random.default_rng([G, n_alive])
+    enc, _, _, params, _ = _field(dev, 1 << 16, 11, table_dtype=torch.float16 if f16 else torch.float32)
+    G3 = G ** 3
+    alive_c = np.sort(rng.choice(G3, n_alive, replace=False)).astype(np.int32)
+    density = torch.from_numpy(rng.uniform(0, 1, K * G3).astype(np.float32)).to(dev)
+    bits = torch.from_numpy(rng.integers(0, 256, K * G3 // 8).astype(np.uint8)).to(dev)
+    w = params.half() if f16 else params
+    desc = _lib.occupancy_update_descriptor(enc.descriptor(0, 1.0), G, K, cas, n_alive, update_all,
+                                            _lib.DTYPE_F16 if f16 else _lib.DTYPE_F32, SEED, STEP)
+    got = []
+    for target in ("occupancy_grid_update", "occupancy_grid_update_staged"):
+        dens = density.clone()
+        prefix = torch.full((G3 // 64 + 1,), -1, dtype=torch.int32, device=dev)
+        buffers = [torch.from_numpy(alive_c).to(dev), bits, enc.table.detach(), w, dens, prefix]
+        if target.endswith("staged"):
+            buffers.append(torch.empty(_lib.occupancy_update_workspace_bytes(n_alive), dtype=torch.uint8, device=dev))
+        _lib.call(target, buffers, desc)
+        got.append((dens, prefix))
+    assert not torch.equal(got[0][0], density)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    if not update_all:
+        words = bits.cpu().numpy().reshape(K, -1)[cas].view("<u8")
+        pop = np.array([bin(int(x)).count("1") for x in words], np.int64)
+        np.testing.assert_array_equal(got[1][1].cpu().numpy(), np.concatenate([[0], np.cumsum(pop)]))
