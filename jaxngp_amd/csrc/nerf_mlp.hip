@@ -245,7 +245,23 @@ __device__ __forceinline__ void store_drgbs(float *__restrict__ drgbs, size_t s,
     if (live) drgbs[4 * s + g] = g == 0 ? e : 1.0f / (1.0f + e);
 }
 
-__device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + det_expf(-x)); }
+// The output gradients gin of sample i (in every lane (i, g)) before the activations: of
+// the colours in dr[0..2] of lane (i, 0), of the density in its dsig; dr is 0 in the other
+// lanes.  As in store_drgbs lane (i, g) takes value g.
+__device__ __forceinline__ void head_gradient(const v4f &gin, float o0, const v4f &rr, int i, int g, v4f &dr, float &dsig) {
+    const float a = __shfl(o0, i), b = __shfl(rr[0], i), c = __shfl(rr[1], i), d = __shfl(rr[2], i);
+    const float x = g == 1 ? b : g == 2 ? c : d, up = g == 0 ? gin[0] : g == 1 ? gin[1] : g == 2 ? gin[2] : gin[3];
+    const float e = det_expf(g == 0 ? fminf(fmaxf(a, -15.0f), 15.0f) : -x);
+    const float y = 1.0f / (1.0f + e);
+    dsig = up * e;
+    const float v = up * y * (1.0f - y);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float t = __shfl(v, kTile * (k + 1) + i);
+        dr[k] = g == 0 ? t : 0.0f;
+    }
+    dr[3] = 0.0f;
+}
 
 struct Fwd {
     v4f x[2], h1[4], c[2], h2[4], h3[4], rr;  // c[0] = o (density MLP output), c[1] = SH
@@ -488,16 +504,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         forward_from_x(lds, in.dx, in.dy, in.dz, i, g, f);
         const v4f gin = in.gin;
         // colour head: d(pre-sigmoid), features 0..2 live in lanes g == 0
-        v4f dr = {0.0f, 0.0f, 0.0f, 0.0f};
-        float dsig = 0.0f;
-        if (g == 0) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const float y = sigmoidf(f.rr[c]);
-                dr[c] = gin[c + 1] * y * (1.0f - y);
-            }
-            dsig = gin[0] * det_expf(fminf(fmaxf(f.c[0][0], -15.0f), 15.0f));
-        }
+        v4f dr;
+        float dsig;
+        head_gradient(gin, f.c[0][0], f.rr, i, g, dr, dsig);
         // W5
         tile_to_lds<4>(zs, f.h3, i, g);
         tile_to_lds<1>(ys, &dr, i, g);
@@ -844,16 +853,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         f.x[1] = in.x[1];
         forward_from_x_h(lds, in.dx, in.dy, in.dz, i, g, f);
         const v4f gin = in.gin;
-        v4f dr = {0.0f, 0.0f, 0.0f, 0.0f};
-        float dsig = 0.0f;
-        if (g == 0) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const float y = sigmoidf(f.rr[c]);
-                dr[c] = gin[c + 1] * y * (1.0f - y);
-            }
-            dsig = gin[0] * det_expf(fminf(fmaxf(f.c[0][0], -15.0f), 15.0f));
-        }
+        v4f dr;
+        float dsig;
+        head_gradient(gin, f.c[0][0], f.rr, i, g, dr, dsig);
         // W5
         tile_to_lds_h<4>(zs, f.h3, i, g);
         tile_to_lds_h<1>(ys, &dr, i, g);
