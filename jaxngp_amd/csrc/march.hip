@@ -113,7 +113,9 @@ struct Window {
     float exit;     // exit distance of its cell
     uint64_t word;  // the occupancy word (or byte) of its cell
     uint32_t bit;   // its bit there
+    uint32_t cell;  // its index
     bool live;      // w < t_end
+    bool clear;     // kOne: no plane of the grid within the rounding error (see march_ray_wave)
     // the same in all lanes
     float base, next;  // c_0, c_64
     bool stall;        // the chain stops growing
@@ -171,15 +173,19 @@ __device__ __forceinline__ void chain_window(const MarchParams &p, bool const_st
 }
 
 // The window starting at `base`, its occupancy load issued.  Call with all lanes active.
+template <bool kOne>
 __device__ __forceinline__ Window make_window(const MarchParams &p, const uint8_t *__restrict__ bits, bool word_ok,
-                                              const Ray &r, bool const_step, float k_step, float base) {
+                                              const Ray &r, bool const_step, float k_step, float margin, float base) {
     Window v;
     v.base = base;
     chain_window(p, const_step, k_step, base, v.w, v.next, v.stall);
     v.live = v.w < r.t1;
     const float px = r.ox + v.w * r.dx, py = r.oy + v.w * r.dy, pz = r.oz + v.w * r.dz;
     float gx, gy, gz, mb;
-    const uint32_t idx = cell_index(p, px, py, pz, step_size(p, v.w), gx, gy, gz, mb);
+    const uint32_t idx = cell_index<kOne>(p, px, py, pz, step_size(p, v.w), gx, gy, gz, mb);
+    v.cell = idx;
+    v.clear = kOne && fmaxf(fabsf(gx - floorf(gx) - 0.5f), fmaxf(fabsf(gy - floorf(gy) - 0.5f),
+                                                                 fabsf(gz - floorf(gz) - 0.5f))) <= 0.5f - margin;
     v.word = 0ull;
     if (word_ok) {
         v.bit = idx & 63u;
@@ -200,7 +206,14 @@ __device__ __forceinline__ float lane_float(float v, int lane) {
 // taking at most cap samples (kWrite: also writes their t; with a record: also keeps
 // it).  Call with all 64 lanes active.  The next window is made, its occupancy load in flight, before this
 // one is walked.
-template <bool kWrite>
+// kOne (a grid of one cascade): the walk crosses a stretch of empty cells at once instead of
+// cell by cell.  Every visited element of a cell has the same exit but for rounding, and the
+// next visited one is the first past it: the first element of the next cell, unless an
+// element lies within the rounding error of a plane between cells, on either side or as a
+// cell's index and exit see it.  So if no element of the window does (`clear`; nine windows
+// in ten), the walk takes the first element of the last empty cell before the next
+// occupied one, and its exit.
+template <bool kWrite, bool kOne>
 __device__ uint32_t march_ray_wave(const MarchParams &p, const uint8_t *__restrict__ bits, bool word_ok, const Ray &r,
                                    float t_start, uint32_t cap, const RaySamples &o, const RayRecord &rec) {
     const int lane = lane_id();
@@ -216,7 +229,13 @@ __device__ uint32_t march_ray_wave(const MarchParams &p, const uint8_t *__restri
         if (rec.words != nullptr && lane == 0) rec.words[0] = 0u;
         return 0;
     }
-    Window v = make_window(p, bits, word_ok, r, const_step, k_step, t_start);
+    // A position carries up to 2^-24 (|o| + t|d| + 1) on an axis, an exit distance that, its
+    // own roundings of as much and the position's again, over |d|: less than 2^-21 of the sum
+    // in all, here in cells.
+    const float reach = fmaxf(fabsf(r.ox) + fabsf(r.t1 * r.dx),
+                              fmaxf(fabsf(r.oy) + fabsf(r.t1 * r.dy), fabsf(r.oz) + fabsf(r.t1 * r.dz)));
+    const float margin = 4.7683716e-7f * (reach + 2.0f) * (0.5f * (float)p.G) / fminf(1.0f, p.bound);
+    Window v = make_window<kOne>(p, bits, word_ok, r, const_step, k_step, margin, t_start);
     for (;;) {
         if (v.stall) {
             // the chain stops growing at or after `base`: the serial loop on one lane
@@ -243,10 +262,18 @@ __device__ uint32_t march_ray_wave(const MarchParams &p, const uint8_t *__restri
         const uint64_t live_m = __ballot(v.live);
         const bool last = (live_m >> (kWave - 1)) == 0ull;  // the chain reaches t_end here
         Window next;
-        if (!last) next = make_window(p, bits, word_ok, r, const_step, k_step, v.next);
+        if (!last) next = make_window<kOne>(p, bits, word_ok, r, const_step, k_step, margin, v.next);
         const uint64_t occ_m = __ballot(v.live && ((v.word >> v.bit) & 1ull));
         const uint32_t n0 = n;
-        uint64_t emit = 0ull;
+        uint64_t emit = 0ull, starts = 0ull;  // first elements of cells
+        bool clear = false;
+        if constexpr (kOne) {
+            constexpr int kWaveShr1 = 0x138;
+            const uint32_t before =
+                (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v.cell, kWaveShr1, 0xf, 0xf, false);
+            starts = __ballot(v.cell != before);
+            clear = __ballot(v.live && !v.clear) == 0ull;
+        }
         int cur = 0;
         while (cur < kWave) {
             if (pending) {
@@ -266,6 +293,11 @@ __device__ uint32_t march_ray_wave(const MarchParams &p, const uint8_t *__restri
                 if (n >= cap) break;
                 cur += run;
             } else {
+                if (kOne && clear) {
+                    const uint64_t ahead = occ_m >> cur;
+                    const uint64_t upto = ahead == 0ull ? ~0ull : (1ull << (cur + __builtin_ctzll(ahead))) - 1ull;
+                    cur = max(cur, kWave - 1 - __builtin_clzll((starts & upto) | 1ull));
+                }
                 thr = lane_float(v.exit, cur);
                 pending = true;
                 cur += 1;
@@ -317,9 +349,13 @@ __device__ __forceinline__ RayRecord record_of(const RecordStore &st, uint32_t i
 // are short of total_samples; what it reads too early costs a block marched in vain, no
 // more.  (Drawing rays from one shared counter instead cost a device atomic on one
 // address per ray, about 10 ns each one after another: 4096 rays took 114 us.)
-// The march is bound by one ray's latency, a chain of windows of about 350
+// The march is bound by one ray's latency, a chain of windows of about 250
 // instructions: few wavefronts in flight lose little and march few rays past the fill.
-// 2^18 rays, total_samples 2^18 filled by the first 3300: MARCH_NOTE.
+// march_rays of 2^18 camera rays, about 20 samples each, into 2^18 slots: 552 us with
+// launches of growing size, 221 in rounds, 146 with empty stretches crossed at once; 4,096
+// rays into more slots than they fill: 292, 149, 101.  (Rounds of 4,096 rays take 162
+// instead of 152, and beside a training step's MLP backward 21 us of the step.)
+template <bool kOne>
 __global__ void __launch_bounds__(kBlock)
     march_count_kernel(MarchParams p, bool word_ok, uint32_t n_rays, uint32_t total_samples, uint32_t block_begin,
                        uint32_t block_end, uint32_t first_counter, const float *__restrict__ rays_o,
@@ -350,7 +386,7 @@ __global__ void __launch_bounds__(kBlock)
             const float t0 = t_starts[i], t1 = t_ends[i];
             if (t1 > t0) {
                 const Ray r = load_ray(rays_o, rays_d, i, t1);
-                n = march_ray_wave<false>(p, bits, word_ok, r, start_t(p, t0, noises[i]), p.n_cap, RaySamples{},
+                n = march_ray_wave<false, kOne>(p, bits, word_ok, r, start_t(p, t0, noises[i]), p.n_cap, RaySamples{},
                                           record_of(records, i));
             }
             if (lane == 0) rays_n_samples[i] = min(n, kPastFill - 1u);
@@ -512,6 +548,7 @@ __device__ __forceinline__ uint64_t ray_start(const uint32_t *__restrict__ rays_
 // where it has none.  Stops at the first ray whose block prefix reaches
 // total_samples (every later ray is past the filled buffer).  Runs before
 // march_finish_kernel overwrites the block slots.
+template <bool kOne>
 __global__ void __launch_bounds__(kBlock)
     march_emit_kernel(MarchParams p, bool word_ok, uint32_t n_rays, uint32_t total_samples,
                       const float *__restrict__ rays_o, const float *__restrict__ rays_d,
@@ -543,7 +580,7 @@ __global__ void __launch_bounds__(kBlock)
                 }
             } else {
                 const Ray r = load_ray(rays_o, rays_d, i, t1);
-                march_ray_wave<true>(p, bits, word_ok, r, start_t(p, t0, noises[i]), min(p.n_cap, n),
+                march_ray_wave<true, kOne>(p, bits, word_ok, r, start_t(p, t0, noises[i]), min(p.n_cap, n),
                                      RaySamples{zs + s}, RayRecord{nullptr, 0u});
             }
         }
@@ -1029,6 +1066,7 @@ extern "C" void march_rays(ngp_stream_t stream_, void **buffers, const char *opa
         check_launch(target);
         return;
     }
+    const bool one = d.K == 1;
     const uint32_t n_blocks = div_up(d.n_rays, kRaysPerBlock);
     constexpr uint32_t kMaxCountBlocks = 2048;
     hipLaunchKernelGGL(march_begin_kernel, dim3(std::min(div_up(d.n_rays, kBlock), 2048u)), dim3(kBlock), 0, stream,
@@ -1047,7 +1085,7 @@ extern "C" void march_rays(ngp_stream_t stream_, void **buffers, const char *opa
     for (int c = 0; c < 2; ++c) {
         const uint32_t begin = c == 0 ? 0 : first_end, end = c == 0 ? first_end : n_blocks;
         if (end <= begin) continue;
-        hipLaunchKernelGGL(march_count_kernel, dim3(std::min(end - begin, c == 0 ? kFirstBlocks : kMaxCountBlocks)),
+        hipLaunchKernelGGL(one ? march_count_kernel<true> : march_count_kernel<false>, dim3(std::min(end - begin, c == 0 ? kFirstBlocks : kMaxCountBlocks)),
                            dim3(kBlock), 0, stream, p, word_ok, d.n_rays, d.total_samples, begin, end,
                            c == 0 ? 0 : kFirstRounds, rays_o, rays_d, t_starts, t_ends, noises, bits, rec, n_samples,
                            startidx);
@@ -1056,7 +1094,7 @@ extern "C" void march_rays(ngp_stream_t stream_, void **buffers, const char *opa
     hipLaunchKernelGGL(march_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, d.n_rays, n_blocks, d.total_samples,
                        n_samples, startidx, next_loc, exceeded);
     if (!check_launch(target)) return;
-    hipLaunchKernelGGL(march_emit_kernel, dim3(std::min(n_blocks, kMaxCountBlocks)), dim3(kBlock), 0, stream, p, word_ok,
+    hipLaunchKernelGGL(one ? march_emit_kernel<true> : march_emit_kernel<false>, dim3(std::min(n_blocks, kMaxCountBlocks)), dim3(kBlock), 0, stream, p, word_ok,
                        d.n_rays, d.total_samples, rays_o, rays_d, t_starts, t_ends, noises, bits, rec,
                        n_samples, startidx, zs);
     if (!check_launch(target)) return;

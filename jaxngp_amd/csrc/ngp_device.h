@@ -121,10 +121,12 @@ __device__ __forceinline__ bool occupied(BitCache &c, const uint8_t *__restrict_
 
 // Occupancy cell of one position (marching.cu:79-98 and 170-176): its index in the
 // bitfield, the float grid coordinate and the mip bound used by the empty-cell skip.
+// kOne: the grid has one cascade.
+template <bool kOne = false>
 __device__ __forceinline__ uint32_t cell_index(const MarchParams &p, float px, float py, float pz, float ds, float &gx,
                                                float &gy, float &gz, float &mip_bound) {
     uint32_t cascade = 0;
-    if (p.K > 1) {
+    if (!kOne && p.K > 1) {
         float m = fmaxf(fabsf(px), fmaxf(fabsf(py), fabsf(pz)));
         uint32_t c1 = clamp_cascade(frexp_exp(m), p.K);
         uint32_t c2 = clamp_cascade(frexp_exp(ds * (float)p.G), p.K);

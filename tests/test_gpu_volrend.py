@@ -242,6 +242,28 @@ def test_march_rays_inference_constant_step_one_cascade(dev, kind, G, diag, boun
         nri, idx, term = np.array([want["next_ray_index"]], np.uint32), want["indices"], np.zeros(n, bool)
 
 
+@pytest.mark.parametrize("G, diag, bound, portion", [(4, 64, 1.0, 0.0), (64, 1024, 1.0, 0.0), (128, 333, 0.7, 0.0),
+                                                     (128, 512, 3.0, 1 / 256)])
+@pytest.mark.parametrize("kind", ["axis", "graze", "inside", "far"])
+def test_march_rays_one_cascade_edges(dev, kind, G, diag, bound, portion):
+    """The walk that crosses stretches of empty cells at once against the step-by-step oracle,
+    every output bit for bit, on rays along and through planes of the grid; samples enough for
+    several rounds of rays, the last of them partial, and for a buffer that fills."""
+    rng = np.random.default_rng([G, len(kind), diag])
+    n = 9003
+    o, d = _crossing_rays(rng, n, G, kind)
+    o *= np.float32(bound)
+    t0 = rng.uniform(0.0, 1.0, n).astype(np.float32)
+    t1 = (t0 + rng.uniform(0.0, 5.5, n)).astype(np.float32)
+    noise = rng.uniform(0, 1, n).astype(np.float32)
+    filled = rng.random(G ** 3 // 64) < 0.3  # blocks: 64 cells in Morton order
+    filled[0] = True
+    bits = np.packbits(np.repeat(filled, 64) & (rng.random(G ** 3) < 0.7), bitorder="little")
+    for total in (1 << 14, 1 << 21):
+        got, want = _march_both(dev, total, diag, 1, G, bound, portion, o, d, t0, t1, noise, bits)
+        _assert_march_equal(got, want)
+
+
 def test_integrate_rays_bit_exact_and_backward(dev):
     rng = np.random.default_rng(5)
     start, ns, bgs, dss, z, drgbs = integrate_inputs(rng, 4096, 200)
