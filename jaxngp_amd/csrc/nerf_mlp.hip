@@ -58,9 +58,20 @@ constexpr int L_END = L_W5 + 64 * S_W5;  // 11264 floats
 static_assert(S_W1 % 16 == 4 && S_W2 % 16 == 4 && S_W3 % 16 == 4 && S_W4 % 16 == 4 && S_W5 % 16 == 4,
               "weight row strides of 4 mod 16");
 
-// per-wave transpose scratch of the backward pass: [16 samples][68]
-constexpr int S_T = 68;
-constexpr int T_FLOATS = kTile * S_T;
+// Per-wave transpose scratch of the backward pass, a tile of 16 samples x 64 features, where
+// the four samples that a lane of dW's MFMAs takes of a feature are one read (f32: 16
+// bytes, f16: 8).  Quad q of feature 16b + 4g + r stands at 256b + 64r + 16g + 4 (q ^ r): a
+// wavefront writes its 64 values of one r, and reads the quads of 16 features, over every
+// bank once.
+constexpr int T_VALUES = kTile * 64;
+
+__device__ __forceinline__ int scratch_write_at(int b, int r, int g, int q, int k) {
+    return 256 * b + 64 * r + 16 * g + 4 * (q ^ r) + k;
+}
+// quad q of feature i of block 0
+__device__ __forceinline__ int scratch_read_at(int i, int q) {
+    return 64 * (i & 3) + 16 * (i >> 2) + 4 * (q ^ (i & 3));
+}
 
 __device__ __forceinline__ v4f mfma(float a, float b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -382,46 +393,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
     }
 }
 
-// Writes a [16 samples x NB*16 features] tile held in MFMA output layout into a
-// per-wave LDS scratch as [sample][feature].
+// Writes a [16 samples x NB*16 features] tile held in MFMA output layout into a per-wave
+// scratch; quad q holds samples q, 4 + q, 8 + q and 12 + q, one of each of dW's K-steps.
 template <int NB>
 __device__ __forceinline__ void tile_to_lds(float *scr, const v4f *z, int i, int g) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b) *reinterpret_cast<v4f *>(scr + i * S_T + 16 * b + 4 * g) = z[b];
-}
-
-// acc[ib*OB + ob] += Z^T dY over the 16 samples of the tile (both in scratch).
-template <int IB, int OB>
-__device__ __forceinline__ void dw_accumulate(v4f *acc, const float *zs, const float *ys, int i, int g) {
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        float a[IB], bb[OB];
-#pragma unroll
-        for (int ib = 0; ib < IB; ++ib) a[ib] = zs[(4 * t + g) * S_T + 16 * ib + i];
-#pragma unroll
-        for (int ob = 0; ob < OB; ++ob) bb[ob] = ys[(4 * t + g) * S_T + 16 * ob + i];
-#pragma unroll
-        for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-            for (int ob = 0; ob < OB; ++ob) acc[ib * OB + ob] = mfma(a[ib], bb[ob], acc[ib * OB + ob]);
-    }
-}
-
-// Adds dW blocks (MFMA layout: lane (j, g) reg r = dW[16ib + 4g + r][16ob + j]) into
-// an LDS array laid out as the flax kernel [in][out_dim].  Every (row, col) is owned
-// by exactly one lane of the calling wave.
-template <int IB, int OB>
-__device__ __forceinline__ void dw_to_lds(float *dst, const v4f *acc, int out_dim, int i, int g) {
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-        for (int ob = 0; ob < OB; ++ob) {
-            const int col = 16 * ob + i;
-            if (col < out_dim) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dst[(16 * ib + 4 * g + r) * out_dim + col] += acc[ib * OB + ob][r];
-            }
-        }
+        for (int r = 0; r < 4; ++r) scr[scratch_write_at(b, r, g, i & 3, i >> 2)] = z[b][r];
 }
 
 // The workgroup's waves split each layer's dW: wave `part` owns column block
@@ -433,18 +412,14 @@ __device__ __forceinline__ void dw_accumulate_part(v4f *acc, const float *scratc
     static_assert(OB == 4 || (OB == 1 && IB == 4), "blocks split over four waves");
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-        const float *zs = scratch + w * 2 * T_FLOATS;
-        const float *ys = zs + T_FLOATS;
+        const float *zs = scratch + w * 2 * T_VALUES + scratch_read_at(i, g);
+        const float *ys = zs + T_VALUES;
+        const v4f y = *reinterpret_cast<const v4f *>(ys + (OB == 4 ? 256 * part : 0));
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int r0 = (4 * t + g) * S_T;
-            if constexpr (OB == 4) {
-                const float bb = ys[r0 + 16 * part + i];
+        for (int ib = 0; ib < (OB == 4 ? IB : 1); ++ib) {
+            const v4f z = *reinterpret_cast<const v4f *>(zs + 256 * (OB == 4 ? ib : part));
 #pragma unroll
-                for (int ib = 0; ib < IB; ++ib) acc[ib] = mfma(zs[r0 + 16 * ib + i], bb, acc[ib]);
-            } else {
-                acc[0] = mfma(zs[r0 + 16 * part + i], ys[r0 + i], acc[0]);
-            }
+            for (int t = 0; t < 4; ++t) acc[ib] = mfma(z[t], y[t], acc[ib]);
         }
     }
 }
@@ -466,18 +441,22 @@ __device__ __forceinline__ void dw_part_to_row(float *dst, const v4f *acc, int o
     }
 }
 
+// Bounded by the f32 matrix unit (464 MFMAs a tile, 103 us for 2^18 samples), with two
+// wavefronts per SIMD between ten barriers a tile to feed it.  A layer's dZ is computed
+// before the barrier that dW's operands wait for, and those are read four samples at a time
+// (scratch_read_at): 2^18 samples 158 -> 150 us, f16 69 -> 67.
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
     mlp_backward_kernel(uint32_t n, bool level_major, const float *__restrict__ enc, const float *__restrict__ dirs,
                         const float *__restrict__ params, const float *__restrict__ dL_ddrgbs,
                         float *__restrict__ dL_denc, float *__restrict__ workspace) {
     __shared__ __align__(16) float lds[L_END];
-    __shared__ float scratch[kWaves * 2 * T_FLOATS];
+    __shared__ __align__(16) float scratch[kWaves * 2 * T_VALUES];
     stage_weights(lds, params);
     const int lane = lane_id();
     const int i = lane & 15, g = lane >> 4;
     const int wv = threadIdx.x / kWave;
-    float *zs = scratch + wv * 2 * T_FLOATS;
-    float *ys = zs + T_FLOATS;
+    float *zs = scratch + wv * 2 * T_VALUES;
+    float *ys = zs + T_VALUES;
     const uint32_t n_tiles = (n + kTile - 1) / kTile;
     // the workgroup takes kWaves consecutive tiles at a time (a tile past the end
     // loads as zeros and contributes nothing), so all its waves meet at the barriers
@@ -510,50 +489,50 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         // W5
         tile_to_lds<4>(zs, f.h3, i, g);
         tile_to_lds<1>(ys, &dr, i, g);
-        __syncthreads();
-        dw_accumulate_part<4, 1>(gW5, scratch, wv, i, g);
         v4f d3[4];
         layer_bwd<64, 16, S_W5>(lds + L_W5, &dr, d3, i, g);
         relu_mask<4>(d3, f.h3);
         __syncthreads();
+        dw_accumulate_part<4, 1>(gW5, scratch, wv, i, g);
+        __syncthreads();
         // W4
         tile_to_lds<4>(zs, f.h2, i, g);
         tile_to_lds<4>(ys, d3, i, g);
-        __syncthreads();
-        dw_accumulate_part<4, 4>(gW4, scratch, wv, i, g);
         v4f d2[4];
         layer_bwd<64, 64, S_W4>(lds + L_W4, d3, d2, i, g);
         relu_mask<4>(d2, f.h2);
         __syncthreads();
+        dw_accumulate_part<4, 4>(gW4, scratch, wv, i, g);
+        __syncthreads();
         // W3
         tile_to_lds<2>(zs, f.c, i, g);
         tile_to_lds<4>(ys, d2, i, g);
-        __syncthreads();
-        dw_accumulate_part<2, 4>(gW3, scratch, wv, i, g);
         v4f dc[2];
         layer_bwd<32, 64, S_W3>(lds + L_W3, d2, dc, i, g);
         if (g == 0) dc[0][0] += dsig;
         __syncthreads();
+        dw_accumulate_part<2, 4>(gW3, scratch, wv, i, g);
+        __syncthreads();
         // W2
         tile_to_lds<4>(zs, f.h1, i, g);
         tile_to_lds<1>(ys, &dc[0], i, g);
-        __syncthreads();
-        dw_accumulate_part<4, 1>(gW2, scratch, wv, i, g);
         v4f d1[4];
         layer_bwd<64, 16, S_W2>(lds + L_W2, &dc[0], d1, i, g);
         relu_mask<4>(d1, f.h1);
         __syncthreads();
+        dw_accumulate_part<4, 1>(gW2, scratch, wv, i, g);
+        __syncthreads();
         // W1
         tile_to_lds<2>(zs, f.x, i, g);
         tile_to_lds<4>(ys, d1, i, g);
-        __syncthreads();
-        dw_accumulate_part<2, 4>(gW1, scratch, wv, i, g);
         v4f dx[2];
         layer_bwd<32, 64, S_W1>(lds + L_W1, d1, dx, i, g);
         if (live) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) store_enc4(dL_denc, level_major, n, s, b, g, dx[b]);
         }
+        __syncthreads();
+        dw_accumulate_part<2, 4>(gW1, scratch, wv, i, g);
         __syncthreads();
     }
 
@@ -760,37 +739,15 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
     }
 }
 
-// acc[ib*OB + ob] += Z^T dY over the tile's 16 samples (K = samples), f16 operands:
-// lane (i, g) takes samples 4g..4g+3 of feature 16ib + i (A) and 16ob + i (B).
-template <int IB, int OB>
-__device__ __forceinline__ void dw_accumulate_h(v4f *acc, const float *zs, const float *ys, int i, int g) {
-    h4 a[IB], bb[OB];
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) a[ib][q] = (_Float16)zs[(4 * g + q) * S_T + 16 * ib + i];
-#pragma unroll
-    for (int ob = 0; ob < OB; ++ob)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) bb[ob][q] = (_Float16)ys[(4 * g + q) * S_T + 16 * ob + i];
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-        for (int ob = 0; ob < OB; ++ob) acc[ib * OB + ob] = mfma_h16(a[ib], bb[ob], acc[ib * OB + ob]);
-}
-
 // tile_to_lds for the f16 backward: the dW MFMAs take f16 operands, so the tile is
 // rounded to f16 once here (the same rounding as at the MFMA) and the scratch
-// takes half the LDS.
+// takes half the LDS.  Quad q holds samples 4q..4q + 3.
 template <int NB>
 __device__ __forceinline__ void tile_to_lds_h(_Float16 *scr, const v4f *z, int i, int g) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        h4 v;
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (_Float16)z[b][r];
-        *reinterpret_cast<h4 *>(scr + i * S_T + 16 * b + 4 * g) = v;
-    }
+        for (int r = 0; r < 4; ++r) scr[scratch_write_at(b, r, g, i >> 2, i & 3)] = (_Float16)z[b][r];
 }
 
 // dw_accumulate_part with f16 operands (K = the tile's 16 samples per MFMA).
@@ -799,18 +756,12 @@ __device__ __forceinline__ void dw_accumulate_part_h(v4f *acc, const _Float16 *s
     static_assert(OB == 4 || (OB == 1 && IB == 4), "blocks split over four waves");
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-        const _Float16 *zs = scratch + w * 2 * T_FLOATS;
-        const _Float16 *ys = zs + T_FLOATS;
-        const int cb = OB == 4 ? 16 * part : 0;  // this wave's output block in ys
-        h4 bb;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) bb[q] = ys[(4 * g + q) * S_T + cb + i];
+        const _Float16 *zs = scratch + w * 2 * T_VALUES + scratch_read_at(i, g);
+        const _Float16 *ys = zs + T_VALUES;
+        const h4 bb = *reinterpret_cast<const h4 *>(ys + (OB == 4 ? 256 * part : 0));
 #pragma unroll
         for (int ib = 0; ib < (OB == 4 ? IB : 1); ++ib) {
-            const int rb = OB == 4 ? 16 * ib : 16 * part;  // input block in zs
-            h4 a;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) a[q] = zs[(4 * g + q) * S_T + rb + i];
+            const h4 a = *reinterpret_cast<const h4 *>(zs + 256 * (OB == 4 ? ib : part));
             acc[ib] = mfma_h16(a, bb, acc[ib]);
         }
     }
@@ -821,13 +772,13 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                           const _Float16 *__restrict__ params, const float *__restrict__ dL_ddrgbs,
                           float *__restrict__ dL_denc, float *__restrict__ workspace) {
     __shared__ __align__(16) _Float16 lds[H_END];
-    __shared__ __align__(16) _Float16 scratch[kWaves * 2 * T_FLOATS];
+    __shared__ __align__(16) _Float16 scratch[kWaves * 2 * T_VALUES];
     stage_weights_h<true>(lds, params);
     const int lane = lane_id();
     const int i = lane & 15, g = lane >> 4;
     const int wv = threadIdx.x / kWave;
-    _Float16 *zs = scratch + wv * 2 * T_FLOATS;
-    _Float16 *ys = zs + T_FLOATS;
+    _Float16 *zs = scratch + wv * 2 * T_VALUES;
+    _Float16 *ys = zs + T_VALUES;
     const uint32_t n_tiles = (n + kTile - 1) / kTile;
     // kWaves consecutive tiles per workgroup step; tiles past the end load as zeros
     const uint32_t n_groups = (n_tiles + kWaves - 1) / kWaves;
@@ -859,48 +810,46 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         // W5
         tile_to_lds_h<4>(zs, f.h3, i, g);
         tile_to_lds_h<1>(ys, &dr, i, g);
-        __syncthreads();
-        dw_accumulate_part_h<4, 1>(gW5, scratch, wv, i, g);
         const h8 drin = pack_h8(dr, zero);
         v4f d3[4];
         layer_bwd_h<4, 1, BT5, true>(lds + H_B5, &drin, d3, i, g);
         relu_mask<4>(d3, f.h3);
         __syncthreads();
+        dw_accumulate_part_h<4, 1>(gW5, scratch, wv, i, g);
+        __syncthreads();
         // W4
         tile_to_lds_h<4>(zs, f.h2, i, g);
         tile_to_lds_h<4>(ys, d3, i, g);
-        __syncthreads();
-        dw_accumulate_part_h<4, 4>(gW4, scratch, wv, i, g);
         const h8 d3in[2] = {pack_h8(d3[0], d3[1]), pack_h8(d3[2], d3[3])};
         v4f d2[4];
         layer_bwd_h<4, 2, BT4, false>(lds + H_B4, d3in, d2, i, g);
         relu_mask<4>(d2, f.h2);
         __syncthreads();
+        dw_accumulate_part_h<4, 4>(gW4, scratch, wv, i, g);
+        __syncthreads();
         // W3
         tile_to_lds_h<2>(zs, f.c, i, g);
         tile_to_lds_h<4>(ys, d2, i, g);
-        __syncthreads();
-        dw_accumulate_part_h<2, 4>(gW3, scratch, wv, i, g);
         const h8 d2in[2] = {pack_h8(d2[0], d2[1]), pack_h8(d2[2], d2[3])};
         v4f dc[2];
         layer_bwd_h<2, 2, BT3, false>(lds + H_B3, d2in, dc, i, g);
         if (g == 0) dc[0][0] += dsig;
         __syncthreads();
+        dw_accumulate_part_h<2, 4>(gW3, scratch, wv, i, g);
+        __syncthreads();
         // W2
         tile_to_lds_h<4>(zs, f.h1, i, g);
         tile_to_lds_h<1>(ys, &dc[0], i, g);
-        __syncthreads();
-        dw_accumulate_part_h<4, 1>(gW2, scratch, wv, i, g);
         const h8 dcin = pack_h8(dc[0], zero);
         v4f d1[4];
         layer_bwd_h<4, 1, BT2, true>(lds + H_B2, &dcin, d1, i, g);
         relu_mask<4>(d1, f.h1);
         __syncthreads();
+        dw_accumulate_part_h<4, 1>(gW2, scratch, wv, i, g);
+        __syncthreads();
         // W1
         tile_to_lds_h<2>(zs, f.x, i, g);
         tile_to_lds_h<4>(ys, d1, i, g);
-        __syncthreads();
-        dw_accumulate_part_h<2, 4>(gW1, scratch, wv, i, g);
         const h8 d1in[2] = {pack_h8(d1[0], d1[1]), pack_h8(d1[2], d1[3])};
         v4f dx[2];
         layer_bwd_h<2, 2, BT1, false>(lds + H_B1, d1in, dx, i, g);
@@ -908,6 +857,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int b = 0; b < 2; ++b) store_enc4(dL_denc, level_major, n, s, b, g, dx[b]);
         }
+        __syncthreads();
+        dw_accumulate_part_h<2, 4>(gW1, scratch, wv, i, g);
         __syncthreads();
     }
 
