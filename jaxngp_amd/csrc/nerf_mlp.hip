@@ -624,38 +624,43 @@ __device__ __forceinline__ h8 join_h4(h4 lo, h4 hi) {
     return h8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
-// Copies the flat f16 parameters into the forward (transposed) and, with
-// kBackward, the backward LDS layouts; padding is zero.
-template <bool kBackward>
-__device__ void stage_weights_h(_Float16 *lds, const _Float16 *__restrict__ params) {
-    const int end = kBackward ? H_END : H_FEND;
-    for (int t = threadIdx.x; t < end; t += kThreads) lds[t] = (_Float16)0.0f;
-    __syncthreads();
-    // W1 [32][64], W2 [64][16], W3 [32][64], W4 [64][64], W5 [64][3] (flax [in][out])
-    for (int t = threadIdx.x; t < 32 * 64; t += kThreads) {
-        const int in = t / 64, out = t % 64;
-        lds[H_F1 + out * FT1 + in] = params[P_W1 + t];
-        lds[H_F3 + out * FT3 + in] = params[P_W3 + t];
-        if (kBackward) {
-            lds[H_B1 + in * BT1 + out] = params[P_W1 + t];
-            lds[H_B3 + in * BT3 + out] = params[P_W3 + t];
+// Copies a weight matrix [IN][OUT] to W^T rows of FT halves and, with BT > 0, to W rows of
+// BT halves; outputs OUT up to ROWS are zero.  Four inputs of one output at a time, so that
+// lanes read consecutive halves and write 8 bytes.
+template <int IN, int OUT, int ROWS, int FT, int BT>
+__device__ __forceinline__ void stage_matrix_h(_Float16 *fwd, _Float16 *bwd, const _Float16 *__restrict__ w) {
+    constexpr int kPer = ROWS * IN / 4 / kThreads;
+    static_assert(ROWS * IN % (4 * kThreads) == 0, "whole quads per thread");
+    h4 v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int t = threadIdx.x + k * kThreads, out = t % ROWS, q = t / ROWS;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const _Float16 x = w[(4 * q + r) * OUT + (ROWS == OUT ? out : min(out, OUT - 1))];
+            v[k][r] = ROWS == OUT || out < OUT ? x : (_Float16)0.0f;
         }
     }
-    for (int t = threadIdx.x; t < 64 * 16; t += kThreads) {
-        const int in = t / 16, out = t % 16;
-        lds[H_F2 + out * FT2 + in] = params[P_W2 + t];
-        if (kBackward) lds[H_B2 + in * BT2 + out] = params[P_W2 + t];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int t = threadIdx.x + k * kThreads, out = t % ROWS, q = t / ROWS;
+        *reinterpret_cast<h4 *>(fwd + out * FT + 4 * q) = v[k];
+        if constexpr (BT > 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bwd[(4 * q + r) * BT + out] = v[k][r];
+        }
     }
-    for (int t = threadIdx.x; t < 64 * 64; t += kThreads) {
-        const int in = t / 64, out = t % 64;
-        lds[H_F4 + out * FT4 + in] = params[P_W4 + t];
-        if (kBackward) lds[H_B4 + in * BT4 + out] = params[P_W4 + t];
-    }
-    for (int t = threadIdx.x; t < 64 * 3; t += kThreads) {
-        const int in = t / 3, out = t % 3;
-        lds[H_F5 + out * FT5 + in] = params[P_W5 + t];
-        if (kBackward) lds[H_B5 + in * BT5 + out] = params[P_W5 + t];
-    }
+}
+
+// Copies the flat f16 parameters into the forward (transposed) and, with
+// kBackward, the backward LDS layouts (flax [in][out]; padding is not read).
+template <bool kBackward>
+__device__ void stage_weights_h(_Float16 *lds, const _Float16 *__restrict__ params) {
+    stage_matrix_h<32, 64, 64, FT1, kBackward ? BT1 : 0>(lds + H_F1, lds + H_B1, params + P_W1);
+    stage_matrix_h<64, 16, 16, FT2, kBackward ? BT2 : 0>(lds + H_F2, lds + H_B2, params + P_W2);
+    stage_matrix_h<32, 64, 64, FT3, kBackward ? BT3 : 0>(lds + H_F3, lds + H_B3, params + P_W3);
+    stage_matrix_h<64, 64, 64, FT4, kBackward ? BT4 : 0>(lds + H_F4, lds + H_B4, params + P_W4);
+    stage_matrix_h<64, 3, 16, FT5, kBackward ? BT5 : 0>(lds + H_F5, lds + H_B5, params + P_W5);
     __syncthreads();
 }
 
