@@ -402,6 +402,23 @@ typedef struct NgpPoolScatterDescriptor {
  * in : idx u32[n], src f32[n, width]   inout: dst f32[n_total, width] */
 void pool_scatter(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
+/* The end of a pool round in one launch: the three scatters of march_rays_inference's and
+ * integrate_rays_inference's results, and the count of terminated rays.  opaque:
+ * NgpPoolScatterDescriptor with width 4.
+ * in : idx u32[n], t_starts f32[n], rgbd f32[n, 4], T f32[n], terminate_cnt u32[1]
+ * inout: t_starts f32[n_total], rays_rgbd f32[n_total, 4], rays_T f32[n_total], total u64[1]
+ *      (both rgbd 16-byte aligned) */
+void pool_round(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
+typedef struct NgpNearFarDescriptor {
+    uint32_t n_rays;
+    float bound;
+} NgpNearFarDescriptor;
+
+/* Entry and exit distances of [-bound, bound]^3 (models/renderers/cuda.py:56-97).
+ * in : rays_o f32[n, 3], rays_d f32[n, 3]   out: t_starts f32[n], t_ends f32[n] */
+void rays_near_far(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
 /* ---------------------------------------------------------------------------
  * Learned proposal (no counterpart in the reference): a hash grid (L = 5, F = 2)
  * and a 10 -> 16 -> 1 MLP predicting density at 64 equal bins of each ray's

@@ -51,6 +51,8 @@ TARGETS = (
     "occupancy_grid_update",
     "occupancy_grid_update_staged",
     "pool_scatter",
+    "pool_round",
+    "rays_near_far",
     "proposal_points",
     "proposal_mlp_forward",
     "proposal_mlp_backward",
@@ -368,6 +370,10 @@ def proposal_train_descriptor(render_desc: bytes, total_samples, n_uniform=0) ->
 
 def proposal_loss_descriptor(n_rays, eps=1e-7) -> bytes:
     return struct.pack("<If", n_rays, eps)
+
+
+def near_far_descriptor(n_rays, bound) -> bytes:
+    return struct.pack("<If", n_rays, bound)
 
 
 def pool_scatter_descriptor(n, n_total, width) -> bytes:

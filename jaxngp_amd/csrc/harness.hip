@@ -288,6 +288,46 @@ __global__ void __launch_bounds__(kBlock)
     if (r < n_total) dst[(size_t)r * width + c] = src[t];
 }
 
+// torch.minimum, torch.maximum: NaN if either operand is NaN
+__device__ __forceinline__ float min_nan(float a, float b) { return a != a ? a : b != b ? b : fminf(a, b); }
+__device__ __forceinline__ float max_nan(float a, float b) { return a != a ? a : b != b ? b : fmaxf(a, b); }
+
+// Entry and exit of [-bound, bound]^3 (cuda.py:56-97), the operations of
+// renderer.make_near_far_from_bound one by one.
+__global__ void __launch_bounds__(kBlock)
+    near_far_kernel(uint32_t n, float bound, const float *__restrict__ rays_o, const float *__restrict__ rays_d,
+                    float *__restrict__ t_starts, float *__restrict__ t_ends) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    float lo = -__builtin_huge_valf(), hi = __builtin_huge_valf();
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float o = rays_o[3 * (size_t)i + a];
+        float d = rays_d[3 * (size_t)i + a];
+        d = signbit(d) ? min_nan(d, -1e-15f) : max_nan(d, 1e-15f);
+        const float ta = (-bound - o) / d, tb = (bound - o) / d;
+        lo = max_nan(lo, min_nan(ta, tb));
+        hi = min_nan(hi, max_nan(ta, tb));
+    }
+    t_starts[i] = max_nan(lo, 0.0f);
+    t_ends[i] = hi;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    pool_round_kernel(uint32_t n, uint32_t n_total, const uint32_t *__restrict__ idx, const float *__restrict__ t_src,
+                      const float4 *__restrict__ rgbd_src, const float *__restrict__ T_src,
+                      const uint32_t *__restrict__ count, float *__restrict__ t_dst, float4 *__restrict__ rgbd_dst,
+                      float *__restrict__ T_dst, uint64_t *__restrict__ total) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i == 0) *total += *count;
+    if (i >= n) return;
+    const uint32_t r = idx[i];
+    if (r >= n_total) return;
+    t_dst[r] = t_src[i];
+    rgbd_dst[r] = rgbd_src[i];
+    T_dst[r] = T_src[i];
+}
+
 }  // namespace
 }  // namespace ngp
 
@@ -427,5 +467,42 @@ extern "C" void pool_scatter(ngp_stream_t stream, void **buffers, const char *op
     hipLaunchKernelGGL(pool_scatter_kernel, dim3((uint32_t)((total + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                        (hipStream_t)stream, d.n, d.n_total, d.width, (const uint32_t *)buffers[0],
                        (const float *)buffers[1], (float *)buffers[2]);
+    check_launch(target);
+}
+
+extern "C" void pool_round(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
+    const char *target = "pool_round";
+    NgpPoolScatterDescriptor d;
+    if (!read_descriptor(opaque, opaque_len, &d, target)) return;
+    if (d.width != 4) {
+        set_error(kBadDescriptor, "%s: width must be 4", target);
+        return;
+    }
+    if (d.n == 0) return;
+    if (!check_buffers(buffers, 9, target)) return;
+    if (((reinterpret_cast<uintptr_t>(buffers[2]) | reinterpret_cast<uintptr_t>(buffers[6])) & 15u) != 0) {
+        set_error(kBadArgument, "%s: the colours must be 16-byte aligned", target);
+        return;
+    }
+    if ((reinterpret_cast<uintptr_t>(buffers[8]) & 7u) != 0) {
+        set_error(kBadArgument, "%s: the total must be 8-byte aligned", target);
+        return;
+    }
+    hipLaunchKernelGGL(pool_round_kernel, dim3(div_up(d.n, kBlock)), dim3(kBlock), 0, (hipStream_t)stream, d.n, d.n_total,
+                       (const uint32_t *)buffers[0], (const float *)buffers[1], (const float4 *)buffers[2],
+                       (const float *)buffers[3], (const uint32_t *)buffers[4], (float *)buffers[5], (float4 *)buffers[6],
+                       (float *)buffers[7], (uint64_t *)buffers[8]);
+    check_launch(target);
+}
+
+extern "C" void rays_near_far(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
+    const char *target = "rays_near_far";
+    NgpNearFarDescriptor d;
+    if (!read_descriptor(opaque, opaque_len, &d, target)) return;
+    if (d.n_rays == 0) return;
+    if (!check_buffers(buffers, 4, target)) return;
+    hipLaunchKernelGGL(near_far_kernel, dim3(div_up(d.n_rays, kBlock)), dim3(kBlock), 0, (hipStream_t)stream, d.n_rays,
+                       d.bound, (const float *)buffers[0], (const float *)buffers[1], (float *)buffers[2],
+                       (float *)buffers[3]);
     check_launch(target);
 }

@@ -687,11 +687,43 @@ __global__ void march_empty_kernel(uint32_t total_samples, uint32_t *next_loc, u
 // ---------------------------------------------------------------------------
 
 // Terminated slots take new ray indices in slot order (the reference hands them
-// out with atomicAdd, marching.cu:300), in three launches without scratch memory:
+// out with atomicAdd, marching.cu:300).  Up to kMaxAssignOnce slots every block counts the
+// terminated ones before its own range by itself, in one launch (2^18 slots: 8 us
+// instead of 11 us); past that, where this would read too much, and with next_in and next_out
+// in one place, in three launches without scratch memory:
 // per-block counts of terminated slots are parked in the first slot of each
 // block's range of indices_out, one workgroup turns them into exclusive prefixes
 // (and writes next_out), and every block then assigns its range.
 constexpr int kAssignBlock = 1024;
+
+constexpr uint32_t kMaxAssignOnce = 1u << 19;
+
+__global__ void __launch_bounds__(kAssignBlock)
+    assign_kernel(uint32_t n_rays, const bool *__restrict__ terminated, const uint32_t *__restrict__ indices_in,
+                  const uint32_t *__restrict__ next_in, uint32_t *__restrict__ next_out,
+                  uint32_t *__restrict__ indices_out) {
+    const uint32_t first = blockIdx.x * kAssignBlock, j = first + threadIdx.x;
+    uint32_t c = 0, before = 0, own = 0;
+    // (bools are 0 or 1; the flags are 16-byte aligned; kLoads of them in flight)
+    constexpr uint32_t kLoads = 8;
+    for (uint32_t q0 = threadIdx.x; q0 < first / 16u; q0 += kLoads * kAssignBlock) {
+        uint4 v[kLoads];
+#pragma unroll
+        for (uint32_t u = 0; u < kLoads; ++u) {
+            const uint32_t q = q0 + u * kAssignBlock;
+            v[u] = q < first / 16u ? reinterpret_cast<const uint4 *>(terminated)[q] : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kLoads; ++u)
+            c += (uint32_t)(__popc(v[u].x) + __popc(v[u].y) + __popc(v[u].z) + __popc(v[u].w));
+    }
+    block_exclusive_scan<kAssignBlock>(c, &before);
+    before += *next_in;
+    const bool t = j < n_rays && terminated[j];
+    const uint32_t at = before + block_exclusive_scan<kAssignBlock>(t ? 1u : 0u, &own);
+    if (j < n_rays) indices_out[j] = t ? at : indices_in[j];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *next_out = before + own;
+}
 
 __global__ void __launch_bounds__(kAssignBlock)
     assign_count_kernel(uint32_t n_rays, const bool *__restrict__ terminated, uint32_t *__restrict__ indices_out) {
@@ -1139,12 +1171,17 @@ extern "C" void march_rays_inference(ngp_stream_t stream_, void **buffers, const
     float *zs = (float *)buffers[14];
     const MarchParams p = make_march_params(d.diagonal_n_steps, d.K, d.G, d.bound, d.stepsize_portion);
     const uint32_t n_assign = div_up(d.n_rays, kAssignBlock);
-    hipLaunchKernelGGL(assign_count_kernel, dim3(n_assign), dim3(kAssignBlock), 0, stream, d.n_rays, terminated,
-                       indices_out);
-    hipLaunchKernelGGL(assign_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, n_assign, next_in, next_out,
-                       indices_out);
-    hipLaunchKernelGGL(assign_write_kernel, dim3(n_assign), dim3(kAssignBlock), 0, stream, d.n_rays, terminated,
-                       indices_in, indices_out);
+    if (d.n_rays <= kMaxAssignOnce && next_in != next_out && (reinterpret_cast<uintptr_t>(terminated) & 15u) == 0) {
+        hipLaunchKernelGGL(assign_kernel, dim3(n_assign), dim3(kAssignBlock), 0, stream, d.n_rays, terminated, indices_in,
+                           next_in, next_out, indices_out);
+    } else {
+        hipLaunchKernelGGL(assign_count_kernel, dim3(n_assign), dim3(kAssignBlock), 0, stream, d.n_rays, terminated,
+                           indices_out);
+        hipLaunchKernelGGL(assign_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, n_assign, next_in, next_out,
+                           indices_out);
+        hipLaunchKernelGGL(assign_write_kernel, dim3(n_assign), dim3(kAssignBlock), 0, stream, d.n_rays, terminated,
+                           indices_in, indices_out);
+    }
     if (!check_launch(target)) return;
     const bool word_ok = bitfield_words_ok(bits, d.K, d.G);
     const bool plain = word_ok && d.K == 1 && d.bound >= 1.0f && d.stepsize_portion == 0.0f;

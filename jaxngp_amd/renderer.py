@@ -137,8 +137,10 @@ def render_rays_inference(model, o: torch.Tensor, d: torch.Tensor, occupancy_bit
     """The ray-pool loop of render_image_inference on explicit rays o, d [n, 3].
     Returns (rays_rgbd [n, 4], rays_bg [n, 3])."""
     dev = o.device
-    t_starts, t_ends = make_near_far_from_bound(model.bound, o, d)
     n_px = o.shape[0]
+    t_starts, t_ends = torch.empty(n_px, device=dev), torch.empty(n_px, device=dev)
+    # make_near_far_from_bound in one launch instead of fifteen
+    _lib.call("rays_near_far", [o, d, t_starts, t_ends], _lib.near_far_descriptor(n_px, model.bound))
     rays_rgbd = torch.zeros(n_px, 4, device=dev)
     rays_T = torch.ones(n_px, device=dev)
     rays_bg = torch.as_tensor(bg, dtype=torch.float32, device=dev).expand(n_px, 3).contiguous()
@@ -157,7 +159,7 @@ def render_rays_inference(model, o: torch.Tensor, d: torch.Tensor, occupancy_bit
     cnt = torch.empty(1, dtype=u32, device=dev)
     rgbd_out = torch.empty(n, 4, device=dev)
     T_out = torch.empty(n, device=dev)
-    total = torch.zeros((), dtype=torch.int64, device=dev)
+    total = torch.zeros(1, dtype=torch.int64, device=dev)
     pe = model.position_encoder
     half = getattr(model, "mlp_half", None) is not None
     params = model.mlp_half if half else model.mlp_params.detach()
@@ -171,15 +173,13 @@ def render_rays_inference(model, o: torch.Tensor, d: torch.Tensor, occupancy_bit
         rounds.append((
             P("march_rays_inference", [o, d, t_starts, t_ends, occupancy_bitfield, nxt[a:a + 1], terminated, idx[a],
                                        nxt[b:b + 1], ib, n_samples, t_out, xyzs, dss, zs], mdesc),
-            P("pool_scatter", [ib, t_out, t_starts], _lib.pool_scatter_descriptor(n, n_px, 1)),
             P("nerf_field_chunks", [xyzs, n_samples, ib, d, pe.table.detach(), params, drgbs], fdesc),
             P("integrate_rays_inference", [rays_bg, rays_rgbd, rays_T, n_samples, ib, dss, zs, drgbs, cnt,
                                            terminated, rgbd_out, T_out],
               _lib.integrating_inference_descriptor(n_px, n, cap)),
-            P("pool_scatter", [ib, rgbd_out, rays_rgbd], _lib.pool_scatter_descriptor(n, n_px, 4)),
-            P("pool_scatter", [ib, T_out, rays_T], _lib.pool_scatter_descriptor(n, n_px, 1)),
+            P("pool_round", [ib, t_out, rgbd_out, T_out, cnt, t_starts, rays_rgbd, rays_T, total],
+              _lib.pool_scatter_descriptor(n, n_px, 4)),
         ))
-    cnt32 = cnt.view(torch.int32)
     n_rendered, r = 0, 0
     while n_rendered < n_px:
         iters = max(1, (n_px - n_rendered) // n)
@@ -187,7 +187,6 @@ def render_rays_inference(model, o: torch.Tensor, d: torch.Tensor, occupancy_bit
         for _ in range(iters):
             for call in rounds[r & 1]:
                 call()
-            total += cnt32[0]
             r += 1
         _lib.check()
         n_rendered = int(total.item())

@@ -168,3 +168,24 @@ def test_guided_proposal_render_at_its_settings():
         print(f"view {i}: plain {p_plain:.2f} dB, guided proposal {p_prop:.2f} dB {st}", flush=True)
         assert st["proposal_rays"] > 0
         assert p_prop > p_plain - 0.3
+
+
+def test_near_far_kernel_equals_the_torch_operations(dev):
+    """The frame renderer's entry and exit distances, bit for bit (the same operations), on rays
+    along planes, axes and edges, with zeros of either sign, infinities and NaN."""
+    from jaxngp_amd import _lib
+    special = torch.tensor([0.0, -0.0, 1.0, -1.0, 0.5, -2.0, 3e38, -1e-39, float("inf"), float("-inf"), float("nan")],
+                           device=dev)
+    g = torch.Generator(device=dev).manual_seed(1)
+    n = 20_011
+    pick = lambda: torch.where(torch.rand(n, 3, generator=g, device=dev) < 0.5,
+                               special[torch.randint(0, special.numel(), (n, 3), generator=g, device=dev)],
+                               torch.randn(n, 3, generator=g, device=dev))
+    for bound in (1.0, 0.3, 2.7):
+        o, d = pick(), pick()
+        got = [torch.empty(n, device=dev) for _ in range(2)]
+        _lib.call("rays_near_far", [o, d, *got], _lib.near_far_descriptor(n, bound))
+        for a, b in zip(got, make_near_far_from_bound(bound, o, d)):
+            nan = torch.isnan(b)
+            assert torch.equal(torch.isnan(a), nan)
+            assert torch.equal(a[~nan], b[~nan])
