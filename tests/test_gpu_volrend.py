@@ -264,6 +264,23 @@ def test_march_rays_one_cascade_edges(dev, kind, G, diag, bound, portion):
         _assert_march_equal(got, want)
 
 
+@pytest.mark.parametrize("n, offset", [(1, 0), (1023, 0), (1025, 0), (3000, 1), (1 << 19, 0), ((1 << 19) + 1, 0)])
+def test_slot_assignment_in_one_launch_or_three(dev, n, offset):
+    """Terminated slots take the next ray indices in slot order, whichever way they are counted:
+    within a block, over blocks, from unaligned flags, up to the one-launch limit and past it."""
+    rng = np.random.default_rng(n)
+    flags = rng.random(n + offset) < 0.4
+    term = T(flags, dev)[offset:]
+    idx = rng.integers(0, 1000, n).astype(np.uint32)
+    rays = torch.zeros(4, 3, device=dev)
+    empty = torch.ones(4, device=dev)  # t_end < t_start: nothing is marched
+    out = volrend.march_rays_inference(64, 1, 4, 1, 1.0, 0.0, rays, rays + 1, empty, empty - 1,
+                                       torch.zeros(8, dtype=torch.uint8, device=dev), U(np.array([7], np.uint32), dev), term, U(idx, dev))
+    want = np.where(flags[offset:], 7 + np.cumsum(flags[offset:]) - 1, idx)
+    np.testing.assert_array_equal(N(out[1]), want.astype(np.uint32))
+    assert int(N(out[0].view(torch.int32))[0]) == 7 + int(flags[offset:].sum())
+
+
 def test_integrate_rays_bit_exact_and_backward(dev):
     rng = np.random.default_rng(5)
     start, ns, bgs, dss, z, drgbs = integrate_inputs(rng, 4096, 200)
