@@ -236,7 +236,7 @@ def run_training(data, cfg, steps: int, warmup: int, dev) -> dict:
             log(f"[{cfg.precision}] warmup step {i}: {tr.metrics()}")
     torch.cuda.synchronize()
     targets = ["march_rays", "hashgrid_encode", "nerf_mlp_forward", "integrate_rays", "integrate_rays_backward",
-               "nerf_mlp_backward", "hashgrid_encode_backward", "hashgrid_encode_backward_adam", "adam_update"]
+               "nerf_mlp_backward", "hashgrid_encode_backward", "hashgrid_encode_backward_adam", "adam_update_two"]
 
     class Timed:
         def __init__(self, call, events):

@@ -631,6 +631,14 @@ typedef struct NgpLossScaleCheckDescriptor {
  * in : grads f32[n]   inout: NgpLossScaleState[1] */
 void loss_scale_check(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
+typedef struct NgpLossScaleCheckTwoDescriptor {
+    uint64_t n0, n1;
+} NgpLossScaleCheckTwoDescriptor;
+
+/* loss_scale_check of two gradients in one launch.
+ * in : gradients f32[n0], f32[n1]   inout: state */
+void loss_scale_check_two(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
 typedef struct NgpLossScaleUpdateDescriptor {
     uint32_t growth_interval; /* finite steps before the scale doubles */
     float min_scale, max_scale;
@@ -660,6 +668,14 @@ typedef struct NgpAdamDescriptor {
  * out: mirror f16[n] (only read when mirror_dtype is NGP_DTYPE_F16; may be NULL);
  * with NGP_LOSS_SCALED, one more input after the mirror slot: NgpLossScaleState[1] */
 void adam_update(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
+typedef struct NgpAdamTwoDescriptor {
+    NgpAdamDescriptor first, second; /* the same flags in both */
+} NgpAdamTwoDescriptor;
+
+/* adam_update of two arrays in one launch: adam_update's buffers 0..4 of the first, then of
+ * the second (mirrors may be NULL), then the loss-scale state if NGP_LOSS_SCALED. */
+void adam_update_two(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
 typedef struct HashGridAdamDescriptor {
     HashGridDescriptor grid; /* as hashgrid_encode_backward (F <= 2, f32 table) */

@@ -45,7 +45,9 @@ TARGETS = (
     "train_bg_grad",
     "train_loss_grad",
     "adam_update",
+    "adam_update_two",
     "loss_scale_check",
+    "loss_scale_check_two",
     "loss_scale_update",
     "nerf_field_chunks",
     "occupancy_grid_update",
@@ -404,6 +406,10 @@ def occupancy_update_descriptor(grid_desc: bytes, G, K, cascade, n_alive, update
 
 def loss_scale_check_descriptor(n) -> bytes:
     return struct.pack("<Q", n)
+
+
+def loss_scale_check_two_descriptor(n0, n1) -> bytes:
+    return struct.pack("<QQ", n0, n1)
 
 
 def loss_scale_update_descriptor(growth_interval=2000, min_scale=1.0, max_scale=2.0 ** 24) -> bytes:

@@ -915,10 +915,11 @@ __device__ __forceinline__ v4f encode_two_levels(const HashGridDescriptor &d, co
 // A pool round's samples stand in a third of the entries, a whole slot or nothing, so a
 // wavefront packs them: it looks at 64 entries at a time, writes the dead ones' zeros,
 // appends the live ones to a queue of its own in LDS and takes tiles of 16 from that.
-// Bounded by the gathers' misses in L2 (every XCD reads every level of the table, unlike in
-// the encoder): 753,000 samples of 2^21 entries 292 -> 260 us; batches of 64 samples level
-// by level with two rows to a load (270), four wavefronts per SIMD (268) and contiguous
-// entries per wavefront (274) end at the same rate.  A round without samples 46 -> 20 us
+// No one thing bounds it: the matrix unit is busy half of the time, the vector unit a
+// third, the gathers' address unit half, and six in ten L2 requests miss (every XCD reads
+// every level, unlike in the encoder).  753,000 samples of 2^21 entries 292 -> 260 us; batches of 64 samples level
+// by level with two rows to a load (270), four wavefronts per SIMD (268), contiguous
+// entries per wavefront (274) and per XCD (260) end at the same rate.  A round without samples 46 -> 20 us
 // (the zeros, and the 64-bit division per entry that went).
 constexpr int kQueue = kWave + kTile;
 // Workgroups in a launch, four times what the chip holds: the wavefronts' entries hold

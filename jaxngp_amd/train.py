@@ -492,10 +492,12 @@ class Trainer:
                                                             b["hg_ws"]], hdesc) if fused else
                         P("hashgrid_encode_backward", [b["xyzs"], b["denc"], b["dtable"], b["hg_ws"]], hdesc)),
             fused_table=fused,
-            adam_table=P("adam_update", [tab_master, b["dtable"], o["tm"], o["tv"]] +
-                         [mirror if mirror is not None else none] + state, b"", stream=side),
             adam_mlp=P("adam_update", [params, b["dparams"], o["mm"], o["mv"]] +
                        [m.mlp_half if self.fp16 else none] + state, b"", stream=side),
+            adam_two=P("adam_update_two", [tab_master, b["dtable"], o["tm"], o["tv"],
+                                           mirror if mirror is not None else none,
+                                           params, b["dparams"], o["mm"], o["mv"],
+                                           m.mlp_half if self.fp16 else none] + state, b"", stream=side),
             mirror=mirror is not None,
             flags=flags,
         )
@@ -540,10 +542,8 @@ class Trainer:
                 calls["check_bg"] = P("loss_scale_check", [bb["dparams"], self.loss_state],
                                       _lib.loss_scale_check_descriptor(bgp.numel()), stream=side)
         if self.fp16:
-            calls["check_table"] = P("loss_scale_check", [b["dtable"], self.loss_state],
-                                     _lib.loss_scale_check_descriptor(b["dtable"].numel()), stream=side)
-            calls["check_mlp"] = P("loss_scale_check", [b["dparams"], self.loss_state],
-                                   _lib.loss_scale_check_descriptor(N_PARAMS), stream=side)
+            calls["check_two"] = P("loss_scale_check_two", [b["dtable"], b["dparams"], self.loss_state],
+                                   _lib.loss_scale_check_two_descriptor(b["dtable"].numel(), N_PARAMS), stream=side)
             calls["scale_update"] = P("loss_scale_update", [self.loss_state],
                                       _lib.loss_scale_update_descriptor(c.loss_scale_growth_interval), stream=side)
         return calls
@@ -600,7 +600,7 @@ class Trainer:
         lr = lr_at(t - 1, c.lr)
         b1, b2 = 0.9, 0.99
         bp1, bp2 = float(np.float32(b1) ** t), float(np.float32(b2) ** t)
-        n_table = k["adam_table"].keep[0].numel()
+        n_table = k["adam_two"].keep[0].numel()
         for name in order:
             if name == self._pf_before and train_prop:
                 # the proposal's update, on this step's samples and the field's weights at
@@ -632,17 +632,17 @@ class Trainer:
         self.side_stream.wait_event(self._bwd_done)
         with torch.cuda.stream(self.side_stream):
             if self.fp16:
-                k["check_table"]()
-                k["check_mlp"]()
+                k["check_two"]()
                 if bg:
                     k["check_bg"]()
-            if not k["fused_table"]:
-                k["adam_table"](_lib.adam_descriptor(n_table, lr, b1, b2, 1e-15, 1e-15, bp1, bp2, 0.0,
-                                                     mirror_dtype=_lib.DTYPE_F16 if k["mirror"] else _lib.DTYPE_F32,
-                                                     flags=k["flags"]))
-            k["adam_mlp"](_lib.adam_descriptor(N_PARAMS, lr, b1, b2, 1e-15, 1e-15, bp1, bp2, 1e-6,
-                                               mirror_dtype=_lib.DTYPE_F16 if self.fp16 else _lib.DTYPE_F32,
-                                               flags=k["flags"]))
+            mlp = _lib.adam_descriptor(N_PARAMS, lr, b1, b2, 1e-15, 1e-15, bp1, bp2, 1e-6,
+                                       mirror_dtype=_lib.DTYPE_F16 if self.fp16 else _lib.DTYPE_F32, flags=k["flags"])
+            if k["fused_table"]:
+                k["adam_mlp"](mlp)
+            else:
+                k["adam_two"](_lib.adam_descriptor(n_table, lr, b1, b2, 1e-15, 1e-15, bp1, bp2, 0.0,
+                                                   mirror_dtype=_lib.DTYPE_F16 if k["mirror"] else _lib.DTYPE_F32,
+                                                   flags=k["flags"]) + mlp)
             if bg:
                 # params["bg"] is optimised like the NeRF MLP: the "network" Adam and
                 # weight decay 1e-6 (app/nerf/_utils.py:28-76)

@@ -321,3 +321,38 @@ def test_prefetched_samples_equal_a_fresh_run(small_data, guided):
     torch.cuda.synchronize()
     m = tr.metrics()
     assert math.isfinite(m["loss"]) and m["n_valid_rays"] > 0
+
+
+@pytest.mark.parametrize("n0, n1, half, flags, overflow", [(4096, 9408, True, 1, False), (4096, 9408, True, 1, True),
+                                                           (3_000_004, 37, False, 0, False), (1, 4097, True, 0, False)])
+def test_two_updates_in_one_launch_equal_two_launches(dev, n0, n1, half, flags, overflow):
+    """adam_update_two and loss_scale_check_two against the single calls, bit for bit: arrays of
+    one value, of odd and of vector sizes, with and without mirrors, scaled, skipped."""
+    g = torch.Generator(device=dev).manual_seed(n0)
+    state = torch.tensor([1024.0, 0.0, 0.0, 0.0], device=dev)
+    init = [[torch.randn(n, generator=g, device=dev) for _ in range(3)] +
+            [torch.rand(n, generator=g, device=dev), torch.zeros(n, dtype=torch.float16, device=dev)] for n in (n0, n1)]
+    if overflow:
+        init[1][1][-1] = float("inf")
+    none = torch.empty(0, device=dev)
+    dt = _lib.DTYPE_F16 if half else _lib.DTYPE_F32
+    desc = [_lib.adam_descriptor(n, 1e-2, 0.9, 0.99, 1e-15, 1e-15, 0.81, 0.98, wd, mirror_dtype=dt, flags=flags)
+            for n, wd in ((n0, 0.0), (n1, 1e-6))]
+    out = []
+    for two in (False, True):
+        a = [[t.clone() for t in arrays] for arrays in init]
+        st = state.clone()
+        bufs = [x[:4] + [x[4] if half else none] for x in a]
+        if two:
+            _lib.call("loss_scale_check_two", [a[0][1], a[1][1], st], _lib.loss_scale_check_two_descriptor(n0, n1))
+            _lib.call("adam_update_two", bufs[0] + bufs[1] + ([st] if flags else []), desc[0] + desc[1])
+        else:
+            for k, n in ((0, n0), (1, n1)):
+                _lib.call("loss_scale_check", [a[k][1], st], _lib.loss_scale_check_descriptor(n))
+            for k in (0, 1):
+                _lib.call("adam_update", bufs[k] + ([st] if flags else []), desc[k])
+        out.append([st] + a[0] + a[1])
+    assert bool(out[0][0].view(torch.int32)[1]) == overflow
+    assert torch.equal(out[0][1], init[0][0]) == overflow
+    for x, y in zip(*out):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
