@@ -160,6 +160,22 @@ __global__ void __launch_bounds__(kBlock)
     for (uint32_t t = threadIdx.x; t < n * L; t += kBlock) pm[(size_t)p0 * L + t] = tile[t / L * row + t % L];
 }
 
+// [n, L * F] gradients -> [L, n, F], for F = 2: the same the other way.  The level's bucket
+// kernel then reads whole lines; point-major it takes 8 bytes of each of 64 lines, and
+// every level reads the lines again (2^18 ray samples f32: bucket 97 -> 70 us for 15 here).
+__global__ void __launch_bounds__(kBlock)
+    gradients_to_levels_kernel(uint32_t n_points, uint32_t L, const float2 *__restrict__ pm, float2 *__restrict__ lm) {
+    __shared__ float2 tile[kTransposePoints * (NGP_HASHGRID_MAX_LEVELS + 1)];
+    const uint32_t p0 = blockIdx.x * kTransposePoints;
+    const uint32_t n = min((uint32_t)kTransposePoints, n_points - p0), row = L + 1;
+    for (uint32_t t = threadIdx.x; t < n * L; t += kBlock) tile[t / L * row + t % L] = pm[(size_t)p0 * L + t];
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < L * kTransposePoints; t += kBlock) {
+        const uint32_t l = t / kTransposePoints, i = t % kTransposePoints;
+        if (i < n) lm[(size_t)l * n_points + p0 + i] = tile[i * row + l];
+    }
+}
+
 // Backward without global atomics.  Device-scope atomics on this chip (float or
 // integer, any scope) retire at ~21-27 G/s for the whole device on scattered
 // addresses, two orders of magnitude below the gather rate, so contributions are
@@ -276,6 +292,9 @@ struct EntryValue {
 
 inline uint32_t value_bytes(uint32_t F, bool half) { return half && F == 2 ? 4 : 4 * F; }
 
+// points (both ways: 77,777 72 and 74 us, 150,000 120 and 105; f16 67 and 70, 116 and 97)
+constexpr uint32_t kTransposeFrom = 3u << 15;
+
 struct BwdPlan {
     uint32_t R, n_slices, n_chunks, n_items;
     uint64_t M;             // n_slices * n_items counters
@@ -290,7 +309,8 @@ struct BwdPlan {
     uint32_t group_shift;  // log2 of the slices in kSliceBytes
     uint32_t s_lo[NGP_HASHGRID_MAX_LEVELS], s_hi[NGP_HASHGRID_MAX_LEVELS];
     uint64_t runs_off, slice_np_off, first_part_off, split_off, rows_off, part_group_off;
-    bool whole;  // no slice can be cut into parts
+    bool whole;      // no slice can be cut into parts
+    bool transpose;  // a point-major gradient is copied level-major first (to partials_off)
 };
 
 // Rows of one slice: R rows of F f64 accumulators fill kSliceBytes of LDS.  A power
@@ -364,7 +384,9 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         p.meta_off = align(p.split_off + 4 * (uint64_t)p.n_slices);  // [0] parts, [1] cut slices
         p.part_slice_off = align(p.meta_off + 8);
         p.partials_off = align(p.part_slice_off + 4 * (uint64_t)p.max_parts);
-        p.part_group_off = align(p.partials_off + (uint64_t)p.max_parts * p.R * d.F * 8);
+        p.transpose = d.F == 2 && d.enc_layout == NGP_ENC_POINT_MAJOR && !p.whole && d.n_points >= kTransposeFrom;
+        const uint64_t lm_bytes = p.transpose ? (uint64_t)d.n_points * d.L * 8 : 0;
+        p.part_group_off = align(p.partials_off + std::max((uint64_t)p.max_parts * p.R * d.F * 8, lm_bytes));
         p.entries_off = align(p.part_group_off + 4 * (uint64_t)p.max_parts);
         p.rows_off = align(p.entries_off + max_entries * value_bytes(d.F, d.table_dtype == NGP_DTYPE_F16));
         p.bytes = p.rows_off + max_entries * sizeof(uint16_t);
@@ -1366,7 +1388,15 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
     uint16_t *entry_rows = reinterpret_cast<uint16_t *>(ws + p.rows_off);
     const size_t lds = (size_t)R * F * sizeof(double);
     constexpr uint32_t kCombineBlocks = 512;
-    hipLaunchKernelGGL((bwd_bucket_kernel<F, kHalf, R>), dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, d, p, pos, g,
+    HashGridDescriptor db = d;
+    if (p.transpose && (reinterpret_cast<uintptr_t>(g) & 7u) == 0) {
+        float *lm = reinterpret_cast<float *>(ws + p.partials_off);
+        hipLaunchKernelGGL(gradients_to_levels_kernel, dim3(div_up(d.n_points, kTransposePoints)), dim3(kBlock), 0, stream,
+                           d.n_points, d.L, (const float2 *)g, (float2 *)lm);
+        g = lm;
+        db.enc_layout = NGP_ENC_LEVEL_MAJOR;
+    }
+    hipLaunchKernelGGL((bwd_bucket_kernel<F, kHalf, R>), dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, db, p, pos, g,
                        runs, values, entry_rows, meta);
     if (!p.whole)
         hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, runs, meta, slice_np,

@@ -364,3 +364,27 @@ def test_fused_table_update_matches_gradient_then_adam(dev):
         same = (p2 == p1).float().mean().item()
         print(f"  params equal bit for bit: {same:.6f}", flush=True)
         assert same > 0.999
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n, L", [((3 << 15) - 1, 16), (3 << 15, 16), ((3 << 15) + 65, 5), (1 << 18, 16)])
+def test_point_major_gradient_on_both_sides_of_the_transpose(dev, n, L, half):
+    """The table gradient of a point-major gradient, copied level-major first from 98,304 points
+    on, against the same gradient given level-major: the same f64 sums up to the order of
+    entries, rounded to f32 at most a few times (1e-6 of the largest row)."""
+    from jaxngp_amd import _lib
+    enc = HashGridEncoder(L=L, T=1 << 15, F=2, N_min=16, N_max=512, generator=torch.Generator().manual_seed(3))
+    if half:
+        enc.table.data = enc.table.data.half()
+    enc = enc.to(dev)
+    g = torch.Generator(device=dev).manual_seed(n)
+    pos = torch.rand(n, 3, generator=g, device=dev) * 2 - 1
+    lm = torch.randn(L, n, 2, generator=g, device=dev)
+    got = []
+    for layout, grad in ((0, lm.permute(1, 0, 2).reshape(n, 2 * L).contiguous()), (1, lm)):
+        d = enc.descriptor(n, 1.0, layout)
+        ws = torch.empty(_lib.hashgrid_backward_workspace_bytes(d), dtype=torch.uint8, device=dev)
+        out = torch.empty(enc.table.shape, device=dev)
+        _lib.call("hashgrid_encode_backward", [pos, grad, out, ws], d)
+        got.append(out)
+    assert (got[0] - got[1]).abs().max() <= 1e-6 * got[1].abs().max()
