@@ -293,6 +293,11 @@ void hashgrid_encode_backward(ngp_stream_t stream, void **buffers, const char *o
  * output).  Returns 0 and sets the last error for an invalid descriptor. */
 size_t hashgrid_encode_backward_workspace_size(const char *opaque, size_t opaque_len);
 
+/* hashgrid_encode_backward with dL_dtable in f16 (16-byte aligned), the f32 sums rounded as
+ * a cast would: for F = 2, an f16 table and the one-pass form, as _supported tells. */
+int hashgrid_encode_backward_f16_supported(const char *opaque, size_t opaque_len);
+void hashgrid_encode_backward_f16(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
 /* Forward of NeRF.__call__ after the position encoder (models/nerfs.py:66-86).
  * opaque: NerfMlpDescriptor.
  * in : encodings f32[S,32] or f32[16,S,2] (enc_layout), dirs f32[S,3],

@@ -33,6 +33,7 @@ TARGETS = (
     "hashgrid_encode",
     "hashgrid_encode_staged",
     "hashgrid_encode_backward",
+    "hashgrid_encode_backward_f16",
     "tcnn_hashgrid_encode",
     "tcnn_hashgrid_encode_backward",
     "sky_sphere_bg",
@@ -95,6 +96,8 @@ def load() -> ctypes.CDLL:
     lib.ngp_version.restype = ctypes.c_char_p
     lib.hashgrid_encode_backward_workspace_size.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
     lib.hashgrid_encode_backward_workspace_size.restype = ctypes.c_size_t
+    lib.hashgrid_encode_backward_f16_supported.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
+    lib.hashgrid_encode_backward_f16_supported.restype = ctypes.c_int
     lib.hashgrid_encode_backward_adam_supported.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
     lib.hashgrid_encode_backward_adam_supported.restype = ctypes.c_int
     lib.sky_sphere_bg_workspace_size.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
@@ -206,6 +209,13 @@ def hashgrid_backward_workspace_bytes(opaque: bytes) -> int:
         _check()
         raise NGPError("hashgrid_encode_backward_workspace_size: invalid descriptor")
     return n
+
+
+def hashgrid_backward_f16_supported(opaque: bytes) -> bool:
+    """Whether hashgrid_encode_backward_f16 takes the HashGridDescriptor `opaque`."""
+    ok = bool(load().hashgrid_encode_backward_f16_supported(opaque, len(opaque)))
+    _check()
+    return ok
 
 
 def hashgrid_backward_adam_supported(opaque: bytes) -> bool:

@@ -1123,12 +1123,17 @@ struct EntryGroup {
 
 constexpr uint32_t kSplitBlocks = 512;  // two to a CU
 
-template <int F, bool kHalf, uint32_t R, bool kAdam>
+// What becomes of a row's sum: stored in f32, an optimizer step, or stored in f16 (the
+// gradient of an f16 table, rounded as a cast of the f32 sum would; a cast of the whole table
+// afterwards took 10-14 us for 6.1 M rows).
+enum { kFloatRows, kAdamRows, kHalfRows };
+
+template <int F, bool kHalf, uint32_t R, int kOut>
 __device__ __forceinline__ void
 reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t part, uint32_t n_parts, uint32_t slot,
             const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
             const uint16_t *__restrict__ entry_rows, double *__restrict__ partials, uint32_t *__restrict__ part_group,
-            float *__restrict__ dtable, const AdamStep &adam, float *__restrict__ adam_p, float *__restrict__ adam_m,
+            void *__restrict__ dtable, const AdamStep &adam, float *__restrict__ adam_p, float *__restrict__ adam_m,
             float *__restrict__ adam_v) {
     typedef EntryGroup<F, kHalf> Group;
     constexpr uint32_t kBucketEntries = bucket_entries(kHalf);
@@ -1195,7 +1200,7 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
     }
     __syncthreads();
     const size_t o = (size_t)s * R * F;
-    if (kAdam && n_parts == 1) {
+    if (kOut == kAdamRows && n_parts == 1) {
         // unrolled so that several rows' params, m and v loads are in flight at once
 #pragma unroll 8
         for (uint32_t t = threadIdx.x; t < rows * F; t += kRunThreads) {
@@ -1212,9 +1217,13 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
         for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) out[t] = reinterpret_cast<const double2 *>(acc)[t];
         return;
     }
-    float *out = dtable + o;
     for (uint32_t t = threadIdx.x; t < rows; t += kRunThreads) {
-        if constexpr (F == 2) {
+        float *out = static_cast<float *>(dtable) + o;
+        if constexpr (kOut == kHalfRows) {
+            static_assert(F == 2, "two features, one store");
+            reinterpret_cast<__half2 *>(static_cast<__half *>(dtable) + o)[t] =
+                __floats2half2_rn((float)acc[t], (float)acc[R + t]);
+        } else if constexpr (F == 2) {
             reinterpret_cast<float2 *>(out)[t] = make_float2((float)acc[t], (float)acc[R + t]);
         } else {
             out[t] = (float)acc[t];
@@ -1222,14 +1231,14 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
     }
 }
 
-template <int F, bool kHalf, uint32_t R, bool kAdam>
+template <int F, bool kHalf, uint32_t R, int kOut>
 __global__ void __launch_bounds__(kRunThreads)
     bwd_reduce_runs_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ meta,
                            const uint32_t *__restrict__ slice_np, const uint32_t *__restrict__ first_part,
                            const uint32_t *__restrict__ part_slice, const uint32_t *__restrict__ runs,
                            const EntryValue<F, kHalf> *__restrict__ values, const uint16_t *__restrict__ entry_rows,
                            double *__restrict__ partials, uint32_t *__restrict__ part_group,
-                           float *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
+                           void *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
                            float *__restrict__ adam_m, float *__restrict__ adam_v) {
     uint32_t s = blockIdx.x;
     if (!p.whole) {
@@ -1237,7 +1246,7 @@ __global__ void __launch_bounds__(kRunThreads)
             const uint32_t n = meta[0];
             for (uint32_t i = blockIdx.x; i < n; i += kSplitBlocks) {
                 const uint32_t cut = part_slice[i];
-                reduce_part<F, kHalf, R, kAdam>(d, p, cut, i - first_part[cut], slice_np[cut], i, runs, values, entry_rows,
+                reduce_part<F, kHalf, R, kOut>(d, p, cut, i - first_part[cut], slice_np[cut], i, runs, values, entry_rows,
                                                 partials, part_group, dtable, adam, adam_p, adam_m, adam_v);
                 __syncthreads();  // the sums are read out
             }
@@ -1246,7 +1255,7 @@ __global__ void __launch_bounds__(kRunThreads)
         s -= kSplitBlocks;
         if (slice_np[s] != 1) return;
     }
-    reduce_part<F, kHalf, R, kAdam>(d, p, s, 0, 1, 0, runs, values, entry_rows, partials, part_group, dtable, adam,
+    reduce_part<F, kHalf, R, kOut>(d, p, s, 0, 1, 0, runs, values, entry_rows, partials, part_group, dtable, adam,
                                     adam_p, adam_m, adam_v);
 }
 
@@ -1254,12 +1263,12 @@ __global__ void __launch_bounds__(kRunThreads)
 // 1 / kCombineSplit of a slice's rows.  With kAdam the sums are not stored: the rows take
 // the optimizer step in place.
 constexpr uint32_t kCombineSplit = 16;
-template <int F, uint32_t R, bool kAdam>
+template <int F, uint32_t R, int kOut>
 __global__ void __launch_bounds__(256)
     bwd_combine_runs_kernel(HashGridDescriptor d, const uint32_t *__restrict__ meta,
                             const uint32_t *__restrict__ slice_np, const uint32_t *__restrict__ first_part,
                             const uint32_t *__restrict__ split, const double *__restrict__ partials,
-                            const uint32_t *__restrict__ part_group, float *__restrict__ dtable, AdamStep adam,
+                            const uint32_t *__restrict__ part_group, void *__restrict__ dtable, AdamStep adam,
                             float *__restrict__ adam_p, float *__restrict__ adam_m, float *__restrict__ adam_v) {
     constexpr uint32_t kPer = R * F / kCombineSplit;
     constexpr uint32_t kBatch = 8;  // partial rows in flight per thread
@@ -1298,13 +1307,15 @@ __global__ void __launch_bounds__(256)
             }
             sum += (float)in_group;
             const size_t o = ((size_t)s * R + r) * F + f;
-            if constexpr (kAdam) {
+            if constexpr (kOut == kAdamRows) {
                 float mk = adam_m[o], vk = adam_v[o];
                 adam_p[o] = adam_step(adam, adam_p[o], sum, mk, vk);
                 adam_m[o] = mk;
                 adam_v[o] = vk;
+            } else if constexpr (kOut == kHalfRows) {
+                static_cast<__half *>(dtable)[o] = __float2half_rn(sum);
             } else {
-                dtable[o] = sum;
+                static_cast<float *>(dtable)[o] = sum;
             }
         }
     }
@@ -1378,7 +1389,8 @@ bool reserve_lds(K kernel, size_t lds, const char *target) {
 // The one-pass form on slices of R rows.
 template <int F, bool kHalf, uint32_t R>
 bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStream_t stream, const float *pos,
-                          const float *g, float *dtable, uint8_t *ws, const char *target, const FusedAdam *fused) {
+                          const float *g, void *dtable, uint8_t *ws, const char *target, const FusedAdam *fused,
+                          bool half_rows) {
     auto word = [&](uint64_t off) { return reinterpret_cast<uint32_t *>(ws + off); };
     uint32_t *runs = word(p.runs_off), *meta = word(p.meta_off), *slice_np = word(p.slice_np_off);
     uint32_t *first_part = word(p.first_part_off), *split = word(p.split_off), *part_slice = word(p.part_slice_off);
@@ -1402,26 +1414,30 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
         hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, runs, meta, slice_np,
                            first_part, part_slice, split);
     const dim3 reduce_grid(p.n_slices + (p.whole ? 0 : kSplitBlocks));
-    auto finish = [&](auto adam, const AdamStep &step, float *ap, float *am, float *av) {
-        constexpr bool kAdam = decltype(adam)::value;
-        const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, kAdam>;
+    auto finish = [&](auto kind, const AdamStep &step, float *ap, float *am, float *av) {
+        constexpr int kOut = decltype(kind)::value;
+        const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, kOut>;
         if (!reserve_lds(reduce, lds, target)) return false;
         hipLaunchKernelGGL(reduce, reduce_grid, dim3(kRunThreads), lds, stream, d, p, meta, slice_np, first_part,
                            part_slice, runs, values, entry_rows, partials, part_group, dtable, step, ap, am, av);
         if (!p.whole)
-            hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, kAdam>), dim3(kCombineBlocks), dim3(256), 0, stream, d, meta,
+            hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, kOut>), dim3(kCombineBlocks), dim3(256), 0, stream, d, meta,
                                slice_np, first_part, split, partials, part_group, dtable, step, ap, am, av);
         return true;
     };
     if constexpr (!kHalf) {
-        if (fused != nullptr) return finish(std::true_type{}, fused->step, fused->p, fused->m, fused->v);
+        if (fused != nullptr)
+            return finish(std::integral_constant<int, kAdamRows>{}, fused->step, fused->p, fused->m, fused->v);
+    } else if constexpr (F == 2) {
+        if (half_rows) return finish(std::integral_constant<int, kHalfRows>{}, AdamStep{}, nullptr, nullptr, nullptr);
     }
-    return finish(std::false_type{}, AdamStep{}, nullptr, nullptr, nullptr);
+    return finish(std::integral_constant<int, kFloatRows>{}, AdamStep{}, nullptr, nullptr, nullptr);
 }
 
 template <int F, bool kHalf>
-bool launch_backward(const HashGridDescriptor &d, hipStream_t stream, const float *pos, const float *g, float *dtable,
-                     uint8_t *ws, const char *target, const FusedAdam *fused = nullptr) {
+bool launch_backward(const HashGridDescriptor &d, hipStream_t stream, const float *pos, const float *g, void *dtable_,
+                     uint8_t *ws, const char *target, const FusedAdam *fused = nullptr, bool half_rows = false) {
+    float *dtable = static_cast<float *>(dtable_);
     const BwdPlan p = make_plan(d);
     uint32_t *meta = reinterpret_cast<uint32_t *>(ws + p.meta_off);
     uint32_t *parts = reinterpret_cast<uint32_t *>(ws + p.parts_off);
@@ -1432,8 +1448,10 @@ bool launch_backward(const HashGridDescriptor &d, hipStream_t stream, const floa
     if constexpr (F <= 2) {
         if (p.bucket) {
             constexpr uint32_t kSmall = kRunSliceBytes / (8 * F), kLarge = kSliceBytes / (8 * F);
-            return p.R == kSmall ? launch_backward_runs<F, kHalf, kSmall>(d, p, stream, pos, g, dtable, ws, target, fused)
-                                 : launch_backward_runs<F, kHalf, kLarge>(d, p, stream, pos, g, dtable, ws, target, fused);
+            return p.R == kSmall ? launch_backward_runs<F, kHalf, kSmall>(d, p, stream, pos, g, dtable_, ws, target, fused,
+                                                                          half_rows)
+                                 : launch_backward_runs<F, kHalf, kLarge>(d, p, stream, pos, g, dtable_, ws, target, fused,
+                                                                          half_rows);
         }
     }
     if (fused != nullptr) {
@@ -1632,12 +1650,28 @@ extern "C" size_t hashgrid_encode_backward_workspace_size(const char *opaque, si
     return (size_t)make_plan(d).bytes;
 }
 
-extern "C" void hashgrid_encode_backward(ngp_stream_t stream_, void **buffers, const char *opaque, size_t opaque_len) {
-    const char *target = "hashgrid_encode_backward";
+static bool half_rows_ok(const HashGridDescriptor &d, const BwdPlan &p) {
+    return d.F == 2 && d.table_dtype == NGP_DTYPE_F16 && p.bucket;
+}
+
+extern "C" int hashgrid_encode_backward_f16_supported(const char *opaque, size_t opaque_len) {
+    HashGridDescriptor d;
+    if (!read_descriptor(opaque, opaque_len, &d, "hashgrid_encode_backward_f16_supported")) return 0;
+    if (!validate(d, "hashgrid_encode_backward_f16_supported")) return 0;
+    return half_rows_ok(d, make_plan(d)) ? 1 : 0;
+}
+
+// Both table gradients: rows in f32, or (half_rows) in f16.
+static void encode_backward(ngp_stream_t stream_, void **buffers, const char *opaque, size_t opaque_len,
+                            const char *target, bool half_rows) {
     HashGridDescriptor d;
     if (!read_descriptor(opaque, opaque_len, &d, target)) return;
     if (!validate(d, target)) return;
     const BwdPlan plan = make_plan(d);
+    if (half_rows && !half_rows_ok(d, plan)) {
+        set_error(kBadDescriptor, "%s: needs F = 2, an f16 table and the one-pass table gradient", target);
+        return;
+    }
     if (plan.n_slices > kMaxSlices) {
         set_error(kBadDescriptor, "%s: table of %u rows exceeds %u row slices", target, d.n_rows, kMaxSlices);
         return;
@@ -1654,7 +1688,7 @@ extern "C" void hashgrid_encode_backward(ngp_stream_t stream_, void **buffers, c
     float *dtable = (float *)buffers[2];
     if (d.n_points == 0) {
         // no contributions: the gradient is zero
-        const size_t n = (size_t)d.n_rows * d.F;
+        const size_t n = (size_t)d.n_rows * d.F / (half_rows ? 2 : 1);  // in floats
         const bool vec = (reinterpret_cast<uintptr_t>(dtable) & 15u) == 0;
         const size_t n4 = vec ? n / 4 : 0;
         const size_t n_tail = n - 4 * n4;
@@ -1675,7 +1709,7 @@ extern "C" void hashgrid_encode_backward(ngp_stream_t stream_, void **buffers, c
     switch (d.F) {
         case 1: ok = launch_backward<1, false>(d, stream, pos, g, dtable, ws, target); break;
         case 2:
-            ok = half ? launch_backward<2, true>(d, stream, pos, g, dtable, ws, target)
+            ok = half ? launch_backward<2, true>(d, stream, pos, g, dtable, ws, target, nullptr, half_rows)
                       : launch_backward<2, false>(d, stream, pos, g, dtable, ws, target);
             break;
         case 4:
@@ -1686,4 +1720,13 @@ extern "C" void hashgrid_encode_backward(ngp_stream_t stream_, void **buffers, c
     }
     if (!ok) return;
     check_launch(target);
+}
+
+extern "C" void hashgrid_encode_backward(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
+    encode_backward(stream, buffers, opaque, opaque_len, "hashgrid_encode_backward", false);
+}
+
+extern "C" void hashgrid_encode_backward_f16(ngp_stream_t stream, void **buffers, const char *opaque,
+                                             size_t opaque_len) {
+    encode_backward(stream, buffers, opaque, opaque_len, "hashgrid_encode_backward_f16", true);
 }

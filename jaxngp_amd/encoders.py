@@ -89,10 +89,13 @@ class _HashGridFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         (pos,) = ctx.saved_tensors
-        dtable = torch.empty(ctx.table_shape, dtype=torch.float32, device=pos.device)
         desc = ctx.desc_fn(pos.shape[0])
+        # the rows of an f16 table's gradient are stored in f16: a cast reads and writes all of them again
+        half = ctx.table_dtype == torch.float16 and _lib.hashgrid_backward_f16_supported(desc)
+        dtable = torch.empty(ctx.table_shape, dtype=torch.float16 if half else torch.float32, device=pos.device)
         ws = torch.empty(_lib.hashgrid_backward_workspace_bytes(desc), dtype=torch.uint8, device=pos.device)
-        _lib.call("hashgrid_encode_backward", [pos, g.float().contiguous(), dtable, ws], desc)
+        _lib.call("hashgrid_encode_backward_f16" if half else "hashgrid_encode_backward",
+                  [pos, g.float().contiguous(), dtable, ws], desc)
         return None, dtable.to(ctx.table_dtype), None, None, None
 
 

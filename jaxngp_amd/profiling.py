@@ -32,13 +32,13 @@ TARGET_KERNELS = {
     "march_rays": (["march_begin_kernel", "march_count_kernel", "march_scan_kernel", "march_emit_kernel",
                     "march_fill_kernel", "march_finish_kernel", "march_empty_kernel"], "march_scan_kernel"),
     "hashgrid_encode": (["hashgrid_fwd_kernel", "encodings_to_points_kernel"], "hashgrid_fwd_kernel"),
-    "hashgrid_encode_backward": (["gradients_to_levels_kernel", "bwd_bucket_kernel", "bwd_slice_parts_kernel", "bwd_combine_runs_kernel",
-                                  "bwd_reduce_runs_kernel", "bwd_count_kernel", "scan_sums_kernel",
-                                  "scan_apply_kernel", "plan_parts_kernel", "bwd_scatter_kernel", "bwd_reduce_kernel",
-                                  "bwd_combine_kernel", "zero_table_kernel"], "bwd_reduce_runs_kernel"),
+    "hashgrid_encode_backward": (["gradients_to_levels_kernel", "bwd_bucket_kernel", "bwd_slice_parts_kernel",
+                                  "bwd_combine_runs_kernel", "bwd_reduce_runs_kernel", "bwd_count_kernel",
+                                  "scan_sums_kernel", "scan_apply_kernel", "plan_parts_kernel", "bwd_scatter_kernel",
+                                  "bwd_reduce_kernel", "bwd_combine_kernel", "zero_table_kernel"], "bwd_reduce_runs_kernel"),
     # the same kernels with the table's optimizer step in the reduce and combine passes
-    "hashgrid_encode_backward_adam": (["gradients_to_levels_kernel", "bwd_bucket_kernel", "bwd_slice_parts_kernel", "bwd_combine_runs_kernel",
-                                       "bwd_reduce_runs_kernel", "adam_zero_grad_kernel"], "bwd_reduce_runs_kernel"),
+    "hashgrid_encode_backward_adam": (["gradients_to_levels_kernel", "bwd_bucket_kernel", "bwd_slice_parts_kernel",
+                                       "bwd_combine_runs_kernel", "bwd_reduce_runs_kernel", "adam_zero_grad_kernel"], "bwd_reduce_runs_kernel"),
     "nerf_mlp_forward": (["mlp_forward_kernel", "mlp_forward_h_kernel"], None),
     "nerf_mlp_backward": (["mlp_backward_kernel", "mlp_backward_h_kernel", "sum_rows_kernel"], "sum_rows_kernel"),
     "integrate_rays": (["integrate_kernel"], "integrate_kernel"),

@@ -388,3 +388,29 @@ def test_point_major_gradient_on_both_sides_of_the_transpose(dev, n, L, half):
         _lib.call("hashgrid_encode_backward", [pos, grad, out, ws], d)
         got.append(out)
     assert (got[0] - got[1]).abs().max() <= 1e-6 * got[1].abs().max()
+
+
+@pytest.mark.parametrize("n, T", [(0, 1 << 15), (1, 1 << 15), (1000, 1 << 19), (77_777, 1 << 15), (130_000, 1 << 19)])
+def test_f16_rows_equal_the_cast_of_f32_rows(dev, n, T):
+    """hashgrid_encode_backward_f16 against a cast of hashgrid_encode_backward's rows: no points,
+    slices in one part, cut slices and both kinds of launches.  The f32 sums may differ in
+    their last bits (the order of an f64 sum), so at most one f16 step, in few rows."""
+    from jaxngp_amd import _lib
+    enc = HashGridEncoder(L=16, T=T, F=2, N_min=16, N_max=2048, generator=torch.Generator().manual_seed(3))
+    enc.table.data = enc.table.data.half()
+    enc = enc.to(dev)
+    g = torch.Generator(device=dev).manual_seed(n)
+    pos = torch.rand(n, 3, generator=g, device=dev) * 2 - 1
+    grad = torch.randn(n, 32, generator=g, device=dev)
+    if n > 1:
+        grad[0] = 1e6  # past f16: inf in both
+    d = enc.descriptor(n, 1.0)
+    assert _lib.hashgrid_backward_f16_supported(d)
+    ws = torch.empty(_lib.hashgrid_backward_workspace_bytes(d), dtype=torch.uint8, device=dev)
+    out = [torch.full(enc.table.shape, 3.0, dtype=dt, device=dev) for dt in (torch.float32, torch.float16)]
+    _lib.call("hashgrid_encode_backward", [pos, grad, out[0], ws], d)
+    _lib.call("hashgrid_encode_backward_f16", [pos, grad, out[1], ws], d)
+    want, got = out[0].half(), out[1]
+    apart = (want.view(torch.int16).int() - got.view(torch.int16).int()).abs()
+    assert int(apart.max()) <= 1 and float((apart > 0).float().mean()) < 1e-3
+    assert n < 2 or bool(torch.isinf(got).any())
