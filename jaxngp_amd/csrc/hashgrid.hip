@@ -341,9 +341,11 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
     const int ew = entry_words_host(d.F, d.table_dtype == NGP_DTYPE_F16);
     const bool half_values = d.F == 2 && d.table_dtype == NGP_DTYPE_F16;
     p.n_bchunks = std::max<uint32_t>(1, div_up(d.n_points, bucket_points(half_values)));
-    // (entry indexes within a level are 32 bits)
-    p.bucket = (plan_slices(d, kRunSliceBytes, p) || plan_slices(d, kSliceBytes, p)) &&
-               (uint64_t)p.n_bchunks * bucket_entries(half_values) <= 0xffffffffull;
+    // (entry indexes within a level are 32 bits; the small slices of a table past half of
+    // kMaxSlices * kSliceBytes would be more than kMaxSlices; the sort below takes kSliceBytes)
+    const bool short_index = (uint64_t)p.n_bchunks * bucket_entries(half_values) <= 0xffffffffull;
+    p.bucket = short_index && plan_slices(d, kRunSliceBytes, p) && p.n_slices <= kMaxSlices;
+    if (!p.bucket) p.bucket = plan_slices(d, kSliceBytes, p) && short_index;
     if (p.bucket) {
         p.n_bitems = d.L * p.n_bchunks;
         const uint64_t runs = (uint64_t)p.n_bitems * p.span_stride;

@@ -157,6 +157,24 @@ def test_hashgrid_backward_workspace_size():
     assert _lib.last_error() == (0, "")
 
 
+@pytest.mark.parametrize("L, T, F", [(20, 2 ** 21, 2), (32, 2 ** 21, 2), (20, 2 ** 22, 1), (16, 2 ** 22, 2)])
+@pytest.mark.parametrize("dt", [0, 1])
+def test_hashgrid_backward_takes_large_tables(L, T, F, dt):
+    """Tables of more rows than 8,192 slices of 64 KiB, but not of 128 KiB, hold are taken: the
+    first complaint is about the buffers.  Past that they are refused."""
+    from jaxngp_amd.encoders import level_table
+    lv = level_table(L, T, 256, 2 ** 14)
+    rows = 8192 * 16384 // F
+    assert rows // 2 < lv.n_rows <= rows
+    desc = lambda n, n_rows, offsets: _lib.hashgrid_descriptor(
+        n, L, F, T, lv.first_hash_level, dt, n_rows, 1.0, list(lv.scales), lv.resolutions, offsets)
+    for n in (0, 1000, 2 ** 18):
+        with pytest.raises(_lib.NGPError, match="buffer . is NULL"):
+            _lib.call_raw("hashgrid_encode_backward", [0] * 4, desc(n, lv.n_rows, lv.offsets))
+    with pytest.raises(_lib.NGPError, match="slices"):
+        _lib.call_raw("hashgrid_encode_backward", [0] * 4, desc(1000, rows + 1, list(lv.offsets[:-1]) + [rows + 1]))
+
+
 def test_sky_sphere_host_checks():
     """Parameter count, workspace size and descriptor errors need no GPU."""
     lib = _lib.load()
