@@ -212,7 +212,7 @@ def steady_state(tr, steps: int = 200) -> dict:
 
 CALIBRATION_STEPS = 30
 ROOFLINE_CANDIDATES = ("hashgrid_encode", "hashgrid_encode_backward", "hashgrid_encode_backward_adam", "march_rays",
-                       "integrate_rays", "integrate_rays_backward", "nerf_mlp_forward", "nerf_mlp_backward")
+                       "train_integrate", "nerf_mlp_forward", "nerf_mlp_backward")
 
 
 def run_training(data, cfg, steps: int, warmup: int, dev) -> dict:
@@ -235,7 +235,7 @@ def run_training(data, cfg, steps: int, warmup: int, dev) -> dict:
             torch.cuda.synchronize()
             log(f"[{cfg.precision}] warmup step {i}: {tr.metrics()}")
     torch.cuda.synchronize()
-    targets = ["march_rays", "hashgrid_encode", "nerf_mlp_forward", "integrate_rays", "integrate_rays_backward",
+    targets = ["march_rays", "hashgrid_encode", "nerf_mlp_forward", "train_integrate",
                "nerf_mlp_backward", "hashgrid_encode_backward", "hashgrid_encode_backward_adam", "adam_update_two"]
 
     class Timed:
@@ -459,8 +459,8 @@ def main() -> None:
         "hashgrid_encode_backward_adam": ("hbm", S * ENC_BYTES_PER_POINT +
                                           tr.model.position_encoder.table.numel() * ADAM_BYTES_PER_PARAM),
         "march_rays": ("hbm", spp * MARCH_BYTES_PER_SAMPLE + n_rays * MARCH_BYTES_PER_RAY),
-        "integrate_rays": ("hbm", S * INT_FWD_BYTES_PER_SAMPLE + n_rays * INT_FWD_BYTES_PER_RAY),
-        "integrate_rays_backward": ("hbm", S * INT_BWD_BYTES_PER_SAMPLE + n_rays * INT_BWD_BYTES_PER_RAY),
+        "train_integrate": ("hbm", S * (INT_FWD_BYTES_PER_SAMPLE + INT_BWD_BYTES_PER_SAMPLE)
+                            + n_rays * (INT_FWD_BYTES_PER_RAY + INT_BWD_BYTES_PER_RAY)),
         "nerf_mlp_forward": ("mfma", S * MLP_FWD_FLOP),
         "nerf_mlp_backward": ("mfma", S * MLP_FWD_FLOP * 3),
     }

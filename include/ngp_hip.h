@@ -627,6 +627,24 @@ typedef struct NgpLossDescriptor {
  * with NGP_LOSS_SCALED, one more input: NgpLossScaleState[1] */
 void train_loss_grad(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
+typedef struct NgpTrainIntegrateDescriptor {
+    uint32_t n_rays;        /* positive */
+    uint32_t total_samples; /* positive */
+    float near_distance;    /* as integrate_rays_backward */
+    float delta;            /* as train_loss_grad */
+    uint32_t flags;         /* as train_loss_grad */
+} NgpTrainIntegrateDescriptor;
+
+/* integrate_rays, train_loss_grad and integrate_rays_backward of one batch in two launches:
+ * the same values, the loss up to the order of its sum.
+ * in : rays_sample_startidx u32[n], rays_n_samples u32[n], bgs f32[n,3], dss f32[S],
+ *      z_vals f32[S], drgbs f32[S,4], gt_rgb f32[n,3], ray_is_valid bool[n]
+ * out: measured_batch_size u32[1], final_rgbds f32[n,4], final_opacities f32[n],
+ *      n_valid_rays u32[1], dL_dfinal_rgbds f32[n,4], loss f32[1], dL_dbgs f32[n,3],
+ *      dL_dz_vals f32[S], dL_ddrgbs f32[S,4] (every [.,4] 16-byte aligned)
+ * with NGP_LOSS_SCALED, one more input: NgpLossScaleState[1] */
+void train_integrate(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
+
 typedef struct NgpLossScaleCheckDescriptor {
     uint64_t n;
 } NgpLossScaleCheckDescriptor;

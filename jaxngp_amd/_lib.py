@@ -45,6 +45,7 @@ TARGETS = (
     "train_gt_blend",
     "train_bg_grad",
     "train_loss_grad",
+    "train_integrate",
     "adam_update",
     "adam_update_two",
     "loss_scale_check",
@@ -382,6 +383,10 @@ def proposal_train_descriptor(render_desc: bytes, total_samples, n_uniform=0) ->
 
 def proposal_loss_descriptor(n_rays, eps=1e-7) -> bytes:
     return struct.pack("<If", n_rays, eps)
+
+
+def train_integrate_descriptor(n_rays, total_samples, near_distance, delta, flags=0) -> bytes:
+    return struct.pack("<IIffI", n_rays, total_samples, near_distance, delta, flags)
 
 
 def near_far_descriptor(n_rays, bound) -> bytes:

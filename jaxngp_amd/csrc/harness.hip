@@ -14,6 +14,7 @@
 // so a step is reproducible from its inputs and needs no generator state.
 #include <hip/hip_fp16.h>
 
+#include "loss_device.h"
 #include "ngp_common.h"
 #include "rng_device.h"
 
@@ -134,47 +135,19 @@ __global__ void zero_u32_kernel(uint32_t *p, int n) {
 }
 
 // One workgroup counts the valid rays and writes the count and a zero loss
-// accumulator, so the loss needs no separate clearing launches (the batch's flags
-// are a few hundred KB; 16 bytes per load).
+// accumulator, so the loss needs no separate clearing launches.
 constexpr int kCountThreads = 1024;
 __global__ void __launch_bounds__(kCountThreads) count_valid_kernel(uint32_t n, const bool *__restrict__ flags,
                                                                     uint32_t *__restrict__ count,
                                                                     float *__restrict__ loss) {
     __shared__ uint32_t wsum[kCountThreads / kWave];
-    const uint8_t *f = reinterpret_cast<const uint8_t *>(flags);
-    uint32_t c = 0;
-    const uint32_t n16 = (reinterpret_cast<uintptr_t>(f) & 15u) == 0 ? n / 16 : 0;
-    // eight 16-byte loads in flight per thread (one round for 2^17 flags)
-    constexpr uint32_t kU = 8;
-    for (uint32_t q0 = 0; q0 < n16; q0 += kU * kCountThreads) {
-        uint4 v[kU];
-#pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) {
-            const uint32_t q = q0 + u * kCountThreads + threadIdx.x;
-            v[u] = q < n16 ? reinterpret_cast<const uint4 *>(f)[q] : make_uint4(0u, 0u, 0u, 0u);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) {
-            // bools are 0 or 1: add the bytes of each word
-            const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                c += (w[k] & 0xffu) + ((w[k] >> 8) & 0xffu) + ((w[k] >> 16) & 0xffu) + (w[k] >> 24);
-        }
-    }
-    for (uint32_t i = 16 * n16 + threadIdx.x; i < n; i += kCountThreads) c += f[i] ? 1u : 0u;
-    c = wave_sum(c);
-    if (lane_id() == 0) wsum[threadIdx.x / kWave] = c;
-    __syncthreads();
+    const uint32_t t = count_flags<kCountThreads>(n, flags, wsum);
     if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int w = 0; w < kCountThreads / kWave; ++w) t += wsum[w];
         *count = t;
         *loss = 0.0f;
     }
 }
 
-// optax.huber_loss(pred, target, delta): 0.5 e^2 if |e| <= delta else delta (|e| - delta/2)
 __global__ void __launch_bounds__(kBlock)
     loss_grad_kernel(uint32_t n, float delta, const float *__restrict__ rgbd, const float *__restrict__ gt,
                      const bool *__restrict__ valid, const uint32_t *__restrict__ n_valid,
@@ -187,17 +160,8 @@ __global__ void __launch_bounds__(kBlock)
         const float ls = scale_state != nullptr ? scale_state->scale : 1.0f;
         float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (valid[i]) {
-            float e[3], h = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                e[c] = rgbd[4 * (size_t)i + c] - gt[3 * (size_t)i + c];
-                const float ae = fabsf(e[c]);
-                h += ae <= delta ? 0.5f * e[c] * e[c] : delta * (ae - 0.5f * delta);
-            }
-            l = (h / 3.0f) / nv;
-            const float s = 1.0f / (3.0f * nv);
-            g = make_float4((fminf(fmaxf(e[0], -delta), delta) * s) * ls, (fminf(fmaxf(e[1], -delta), delta) * s) * ls,
-                            (fminf(fmaxf(e[2], -delta), delta) * s) * ls, 0.0f);
+            const float *c = rgbd + 4 * (size_t)i;
+            l = huber_ray(c[0], c[1], c[2], gt + 3 * (size_t)i, delta, nv, ls, g);
         }
         *reinterpret_cast<float4 *>(dL_drgbd + 4 * (size_t)i) = g;
     }

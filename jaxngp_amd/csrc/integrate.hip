@@ -11,6 +11,7 @@
 // the chunk, and the colour and depth sums run in sample order in four lanes.  Inference integration keeps one thread per pool slot
 // (at most march_steps_cap samples each).  Counters are reduced per wavefront and
 // added with one atomic per wave.
+#include "loss_device.h"
 #include "ngp_common.h"
 #include "ngp_device.h"
 
@@ -425,10 +426,230 @@ void zero_floats2(float *a, size_t na, float *b, size_t nb, hipStream_t stream) 
     hipLaunchKernelGGL(fill_zero2_kernel, dim3(grid), dim3(256), 0, stream, zero_range_of(a, na), zero_range_of(b, nb));
 }
 
+// What train_integrate needs before its rays: workgroup 0 counts the valid rays and clears
+// the counter and the loss, the others clear the gradients of the samples.  One launch of
+// 9 us where clearing the counter, counting and clearing the gradients were three (19).
+constexpr int kPrepareThreads = 1024;
+__global__ void __launch_bounds__(kPrepareThreads)
+    train_prepare_kernel(uint32_t n_rays, const bool *__restrict__ valid, uint32_t *__restrict__ n_valid,
+                         uint32_t *__restrict__ measured, float *__restrict__ loss, ZeroRange a, ZeroRange b) {
+    if (blockIdx.x == 0) {
+        __shared__ uint32_t wsum[kPrepareThreads / kWave];
+        const uint32_t t = count_flags<kPrepareThreads>(n_rays, valid, wsum);
+        if (threadIdx.x == 0) {
+            *n_valid = t;
+            *measured = 0u;
+            *loss = 0.0f;
+        }
+        return;
+    }
+    const size_t stride = (size_t)(gridDim.x - 1) * kPrepareThreads;
+    const size_t first = (size_t)(blockIdx.x - 1) * kPrepareThreads + threadIdx.x;
+    zero_range(a, first, stride);
+    zero_range(b, first, stride);
+}
+
+// integrate_kernel, the loss of its rays and integrate_backward_kernel in one: a ray's
+// wavefront has its colour, so it takes the gradient at once and goes back over its samples,
+// with the same operations in the same order.  The three are bound by one ray's chain and by
+// being launched, not by bytes.  A ray of one chunk keeps its chunk in registers (the forward
+// then leaves the prefix sums); longer ones run the chain again, as integrate_backward_kernel.
+__global__ void __launch_bounds__(kBlock)
+    train_integrate_kernel(NgpTrainIntegrateDescriptor d, const uint32_t *__restrict__ startidx,
+                           const uint32_t *__restrict__ nsamp, const float *__restrict__ bgs,
+                           const float *__restrict__ dss, const float *__restrict__ zs, const float *__restrict__ drgbs,
+                           const float *__restrict__ gt, const bool *__restrict__ valid,
+                           const uint32_t *__restrict__ n_valid, const NgpLossScaleState *__restrict__ scale_state,
+                           uint32_t *__restrict__ measured, float *__restrict__ rgbd_out,
+                           float *__restrict__ opacity_out, float *__restrict__ dL_drgbd, float *__restrict__ loss,
+                           float *__restrict__ dL_dbgs, float *__restrict__ dL_dz, float *__restrict__ dL_ddrgbs) {
+    __shared__ __align__(16) float rows_all[kBlock / kWave][kRows];
+    float *rows = rows_all[threadIdx.x / kWave];
+    float *prods = rows + 2 * kRow;
+    const int lane = lane_id();
+    const uint32_t n_waves = gridDim.x * (kBlock / kWave);
+    const uint32_t wave = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    const float nv = (float)max(*n_valid, 1u);
+    const float ls = scale_state != nullptr ? scale_state->scale : 1.0f;
+    uint32_t composited = 0;
+    float l = 0.0f;  // this lane's rays
+    for (uint64_t first = wave; first < d.n_rays; first += (uint64_t)kWave * n_waves) {
+        const RayBatch rb = load_ray_batch(first, n_waves, d.n_rays, startidx, nsamp, d.total_samples);
+        if (rb.in && rb.n == 0) {  // T = 1: background, opacity 0, a gradient of the background only
+            const float r = 0.0f + bgs[3 * rb.ray], g = 0.0f + bgs[3 * rb.ray + 1], b = 0.0f + bgs[3 * rb.ray + 2];
+            float4 gr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (valid[rb.ray]) l += huber_ray(r, g, b, gt + 3 * rb.ray, d.delta, nv, ls, gr);
+            opacity_out[rb.ray] = 0.0f;
+            *reinterpret_cast<float4 *>(rgbd_out + 4 * rb.ray) = make_float4(r, g, b, 0.0f);
+            *reinterpret_cast<float4 *>(dL_drgbd + 4 * rb.ray) = gr;
+            dL_dbgs[3 * rb.ray + 0] = 1.0f * gr.x;
+            dL_dbgs[3 * rb.ray + 1] = 1.0f * gr.y;
+            dL_dbgs[3 * rb.ray + 2] = 1.0f * gr.z;
+        }
+        for (uint64_t todo = __ballot(rb.in && rb.n > 0); todo != 0; todo &= todo - 1) {
+            const int src = __builtin_ctzll(todo);
+            const uint32_t ray = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rb.ray, src);
+            const size_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rb.s0, src);
+            const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)rb.n, src);
+            const bool one = n <= (uint32_t)kWave;
+            const bool ray_valid = valid[ray];
+            const float bg0 = bgs[3 * (size_t)ray], bg1 = bgs[3 * (size_t)ray + 1], bg2 = bgs[3 * (size_t)ray + 2];
+            Chunk ch;
+            float T, acc, alpha, om, Tq;
+            int stop;
+            // one chunk's chain: products of the samples before the stop, running sums in acc
+            const auto chain = [&](int m, bool prefix) {
+                alpha = lane < m ? 1.0f - det_expf(-ch.c.x * ch.ds) : 0.0f;
+                om = lane < m ? 1.0f - alpha : 1.0f;
+                stop = transmittance_chunk(rows, om, m, T, Tq);
+                const float w = Tq * alpha;
+                const bool in = lane < stop;
+                prods[lane] = in ? w * ch.c.y : 0.0f;
+                prods[kRow + lane] = in ? w * ch.c.z : 0.0f;
+                prods[2 * kRow + lane] = in ? w * ch.c.w : 0.0f;
+                prods[3 * kRow + lane] = in ? w * ch.z : 0.0f;
+                __builtin_amdgcn_wave_barrier();
+                ordered_sums(prods, acc, prefix);
+                __builtin_amdgcn_wave_barrier();
+            };
+            T = 1.0f;
+            acc = 0.0f;  // lane ch < 4: running r, g, b, depth
+            const Chunk chunk0 = load_chunk(drgbs, zs, dss, s0, 0, n);
+            Chunk next = chunk0;
+            for (uint32_t c0 = 0; c0 < n && T > kTThreshold; c0 += kWave) {
+                ch = next;
+                if (c0 + kWave < n) next = load_chunk(drgbs, zs, dss, s0, c0 + kWave, n);
+                chain((int)min(n - c0, (uint32_t)kWave), one);
+                composited += (uint32_t)stop;
+            }
+            const float op = 1.0f - T;
+            float out;  // lane c < 4: channel c
+            if (T <= kTThreshold) {
+                const float inv = 1.0f / op;
+                out = acc * inv;
+            } else {
+                const float bg = lane == 0 ? bg0 : (lane == 1 ? bg1 : bg2);
+                out = lane < 3 ? acc + T * bg : acc;
+            }
+            const float4 R =
+                make_float4(lane_value(out, 0), lane_value(out, 1), lane_value(out, 2), lane_value(out, 3));
+            float4 gr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (ray_valid) {
+                const float lr = huber_ray(R.x, R.y, R.z, gt + 3 * (size_t)ray, d.delta, nv, ls, gr);
+                if (lane == 0) l += lr;
+            }
+            if (lane == 0) {
+                const bool live = T > kTThreshold;
+                opacity_out[ray] = op;
+                *reinterpret_cast<float4 *>(rgbd_out + 4 * (size_t)ray) = R;
+                *reinterpret_cast<float4 *>(dL_drgbd + 4 * (size_t)ray) = gr;
+                dL_dbgs[3 * (size_t)ray + 0] = live ? T * gr.x : 0.0f;
+                dL_dbgs[3 * (size_t)ray + 1] = live ? T * gr.y : 0.0f;
+                dL_dbgs[3 * (size_t)ray + 2] = live ? T * gr.z : 0.0f;
+            }
+            const bool terminated = op >= 1.0f - kTThreshold;
+            const float bgk = terminated ? 0.0f : 1.0f - op;
+            // the gradients of the chunk at c0, from its chain with prefix sums
+            const auto back = [&](uint32_t c0) {
+                const float w = Tq * alpha;
+                const float T1 = Tq * om;  // T_{i+1} enters the gradient (integrating.cu:190-192)
+                if (lane < stop) {
+                    const float my_r = prods[lane], my_g = prods[kRow + lane], my_b = prods[2 * kRow + lane],
+                                my_d = prods[3 * kRow + lane];
+                    const size_t s = s0 + c0 + lane;
+                    dL_dz[s] = w * gr.w;
+                    const float a0 = gr.x * ((T1 * ch.c.y - (R.x - my_r)) - bg0 * bgk);
+                    const float a1 = gr.y * ((T1 * ch.c.z - (R.y - my_g)) - bg1 * bgk);
+                    const float a2 = gr.z * ((T1 * ch.c.w - (R.z - my_b)) - bg2 * bgk);
+                    const float a3 = gr.w * (T1 * ch.z - (R.w - my_d));
+                    const float dsig = ch.ds * (((a0 + a1) + a2) + a3);
+                    const float reg = ((double)ch.c.x > 4e-5 && ch.z < d.near_distance) ? 1e-4f : 0.0f;
+                    const float gs = fminf(ch.z * ch.z, 1.0f);
+                    *reinterpret_cast<float4 *>(dL_ddrgbs + 4 * s) =
+                        make_float4(gs * dsig + reg, w * gr.x, w * gr.y, w * gr.z);
+                }
+                __builtin_amdgcn_wave_barrier();
+            };
+            if (one) {
+                back(0);
+                continue;
+            }
+            T = 1.0f;
+            acc = 0.0f;
+            next = chunk0;
+            for (uint32_t c0 = 0; c0 < n && T > kTThreshold; c0 += kWave) {
+                ch = next;
+                if (c0 + kWave < n) next = load_chunk(drgbs, zs, dss, s0, c0 + kWave, n);
+                chain((int)min(n - c0, (uint32_t)kWave), true);
+                back(c0);
+            }
+        }
+    }
+    // one device atomic per workgroup and counter, as integrate_kernel
+    __shared__ uint32_t wave_n[kBlock / kWave];
+    __shared__ float wave_l[kBlock / kWave];
+#pragma unroll
+    for (int k = kWave / 2; k > 0; k >>= 1) l += __shfl_xor(l, k, kWave);
+    if (lane == 0) {
+        wave_n[threadIdx.x / kWave] = composited;
+        wave_l[threadIdx.x / kWave] = l;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t tot = 0;
+        float tot_l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kBlock / kWave; ++w) {
+            tot += wave_n[w];
+            tot_l += wave_l[w];
+        }
+        if (tot != 0) atomicAdd(measured, tot);
+        if (tot_l != 0.0f) atomicAdd(loss, tot_l);
+    }
+}
+
 }  // namespace
 }  // namespace ngp
 
 using namespace ngp;
+
+extern "C" void train_integrate(ngp_stream_t stream_, void **buffers, const char *opaque, size_t opaque_len) {
+    const char *target = "train_integrate";
+    NgpTrainIntegrateDescriptor d;
+    if (!read_descriptor(opaque, opaque_len, &d, target)) return;
+    if (d.flags & ~NGP_LOSS_SCALED) {
+        set_error(kBadDescriptor, "%s: unknown flags %u", target, d.flags);
+        return;
+    }
+    if (d.n_rays == 0 || d.total_samples == 0) {
+        set_error(kBadDescriptor, "%s: n_rays and total_samples must be positive", target);
+        return;
+    }
+    const bool scaled = (d.flags & NGP_LOSS_SCALED) != 0;
+    if (!check_buffers(buffers, 17, target)) return;
+    if (scaled && !check_buffer_list(buffers, {17}, target)) return;
+    for (int i : {5, 9, 12, 16}) {
+        if (!aligned16(buffers[i])) {
+            set_error(kBadArgument, "%s: buffer %d must be 16-byte aligned", target, i);
+            return;
+        }
+    }
+    hipStream_t stream = (hipStream_t)stream_;
+    const size_t S = d.total_samples;
+    const uint32_t clear = (uint32_t)std::min<size_t>((S + kPrepareThreads - 1) / kPrepareThreads, 1024);
+    hipLaunchKernelGGL(train_prepare_kernel, dim3(1 + clear), dim3(kPrepareThreads), 0, stream, d.n_rays,
+                       (const bool *)buffers[7], (uint32_t *)buffers[11], (uint32_t *)buffers[8], (float *)buffers[13],
+                       zero_range_of((float *)buffers[15], S), zero_range_of((float *)buffers[16], 4 * S));
+    if (!check_launch(target)) return;
+    hipLaunchKernelGGL(train_integrate_kernel, dim3(wave_grid(d.n_rays)), dim3(kBlock), 0, stream, d,
+                       (const uint32_t *)buffers[0], (const uint32_t *)buffers[1], (const float *)buffers[2],
+                       (const float *)buffers[3], (const float *)buffers[4], (const float *)buffers[5],
+                       (const float *)buffers[6], (const bool *)buffers[7], (const uint32_t *)buffers[11],
+                       scaled ? (const NgpLossScaleState *)buffers[17] : nullptr, (uint32_t *)buffers[8],
+                       (float *)buffers[9], (float *)buffers[10], (float *)buffers[12], (float *)buffers[13],
+                       (float *)buffers[14], (float *)buffers[15], (float *)buffers[16]);
+    check_launch(target);
+}
 
 extern "C" void integrate_rays(ngp_stream_t stream_, void **buffers, const char *opaque, size_t opaque_len) {
     const char *target = "integrate_rays";

@@ -42,6 +42,7 @@ TARGET_KERNELS = {
     "nerf_mlp_forward": (["mlp_forward_kernel", "mlp_forward_h_kernel"], None),
     "nerf_mlp_backward": (["mlp_backward_kernel", "mlp_backward_h_kernel", "sum_rows_kernel"], "sum_rows_kernel"),
     "integrate_rays": (["integrate_kernel"], "integrate_kernel"),
+    "train_integrate": (["train_prepare_kernel", "train_integrate_kernel"], "train_integrate_kernel"),
     "integrate_rays_backward": (["integrate_backward_kernel", "fill_zero2_kernel"], "integrate_backward_kernel"),
     "occupancy_grid_update": (["ogrid_update_kernel", "ogrid_decay_kernel", "ogrid_prefix_kernel",
                                "ogrid_points_kernel", "ogrid_density_kernel"], "ogrid_decay_kernel"),

@@ -12,7 +12,7 @@ A step is the sequence of C-ABI targets below on preallocated device buffers, al
 enqueued on the current stream with no host synchronisation (encodings and their
 gradients use the level-major [16, S, 2] layout between the encoder and the MLP):
   train_make_rays -> march_rays -> hashgrid_encode -> nerf_mlp_forward ->
-  integrate_rays -> train_loss_grad -> integrate_rays_backward ->
+  train_integrate (integrate_rays, train_loss_grad and integrate_rays_backward in one) ->
   nerf_mlp_backward -> hashgrid_encode_backward -> adam_update (table, MLP)
 """
 from __future__ import annotations
@@ -478,14 +478,11 @@ class Trainer:
             guided=guided if c.proposal_guided else None,
             encode=P("hashgrid_encode", [b["xyzs"], table, b["enc"]], hdesc),
             mlp=P("nerf_mlp_forward", [b["enc"], b["dirs"], mlp_w, b["drgbs"]], _lib.nerf_mlp_descriptor(S, 0, LM, pd)),
-            integrate=P("integrate_rays", [b["start"], b["ns"], b["bgs"], b["dss"], b["zs"], b["drgbs"], b["measured"],
-                                           b["rgbd"], b["op"]], _lib.integrating_descriptor(n, S)),
-            loss=P("train_loss_grad", [b["rgbd"], b["gt"], b["valid"], b["n_valid"], b["g_rgbd"], b["loss"]] + state,
-                   _lib.loss_descriptor(n, 0.1, flags)),
-            integrate_bwd=P("integrate_rays_backward", [b["start"], b["ns"], b["bgs"], b["dss"], b["zs"], b["drgbs"],
-                                                        b["rgbd"], b["op"], b["g_rgbd"], b["dbgs"], b["dz"],
-                                                        b["ddrgbs"]],
-                            _lib.integrating_backward_descriptor(n, S, c.near)),
+            # integrate_rays, train_loss_grad and integrate_rays_backward
+            integrate=P("train_integrate", [b["start"], b["ns"], b["bgs"], b["dss"], b["zs"], b["drgbs"], b["gt"],
+                                            b["valid"], b["measured"], b["rgbd"], b["op"], b["n_valid"], b["g_rgbd"],
+                                            b["loss"], b["dbgs"], b["dz"], b["ddrgbs"]] + state,
+                        _lib.train_integrate_descriptor(n, S, c.near, 0.1, flags)),
             mlp_bwd=P("nerf_mlp_backward", [b["enc"], b["dirs"], mlp_w, b["ddrgbs"], b["denc"], b["dparams"],
                                             b["ws"]], _lib.nerf_mlp_descriptor(S, b["ws"].shape[0], LM, pd)),
             encode_bwd=(P("hashgrid_encode_backward_adam", [b["xyzs"], b["denc"], table, o["tm"], o["tv"],
@@ -551,9 +548,8 @@ class Trainer:
     def step(self) -> None:
         """One training step (app/nerf/_utils.py:80-170), then the grid cadence.
         Kernel order: train_make_rays -> march_rays (or the guided sampler) -> (wait for
-        the previous update) -> hashgrid_encode -> nerf_mlp_forward -> integrate_rays ->
-        train_loss_grad -> integrate_rays_backward -> nerf_mlp_backward ->
-        hashgrid_encode_backward, then adam_update (table, MLP) on the side stream.
+        the previous update) -> hashgrid_encode -> nerf_mlp_forward -> train_integrate ->
+        nerf_mlp_backward -> hashgrid_encode_backward, then adam_update (table, MLP) on the side stream.
         With `prefetch_march`, the next step's train_make_rays and sampler are issued on
         the prefetch stream into the other buffer set before this step's MLP backward, so
         the latency-bound marcher overlaps the MLP backward, the table gradient and the
@@ -565,7 +561,7 @@ class Trainer:
         before the next step changes what it reads (see _prefetchable), and is dropped
         if the grid's bitfield was replaced meanwhile.  With a background model,
         sky_sphere_bg + train_gt_blend follow the wait and train_bg_grad +
-        sky_sphere_bg_backward follow integrate_rays_backward.  Readers of the
+        sky_sphere_bg_backward follow train_integrate.  Readers of the
         parameters outside the step go through `model`, `bg_model` or `sync()`."""
         c = self.cfg
         if self._calls is None:
@@ -590,11 +586,11 @@ class Trainer:
         # on the side stream; everything after waits for it
         self.sync()
         bg = self._bg_model is not None
-        order = ("encode", "mlp", "integrate", "loss", "integrate_bwd", "mlp_bwd", "encode_bwd")
+        order = ("encode", "mlp", "integrate", "mlp_bwd", "encode_bwd")
         if bg:
             # per-ray backgrounds from the model, the ground truth blended over them, and
             # their gradient after the integrator's (app/nerf/_utils.py:128-150)
-            order = ("bg_fwd", "bg_blend") + order[:5] + ("bg_grad", "bg_bwd") + order[5:]
+            order = ("bg_fwd", "bg_blend") + order[:3] + ("bg_grad", "bg_bwd") + order[3:]
         train_prop = self.prop is not None and s0 % c.proposal_every == 0
         t = s0 + 1  # the optimizer's step count after this step
         lr = lr_at(t - 1, c.lr)

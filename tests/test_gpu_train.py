@@ -356,3 +356,47 @@ def test_two_updates_in_one_launch_equal_two_launches(dev, n0, n1, half, flags, 
     assert torch.equal(out[0][1], init[0][0]) == overflow
     for x, y in zip(*out):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("n_rays, counts, scaled", [
+    (1, (1,), False), (5, (0, 1, 63, 64, 65), True), (300, (0, 64, 129, 500), False), (4099, (64,), True),
+    (70_001, (0, 0, 0, 3), False)])
+def test_train_integrate_matches_its_three_parts(n_rays, counts, scaled):
+    """train_integrate against integrate_rays, train_loss_grad and integrate_rays_backward on rays
+    of no, one and several chunks, transparent and opaque, valid or not, the last past the
+    arrays' end: every output bit for bit, the loss within the rounding of a sum of n_rays
+    positive terms in any order."""
+    from jaxngp_amd import _lib
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(n_rays)
+    ns = torch.tensor(counts, dtype=torch.int64).repeat(-(-n_rays // len(counts)))[:n_rays]
+    start = torch.cumsum(ns, 0) - ns
+    S = max(1, int(ns.sum()) - 1)
+    R = lambda *s: torch.rand(*s, generator=g, device=dev)
+    u32 = lambda t: t.to(torch.int32).to(dev).view(torch.uint32)
+    drgbs = R(S, 4)
+    drgbs[:, 0] *= torch.where(R(S) < 0.5, 1.0, 300.0)
+    ins = [u32(start), u32(ns), R(n_rays, 3), R(S) * 0.02, R(S) * 3, drgbs]
+    gt, valid = R(n_rays, 3), R(n_rays) < 0.9
+    flags = 1 if scaled else 0
+    state = [torch.tensor([512.0, 0.0, 0.0, 0.0], device=dev)] if scaled else []
+    out = lambda: dict(measured=torch.full((1,), 7, dtype=torch.int32, device=dev).view(torch.uint32),
+                       rgbd=torch.full((n_rays, 4), 5.0, device=dev), op=torch.full((n_rays,), 5.0, device=dev),
+                       n_valid=torch.full((1,), 7, dtype=torch.int32, device=dev).view(torch.uint32),
+                       g=torch.full((n_rays, 4), 5.0, device=dev), loss=torch.full((1,), 5.0, device=dev),
+                       dbgs=torch.full((n_rays, 3), 5.0, device=dev), dz=torch.full((S,), 5.0, device=dev),
+                       dd=torch.full((S, 4), 5.0, device=dev))
+    a, b = out(), out()
+    _lib.call("integrate_rays", ins + [a["measured"], a["rgbd"], a["op"]], _lib.integrating_descriptor(n_rays, S))
+    _lib.call("train_loss_grad", [a["rgbd"], gt, valid, a["n_valid"], a["g"], a["loss"]] + state,
+              _lib.loss_descriptor(n_rays, 0.1, flags))
+    _lib.call("integrate_rays_backward", ins + [a["rgbd"], a["op"], a["g"], a["dbgs"], a["dz"], a["dd"]],
+              _lib.integrating_backward_descriptor(n_rays, S, 0.3))
+    _lib.call("train_integrate", ins + [gt, valid] + list(b.values()) + state,
+              _lib.train_integrate_descriptor(n_rays, S, 0.3, 0.1, flags))
+    for k in a:
+        if k == "loss":
+            assert abs(float(a[k]) - float(b[k])) <= 2 * n_rays * 2.0 ** -24 * float(a[k])
+        else:
+            x, y = a[k].cpu(), b[k].cpu()
+            assert torch.equal(x.view(torch.int32), y.view(torch.int32)), k
