@@ -636,7 +636,8 @@ typedef struct NgpTrainIntegrateDescriptor {
 } NgpTrainIntegrateDescriptor;
 
 /* integrate_rays, train_loss_grad and integrate_rays_backward of one batch in two launches:
- * the same values, the loss up to the order of its sum.
+ * the same values, the loss up to the order of its sum.  The rays' sample ranges must not
+ * overlap (march_rays' and proposal_train_samples' do not).
  * in : rays_sample_startidx u32[n], rays_n_samples u32[n], bgs f32[n,3], dss f32[S],
  *      z_vals f32[S], drgbs f32[S,4], gt_rgb f32[n,3], ray_is_valid bool[n]
  * out: measured_batch_size u32[1], final_rgbds f32[n,4], final_opacities f32[n],

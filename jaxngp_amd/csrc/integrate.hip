@@ -452,8 +452,9 @@ __global__ void __launch_bounds__(kPrepareThreads)
 // integrate_kernel, the loss of its rays and integrate_backward_kernel in one: a ray's
 // wavefront has its colour, so it takes the gradient at once and goes back over its samples,
 // with the same operations in the same order.  The three are bound by one ray's chain and by
-// being launched, not by bytes.  A ray of one chunk keeps its chunk in registers (the forward
-// then leaves the prefix sums); longer ones run the chain again, as integrate_backward_kernel.
+// being launched, not by bytes.  The chain runs once: it leaves each sample's T and running
+// sums where the sample's gradients will be (registers for a ray of one chunk), and the way
+// back is one independent pass over them.  Rays' ranges must therefore not overlap.
 __global__ void __launch_bounds__(kBlock)
     train_integrate_kernel(NgpTrainIntegrateDescriptor d, const uint32_t *__restrict__ startidx,
                            const uint32_t *__restrict__ nsamp, const float *__restrict__ bgs,
@@ -494,14 +495,20 @@ __global__ void __launch_bounds__(kBlock)
             const bool one = n <= (uint32_t)kWave;
             const bool ray_valid = valid[ray];
             const float bg0 = bgs[3 * (size_t)ray], bg1 = bgs[3 * (size_t)ray + 1], bg2 = bgs[3 * (size_t)ray + 2];
+            float T = 1.0f, acc = 0.0f;  // lane ch < 4: running r, g, b, depth
             Chunk ch;
-            float T, acc, alpha, om, Tq;
-            int stop;
-            // one chunk's chain: products of the samples before the stop, running sums in acc
-            const auto chain = [&](int m, bool prefix) {
-                alpha = lane < m ? 1.0f - det_expf(-ch.c.x * ch.ds) : 0.0f;
-                om = lane < m ? 1.0f - alpha : 1.0f;
-                stop = transmittance_chunk(rows, om, m, T, Tq);
+            float4 sums = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // up to and including this lane's sample
+            float Tq = 0.0f;
+            uint32_t k = 0;  // composited samples
+            Chunk next = load_chunk(drgbs, zs, dss, s0, 0, n);
+            for (uint32_t c0 = 0; c0 < n && T > kTThreshold; c0 += kWave) {
+                ch = next;
+                if (c0 + kWave < n) next = load_chunk(drgbs, zs, dss, s0, c0 + kWave, n);
+                const int m = (int)min(n - c0, (uint32_t)kWave);
+                const float alpha = lane < m ? 1.0f - det_expf(-ch.c.x * ch.ds) : 0.0f;
+                const float om = lane < m ? 1.0f - alpha : 1.0f;
+                const int stop = transmittance_chunk(rows, om, m, T, Tq);
+                k += (uint32_t)stop;
                 const float w = Tq * alpha;
                 const bool in = lane < stop;
                 prods[lane] = in ? w * ch.c.y : 0.0f;
@@ -509,19 +516,16 @@ __global__ void __launch_bounds__(kBlock)
                 prods[2 * kRow + lane] = in ? w * ch.c.w : 0.0f;
                 prods[3 * kRow + lane] = in ? w * ch.z : 0.0f;
                 __builtin_amdgcn_wave_barrier();
-                ordered_sums(prods, acc, prefix);
+                ordered_sums(prods, acc, true);
                 __builtin_amdgcn_wave_barrier();
-            };
-            T = 1.0f;
-            acc = 0.0f;  // lane ch < 4: running r, g, b, depth
-            const Chunk chunk0 = load_chunk(drgbs, zs, dss, s0, 0, n);
-            Chunk next = chunk0;
-            for (uint32_t c0 = 0; c0 < n && T > kTThreshold; c0 += kWave) {
-                ch = next;
-                if (c0 + kWave < n) next = load_chunk(drgbs, zs, dss, s0, c0 + kWave, n);
-                chain((int)min(n - c0, (uint32_t)kWave), one);
-                composited += (uint32_t)stop;
+                sums = make_float4(prods[lane], prods[kRow + lane], prods[2 * kRow + lane], prods[3 * kRow + lane]);
+                __builtin_amdgcn_wave_barrier();
+                if (!one && in) {
+                    dL_dz[s0 + c0 + lane] = Tq;
+                    *reinterpret_cast<float4 *>(dL_ddrgbs + 4 * (s0 + c0 + lane)) = sums;
+                }
             }
+            composited += k;
             const float op = 1.0f - T;
             float out;  // lane c < 4: channel c
             if (T <= kTThreshold) {
@@ -549,39 +553,27 @@ __global__ void __launch_bounds__(kBlock)
             }
             const bool terminated = op >= 1.0f - kTThreshold;
             const float bgk = terminated ? 0.0f : 1.0f - op;
-            // the gradients of the chunk at c0, from its chain with prefix sums
-            const auto back = [&](uint32_t c0) {
-                const float w = Tq * alpha;
-                const float T1 = Tq * om;  // T_{i+1} enters the gradient (integrating.cu:190-192)
-                if (lane < stop) {
-                    const float my_r = prods[lane], my_g = prods[kRow + lane], my_b = prods[2 * kRow + lane],
-                                my_d = prods[3 * kRow + lane];
-                    const size_t s = s0 + c0 + lane;
-                    dL_dz[s] = w * gr.w;
-                    const float a0 = gr.x * ((T1 * ch.c.y - (R.x - my_r)) - bg0 * bgk);
-                    const float a1 = gr.y * ((T1 * ch.c.z - (R.y - my_g)) - bg1 * bgk);
-                    const float a2 = gr.z * ((T1 * ch.c.w - (R.z - my_b)) - bg2 * bgk);
-                    const float a3 = gr.w * (T1 * ch.z - (R.w - my_d));
-                    const float dsig = ch.ds * (((a0 + a1) + a2) + a3);
-                    const float reg = ((double)ch.c.x > 4e-5 && ch.z < d.near_distance) ? 1e-4f : 0.0f;
-                    const float gs = fminf(ch.z * ch.z, 1.0f);
-                    *reinterpret_cast<float4 *>(dL_ddrgbs + 4 * s) =
-                        make_float4(gs * dsig + reg, w * gr.x, w * gr.y, w * gr.z);
+            for (uint32_t c0 = 0; c0 < k; c0 += kWave) {
+                if (c0 + lane >= k) break;
+                const size_t s = s0 + c0 + lane;
+                if (!one) {
+                    ch = load_chunk(drgbs, zs, dss, s0, c0, k);
+                    Tq = dL_dz[s];
+                    sums = *reinterpret_cast<const float4 *>(dL_ddrgbs + 4 * s);
                 }
-                __builtin_amdgcn_wave_barrier();
-            };
-            if (one) {
-                back(0);
-                continue;
-            }
-            T = 1.0f;
-            acc = 0.0f;
-            next = chunk0;
-            for (uint32_t c0 = 0; c0 < n && T > kTThreshold; c0 += kWave) {
-                ch = next;
-                if (c0 + kWave < n) next = load_chunk(drgbs, zs, dss, s0, c0 + kWave, n);
-                chain((int)min(n - c0, (uint32_t)kWave), true);
-                back(c0);
+                const float alpha = 1.0f - det_expf(-ch.c.x * ch.ds);
+                const float w = Tq * alpha;
+                const float T1 = Tq * (1.0f - alpha);  // T_{i+1} enters the gradient (integrating.cu:190-192)
+                dL_dz[s] = w * gr.w;
+                const float a0 = gr.x * ((T1 * ch.c.y - (R.x - sums.x)) - bg0 * bgk);
+                const float a1 = gr.y * ((T1 * ch.c.z - (R.y - sums.y)) - bg1 * bgk);
+                const float a2 = gr.z * ((T1 * ch.c.w - (R.z - sums.z)) - bg2 * bgk);
+                const float a3 = gr.w * (T1 * ch.z - (R.w - sums.w));
+                const float dsig = ch.ds * (((a0 + a1) + a2) + a3);
+                const float reg = ((double)ch.c.x > 4e-5 && ch.z < d.near_distance) ? 1e-4f : 0.0f;
+                const float gs = fminf(ch.z * ch.z, 1.0f);
+                *reinterpret_cast<float4 *>(dL_ddrgbs + 4 * s) =
+                    make_float4(gs * dsig + reg, w * gr.x, w * gr.y, w * gr.z);
             }
         }
     }
