@@ -135,19 +135,21 @@ __device__ __forceinline__ void ordered_sums(float *prods, float &acc, bool pref
     const int lane = lane_id();
     if (lane < 4) {
         float4 *row = reinterpret_cast<float4 *>(prods + lane * kRow);
+        float4 v[kWave / 4];  // the whole row in registers first, so the reads overlap
+#pragma unroll
+        for (int q = 0; q < kWave / 4; ++q) v[q] = row[q];
         float a = acc;
-#pragma unroll 4
+#pragma unroll
         for (int q = 0; q < kWave / 4; ++q) {
-            float4 v = row[q];
-            a = a + v.x;
-            v.x = a;
-            a = a + v.y;
-            v.y = a;
-            a = a + v.z;
-            v.z = a;
-            a = a + v.w;
-            v.w = a;
-            if (prefix) row[q] = v;
+            a = a + v[q].x;
+            v[q].x = a;
+            a = a + v[q].y;
+            v[q].y = a;
+            a = a + v[q].z;
+            v[q].z = a;
+            a = a + v[q].w;
+            v[q].w = a;
+            if (prefix) row[q] = v[q];
         }
         acc = a;
     }
@@ -476,17 +478,6 @@ __global__ void __launch_bounds__(kBlock)
     float l = 0.0f;  // this lane's rays
     for (uint64_t first = wave; first < d.n_rays; first += (uint64_t)kWave * n_waves) {
         const RayBatch rb = load_ray_batch(first, n_waves, d.n_rays, startidx, nsamp, d.total_samples);
-        if (rb.in && rb.n == 0) {  // T = 1: background, opacity 0, a gradient of the background only
-            const float r = 0.0f + bgs[3 * rb.ray], g = 0.0f + bgs[3 * rb.ray + 1], b = 0.0f + bgs[3 * rb.ray + 2];
-            float4 gr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (valid[rb.ray]) l += huber_ray(r, g, b, gt + 3 * rb.ray, d.delta, nv, ls, gr);
-            opacity_out[rb.ray] = 0.0f;
-            *reinterpret_cast<float4 *>(rgbd_out + 4 * rb.ray) = make_float4(r, g, b, 0.0f);
-            *reinterpret_cast<float4 *>(dL_drgbd + 4 * rb.ray) = gr;
-            dL_dbgs[3 * rb.ray + 0] = 1.0f * gr.x;
-            dL_dbgs[3 * rb.ray + 1] = 1.0f * gr.y;
-            dL_dbgs[3 * rb.ray + 2] = 1.0f * gr.z;
-        }
         for (uint64_t todo = __ballot(rb.in && rb.n > 0); todo != 0; todo &= todo - 1) {
             const int src = __builtin_ctzll(todo);
             const uint32_t ray = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)rb.ray, src);
@@ -576,6 +567,22 @@ __global__ void __launch_bounds__(kBlock)
                     make_float4(gs * dsig + reg, w * gr.x, w * gr.y, w * gr.z);
             }
         }
+    }
+    // Rays without samples (T = 1: background, opacity 0, a gradient of the background only),
+    // neighbours in neighbouring lanes: in the strided batches above every lane's 69 bytes
+    // were lines of their own.  From the last wavefront down, as the first hold the valid rays.
+    const size_t n_threads = (size_t)gridDim.x * kBlock;
+    for (size_t ray = n_threads - 1 - ((size_t)blockIdx.x * kBlock + threadIdx.x); ray < d.n_rays; ray += n_threads) {
+        if (sample_count(startidx[ray], nsamp[ray], d.total_samples) != 0) continue;
+        const float r = 0.0f + bgs[3 * ray], g = 0.0f + bgs[3 * ray + 1], b = 0.0f + bgs[3 * ray + 2];
+        float4 gr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (valid[ray]) l += huber_ray(r, g, b, gt + 3 * ray, d.delta, nv, ls, gr);
+        opacity_out[ray] = 0.0f;
+        *reinterpret_cast<float4 *>(rgbd_out + 4 * ray) = make_float4(r, g, b, 0.0f);
+        *reinterpret_cast<float4 *>(dL_drgbd + 4 * ray) = gr;
+        dL_dbgs[3 * ray + 0] = 1.0f * gr.x;
+        dL_dbgs[3 * ray + 1] = 1.0f * gr.y;
+        dL_dbgs[3 * ray + 2] = 1.0f * gr.z;
     }
     // one device atomic per workgroup and counter, as integrate_kernel
     __shared__ uint32_t wave_n[kBlock / kWave];

@@ -12,7 +12,8 @@ __device__ __forceinline__ uint32_t count_flags(uint32_t n, const bool *__restri
     const uint8_t *f = reinterpret_cast<const uint8_t *>(flags);
     uint32_t c = 0;
     const uint32_t n16 = (reinterpret_cast<uintptr_t>(f) & 15u) == 0 ? n / 16 : 0;
-    // eight 16-byte loads in flight per thread (one round for 2^17 flags)
+    // eight 16-byte loads in flight per thread (one round for 2^17 flags; sixteen do not
+    // fit the registers of a workgroup of 1024 and took 45 us instead of 10)
     constexpr uint32_t kU = 8;
     for (uint32_t q0 = 0; q0 < n16; q0 += kU * kThreads) {
         uint4 v[kU];
@@ -23,11 +24,8 @@ __device__ __forceinline__ uint32_t count_flags(uint32_t n, const bool *__restri
         }
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u) {
-            // bools are 0 or 1: add the bytes of each word
-            const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                c += (w[k] & 0xffu) + ((w[k] >> 8) & 0xffu) + ((w[k] >> 16) & 0xffu) + (w[k] >> 24);
+            // bools are 0 or 1: a word's set bits are its true bytes
+            c += (uint32_t)(__popc(v[u].x) + __popc(v[u].y) + __popc(v[u].z) + __popc(v[u].w));
         }
     }
     for (uint32_t i = 16 * n16 + threadIdx.x; i < n; i += kThreads) c += f[i] ? 1u : 0u;
