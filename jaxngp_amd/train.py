@@ -624,8 +624,12 @@ class Trainer:
         self.step_count += 1
         # the update on the side stream, once the gradients exist; the next step's
         # rays and march run meanwhile
-        self._bwd_done.record(self.main_stream)
-        self.side_stream.wait_event(self._bwd_done)
+        # (in order on the one stream there is nothing to wait for: an event costs the stream
+        # 5 us, the step f32 599 -> 593 us, guided f16 497 -> 490)
+        apart = self.side_stream is not self.main_stream
+        if apart:
+            self._bwd_done.record(self.main_stream)
+            self.side_stream.wait_event(self._bwd_done)
         with torch.cuda.stream(self.side_stream):
             if self.fp16:
                 k["check_two"]()
@@ -646,8 +650,9 @@ class Trainer:
                                                   1e-6, flags=k["flags"]))
             if self.fp16:
                 k["scale_update"]()
-        self._adam_done.record(self.side_stream)
-        self._adam_pending = True
+        if apart:
+            self._adam_done.record(self.side_stream)
+        self._adam_pending = apart
         self._cur = nxt
         _lib.check()
         self.maybe_update_grid()
