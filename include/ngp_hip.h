@@ -627,6 +627,8 @@ typedef struct NgpLossDescriptor {
  * with NGP_LOSS_SCALED, one more input: NgpLossScaleState[1] */
 void train_loss_grad(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
+#define NGP_TRAIN_COUNT_PARTS 32u
+
 typedef struct NgpTrainIntegrateDescriptor {
     uint32_t n_rays;        /* positive */
     uint32_t total_samples; /* positive */
@@ -643,6 +645,7 @@ typedef struct NgpTrainIntegrateDescriptor {
  * out: measured_batch_size u32[1], final_rgbds f32[n,4], final_opacities f32[n],
  *      n_valid_rays u32[1], dL_dfinal_rgbds f32[n,4], loss f32[1], dL_dbgs f32[n,3],
  *      dL_dz_vals f32[S], dL_ddrgbs f32[S,4] (every [.,4] 16-byte aligned)
+ * scratch: u32[NGP_TRAIN_COUNT_PARTS]
  * with NGP_LOSS_SCALED, one more input: NgpLossScaleState[1] */
 void train_integrate(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 

@@ -385,6 +385,9 @@ def proposal_loss_descriptor(n_rays, eps=1e-7) -> bytes:
     return struct.pack("<If", n_rays, eps)
 
 
+TRAIN_COUNT_PARTS = 32
+
+
 def train_integrate_descriptor(n_rays, total_samples, near_distance, delta, flags=0) -> bytes:
     return struct.pack("<IIffI", n_rays, total_samples, near_distance, delta, flags)
 

@@ -190,6 +190,7 @@ class Trainer:
             start=z(n, dtype=u32), idcs=z(S, dtype=u32), xyzs=z(S, 3), dirs=z(S, 3), dss=z(S), zs=z(S),
             enc=z(16, S, 2), drgbs=z(S, 4), measured=cnt[3:4], rgbd=z(n, 4), op=z(n), n_valid=cnt[2:3],
             loss=z(1), g_rgbd=z(n, 4), dbgs=z(n, 3), dz=z(S), ddrgbs=z(S, 4), denc=z(16, S, 2), dparams=z(N_PARAMS),
+            parts=z(_lib.TRAIN_COUNT_PARTS, dtype=u32),
             ws=z(mlp_workspace_blocks(S), N_PARAMS), dtable=z(*self.model.position_encoder.table.shape),
         )
         if cfg.proposal_guided:
@@ -481,7 +482,7 @@ class Trainer:
             # integrate_rays, train_loss_grad and integrate_rays_backward
             integrate=P("train_integrate", [b["start"], b["ns"], b["bgs"], b["dss"], b["zs"], b["drgbs"], b["gt"],
                                             b["valid"], b["measured"], b["rgbd"], b["op"], b["n_valid"], b["g_rgbd"],
-                                            b["loss"], b["dbgs"], b["dz"], b["ddrgbs"]] + state,
+                                            b["loss"], b["dbgs"], b["dz"], b["ddrgbs"], b["parts"]] + state,
                         _lib.train_integrate_descriptor(n, S, c.near, 0.1, flags)),
             mlp_bwd=P("nerf_mlp_backward", [b["enc"], b["dirs"], mlp_w, b["ddrgbs"], b["denc"], b["dparams"],
                                             b["ws"]], _lib.nerf_mlp_descriptor(S, b["ws"].shape[0], LM, pd)),

@@ -386,13 +386,14 @@ def test_train_integrate_matches_its_three_parts(n_rays, counts, scaled):
                        g=torch.full((n_rays, 4), 5.0, device=dev), loss=torch.full((1,), 5.0, device=dev),
                        dbgs=torch.full((n_rays, 3), 5.0, device=dev), dz=torch.full((S,), 5.0, device=dev),
                        dd=torch.full((S, 4), 5.0, device=dev))
+    parts = torch.empty(_lib.TRAIN_COUNT_PARTS, dtype=torch.int32, device=dev)
     a, b = out(), out()
     _lib.call("integrate_rays", ins + [a["measured"], a["rgbd"], a["op"]], _lib.integrating_descriptor(n_rays, S))
     _lib.call("train_loss_grad", [a["rgbd"], gt, valid, a["n_valid"], a["g"], a["loss"]] + state,
               _lib.loss_descriptor(n_rays, 0.1, flags))
     _lib.call("integrate_rays_backward", ins + [a["rgbd"], a["op"], a["g"], a["dbgs"], a["dz"], a["dd"]],
               _lib.integrating_backward_descriptor(n_rays, S, 0.3))
-    _lib.call("train_integrate", ins + [gt, valid] + list(b.values()) + state,
+    _lib.call("train_integrate", ins + [gt, valid] + list(b.values()) + [parts] + state,
               _lib.train_integrate_descriptor(n_rays, S, 0.3, 0.1, flags))
     for k in a:
         if k == "loss":
