@@ -464,6 +464,9 @@ __global__ void __launch_bounds__(kPrepareThreads)
 // being launched, not by bytes.  The chain runs once: it leaves each sample's T and running
 // sums where the sample's gradients will be (registers for a ray of one chunk), and the way
 // back is one independent pass over them.  Rays' ranges must therefore not overlap.
+// A training batch of 2^18 samples, 1,450 rays of 2^18 with samples: 66 us as six kernels, 38-45
+// with the chain run twice, now 27 and 6 for train_prepare_kernel; what is left is the longest
+// ray's chain, 64 dependent products and sums a chunk.
 __global__ void __launch_bounds__(kBlock)
     train_integrate_kernel(NgpTrainIntegrateDescriptor d, const uint32_t *__restrict__ startidx,
                            const uint32_t *__restrict__ nsamp, const float *__restrict__ bgs,
