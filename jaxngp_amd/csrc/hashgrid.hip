@@ -243,18 +243,23 @@ __device__ __forceinline__ float entry_value(const uint32_t *w, int f) {
     }
 }
 
-// The last row level l's vertices can address.  A dense level's vertex
-// coordinates reach res (a point on the upper face), so its rows run up to
-// res + res^2 + res^3 past the level's offset, into the next level's rows, as the
-// reference's indices do; hashed rows stay below offset + T.  Clamped to the table.
-__host__ __device__ inline uint32_t level_last_row(const HashGridDescriptor &d, uint32_t l) {
-    const uint64_t res = d.resolutions[l];
-    uint64_t local = (uint64_t)d.T - 1u;
-    if (l < d.first_hash_level) local = std::min<uint64_t>(local, res + res * res + res * res * res);
-    return (uint32_t)std::min<uint64_t>((uint64_t)d.offsets[l] + local, (uint64_t)d.n_rows - 1u);
+// The last row level l's vertices can address: rows are taken modulo T, so a point outside
+// the box reaches any of the T rows from the level's offset on, past a dense level's own, as
+// the reference's indices do.  Clamped to the table.
+inline uint32_t level_last_row(const HashGridDescriptor &d, uint32_t l) {
+    return (uint32_t)std::min<uint64_t>((uint64_t)d.offsets[l] + d.T - 1u, (uint64_t)d.n_rows - 1u);
 }
 
-// The one-pass table gradient (F <= 2, every level's rows within kStageSlices
+// The last one that points of the box address.  A dense level's vertex coordinates reach
+// res (a point on the upper face), so its rows run up to res + res^2 + res^3 past the
+// level's offset, into the next level's.
+inline uint32_t level_last_box_row(const HashGridDescriptor &d, uint32_t l) {
+    const uint64_t res = d.resolutions[l];
+    const uint64_t local = l < d.first_hash_level ? res + res * res + res * res * res : ~0ull >> 1;
+    return (uint32_t)std::min<uint64_t>(d.offsets[l] + local, level_last_row(d, l));
+}
+
+// The one-pass table gradient (F <= 2, every level's rows of the box within kStageSlices
 // slices): work item = (level, bucket_points consecutive points).  Its entries are kept
 // in two arrays, the F values (f32, or one half2 for an f16 table with F = 2) and the
 // 16-bit row within the slice: 10 or 6 bytes instead of 12 or 8.
@@ -265,7 +270,7 @@ constexpr int kBucketThreads = 512;
 constexpr int bucket_phases(bool half_values) { return half_values ? 1 : 2; }
 constexpr uint32_t bucket_points(bool half_values) { return kBucketThreads * bucket_phases(half_values); }
 constexpr uint32_t bucket_entries(bool half_values) { return bucket_points(half_values) * 8; }  // one item's at most
-constexpr uint32_t kStageSlices = 1024;                 // slices one level may span
+constexpr uint32_t kStageSlices = 1024;                 // slices one level may span inside the box
 
 constexpr uint32_t kStageEntries = 4096;                // entries staged in LDS at a time
 
@@ -302,13 +307,15 @@ struct BwdPlan {
     uint32_t max_parts;     // upper bound of the reduce grid
     uint64_t counts_off, sums_off, meta_off, parts_off, part_slice_off, partials_off, entries_off, bytes;
     // one-pass path: items of bucket_points points, each level's slices
-    // [s_lo[l], s_hi[l]], per item and slice of its level the run's start and length
+    // [s_lo[l], s_hi[l]] (all it can reach), per item and slice of its level the run's start
+    // and length
     bool bucket;
+    bool wide;  // a level reaches more than kStageSlices slices, outside the box
     uint32_t n_bchunks, n_bitems, span_stride;
     uint32_t run_part;     // entries one workgroup of the reducer sums
     uint32_t group_shift;  // log2 of the slices in kSliceBytes
     uint32_t s_lo[NGP_HASHGRID_MAX_LEVELS], s_hi[NGP_HASHGRID_MAX_LEVELS];
-    uint64_t runs_off, slice_np_off, first_part_off, split_off, rows_off, part_group_off;
+    uint64_t runs_off, slice_np_off, first_part_off, split_off, levels_off, rows_off, part_group_off;
     bool whole;      // no slice can be cut into parts
     bool transpose;  // a point-major gradient is copied level-major first (to partials_off)
 };
@@ -322,17 +329,22 @@ constexpr uint32_t slice_rows() {
 }
 
 // Slices of kRunSliceBytes for the one-pass form where every level then spans at most
-// kStageSlices slices, else of kSliceBytes; whether either fits.
-inline bool plan_slices(const HashGridDescriptor &d, uint32_t slice_bytes, BwdPlan &p) {
+// kStageSlices slices for points of the box, else of kSliceBytes; whether either fits.
+// box_hi: the levels' last slices for points of the box.
+inline bool plan_slices(const HashGridDescriptor &d, uint32_t slice_bytes, BwdPlan &p, uint32_t *box_hi) {
     p.R = slice_bytes / (8 * d.F);
     p.n_slices = div_up(d.n_rows, p.R);
     p.span_stride = 1;
+    uint32_t box_span = 1;
     for (uint32_t l = 0; l < d.L; ++l) {
         p.s_lo[l] = d.offsets[l] / p.R;
         p.s_hi[l] = level_last_row(d, l) / p.R;
         p.span_stride = std::max(p.span_stride, p.s_hi[l] - p.s_lo[l] + 1u);
+        box_hi[l] = level_last_box_row(d, l) / p.R;
+        box_span = std::max(box_span, box_hi[l] - p.s_lo[l] + 1u);
     }
-    return d.F <= 2 && p.span_stride <= kStageSlices;
+    p.wide = p.span_stride > kStageSlices;
+    return d.F <= 2 && box_span <= kStageSlices;
 }
 
 inline BwdPlan make_plan(const HashGridDescriptor &d) {
@@ -344,8 +356,9 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
     // (entry indexes within a level are 32 bits; the small slices of a table past half of
     // kMaxSlices * kSliceBytes would be more than kMaxSlices; the sort below takes kSliceBytes)
     const bool short_index = (uint64_t)p.n_bchunks * bucket_entries(half_values) <= 0xffffffffull;
-    p.bucket = short_index && plan_slices(d, kRunSliceBytes, p) && p.n_slices <= kMaxSlices;
-    if (!p.bucket) p.bucket = plan_slices(d, kSliceBytes, p) && short_index;
+    uint32_t box_hi[NGP_HASHGRID_MAX_LEVELS];
+    p.bucket = short_index && plan_slices(d, kRunSliceBytes, p, box_hi) && p.n_slices <= kMaxSlices;
+    if (!p.bucket) p.bucket = plan_slices(d, kSliceBytes, p, box_hi) && short_index;
     if (p.bucket) {
         p.n_bitems = d.L * p.n_bchunks;
         const uint64_t runs = (uint64_t)p.n_bitems * p.span_stride;
@@ -358,8 +371,8 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         const uint64_t mean = (uint64_t)d.n_points * 8 * p.R / d.T;
         p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 2 + 1023) / 1024 * 1024));
         p.group_shift = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
-        // Few points: even all contributions of all levels that share a group of slices
-        // make one part, so nothing is counted, cut or combined: two launches, not four
+        // Few points: even all contributions of all levels that share a group of slices inside
+        // the box make one part, so nothing is counted, cut or combined: two launches, not four
         // (2000 ray samples f32: 35 -> 26 us; the line is where a group could be cut, and
         // with every point in a fifth of the box 4000 points take 73 us on either side).
         uint32_t sharing = 0;
@@ -367,7 +380,7 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
             uint32_t n = 0;
             for (uint32_t k = 0; k < d.L; ++k)
                 n += (p.s_lo[k] >> p.group_shift) <= (p.s_lo[l] >> p.group_shift) &&
-                     (p.s_hi[k] >> p.group_shift) >= (p.s_lo[l] >> p.group_shift);
+                     (box_hi[k] >> p.group_shift) >= (p.s_lo[l] >> p.group_shift);
             sharing = std::max(sharing, n);
         }
         p.whole = (uint64_t)d.n_points * 8 * sharing <= kPart;
@@ -383,7 +396,8 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         p.slice_np_off = align(p.runs_off + 4 * runs);
         p.first_part_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
         p.split_off = align(p.first_part_off + 4 * (uint64_t)p.n_slices);
-        p.meta_off = align(p.split_off + 4 * (uint64_t)p.n_slices);  // [0] parts, [1] cut slices
+        p.levels_off = align(p.split_off + 4 * (uint64_t)p.n_slices);
+        p.meta_off = align(p.levels_off + 4 * (uint64_t)p.n_slices);  // [0] parts, [1] cut slices
         p.part_slice_off = align(p.meta_off + 8);
         p.partials_off = align(p.part_slice_off + 4 * (uint64_t)p.max_parts);
         p.transpose = d.F == 2 && d.enc_layout == NGP_ENC_POINT_MAJOR && !p.whole && d.n_points >= kTransposeFrom;
@@ -741,8 +755,9 @@ __device__ __forceinline__ void sum_runs(float *v, const CellRuns &r) {
 // LDS-atomic order; the reducer's sums do not depend on it beyond f64 rounding.
 // 2^18 ray samples: f32 110 -> 68 us, f16 90 -> 50 us.  It was bound by the run merge
 // (each corner found its own runs: 626 vector instructions a wavefront and level) and,
-// once that was cheaper (86 us), by 17 M scattered 12-byte stores.
-template <int F, bool kHalf, uint32_t R>
+// once that was cheaper (86 us), by 17 M scattered 12-byte stores.  kSlices: counters for as
+// many slices as a level can reach; the last of them, kMaxSlices, take 32 KiB of LDS.
+template <int F, bool kHalf, uint32_t R, uint32_t kSlices>
 __global__ void __launch_bounds__(kBucketThreads)
     bwd_bucket_kernel(HashGridDescriptor d, BwdPlan p, const float *__restrict__ pos,
                       const float *__restrict__ dL_denc, uint32_t *__restrict__ runs_out,
@@ -752,16 +767,16 @@ __global__ void __launch_bounds__(kBucketThreads)
     constexpr int kBucketPhases = bucket_phases(kHalf);
     constexpr uint32_t kBucketPoints = bucket_points(kHalf), kBucketEntries = bucket_entries(kHalf);
     static_assert(R <= 0x10000u, "rows within a slice fit 16 bits");
-    constexpr int kPer = kStageSlices / kBucketThreads;
-    static_assert(kPer * kBucketThreads == kStageSlices, "whole slice counters per thread");
-    __shared__ uint32_t cnt[kStageSlices];
+    constexpr int kPer = kSlices / kBucketThreads;
+    static_assert(kPer * kBucketThreads == kSlices, "whole slice counters per thread");
+    __shared__ uint32_t cnt[kSlices];
     __shared__ __align__(16) Value stage_v[kStageEntries];
     __shared__ __align__(16) uint16_t stage_r[kStageEntries];
     const uint32_t item = blockIdx.x;
     if (item == 0 && threadIdx.x < 2) meta[threadIdx.x] = 0u;  // for bwd_slice_parts_kernel
     const uint32_t l = item / p.n_bchunks, k = item % p.n_bchunks;
     const uint32_t s_lo = p.s_lo[l];
-    const uint32_t span = p.s_hi[l] - s_lo + 1u;  // <= kStageSlices (host check)
+    const uint32_t span = p.s_hi[l] - s_lo + 1u;  // <= kSlices (host check)
     const bool pow2 = (d.T & (d.T - 1u)) == 0;
     const bool level_major = d.enc_layout == NGP_ENC_LEVEL_MAJOR;
     const float scale = d.scales[l];
@@ -915,38 +930,45 @@ __device__ __forceinline__ uint32_t slice_run_length(const BwdPlan &p, const uin
 
 // One-pass table gradient, part 2: the number of parts of slice s, from the run lengths of
 // every item whose level reaches s or the other slice of its group, and for a slice of
-// several a slot for each and its place in the list of cut slices.
+// several a slot for each and its place in the list of cut slices.  Also the levels that
+// have entries in s: outside the box a dense level reaches many slices, inside few.
 __global__ void __launch_bounds__(256)
     bwd_slice_parts_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ runs,
                            uint32_t *__restrict__ meta, uint32_t *__restrict__ slice_np,
                            uint32_t *__restrict__ first_part, uint32_t *__restrict__ part_slice,
-                           uint32_t *__restrict__ split) {
+                           uint32_t *__restrict__ split, uint32_t *__restrict__ slice_levels) {
     const uint32_t s = blockIdx.x, other = p.group_shift ? s ^ 1u : s;
-    uint32_t own = 0, both = 0;
+    uint32_t own = 0, both = 0, levels = 0;
     for (uint32_t l = 0; l < d.L; ++l) {
         const bool here = s >= p.s_lo[l] && s <= p.s_hi[l], there = other >= p.s_lo[l] && other <= p.s_hi[l];
         if (!here && !there) continue;
+        const uint32_t before = own;
         for (uint32_t k = threadIdx.x; k < p.n_bchunks; k += 256) {
             const uint32_t n = here ? run_length(runs[run_index(p, l, s - p.s_lo[l], k)]) : 0u;
             own += n;
             both += n;
             if (p.group_shift && there) both += run_length(runs[run_index(p, l, other - p.s_lo[l], k)]);
         }
+        if (__ballot(own != before) != 0ull) levels |= 1u << l;
     }
-    __shared__ uint32_t ws[2][256 / kWave];
+    __shared__ uint32_t ws[3][256 / kWave];
     own = wave_sum(own);
     both = wave_sum(both);
     if (lane_id() == 0) {
         ws[0][threadIdx.x / kWave] = own;
         ws[1][threadIdx.x / kWave] = both;
+        ws[2][threadIdx.x / kWave] = levels;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         uint64_t t = 0, g = 0;
+        uint32_t m = 0;
         for (int w = 0; w < 256 / kWave; ++w) {
             t += ws[0][w];
             g += ws[1][w];
+            m |= ws[2][w];
         }
+        slice_levels[s] = m;
         const uint32_t n = n_cuts(t, p.run_part) + n_cuts(g, kPart) - 1u;
         slice_np[s] = n;
         if (n > 1) {  // which slot a part gets does not matter to its sums
@@ -1133,7 +1155,7 @@ enum { kFloatRows, kAdamRows, kHalfRows };
 template <int F, bool kHalf, uint32_t R, int kOut>
 __device__ __forceinline__ void
 reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t part, uint32_t n_parts, uint32_t slot,
-            const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
+            uint32_t own_levels, uint32_t levels, const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
             const uint16_t *__restrict__ entry_rows, double *__restrict__ partials, uint32_t *__restrict__ part_group,
             void *__restrict__ dtable, const AdamStep &adam, float *__restrict__ adam_p, float *__restrict__ adam_m,
             float *__restrict__ adam_v) {
@@ -1156,9 +1178,9 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
     if (threadIdx.x == 0) my_group = 0xffffffffu;
     uint32_t carry = 0, carry_group = 0;  // entries of the items visited before
     const uint32_t other = p.group_shift ? s ^ 1u : s;
-    for (uint32_t l = 0; l < d.L; ++l) {
-        const bool here = s >= p.s_lo[l] && s <= p.s_hi[l];
-        if (!here && (n_parts == 1 || other < p.s_lo[l] || other > p.s_hi[l])) continue;
+    for (uint32_t left = levels; left != 0; left &= left - 1u) {
+        const uint32_t l = (uint32_t)__builtin_ctz(left);
+        const bool here = (own_levels >> l) & 1u;
         const uint32_t *level_runs = runs + (here ? run_index(p, l, s - p.s_lo[l], 0) : 0);
         for (uint32_t k0 = 0; k0 < p.n_bchunks; k0 += kRunThreads) {
             const uint32_t n_k = min(p.n_bchunks - k0, (uint32_t)kRunThreads);
@@ -1233,11 +1255,27 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
     }
 }
 
+// The levels that have entries in slice s, in every lane, read from the runs of few items.
+__device__ __forceinline__ uint32_t levels_of(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s,
+                                              const uint32_t *__restrict__ runs) {
+    static_assert(2 * NGP_HASHGRID_MAX_LEVELS == kWave, "two lanes a level");
+    const uint32_t l = lane_id() % NGP_HASHGRID_MAX_LEVELS;
+    uint32_t any = 0;
+    if (l < d.L && s >= p.s_lo[l] && s <= p.s_hi[l]) {
+#pragma unroll 4
+        for (uint32_t k = lane_id() / NGP_HASHGRID_MAX_LEVELS; k < p.n_bchunks; k += 2)
+            any |= run_length(runs[run_index(p, l, s - p.s_lo[l], k)]);
+    }
+    const uint64_t m = __ballot(any != 0u);
+    return (uint32_t)m | (uint32_t)(m >> 32);
+}
+
 template <int F, bool kHalf, uint32_t R, int kOut>
 __global__ void __launch_bounds__(kRunThreads)
     bwd_reduce_runs_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ meta,
                            const uint32_t *__restrict__ slice_np, const uint32_t *__restrict__ first_part,
-                           const uint32_t *__restrict__ part_slice, const uint32_t *__restrict__ runs,
+                           const uint32_t *__restrict__ part_slice, const uint32_t *__restrict__ slice_levels,
+                           const uint32_t *__restrict__ runs,
                            const EntryValue<F, kHalf> *__restrict__ values, const uint16_t *__restrict__ entry_rows,
                            double *__restrict__ partials, uint32_t *__restrict__ part_group,
                            void *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
@@ -1247,9 +1285,11 @@ __global__ void __launch_bounds__(kRunThreads)
         if (blockIdx.x < kSplitBlocks) {
             const uint32_t n = meta[0];
             for (uint32_t i = blockIdx.x; i < n; i += kSplitBlocks) {
-                const uint32_t cut = part_slice[i];
-                reduce_part<F, kHalf, R, kOut>(d, p, cut, i - first_part[cut], slice_np[cut], i, runs, values, entry_rows,
-                                                partials, part_group, dtable, adam, adam_p, adam_m, adam_v);
+                const uint32_t cut = part_slice[i], other = cut ^ 1u;
+                const uint32_t own = slice_levels[cut];
+                const uint32_t all = own | (p.group_shift && other < p.n_slices ? slice_levels[other] : 0u);
+                reduce_part<F, kHalf, R, kOut>(d, p, cut, i - first_part[cut], slice_np[cut], i, own, all, runs, values,
+                                                entry_rows, partials, part_group, dtable, adam, adam_p, adam_m, adam_v);
                 __syncthreads();  // the sums are read out
             }
             return;
@@ -1257,8 +1297,9 @@ __global__ void __launch_bounds__(kRunThreads)
         s -= kSplitBlocks;
         if (slice_np[s] != 1) return;
     }
-    reduce_part<F, kHalf, R, kOut>(d, p, s, 0, 1, 0, runs, values, entry_rows, partials, part_group, dtable, adam,
-                                    adam_p, adam_m, adam_v);
+    const uint32_t levels = __builtin_amdgcn_readfirstlane(p.whole ? levels_of(d, p, s, runs) : slice_levels[s]);
+    reduce_part<F, kHalf, R, kOut>(d, p, s, 0, 1, 0, levels, levels, runs, values, entry_rows, partials, part_group,
+                                    dtable, adam, adam_p, adam_m, adam_v);
 }
 
 // One-pass table gradient, part 4: slices of several parts, in pieces of
@@ -1396,7 +1437,7 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
     auto word = [&](uint64_t off) { return reinterpret_cast<uint32_t *>(ws + off); };
     uint32_t *runs = word(p.runs_off), *meta = word(p.meta_off), *slice_np = word(p.slice_np_off);
     uint32_t *first_part = word(p.first_part_off), *split = word(p.split_off), *part_slice = word(p.part_slice_off);
-    uint32_t *part_group = word(p.part_group_off);
+    uint32_t *part_group = word(p.part_group_off), *slice_levels = word(p.levels_off);
     double *partials = reinterpret_cast<double *>(ws + p.partials_off);
     auto *values = reinterpret_cast<EntryValue<F, kHalf> *>(ws + p.entries_off);
     uint16_t *entry_rows = reinterpret_cast<uint16_t *>(ws + p.rows_off);
@@ -1410,18 +1451,18 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
         g = lm;
         db.enc_layout = NGP_ENC_LEVEL_MAJOR;
     }
-    hipLaunchKernelGGL((bwd_bucket_kernel<F, kHalf, R>), dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, db, p, pos, g,
-                       runs, values, entry_rows, meta);
+    hipLaunchKernelGGL((p.wide ? bwd_bucket_kernel<F, kHalf, R, kMaxSlices> : bwd_bucket_kernel<F, kHalf, R, kStageSlices>),
+                       dim3(p.n_bitems), dim3(kBucketThreads), 0, stream, db, p, pos, g, runs, values, entry_rows, meta);
     if (!p.whole)
         hipLaunchKernelGGL(bwd_slice_parts_kernel, dim3(p.n_slices), dim3(256), 0, stream, d, p, runs, meta, slice_np,
-                           first_part, part_slice, split);
+                           first_part, part_slice, split, slice_levels);
     const dim3 reduce_grid(p.n_slices + (p.whole ? 0 : kSplitBlocks));
     auto finish = [&](auto kind, const AdamStep &step, float *ap, float *am, float *av) {
         constexpr int kOut = decltype(kind)::value;
         const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, kOut>;
         if (!reserve_lds(reduce, lds, target)) return false;
         hipLaunchKernelGGL(reduce, reduce_grid, dim3(kRunThreads), lds, stream, d, p, meta, slice_np, first_part,
-                           part_slice, runs, values, entry_rows, partials, part_group, dtable, step, ap, am, av);
+                           part_slice, slice_levels, runs, values, entry_rows, partials, part_group, dtable, step, ap, am, av);
         if (!p.whole)
             hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, kOut>), dim3(kCombineBlocks), dim3(256), 0, stream, d, meta,
                                slice_np, first_part, split, partials, part_group, dtable, step, ap, am, av);

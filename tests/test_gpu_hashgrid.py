@@ -198,6 +198,47 @@ def _backward_raw(enc, pos_t, g_t):
     return d
 
 
+@pytest.mark.parametrize("cfg,half", [
+    (CONFIGS["l16_t2e19"], False), (CONFIGS["l16_t2e19"], True),
+    (dict(L=16, T=2 ** 19, F=1, N_min=16, N_max=2048), False),
+    (dict(L=2, T=2 ** 23, F=2, N_min=150, N_max=160), False),  # slices of 64 KiB, level 0 reaches 1,824
+    (dict(L=3, T=2 ** 23, F=2, N_min=150, N_max=200), True),  # of 128 KiB, level 1 reaches 1,025
+])
+@pytest.mark.parametrize("N", [16, 2048, 20000])
+def test_backward_of_points_outside_the_box(dev, cfg, half, N):
+    """Points outside [-bound, bound] read rows modulo T, any of the T from a dense level's
+    offset on, and their gradient goes to the rows that they read: past the upper corner
+    against the oracle (the bound of test_hashgrid_forward_backward; for f16 half an ulp more of
+    each entry, of which a row has at most 8 N, and of the row), past the lower one, where the
+    oracle's conversion of negative coordinates is undefined, as the adjoint of the forward."""
+    enc = HashGridEncoder(**cfg, param_dtype=torch.float16 if half else torch.float32,
+                          generator=torch.Generator().manual_seed(1)).to(dev)
+    rng = np.random.default_rng(N)
+    LF = cfg["L"] * cfg["F"]
+    g = rng.normal(size=(N, LF)).astype(np.float32)
+    far = rng.choice([1.0, 1.05, 1.3, 1.5, 40.0], (N, 1))
+    pos = (rng.uniform(0.9, 1, (N, 3)) * far).astype(np.float32)
+
+    def table_grad(p, up):
+        enc.table.grad = None
+        out, _ = enc(torch.from_numpy(p).to(dev), 1.0)
+        out.backward(torch.from_numpy(up).to(dev))
+        return out.detach().cpu().double().numpy(), enc.table.grad.detach().cpu().double().numpy()
+
+    _, got = table_grad(pos, g)
+    want, absw = _c_backward(enc, pos, g), _c_backward(enc, pos, np.abs(g))
+    assert (got[absw == 0] == 0).all()
+    tol = 1e-5 * absw + 1e-30
+    if half:
+        tol += 2.0 ** -11 * (absw + np.abs(want)) + 8 * N * 2.0 ** -25
+    assert (np.abs(got - want) <= tol).all()
+    if not half:
+        out, d = table_grad(-pos, g)
+        _, dabs = table_grad(-pos, np.abs(g))
+        t = enc.table.detach().cpu().double().numpy()
+        assert abs((out * g).sum() - (d * t).sum()) <= 2e-5 * (dabs * np.abs(t)).sum()
+
+
 @pytest.mark.parametrize("kind,N", [("random", 1), ("ray", 63), ("one_cell", 64), ("ray", 65), ("ray", 513),
                                     ("random", 1025), ("one_cell", 5000), ("random", 30000)])
 def test_backward_item_and_run_edges(dev, kind, N):
