@@ -290,7 +290,8 @@ void hashgrid_encode_backward(ngp_stream_t stream, void **buffers, const char *o
 
 /* Bytes of the workspace hashgrid_encode_backward needs for the descriptor
  * `opaque` (no counterpart in the reference, whose scatter uses atomics on the
- * output).  Returns 0 and sets the last error for an invalid descriptor. */
+ * output).  Never less for more points, all else equal: a workspace serves every
+ * smaller batch too.  Returns 0 and sets the last error for an invalid descriptor. */
 size_t hashgrid_encode_backward_workspace_size(const char *opaque, size_t opaque_len);
 
 /* hashgrid_encode_backward with dL_dtable in f16 (16-byte aligned), the f32 sums rounded as

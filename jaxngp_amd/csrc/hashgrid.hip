@@ -196,6 +196,7 @@ constexpr int kChunk = 2048;         // points per work item
 constexpr int kItemThreads = 256;    // 8 points per thread per item
 constexpr int kReduceThreads = 1024;
 constexpr uint32_t kPart = 65536;    // entries one reduce workgroup sums
+constexpr uint32_t kMinPart = 8192;  // of the one-pass form, at least
 constexpr uint32_t kMaxSlices = 8192;
 constexpr uint32_t kSliceBytes = 131072;
 constexpr uint32_t kRunSliceBytes = 65536;  // one-pass form: two reduce workgroups per CU
@@ -347,6 +348,8 @@ inline bool plan_slices(const HashGridDescriptor &d, uint32_t slice_bytes, BwdPl
     return d.F <= 2 && box_span <= kStageSlices;
 }
 
+inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+
 inline BwdPlan make_plan(const HashGridDescriptor &d) {
     auto align = [](uint64_t x) { return (x + 255) / 256 * 256; };
     BwdPlan p{};
@@ -368,8 +371,8 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         // levels, whose entries also collide more in the LDS atomics, are cut (2^18 points
         // f32: 145 us, with parts of four slices 170, of one and a quarter 142; those take
         // a fifth more workspace, for parts that may be full of one slice's entries).
-        const uint64_t mean = (uint64_t)d.n_points * 8 * p.R / d.T;
-        p.run_part = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(8192, (mean * 5 / 2 + 1023) / 1024 * 1024));
+        p.run_part = (uint32_t)std::min<uint64_t>(
+            kPart, std::max<uint64_t>(kMinPart, ceil_div(20ull * d.n_points * p.R, 1024ull * d.T) * 1024));
         p.group_shift = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
         // Few points: even all contributions of all levels that share a group of slices inside
         // the box make one part, so nothing is counted, cut or combined: two launches, not four
@@ -388,7 +391,10 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         // its group more than kPart.  A group of g <= kPart entries then has at most
         // 2 (g - 1) / run_part parts, a larger one, of two slices, at most
         // 2 + (g - 1) / run_part + 2 (g - 1) / kPart, so at most (1 / run_part + 4 / kPart) g.
-        const uint64_t A = (max_entries + p.run_part - 1) / p.run_part, B = (max_entries + kPart - 1) / kPart;
+        // A bounds E / run_part by what it is before run_part is rounded up, 2 L T / (5 R) or
+        // where the limits are, so that a batch of fewer points never needs more workspace.
+        const uint64_t E = 8ull * d.n_points * d.L, B = ceil_div(E, kPart);
+        const uint64_t A = std::min(ceil_div(E, kMinPart), std::max(B, ceil_div(2ull * d.L * d.T, 5ull * p.R)));
         const uint32_t shared = 1u << p.group_shift;  // slices of a group
         const uint64_t dense = std::max<uint64_t>(2 * A, A + 2 * shared * B), sparse = p.n_slices + A + shared * B;
         p.max_parts = p.whole ? 0 : (uint32_t)std::min(dense, sparse);

@@ -157,6 +157,22 @@ def test_hashgrid_backward_workspace_size():
     assert _lib.last_error() == (0, "")
 
 
+@pytest.mark.parametrize("L, T, F", [(16, 2 ** 19, 2), (16, 2 ** 19, 1), (5, 2 ** 17, 2), (16, 2 ** 22, 2),
+                                     (32, 2 ** 21, 2), (16, 999, 2), (8, 2 ** 12, 4)])
+@pytest.mark.parametrize("dt", [0, 1])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_hashgrid_backward_workspace_grows_with_the_points(L, T, F, dt, layout):
+    """A workspace for a batch serves every smaller batch: host-only sizes over the whole range
+    of plans, around wavefronts, items and steps of the parts."""
+    from jaxngp_amd.encoders import level_table
+    lv = level_table(L, T, 16, 2048)
+    size = lambda n: _lib.hashgrid_backward_workspace_bytes(_lib.hashgrid_descriptor(
+        n, L, F, T, lv.first_hash_level, dt, lv.n_rows, 1.0, list(lv.scales), lv.resolutions, lv.offsets, layout))
+    points = list(range(0, 4096, 61)) + list(range(4096, 600_000, 511)) + [2 ** 20 - 1, 2 ** 20, 2 ** 22, 2 ** 23 - 1]
+    sizes = [size(n) for n in points]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+
+
 @pytest.mark.parametrize("L, T, F", [(20, 2 ** 21, 2), (32, 2 ** 21, 2), (20, 2 ** 22, 1), (16, 2 ** 22, 2)])
 @pytest.mark.parametrize("dt", [0, 1])
 def test_hashgrid_backward_takes_large_tables(L, T, F, dt):
