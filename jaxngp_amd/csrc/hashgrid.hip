@@ -197,6 +197,7 @@ constexpr int kItemThreads = 256;    // 8 points per thread per item
 constexpr int kReduceThreads = 1024;
 constexpr uint32_t kPart = 65536;    // entries one reduce workgroup sums
 constexpr uint32_t kMinPart = 8192;  // of the one-pass form, at least
+constexpr uint32_t kFullParts = 768;  // of one batch, at most, while kPart is enough
 constexpr uint32_t kMaxSlices = 8192;
 constexpr uint32_t kSliceBytes = 131072;
 constexpr uint32_t kRunSliceBytes = 65536;  // one-pass form: two reduce workgroups per CU
@@ -313,10 +314,9 @@ struct BwdPlan {
     bool bucket;
     bool wide;  // a level reaches more than kStageSlices slices, outside the box
     uint32_t n_bchunks, n_bitems, span_stride;
-    uint32_t run_part;     // entries one workgroup of the reducer sums
-    uint32_t group_shift;  // log2 of the slices in kSliceBytes
+    uint32_t run_part;  // entries one workgroup of the reducer sums
     uint32_t s_lo[NGP_HASHGRID_MAX_LEVELS], s_hi[NGP_HASHGRID_MAX_LEVELS];
-    uint64_t runs_off, slice_np_off, first_part_off, split_off, levels_off, rows_off, part_group_off;
+    uint64_t runs_off, slice_np_off, first_part_off, split_off, levels_off, rows_off;
     bool whole;      // no slice can be cut into parts
     bool transpose;  // a point-major gradient is copied level-major first (to partials_off)
 };
@@ -366,38 +366,39 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         p.n_bitems = d.L * p.n_bchunks;
         const uint64_t runs = (uint64_t)p.n_bitems * p.span_stride;
         const uint64_t max_entries = (uint64_t)p.n_bitems * bucket_entries(half_values);
-        // A hashed level spreads 8 contributions a point evenly over its slices; a part holds
-        // two and a half such slices, so these stay whole and the fuller slices of coarse
-        // levels, whose entries also collide more in the LDS atomics, are cut (2^18 points
-        // f32: 145 us, with parts of four slices 170, of one and a quarter 142; those take
-        // a fifth more workspace, for parts that may be full of one slice's entries).
-        p.run_part = (uint32_t)std::min<uint64_t>(
-            kPart, std::max<uint64_t>(kMinPart, ceil_div(20ull * d.n_points * p.R, 1024ull * d.T) * 1024));
-        p.group_shift = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
-        // Few points: even all contributions of all levels that share a group of slices inside
+        // A batch's entries make at most kFullParts full parts, one and a half to a workgroup
+        // that the chip holds: the slices of coarse levels, which hold most entries and whose
+        // entries also collide more in the LDS atomics, are cut until the reducer's last round
+        // is short, and a part costs its R * F f64 of the workspace.  A hashed level spreads 8
+        // contributions a point evenly over its slices; where cutting all of these would only
+        // double the parts, a part takes one of them whole, with a quarter to spare.  2^18 points
+        // f32, L = 16, T = 2^19, all kernels, along rays and at random: 145 and 213 us; 512 parts
+        // 165 and 215, 1,024 139 and 224, 2,048 175 and 318.  T = 2^17, 40,000 at random: 70,
+        // with its hashed slices cut 106.  (Parts of 2.5 slices, cut once more where the sums were
+        // grouped: T = 2^19 147 and 250, 2^17 213 and 319, 2^22 302 and 680, now 257 and 359.)
+        const uint64_t E = 8ull * d.n_points * d.L, mean4 = 32ull * d.n_points * p.R;  // 4 T times the mean
+        uint64_t want = ceil_div(E, 1024ull * kFullParts);
+        if (mean4 / d.T * 5 <= std::min<uint64_t>(16ull * kPart, 32 * E / kFullParts))
+            want = std::max(want, ceil_div(mean4 * 5, 16384ull * d.T));
+        p.run_part = (uint32_t)std::min<uint64_t>(kPart, std::max<uint64_t>(kMinPart, want * 1024));
+        // Few points: even all contributions of all levels that share kSliceBytes of rows inside
         // the box make one part, so nothing is counted, cut or combined: two launches, not four
-        // (2000 ray samples f32: 35 -> 26 us; the line is where a group could be cut, and
-        // with every point in a fifth of the box 4000 points take 73 us on either side).
+        // (2000 ray samples f32: 35 -> 26 us; with every point in a fifth of the box 4000 points
+        // take 73 us on either side).
+        const uint32_t pair = p.R * d.F * 8 == kSliceBytes ? 0 : 1;
         uint32_t sharing = 0;
         for (uint32_t l = 0; l < d.L; ++l) {
             uint32_t n = 0;
             for (uint32_t k = 0; k < d.L; ++k)
-                n += (p.s_lo[k] >> p.group_shift) <= (p.s_lo[l] >> p.group_shift) &&
-                     (box_hi[k] >> p.group_shift) >= (p.s_lo[l] >> p.group_shift);
+                n += p.s_lo[k] >> pair <= p.s_lo[l] >> pair && box_hi[k] >> pair >= p.s_lo[l] >> pair;
             sharing = std::max(sharing, n);
         }
         p.whole = (uint64_t)d.n_points * 8 * sharing <= kPart;
-        // Parts of cut slices: a slice is cut where it holds more than run_part entries or
-        // its group more than kPart.  A group of g <= kPart entries then has at most
-        // 2 (g - 1) / run_part parts, a larger one, of two slices, at most
-        // 2 + (g - 1) / run_part + 2 (g - 1) / kPart, so at most (1 / run_part + 4 / kPart) g.
-        // A bounds E / run_part by what it is before run_part is rounded up, 2 L T / (5 R) or
-        // where the limits are, so that a batch of fewer points never needs more workspace.
-        const uint64_t E = 8ull * d.n_points * d.L, B = ceil_div(E, kPart);
-        const uint64_t A = std::min(ceil_div(E, kMinPart), std::max(B, ceil_div(2ull * d.L * d.T, 5ull * p.R)));
-        const uint32_t shared = 1u << p.group_shift;  // slices of a group
-        const uint64_t dense = std::max<uint64_t>(2 * A, A + 2 * shared * B), sparse = p.n_slices + A + shared * B;
-        p.max_parts = p.whole ? 0 : (uint32_t)std::min(dense, sparse);
+        // Parts of cut slices: one of t > run_part entries has at most 2 (t - 1) / run_part, and
+        // at most 1 + t / run_part.  A bounds E / run_part by what it is before run_part is rounded
+        // up, so that a batch of fewer points never needs more workspace.
+        const uint64_t A = std::min(ceil_div(E, kMinPart), std::max<uint64_t>(ceil_div(E, kPart), kFullParts));
+        p.max_parts = p.whole ? 0 : (uint32_t)std::min(2 * A, p.n_slices + A);
         p.runs_off = 0;
         p.slice_np_off = align(p.runs_off + 4 * runs);
         p.first_part_off = align(p.slice_np_off + 4 * (uint64_t)p.n_slices);
@@ -408,8 +409,7 @@ inline BwdPlan make_plan(const HashGridDescriptor &d) {
         p.partials_off = align(p.part_slice_off + 4 * (uint64_t)p.max_parts);
         p.transpose = d.F == 2 && d.enc_layout == NGP_ENC_POINT_MAJOR && !p.whole && d.n_points >= kTransposeFrom;
         const uint64_t lm_bytes = p.transpose ? (uint64_t)d.n_points * d.L * 8 : 0;
-        p.part_group_off = align(p.partials_off + std::max((uint64_t)p.max_parts * p.R * d.F * 8, lm_bytes));
-        p.entries_off = align(p.part_group_off + 4 * (uint64_t)p.max_parts);
+        p.entries_off = align(p.partials_off + std::max((uint64_t)p.max_parts * p.R * d.F * 8, lm_bytes));
         p.rows_off = align(p.entries_off + max_entries * value_bytes(d.F, d.table_dtype == NGP_DTYPE_F16));
         p.bytes = p.rows_off + max_entries * sizeof(uint16_t);
         return p;
@@ -915,67 +915,41 @@ __global__ void __launch_bounds__(kBucketThreads)
     }
 }
 
-// How a slice's entries are summed.  Its items, in (level, chunk) order, are cut in two
-// ways by exclusive prefixes of run lengths: into work, of run_part entries of the slice
-// (one workgroup's), and into groups, of kPart entries of the kSliceBytes of rows the
-// slice lies in (with all their runs, and whole items of kGroupPoints points).  Each
-// group's sum is rounded to f32 once and the groups are added in f32; within a group the
-// parts' sums stay f64, so the result does not depend on run_part.  Both cuts only move
-// forward over the items, so work + group numbers the parts.
-constexpr uint32_t kGroupPoints = 1024;
-
-__device__ __forceinline__ uint32_t n_cuts(uint64_t entries, uint32_t per) {
-    return entries == 0 ? 1u : (uint32_t)((entries + per - 1) / per);
-}
-
-// Run length of item (l, k) in slice s; 0 if level l does not reach it.
-__device__ __forceinline__ uint32_t slice_run_length(const BwdPlan &p, const uint32_t *__restrict__ runs, uint32_t l,
-                                                     uint32_t s, uint32_t k) {
-    return s < p.s_lo[l] || s > p.s_hi[l] ? 0u : run_length(runs[run_index(p, l, s - p.s_lo[l], k)]);
-}
-
-// One-pass table gradient, part 2: the number of parts of slice s, from the run lengths of
-// every item whose level reaches s or the other slice of its group, and for a slice of
-// several a slot for each and its place in the list of cut slices.  Also the levels that
-// have entries in s: outside the box a dense level reaches many slices, inside few.
+// One-pass table gradient, part 2: the number of parts of slice s, run_part entries each in
+// (level, chunk) order of the items, from the run lengths of every item whose level reaches
+// it, and for a slice of several a slot for each and its place in the list of cut slices.
+// Also the levels that have entries in s: outside the box a dense level reaches many slices,
+// inside few.
 __global__ void __launch_bounds__(256)
     bwd_slice_parts_kernel(HashGridDescriptor d, BwdPlan p, const uint32_t *__restrict__ runs,
                            uint32_t *__restrict__ meta, uint32_t *__restrict__ slice_np,
                            uint32_t *__restrict__ first_part, uint32_t *__restrict__ part_slice,
                            uint32_t *__restrict__ split, uint32_t *__restrict__ slice_levels) {
-    const uint32_t s = blockIdx.x, other = p.group_shift ? s ^ 1u : s;
-    uint32_t own = 0, both = 0, levels = 0;
+    const uint32_t s = blockIdx.x;
+    uint32_t own = 0, levels = 0;
     for (uint32_t l = 0; l < d.L; ++l) {
-        const bool here = s >= p.s_lo[l] && s <= p.s_hi[l], there = other >= p.s_lo[l] && other <= p.s_hi[l];
-        if (!here && !there) continue;
+        if (s < p.s_lo[l] || s > p.s_hi[l]) continue;
         const uint32_t before = own;
-        for (uint32_t k = threadIdx.x; k < p.n_bchunks; k += 256) {
-            const uint32_t n = here ? run_length(runs[run_index(p, l, s - p.s_lo[l], k)]) : 0u;
-            own += n;
-            both += n;
-            if (p.group_shift && there) both += run_length(runs[run_index(p, l, other - p.s_lo[l], k)]);
-        }
+        for (uint32_t k = threadIdx.x; k < p.n_bchunks; k += 256)
+            own += run_length(runs[run_index(p, l, s - p.s_lo[l], k)]);
         if (__ballot(own != before) != 0ull) levels |= 1u << l;
     }
-    __shared__ uint32_t ws[3][256 / kWave];
+    __shared__ uint32_t ws[2][256 / kWave];
     own = wave_sum(own);
-    both = wave_sum(both);
     if (lane_id() == 0) {
         ws[0][threadIdx.x / kWave] = own;
-        ws[1][threadIdx.x / kWave] = both;
-        ws[2][threadIdx.x / kWave] = levels;
+        ws[1][threadIdx.x / kWave] = levels;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint64_t t = 0, g = 0;
+        uint64_t t = 0;
         uint32_t m = 0;
         for (int w = 0; w < 256 / kWave; ++w) {
             t += ws[0][w];
-            g += ws[1][w];
-            m |= ws[2][w];
+            m |= ws[1][w];
         }
         slice_levels[s] = m;
-        const uint32_t n = n_cuts(t, p.run_part) + n_cuts(g, kPart) - 1u;
+        const uint32_t n = t == 0 ? 1u : (uint32_t)((t + p.run_part - 1) / p.run_part);
         slice_np[s] = n;
         if (n > 1) {  // which slot a part gets does not matter to its sums
             const uint32_t at = atomicAdd(meta, n);
@@ -1072,13 +1046,14 @@ __global__ void __launch_bounds__(kReduceThreads)
 // pushing each run's lane number to the lane of its first entry and a running maximum
 // (RunSequence).  kSteps such groups are loaded before the previous ones are added.  A
 // whole slice (nearly all of them) needs no barrier between its runs; a part of a cut
-// slice first finds its items by the prefixes of their run lengths (see n_cuts).
+// slice first finds its items by the prefixes of their run lengths: those that start within
+// it.  Its sums stay f64 until the parts are added, so the result does not depend on the cut.
 // With kAdam, a slice summed in one part is not stored: its rows take the optimizer
 // step in place (params, m, v), and bwd_combine_runs does the same for the others.
 // 2^18 ray samples, f32: 82 -> 65 us, of which the atomics themselves need 27 (34 M f64
 // adds at 1.27 T/s); slices of 64 KiB, two workgroups to a CU, so that one clears or
 // stores its rows while the other adds (128 KiB slices: 80 us); 1,024 points: 29 -> 17.
-// All four parts: f32 190 -> 147 us, f16 176 -> 129; 1,024 points, two parts: 44 -> 28.
+// All four parts: f32 190 -> 145 us, f16 176 -> 125; 1,024 points, two parts: 44 -> 25.
 struct RunSequence {
     uint32_t *marks;        // 64 words of LDS of the wavefront's own, tags below `tag`
     uint32_t tag;           // of the latest group of 64 places
@@ -1161,16 +1136,14 @@ enum { kFloatRows, kAdamRows, kHalfRows };
 template <int F, bool kHalf, uint32_t R, int kOut>
 __device__ __forceinline__ void
 reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t part, uint32_t n_parts, uint32_t slot,
-            uint32_t own_levels, uint32_t levels, const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
-            const uint16_t *__restrict__ entry_rows, double *__restrict__ partials, uint32_t *__restrict__ part_group,
-            void *__restrict__ dtable, const AdamStep &adam, float *__restrict__ adam_p, float *__restrict__ adam_m,
+            uint32_t levels, const uint32_t *__restrict__ runs, const EntryValue<F, kHalf> *__restrict__ values,
+            const uint16_t *__restrict__ entry_rows, double *__restrict__ partials, void *__restrict__ dtable, const AdamStep &adam, float *__restrict__ adam_p, float *__restrict__ adam_m,
             float *__restrict__ adam_v) {
     typedef EntryGroup<F, kHalf> Group;
     constexpr uint32_t kBucketEntries = bucket_entries(kHalf);
     constexpr uint32_t kWaves = kRunThreads / kWave;
     extern __shared__ double acc[];
     __shared__ uint32_t chosen[kRunThreads];
-    __shared__ uint32_t my_group;
     __shared__ uint32_t marks[kWaves][kWave];
     const uint32_t rows = min(d.n_rows - s * R, R);
     for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) reinterpret_cast<double2 *>(acc)[t] = double2{0.0, 0.0};
@@ -1181,13 +1154,10 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
     seq.marks = marks[wave];
     seq.tag = 0;
     seq.marks[lane] = 0u;
-    if (threadIdx.x == 0) my_group = 0xffffffffu;
-    uint32_t carry = 0, carry_group = 0;  // entries of the items visited before
-    const uint32_t other = p.group_shift ? s ^ 1u : s;
+    uint32_t carry = 0;  // entries of the items visited before
     for (uint32_t left = levels; left != 0; left &= left - 1u) {
         const uint32_t l = (uint32_t)__builtin_ctz(left);
-        const bool here = (own_levels >> l) & 1u;
-        const uint32_t *level_runs = runs + (here ? run_index(p, l, s - p.s_lo[l], 0) : 0);
+        const uint32_t *level_runs = runs + run_index(p, l, s - p.s_lo[l], 0);
         for (uint32_t k0 = 0; k0 < p.n_bchunks; k0 += kRunThreads) {
             const uint32_t n_k = min(p.n_bchunks - k0, (uint32_t)kRunThreads);
             const uint32_t k = wave + lane * kWaves;  // this lane's run of the tile
@@ -1195,23 +1165,11 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
             if (n_parts == 1) {
                 if (k < n_k) my_run = level_runs[k0 + k];
             } else {
-                const uint32_t r = here && threadIdx.x < n_k ? level_runs[k0 + threadIdx.x] : 0u;
-                uint32_t g = run_length(r), tot, tot_group;
-                if (p.group_shift && threadIdx.x < n_k) g += slice_run_length(p, runs, l, other, k0 + threadIdx.x);
+                const uint32_t r = threadIdx.x < n_k ? level_runs[k0 + threadIdx.x] : 0u;
+                uint32_t tot;
                 const uint32_t ex = block_exclusive_scan<kRunThreads>(run_length(r), &tot);
-                uint32_t ex_group = block_exclusive_scan<kRunThreads>(g, &tot_group);
-                if constexpr (bucket_points(kHalf) < kGroupPoints) {
-                    // the second item of a group's kGroupPoints goes with the first
-                    static_assert(2 * bucket_points(kHalf) == kGroupPoints, "two items");
-                    const uint32_t before = __shfl_up(g, 1, kWave);
-                    if (threadIdx.x & 1u) ex_group -= before;
-                }
-                const uint32_t group = (carry_group + ex_group) / kPart;
-                const bool mine = r >> 16 != 0u && (carry + ex) / p.run_part + group == part;
-                chosen[threadIdx.x] = mine ? r : 0u;
-                if (mine) my_group = group;  // the same for all of the part's items
+                chosen[threadIdx.x] = run_length(r) != 0u && (carry + ex) / p.run_part == part ? r : 0u;
                 carry += tot;
-                carry_group += tot_group;
                 __syncthreads();
                 my_run = chosen[k];
                 __syncthreads();  // rewritten by the next tile
@@ -1242,7 +1200,6 @@ reduce_part(const HashGridDescriptor &d, const BwdPlan &p, uint32_t s, uint32_t 
         return;
     }
     if (n_parts > 1) {
-        if (threadIdx.x == 0) part_group[slot] = my_group;
         double2 *out = reinterpret_cast<double2 *>(partials + (size_t)slot * R * F);
         for (uint32_t t = threadIdx.x; t < R * F / 2; t += kRunThreads) out[t] = reinterpret_cast<const double2 *>(acc)[t];
         return;
@@ -1283,19 +1240,16 @@ __global__ void __launch_bounds__(kRunThreads)
                            const uint32_t *__restrict__ part_slice, const uint32_t *__restrict__ slice_levels,
                            const uint32_t *__restrict__ runs,
                            const EntryValue<F, kHalf> *__restrict__ values, const uint16_t *__restrict__ entry_rows,
-                           double *__restrict__ partials, uint32_t *__restrict__ part_group,
-                           void *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
+                           double *__restrict__ partials, void *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p,
                            float *__restrict__ adam_m, float *__restrict__ adam_v) {
     uint32_t s = blockIdx.x;
     if (!p.whole) {
         if (blockIdx.x < kSplitBlocks) {
             const uint32_t n = meta[0];
             for (uint32_t i = blockIdx.x; i < n; i += kSplitBlocks) {
-                const uint32_t cut = part_slice[i], other = cut ^ 1u;
-                const uint32_t own = slice_levels[cut];
-                const uint32_t all = own | (p.group_shift && other < p.n_slices ? slice_levels[other] : 0u);
-                reduce_part<F, kHalf, R, kOut>(d, p, cut, i - first_part[cut], slice_np[cut], i, own, all, runs, values,
-                                                entry_rows, partials, part_group, dtable, adam, adam_p, adam_m, adam_v);
+                const uint32_t cut = part_slice[i];
+                reduce_part<F, kHalf, R, kOut>(d, p, cut, i - first_part[cut], slice_np[cut], i, slice_levels[cut], runs,
+                                                values, entry_rows, partials, dtable, adam, adam_p, adam_m, adam_v);
                 __syncthreads();  // the sums are read out
             }
             return;
@@ -1304,8 +1258,8 @@ __global__ void __launch_bounds__(kRunThreads)
         if (slice_np[s] != 1) return;
     }
     const uint32_t levels = __builtin_amdgcn_readfirstlane(p.whole ? levels_of(d, p, s, runs) : slice_levels[s]);
-    reduce_part<F, kHalf, R, kOut>(d, p, s, 0, 1, 0, levels, levels, runs, values, entry_rows, partials, part_group,
-                                    dtable, adam, adam_p, adam_m, adam_v);
+    reduce_part<F, kHalf, R, kOut>(d, p, s, 0, 1, 0, levels, runs, values, entry_rows, partials, dtable, adam, adam_p,
+                                    adam_m, adam_v);
 }
 
 // One-pass table gradient, part 4: slices of several parts, in pieces of
@@ -1317,8 +1271,7 @@ __global__ void __launch_bounds__(256)
     bwd_combine_runs_kernel(HashGridDescriptor d, const uint32_t *__restrict__ meta,
                             const uint32_t *__restrict__ slice_np, const uint32_t *__restrict__ first_part,
                             const uint32_t *__restrict__ split, const double *__restrict__ partials,
-                            const uint32_t *__restrict__ part_group, void *__restrict__ dtable, AdamStep adam,
-                            float *__restrict__ adam_p, float *__restrict__ adam_m, float *__restrict__ adam_v) {
+                            void *__restrict__ dtable, AdamStep adam, float *__restrict__ adam_p, float *__restrict__ adam_m, float *__restrict__ adam_v) {
     constexpr uint32_t kPer = R * F / kCombineSplit;
     constexpr uint32_t kBatch = 8;  // partial rows in flight per thread
     const uint32_t n_tasks = meta[1] * kCombineSplit;
@@ -1330,31 +1283,17 @@ __global__ void __launch_bounds__(256)
         for (uint32_t t = piece * kPer + threadIdx.x; t < (piece + 1) * kPer; t += 256) {
             const uint32_t f = t / R, r = t % R;
             if (r >= rows) continue;
-            float sum = 0.0f;
-            double in_group = 0.0;
-            uint32_t group = 0xffffffffu;
+            double all = 0.0;
             for (uint32_t q0 = 0; q0 < n_parts; q0 += kBatch) {
                 double v[kBatch];
-                uint32_t g[kBatch];
 #pragma unroll
-                for (uint32_t j = 0; j < kBatch; ++j) {
-                    const uint32_t q = p0 + min(q0 + j, n_parts - 1u);
-                    g[j] = part_group[q];
-                    v[j] = partials[(size_t)q * R * F + t];
-                }
+                for (uint32_t j = 0; j < kBatch; ++j)
+                    v[j] = partials[(size_t)(p0 + min(q0 + j, n_parts - 1u)) * R * F + t];
 #pragma unroll
-                for (uint32_t j = 0; j < kBatch; ++j) {
-                    // 0xffffffff: a part without items (both cuts moved on together)
-                    if (q0 + j >= n_parts || g[j] == 0xffffffffu) continue;
-                    if (g[j] != group) {
-                        sum += (float)in_group;
-                        in_group = 0.0;
-                        group = g[j];
-                    }
-                    in_group += v[j];
-                }
+                for (uint32_t j = 0; j < kBatch; ++j)
+                    if (q0 + j < n_parts) all += v[j];
             }
-            sum += (float)in_group;
+            const float sum = (float)all;
             const size_t o = ((size_t)s * R + r) * F + f;
             if constexpr (kOut == kAdamRows) {
                 float mk = adam_m[o], vk = adam_v[o];
@@ -1443,7 +1382,7 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
     auto word = [&](uint64_t off) { return reinterpret_cast<uint32_t *>(ws + off); };
     uint32_t *runs = word(p.runs_off), *meta = word(p.meta_off), *slice_np = word(p.slice_np_off);
     uint32_t *first_part = word(p.first_part_off), *split = word(p.split_off), *part_slice = word(p.part_slice_off);
-    uint32_t *part_group = word(p.part_group_off), *slice_levels = word(p.levels_off);
+    uint32_t *slice_levels = word(p.levels_off);
     double *partials = reinterpret_cast<double *>(ws + p.partials_off);
     auto *values = reinterpret_cast<EntryValue<F, kHalf> *>(ws + p.entries_off);
     uint16_t *entry_rows = reinterpret_cast<uint16_t *>(ws + p.rows_off);
@@ -1468,10 +1407,10 @@ bool launch_backward_runs(const HashGridDescriptor &d, const BwdPlan &p, hipStre
         const auto reduce = bwd_reduce_runs_kernel<F, kHalf, R, kOut>;
         if (!reserve_lds(reduce, lds, target)) return false;
         hipLaunchKernelGGL(reduce, reduce_grid, dim3(kRunThreads), lds, stream, d, p, meta, slice_np, first_part,
-                           part_slice, slice_levels, runs, values, entry_rows, partials, part_group, dtable, step, ap, am, av);
+                           part_slice, slice_levels, runs, values, entry_rows, partials, dtable, step, ap, am, av);
         if (!p.whole)
             hipLaunchKernelGGL((bwd_combine_runs_kernel<F, R, kOut>), dim3(kCombineBlocks), dim3(256), 0, stream, d, meta,
-                               slice_np, first_part, split, partials, part_group, dtable, step, ap, am, av);
+                               slice_np, first_part, split, partials, dtable, step, ap, am, av);
         return true;
     };
     if constexpr (!kHalf) {

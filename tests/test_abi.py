@@ -173,6 +173,25 @@ def test_hashgrid_backward_workspace_grows_with_the_points(L, T, F, dt, layout):
     assert all(a <= b for a, b in zip(sizes, sizes[1:]))
 
 
+@pytest.mark.parametrize("L, T, n, slice_kib", [(16, 2 ** 19, 2 ** 18, 64), (16, 2 ** 17, 2 ** 18, 64),
+                                                (16, 2 ** 22, 2 ** 17, 128), (16, 2 ** 22, 2 ** 18, 128),
+                                                (32, 2 ** 21, 2 ** 18, 128)])
+@pytest.mark.parametrize("dt", [0, 1])
+def test_hashgrid_backward_workspace_is_mostly_entries(L, T, n, slice_kib, dt):
+    """Beside a batch's entries (10 or 6 bytes each) and their runs, at most 2 x 768 partial
+    sums of a slice (more only where 768 parts of 65,536 entries do not hold them) and 20 bytes
+    a slice or part: no table asks for several times its entries."""
+    from jaxngp_amd.encoders import level_table
+    lv = level_table(L, T, 16, 2048)
+    size = _lib.hashgrid_backward_workspace_bytes(_lib.hashgrid_descriptor(
+        n, L, 2, T, lv.first_hash_level, dt, lv.n_rows, 1.0, list(lv.scales), lv.resolutions, lv.offsets, 1))
+    slice_rows = slice_kib * 1024 // 16
+    entries = n * L * 8 * (6 if dt else 10)
+    runs = 4 * L * (T // slice_rows + 1) * (n // (512 if dt else 1024))
+    parts = 2 * max(768, n * L * 8 // 65536) * (slice_kib * 1024 + 20) + 20 * (lv.n_rows // slice_rows + 1)
+    assert size <= entries + runs + parts + 4096
+
+
 @pytest.mark.parametrize("L, T, F", [(20, 2 ** 21, 2), (32, 2 ** 21, 2), (20, 2 ** 22, 1), (16, 2 ** 22, 2)])
 @pytest.mark.parametrize("dt", [0, 1])
 def test_hashgrid_backward_takes_large_tables(L, T, F, dt):
