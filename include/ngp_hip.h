@@ -271,11 +271,12 @@ void integrate_rays_inference(ngp_stream_t stream, void **buffers, const char *o
  *      (NGP_ENC_LEVEL_MAJOR) */
 void hashgrid_encode(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
-/* hashgrid_encode for point-major encodings of F = 2 features by way of a level-major
- * workspace: the same values, in full cache lines (worth it from about 2^15 points).
+/* hashgrid_encode for point-major encodings of F = 2 or 4 features by way of a level-major
+ * workspace: the same values, in full cache lines (worth it from about 2^23 / L^2 points on,
+ * of 8 levels or more).
  * in : positions f32[N,3], table as hashgrid_encode
- * out: encodings f32[N, L*2] (8-byte aligned)
- * scratch: workspace f32[L, N, 2] (8-byte aligned) */
+ * out: encodings f32[N, L*F] (4 F-byte aligned)
+ * scratch: workspace f32[L, N, F] (4 F-byte aligned) */
 void hashgrid_encode_staged(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
 /* Table gradient of HashGridEncoder (the VJP of the gather at encoders.py:226 and

@@ -36,17 +36,23 @@ constexpr int kBlock = 256;
 // against a mean of 57).  Four pairs of XCDs instead deal the levels in snake order
 // from the finest down, each XCD of a pair taking every second group of points: the
 // sums of the four sets are within 6% of the mean for ray samples, and random points,
-// where all hashed levels cost alike, get 2 or 3 of the 11 per pair.
+// where all hashed levels cost alike, get 2 or 3 of the 11 per pair.  Fewer levels leave
+// some of four sets with nothing or with one level more than the rest, so they are dealt to
+// two sets of four XCDs, or one after the other to all eight (level_sets).
 constexpr uint32_t kXcds = 8;
+constexpr uint64_t kL2Bytes = 4u << 20;
 constexpr int kLmPointsPerThread = 2;
 constexpr int kPointsPerBlock = kBlock * kLmPointsPerThread;
 
-constexpr uint32_t kLevelSets = kXcds / 2;
+// 2^18 ray samples, f32, level-major, with 1, 2 and 4 sets: 3 levels 10.5, 9.9 and 16.1 us;
+// 5 levels of up to 2^19 rows 20.6, 22.1 and 27.8; 8 levels 23.9, 23.0 and 27.6; 12 levels
+// 41.8, 38.8 and 41.0 (32,768 of them 10.8, 9.7 and 8.6); 16 levels 63.0, 58.9 and 56.7.
+__host__ __device__ inline uint32_t level_sets(uint32_t L) { return L >= 12 ? 4u : L >= 6 ? 2u : 1u; }
 
-// Point groups of one XCD and level: every second group of kPointsPerBlock points.
-__host__ __device__ inline uint32_t half_groups(uint32_t n_points) {
+// Point groups (of kPointsPerBlock points) of one XCD and level.
+__host__ __device__ inline uint32_t xcd_groups(uint32_t n_points, uint32_t sets) {
     const uint64_t n_pg = ((uint64_t)n_points + kPointsPerBlock - 1) / kPointsPerBlock;
-    return (uint32_t)((n_pg + 1) / 2);
+    return (uint32_t)((n_pg * sets + kXcds - 1) / kXcds);
 }
 
 struct LevelBlock {
@@ -55,21 +61,23 @@ struct LevelBlock {
 };
 
 __device__ __forceinline__ LevelBlock level_block(uint32_t n_points, uint32_t L) {
-    const uint32_t n_half = half_groups(n_points);
+    const uint32_t sets = level_sets(L), n_groups = xcd_groups(n_points, sets);
     const uint32_t b = blockIdx.x;
     const uint32_t x = b % kXcds, rest = b / kXcds;
-    const uint32_t i = rest % n_half, phase = rest / n_half;
-    const uint32_t s = x % kLevelSets;
-    const uint32_t k = phase * kLevelSets + ((phase & 1u) ? kLevelSets - 1u - s : s);
+    const uint32_t i = rest % n_groups, phase = rest / n_groups;
+    const uint32_t s = x % sets;
+    const uint32_t k = phase * sets + ((phase & 1u) ? sets - 1u - s : s);
+    const uint64_t point0 = (uint64_t)(kXcds / sets * i + x / sets) * kPointsPerBlock;
     LevelBlock lb;
     lb.level = L - 1u - k;
-    lb.point0 = (2u * i + x / kLevelSets) * kPointsPerBlock;
-    lb.live = k < L && lb.point0 < n_points;
+    lb.point0 = (uint32_t)point0;
+    lb.live = k < L && point0 < n_points;
     return lb;
 }
 
 inline uint32_t level_grid(uint32_t n_points, uint32_t L) {
-    return kXcds * half_groups(n_points) * div_up(L, kLevelSets);
+    const uint32_t sets = level_sets(L);
+    return kXcds * xcd_groups(n_points, sets) * div_up(L, sets);
 }
 
 // Forward: each thread takes kLmPointsPerThread points of the block's level, kBlock
@@ -143,13 +151,51 @@ __global__ void __launch_bounds__(kBlock)
     });
 }
 
-// [L, n, F] encodings -> [n, L * F], for F = 2: a workgroup takes kTransposePoints
-// points, reads each level's run (512 bytes) and writes the points' rows, both coalesced,
-// through LDS.
-constexpr int kTransposePoints = 64;
+// Point-major forward with the levels of a point in neighbouring lanes: its row is written
+// in whole lines, and no level stays in an L2.  For levels so large that they would not.
+// 2^18 ray samples, f32, against the kernel above: T = 2^22, F = 2 123 and 181 us, T = 2^19,
+// F = 8 168 and 254 (2^14: 15 and 19); a level of two L2s, T = 2^20, F = 2: 111 and 113, and at
+// random 289 and 182.
+template <int F, typename TT>
 __global__ void __launch_bounds__(kBlock)
-    encodings_to_points_kernel(uint32_t n_points, uint32_t L, const float2 *__restrict__ lm, float2 *__restrict__ pm) {
-    __shared__ float2 tile[kTransposePoints * (NGP_HASHGRID_MAX_LEVELS + 1)];
+    hashgrid_fwd_points_kernel(HashGridDescriptor d, const float *__restrict__ pos, const TT *__restrict__ table,
+                               float *__restrict__ enc) {
+    __shared__ LevelTables lt;
+    if (threadIdx.x < d.L) {
+        lt.scale[threadIdx.x] = d.scales[threadIdx.x];
+        lt.res[threadIdx.x] = d.resolutions[threadIdx.x];
+        lt.offset[threadIdx.x] = d.offsets[threadIdx.x];
+    }
+    __syncthreads();
+    const uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (t >= (uint64_t)d.n_points * d.L) return;
+    const uint32_t n = (uint32_t)(t / d.L), l = (uint32_t)(t % d.L);
+    float p[3];
+    normalise(make_divisor(2.0f * d.bound), d.bound, pos + 3 * (size_t)n, p);
+    uint32_t idx[8];
+    float w[8], acc[F];
+    level_vertices(p[0], p[1], p[2], lt.scale[l], lt.res[l], l < d.first_hash_level, d.T, (d.T & (d.T - 1u)) == 0,
+                   lt.offset[l], d.n_rows - 1u, idx, w);
+#pragma unroll
+    for (int f = 0; f < F; ++f) acc[f] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const TT *row = table + (size_t)idx[c] * F;
+#pragma unroll
+        for (int f = 0; f < F; ++f) acc[f] = acc[f] + to_f32<TT>(row[f]) * w[c];
+    }
+#pragma unroll
+    for (int f = 0; f < F; ++f) enc[t * F + f] = acc[f];
+}
+
+// [L, n, F] encodings -> [n, L * F], Vec one point's F features: a workgroup takes
+// kTransposePoints points, reads each level's run (512 bytes for F = 2) and writes the
+// points' rows, both coalesced, through LDS.
+constexpr int kTransposePoints = 64;
+template <typename Vec>
+__global__ void __launch_bounds__(kBlock)
+    encodings_to_points_kernel(uint32_t n_points, uint32_t L, const Vec *__restrict__ lm, Vec *__restrict__ pm) {
+    __shared__ Vec tile[kTransposePoints * (NGP_HASHGRID_MAX_LEVELS + 1)];
     const uint32_t p0 = blockIdx.x * kTransposePoints;
     const uint32_t n = min((uint32_t)kTransposePoints, n_points - p0), row = L + 1;
     for (uint32_t t = threadIdx.x; t < L * kTransposePoints; t += kBlock) {
@@ -1512,9 +1558,24 @@ bool validate(const HashGridDescriptor &d, const char *target) {
 template <typename TT>
 void launch_fwd(const HashGridDescriptor &d, hipStream_t s, const float *pos, const void *table, float *enc) {
     const TT *t = static_cast<const TT *>(table);
+    const dim3 b(kBlock);
+    // (few points fill the chip with neither, and the other kernel's blocks are shorter)
+    const uint64_t level_bytes = (uint64_t)d.T * d.F * sizeof(TT);
+    const uint64_t threads = (uint64_t)d.n_points * d.L;
+    if (d.enc_layout == NGP_ENC_POINT_MAJOR && level_bytes > 2 * kL2Bytes && (uint64_t)d.n_points * d.F >= 1u << 17 &&
+        threads <= 0xffffff00ull) {
+        const dim3 g(div_up(threads, kBlock));
+        switch (d.F) {
+            case 1: hipLaunchKernelGGL((hashgrid_fwd_points_kernel<1, TT>), g, b, 0, s, d, pos, t, enc); break;
+            case 2: hipLaunchKernelGGL((hashgrid_fwd_points_kernel<2, TT>), g, b, 0, s, d, pos, t, enc); break;
+            case 4: hipLaunchKernelGGL((hashgrid_fwd_points_kernel<4, TT>), g, b, 0, s, d, pos, t, enc); break;
+            default: hipLaunchKernelGGL((hashgrid_fwd_points_kernel<8, TT>), g, b, 0, s, d, pos, t, enc); break;
+        }
+        return;
+    }
     // the grouped gather writes a row's two features as one 8-byte vector
     const bool groups = grouped_rows_ok(d, table) && (reinterpret_cast<uintptr_t>(enc) & 7u) == 0;
-    const dim3 g(level_grid(d.n_points, d.L)), b(kBlock);
+    const dim3 g(level_grid(d.n_points, d.L));
     switch (d.F) {
         case 1: hipLaunchKernelGGL((hashgrid_fwd_kernel<1, TT, false>), g, b, 0, s, d, pos, t, enc); break;
         case 2:
@@ -1551,14 +1612,14 @@ extern "C" void hashgrid_encode_staged(ngp_stream_t stream_, void **buffers, con
     HashGridDescriptor d;
     if (!read_descriptor(opaque, opaque_len, &d, target)) return;
     if (!validate(d, target)) return;
-    if (d.F != 2 || d.enc_layout != NGP_ENC_POINT_MAJOR) {
-        set_error(kBadDescriptor, "%s: F must be 2 and enc_layout 0 (point-major)", target);
+    if (!(d.F == 2 || d.F == 4) || d.enc_layout != NGP_ENC_POINT_MAJOR) {
+        set_error(kBadDescriptor, "%s: F must be 2 or 4 and enc_layout 0 (point-major)", target);
         return;
     }
     if (d.n_points == 0) return;
     if (!check_buffers(buffers, 4, target)) return;
-    if (((reinterpret_cast<uintptr_t>(buffers[2]) | reinterpret_cast<uintptr_t>(buffers[3])) & 7u) != 0) {
-        set_error(kBadArgument, "%s: encodings and the workspace must be 8-byte aligned", target);
+    if (((reinterpret_cast<uintptr_t>(buffers[2]) | reinterpret_cast<uintptr_t>(buffers[3])) & (4 * d.F - 1u)) != 0) {
+        set_error(kBadArgument, "%s: encodings and the workspace must be %u-byte aligned", target, 4 * d.F);
         return;
     }
     hipStream_t stream = (hipStream_t)stream_;
@@ -1569,8 +1630,13 @@ extern "C" void hashgrid_encode_staged(ngp_stream_t stream_, void **buffers, con
     if (d.table_dtype == NGP_DTYPE_F32) launch_fwd<float>(dl, stream, pos, buffers[1], lm);
     else launch_fwd<__half>(dl, stream, pos, buffers[1], lm);
     if (!check_launch(target)) return;
-    hipLaunchKernelGGL(encodings_to_points_kernel, dim3(div_up(d.n_points, kTransposePoints)), dim3(kBlock), 0, stream,
-                       d.n_points, d.L, (const float2 *)lm, (float2 *)buffers[2]);
+    const dim3 g(div_up(d.n_points, kTransposePoints)), b(kBlock);
+    if (d.F == 2)
+        hipLaunchKernelGGL(encodings_to_points_kernel<float2>, g, b, 0, stream, d.n_points, d.L, (const float2 *)lm,
+                           (float2 *)buffers[2]);
+    else
+        hipLaunchKernelGGL(encodings_to_points_kernel<float4>, g, b, 0, stream, d.n_points, d.L, (const float4 *)lm,
+                           (float4 *)buffers[2]);
     check_launch(target);
 }
 

@@ -63,12 +63,16 @@ def level_table(L: int, T: int, N_min: int, N_max: int, dim: int = 3) -> LevelTa
     return LevelTable(b, tuple(scales), tuple(res), tuple(offsets), first)
 
 
-# From this many points on, point-major encodings go through a level-major workspace:
-# written point by point, 8 bytes at a stride of 128, every cache line reaches memory in
-# pieces.  2^18 points, f32, a new output each call: 130 us point by point, 115 with a
-# wavefront of 4 points x 16 levels (whole lines, but every level in every L2), 78 staged;
-# below the line the pieces cost less than the second launch and the workspace.
-STAGED_POINTS = 1 << 15
+# Point-major encodings of several levels and many points go through a level-major
+# workspace: written point by point, 8 bytes at a stride of 128, every cache line reaches
+# memory in pieces.  2^18 points, f32, a new output each call: 130 us point by point, 115 with
+# a wavefront of 4 points x 16 levels (whole lines, but every level in every L2), 78 staged.
+# Fewer points, and even more so fewer levels, do not pay for the second launch: GPU time of
+# 16 levels at 32,768 ray samples 17 us both ways (at random 25 and 23), of 12 levels at
+# 65,536 20 and 18, of 8 levels at 2^16, 2^17 and 2^18 10 and 13, 19 and 19, 36 and 30, and of
+# 5 levels at 2^18 24 and 26.
+def _staged(n_points: int, levels: int, n_features: int) -> bool:
+    return n_features in (2, 4) and levels >= 8 and n_points * levels * levels >= 1 << 23
 
 
 class _HashGridFn(torch.autograd.Function):
@@ -76,7 +80,7 @@ class _HashGridFn(torch.autograd.Function):
     def forward(ctx, pos, table, desc_fn, n_out, n_features):
         N = pos.shape[0]
         enc = torch.empty(N, n_out, dtype=torch.float32, device=pos.device)
-        if n_features == 2 and N >= STAGED_POINTS:
+        if _staged(N, n_out // n_features, n_features):
             _lib.call("hashgrid_encode_staged", [pos, table.contiguous(), enc, torch.empty_like(enc)], desc_fn(N))
         elif N:
             _lib.call("hashgrid_encode", [pos, table.contiguous(), enc], desc_fn(N))

@@ -188,6 +188,35 @@ def test_grouped_rows_match_row_by_row_and_staged(dev, T, N, half):
         np.testing.assert_array_equal(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("L, T, F, N, half", [
+    (2, 2 ** 14, 2, 4097, False), (5, 2 ** 15, 1, 4096, False), (6, 2 ** 15, 2, 8193, True), (7, 2 ** 14, 4, 1, False),
+    (11, 2 ** 15, 2, 2049, False), (12, 2 ** 15, 2, 1025, False), (8, 2 ** 15, 4, 4095, True), (16, 2 ** 14, 8, 777, False),
+    # levels of more than two L2s: neighbouring lanes take a point's levels from n F = 2^17 on
+    (3, 2 ** 21, 2, 2 ** 16 - 1, False), (3, 2 ** 21, 2, 2 ** 16, False), (3, 2 ** 19, 8, 2 ** 14 + 5, False),
+    (3, 2 ** 22, 4, 2 ** 15 + 1, True), (3, 2 ** 22, 1, 2 ** 17 + 1, False)])
+def test_forward_over_the_ways_levels_are_dealt(dev, L, T, F, N, half):
+    """One, two and four sets of levels over the XCDs, a last set that is not full, one block
+    and several, and large levels: both layouts and the staged output, bit for bit."""
+    from jaxngp_amd import _lib
+    enc = HashGridEncoder(L=L, T=T, F=F, N_min=16, N_max=512, param_dtype=torch.float16 if half else torch.float32,
+                          generator=torch.Generator().manual_seed(1)).to(dev)
+    with torch.no_grad():
+        enc.table.uniform_(-1, 1)
+    pos_np = np.random.default_rng(N).uniform(-1, 1, (N, 3)).astype(np.float32)
+    pos = torch.from_numpy(pos_np).to(dev)
+    table = enc.table.detach()
+    want = _c_forward(enc, pos_np, table.float().cpu().numpy())
+    for layout in (_lib.ENC_POINT_MAJOR, _lib.ENC_LEVEL_MAJOR):
+        out = torch.empty(L * N * F, device=dev)
+        _lib.call("hashgrid_encode", [pos, table, out], enc.descriptor(N, 1.0, layout))
+        got = out.view(L, N, F).permute(1, 0, 2) if layout == _lib.ENC_LEVEL_MAJOR else out
+        np.testing.assert_array_equal(got.reshape(N, L * F).cpu().numpy(), want)
+    if F in (2, 4):
+        out, ws = torch.empty(N, L * F, device=dev), torch.empty(N, L * F, device=dev)
+        _lib.call("hashgrid_encode_staged", [pos, table, out, ws], enc.descriptor(N, 1.0))
+        np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
 def _backward_raw(enc, pos_t, g_t):
     from jaxngp_amd import _lib
     N = pos_t.shape[0]
