@@ -276,7 +276,8 @@ void hashgrid_encode(ngp_stream_t stream, void **buffers, const char *opaque, si
  * of 8 levels or more).
  * in : positions f32[N,3], table as hashgrid_encode
  * out: encodings f32[N, L*F] (4 F-byte aligned)
- * scratch: workspace f32[L, N, F] (4 F-byte aligned) */
+ * scratch: workspace f32[L, min(N, NGP_ENCODE_STAGE_POINTS), F] (4 F-byte aligned) */
+#define NGP_ENCODE_STAGE_POINTS (1u << 21)
 void hashgrid_encode_staged(ngp_stream_t stream, void **buffers, const char *opaque, size_t opaque_len);
 
 /* Table gradient of HashGridEncoder (the VJP of the gather at encoders.py:226 and

@@ -405,6 +405,7 @@ def field_chunks_descriptor(grid_desc: bytes, n_slots, cap, n_total_rays, param_
     return grid_desc + struct.pack("<4I", n_slots, cap, n_total_rays, param_dtype)
 
 
+ENCODE_STAGE_POINTS = 1 << 21
 OGRID_STAGE_POINTS = 1 << 20
 OGRID_STAGE_BYTES = 144
 

@@ -1627,17 +1627,24 @@ extern "C" void hashgrid_encode_staged(ngp_stream_t stream_, void **buffers, con
     float *lm = (float *)buffers[3];
     HashGridDescriptor dl = d;
     dl.enc_layout = NGP_ENC_LEVEL_MAJOR;
-    if (d.table_dtype == NGP_DTYPE_F32) launch_fwd<float>(dl, stream, pos, buffers[1], lm);
-    else launch_fwd<__half>(dl, stream, pos, buffers[1], lm);
-    if (!check_launch(target)) return;
-    const dim3 g(div_up(d.n_points, kTransposePoints)), b(kBlock);
-    if (d.F == 2)
-        hipLaunchKernelGGL(encodings_to_points_kernel<float2>, g, b, 0, stream, d.n_points, d.L, (const float2 *)lm,
-                           (float2 *)buffers[2]);
-    else
-        hipLaunchKernelGGL(encodings_to_points_kernel<float4>, g, b, 0, stream, d.n_points, d.L, (const float4 *)lm,
-                           (float4 *)buffers[2]);
-    check_launch(target);
+    // pieces, so that the workspace does not grow with the points past 256 MiB (L = 16, F = 2)
+    for (uint32_t n0 = 0; n0 < d.n_points;) {
+        dl.n_points = std::min(d.n_points - n0, NGP_ENCODE_STAGE_POINTS);
+        const float *p = pos + 3 * (size_t)n0;
+        float *out = (float *)buffers[2] + (size_t)n0 * d.L * d.F;
+        if (d.table_dtype == NGP_DTYPE_F32) launch_fwd<float>(dl, stream, p, buffers[1], lm);
+        else launch_fwd<__half>(dl, stream, p, buffers[1], lm);
+        if (!check_launch(target)) return;
+        const dim3 g(div_up(dl.n_points, kTransposePoints)), b(kBlock);
+        if (d.F == 2)
+            hipLaunchKernelGGL(encodings_to_points_kernel<float2>, g, b, 0, stream, dl.n_points, d.L, (const float2 *)lm,
+                               (float2 *)out);
+        else
+            hipLaunchKernelGGL(encodings_to_points_kernel<float4>, g, b, 0, stream, dl.n_points, d.L, (const float4 *)lm,
+                               (float4 *)out);
+        if (!check_launch(target)) return;
+        n0 += dl.n_points;
+    }
 }
 
 extern "C" int hashgrid_encode_backward_adam_supported(const char *opaque, size_t opaque_len) {

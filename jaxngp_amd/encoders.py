@@ -81,7 +81,8 @@ class _HashGridFn(torch.autograd.Function):
         N = pos.shape[0]
         enc = torch.empty(N, n_out, dtype=torch.float32, device=pos.device)
         if _staged(N, n_out // n_features, n_features):
-            _lib.call("hashgrid_encode_staged", [pos, table.contiguous(), enc, torch.empty_like(enc)], desc_fn(N))
+            ws = torch.empty(min(N, _lib.ENCODE_STAGE_POINTS) * n_out, dtype=torch.float32, device=pos.device)
+            _lib.call("hashgrid_encode_staged", [pos, table.contiguous(), enc, ws], desc_fn(N))
         elif N:
             _lib.call("hashgrid_encode", [pos, table.contiguous(), enc], desc_fn(N))
         ctx.save_for_backward(pos)

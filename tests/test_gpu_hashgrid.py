@@ -217,6 +217,24 @@ def test_forward_over_the_ways_levels_are_dealt(dev, L, T, F, N, half):
         np.testing.assert_array_equal(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("F, half", [(2, False), (4, True)])
+def test_staged_forward_in_pieces(dev, F, half):
+    """More points than the workspace of the staged forward takes at once: two whole pieces and
+    a rest of one point, with nothing written past the workspace, bit for bit as point by point."""
+    from jaxngp_amd import _lib
+    piece = _lib.ENCODE_STAGE_POINTS
+    N, L = 2 * piece + 1, 3
+    enc = HashGridEncoder(L=L, T=2 ** 12, F=F, N_min=8, N_max=64, param_dtype=torch.float16 if half else torch.float32,
+                          generator=torch.Generator().manual_seed(1)).to(dev)
+    pos = torch.rand(N, 3, generator=torch.Generator(device=dev).manual_seed(2), device=dev) * 2 - 1
+    out, want = torch.empty(N, L * F, device=dev), torch.empty(N, L * F, device=dev)
+    ws = torch.full((L * piece * F + 64,), 7.0, device=dev)
+    _lib.call("hashgrid_encode_staged", [pos, enc.table.detach(), out, ws], enc.descriptor(N, 1.0))
+    _lib.call("hashgrid_encode", [pos, enc.table.detach(), want], enc.descriptor(N, 1.0))
+    assert torch.equal(out, want)
+    assert (ws[L * piece * F:] == 7.0).all()
+
+
 def _backward_raw(enc, pos_t, g_t):
     from jaxngp_amd import _lib
     N = pos_t.shape[0]
