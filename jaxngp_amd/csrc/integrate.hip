@@ -321,15 +321,16 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
-constexpr int kInferenceBlock = 1024;
-__global__ void __launch_bounds__(kInferenceBlock)
+// One thread per slot, one atomic per workgroup of kThreads (see inference_threads).
+template <int kThreads>
+__global__ void __launch_bounds__(kThreads)
     integrate_inference_kernel(uint32_t n_total_rays, uint32_t n_rays, uint32_t cap, const float *__restrict__ rays_bg,
                                const float *__restrict__ rays_rgbd, const float *__restrict__ rays_T,
                                const uint32_t *__restrict__ n_samples, const uint32_t *__restrict__ indices,
                                const float *__restrict__ dss, const float *__restrict__ zs,
                                const float *__restrict__ drgbs, uint32_t *__restrict__ terminate_cnt,
                                bool *__restrict__ terminated, float *__restrict__ rgbd_out, float *__restrict__ T_out) {
-    const uint32_t i = blockIdx.x * kInferenceBlock + threadIdx.x;
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
     uint32_t term = 0;
     if (i < n_rays) {
         const uint32_t n = min(n_samples[i], cap);
@@ -371,18 +372,24 @@ __global__ void __launch_bounds__(kInferenceBlock)
         T_out[i] = Tout;
     }
     // one atomic per workgroup: they follow one another at about 10 ns each (a round of 2^18
-    // slots that all end, one per wavefront: 51 us, now 9)
-    __shared__ uint32_t wave_n[kInferenceBlock / kWave];
+    // slots that all end, one per wavefront: 51 us, now 9 with workgroups of 1,024)
+    __shared__ uint32_t wave_n[kThreads / kWave];
     const uint32_t ws = wave_sum(term);
     if (lane_id() == 0) wave_n[threadIdx.x / kWave] = ws;
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t tot = 0;
 #pragma unroll
-        for (int w = 0; w < kInferenceBlock / kWave; ++w) tot += wave_n[w];
+        for (int w = 0; w < kThreads / kWave; ++w) tot += wave_n[w];
         if (tot != 0) atomicAdd(terminate_cnt, tot);
     }
 }
+
+// Many slots of few samples: large workgroups, so that the atomics are few.  Few slots, or
+// slots of many samples, which take longer than the atomics: small ones, on more CUs.  us
+// with 256 and 1,024 threads: 2^18 slots of up to 8 35 and 29, of 16 83 and 76, of 64 406 and
+// 433; 2^17 of 8 15.5 and 14.2, of 16 30 and 31; 2^14 of 64 27 and 51; 4,096 of 200 74 and 157.
+inline int inference_threads(uint32_t n_slots, uint32_t cap) { return n_slots >= (uint64_t)cap << 14 ? 1024 : 256; }
 
 // Workgroups for one-wavefront-per-ray kernels: enough wavefronts to fill the chip
 // several times over; wavefronts loop over further rays.
@@ -731,7 +738,9 @@ extern "C" void integrate_rays_inference(ngp_stream_t stream_, void **buffers, c
     uint32_t *cnt = (uint32_t *)buffers[8];
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, cnt);
     if (d.n_rays > 0) {
-        hipLaunchKernelGGL(integrate_inference_kernel, dim3(div_up(d.n_rays, kInferenceBlock)), dim3(kInferenceBlock), 0, stream,
+        const int threads = inference_threads(d.n_rays, d.march_steps_cap);
+        hipLaunchKernelGGL((threads == 1024 ? integrate_inference_kernel<1024> : integrate_inference_kernel<256>),
+                           dim3(div_up(d.n_rays, threads)), dim3(threads), 0, stream,
                            d.n_total_rays, d.n_rays, d.march_steps_cap, (const float *)buffers[0],
                            (const float *)buffers[1], (const float *)buffers[2], (const uint32_t *)buffers[3],
                            (const uint32_t *)buffers[4], (const float *)buffers[5], (const float *)buffers[6],

@@ -410,3 +410,29 @@ def test_integrate_rays_inference_bit_exact(dev):
     want_T[idx[keep]] = T_o[keep]
     np.testing.assert_array_equal(N(rgbd), want_rgbd)
     np.testing.assert_array_equal(N(Tn), want_T)
+
+
+@pytest.mark.parametrize("n, cap", [((1 << 14) - 1, 1), (1 << 14, 1), ((3 << 14) - 1, 3), ((3 << 14) + 1, 3), (257, 70)])
+def test_integrate_rays_inference_both_workgroup_sizes(dev, n, cap):
+    """Both sides of the line between workgroups of 256 and 1,024 threads, with a part of a
+    workgroup at the end, bit for bit against the oracle; the terminated rays are counted."""
+    rng = np.random.default_rng(n)
+    n_total = 2 * n
+    ns = rng.integers(0, cap + 1, n).astype(np.uint32)
+    idx = rng.permutation(n_total + n // 2)[:n].astype(np.uint32)  # some past the last ray
+    bg = rng.uniform(0, 1, (n_total, 3)).astype(np.float32)
+    rgbd = rng.uniform(0, 1, (n_total, 4)).astype(np.float32)
+    trans = rng.uniform(0.0002, 1, n_total).astype(np.float32)
+    dss = np.full((n, cap), 0.01, np.float32)
+    z = rng.uniform(1, 2, (n, cap)).astype(np.float32)
+    drgbs = rng.uniform(0, 1, (n, cap, 4)).astype(np.float32)
+    drgbs[..., 0] *= rng.choice([1.0, 1000.0], (n, 1)).astype(np.float32)
+    got = volrend.integrate_rays_inference(T(bg, dev), T(rgbd, dev), T(trans, dev), U(ns, dev), U(idx, dev), T(dss, dev),
+                                           T(z, dev), T(drgbs, dev))
+    cnt, term, rgbd_o, T_o = oracle.integrate_rays_inference(bg, rgbd, trans, ns, idx, dss, z, drgbs)
+    assert int(N(got[0].view(torch.int32))) == int(cnt)
+    np.testing.assert_array_equal(N(got[1]), term)
+    keep = idx < n_total
+    rgbd[idx[keep]], trans[idx[keep]] = rgbd_o[keep], T_o[keep]
+    np.testing.assert_array_equal(N(got[2]), rgbd)
+    np.testing.assert_array_equal(N(got[3]), trans)
