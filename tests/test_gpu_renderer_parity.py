@@ -194,3 +194,10 @@ def test_field_chunks_pack_live_entries(dev, n_slots, cap, half):
         with torch.no_grad():
             want[live] = model(xyzs[live].contiguous(), rays_d[ray[slot]].contiguous(), None)[0]
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n_slots, cap", [(8192, 8), (8193, 8), (65537, 1)])
+def test_field_chunks_pack_both_widths(dev, n_slots, cap, half):
+    """Both sides of 65,536 entries, up to which a wavefront takes 16 of them at a time."""
+    test_field_chunks_pack_live_entries(dev, n_slots, cap, half)
