@@ -201,3 +201,12 @@ def test_field_chunks_pack_live_entries(dev, n_slots, cap, half):
 def test_field_chunks_pack_both_widths(dev, n_slots, cap, half):
     """Both sides of 65,536 entries, up to which a wavefront takes 16 of them at a time."""
     test_field_chunks_pack_live_entries(dev, n_slots, cap, half)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n_slots, cap", [(2 ** 17 + 5, 8), (12_345, 70)])
+def test_field_chunks_pack_over_several_groups(dev, n_slots, cap, half):
+    """More than 786,432 entries, so that a wavefront takes several groups of 64: live entries
+    left over from one group go in front of the next one's, and slots and places advance by
+    the launch's stride, with a cap that divides 64 and one that does not."""
+    test_field_chunks_pack_live_entries(dev, n_slots, cap, half)
