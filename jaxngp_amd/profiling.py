@@ -31,7 +31,7 @@ import sys
 TARGET_KERNELS = {
     "march_rays": (["march_begin_kernel", "march_count_kernel", "march_scan_kernel", "march_emit_kernel",
                     "march_fill_kernel", "march_finish_kernel", "march_empty_kernel"], "march_scan_kernel"),
-    "hashgrid_encode": (["hashgrid_fwd_kernel", "encodings_to_points_kernel"], "hashgrid_fwd_kernel"),
+    "hashgrid_encode": (["hashgrid_fwd_kernel", "hashgrid_fwd_points_kernel", "encodings_to_points_kernel"], None),
     "hashgrid_encode_backward": (["gradients_to_levels_kernel", "bwd_bucket_kernel", "bwd_slice_parts_kernel",
                                   "bwd_combine_runs_kernel", "bwd_reduce_runs_kernel", "bwd_count_kernel",
                                   "scan_sums_kernel", "scan_apply_kernel", "plan_parts_kernel", "bwd_scatter_kernel",
@@ -45,7 +45,8 @@ TARGET_KERNELS = {
     "train_integrate": (["train_prepare_kernel", "train_integrate_kernel"], "train_integrate_kernel"),
     "integrate_rays_backward": (["integrate_backward_kernel", "fill_zero2_kernel"], "integrate_backward_kernel"),
     "occupancy_grid_update": (["ogrid_update_kernel", "ogrid_decay_kernel", "ogrid_prefix_kernel",
-                               "ogrid_points_kernel", "ogrid_density_kernel"], "ogrid_decay_kernel"),
+                               "ogrid_points_kernel", "ogrid_points_kernel+", "ogrid_hashgrid_fwd_kernel",
+                               "ogrid_density_kernel"], "ogrid_points_kernel"),
     "proposal_train_samples": (["proposal_train_kernel", "proposal_train_scan_kernel", "proposal_train_write_kernel",
                                 "proposal_train_tail_kernel"], "proposal_train_scan_kernel"),
 }
@@ -70,6 +71,27 @@ def _base(name: str) -> str:
     return _short(name).split("<")[0]
 
 
+def _dispatches(path: str):
+    """(kernel, counter, value) of a counter file's rows.  The occupancy update's kernels are
+    told by what was dispatched before them: the encoder launches of its chunks are
+    `ogrid_hashgrid_fwd_kernel`, not the encoder's own, and the chunks of an update after its
+    first `ogrid_points_kernel+`, so that `ogrid_points_kernel` counts updates."""
+    rows = list(csv.DictReader(open(path)))
+    names = {int(r["Dispatch_Id"]): _base(r["Kernel_Name"]) for r in rows}
+    label, before = {}, None
+    for i in sorted(names):
+        k = names[i]
+        if k == "hashgrid_fwd_kernel" and before == "ogrid_points_kernel":
+            label[i] = "ogrid_hashgrid_fwd_kernel"
+        elif k == "ogrid_points_kernel" and before == "ogrid_density_kernel":
+            label[i] = "ogrid_points_kernel+"
+        else:
+            label[i] = k
+        before = k
+    for r in rows:
+        yield label[int(r["Dispatch_Id"])], r["Counter_Name"], float(r["Counter_Value"] or 0)
+
+
 def stats(path: str, top: int = 40) -> str:
     rows = list(csv.DictReader(open(path)))
     tot = sum(float(r["TotalDurationNs"]) for r in rows)
@@ -86,12 +108,12 @@ def _counter(d: str, name: str | None = None) -> dict:
     counter `name` (all rows when None: a run of one counter)"""
     agg = collections.defaultdict(lambda: [0, 0.0])
     for f in glob.glob(d + "/**/*counter_collection*.csv", recursive=True):
-        for r in csv.DictReader(open(f)):
-            if name is not None and r["Counter_Name"] != name:
+        for kernel, counter, value in _dispatches(f):
+            if name is not None and counter != name:
                 continue
-            a = agg[_base(r["Kernel_Name"])]
+            a = agg[kernel]
             a[0] += 1
-            a[1] += float(r["Counter_Value"] or 0)
+            a[1] += value
     return agg
 
 
@@ -153,10 +175,10 @@ def _read_keyed(path: str, key: str) -> dict:
 def counters(pmc_dir: str) -> str:
     rows = collections.defaultdict(lambda: collections.defaultdict(lambda: [0, 0.0]))
     for f in glob.glob(pmc_dir + "/**/*counter_collection*.csv", recursive=True):
-        for r in csv.DictReader(open(f)):
-            a = rows[_base(r["Kernel_Name"])][r["Counter_Name"]]
+        for kernel, counter, value in _dispatches(f):
+            a = rows[kernel][counter]
             a[0] += 1
-            a[1] += float(r["Counter_Value"] or 0)
+            a[1] += value
     ours = {k for ks, _ in TARGET_KERNELS.values() for k in ks} | set(EXTRA_KERNELS)
     names = sorted({c for k in rows if k in ours for c in rows[k]})
     out = [f"{'kernel (average per dispatch)':32s} {'dispatches':>10s} " + " ".join(f"{c:>26s}" for c in names)]

@@ -48,6 +48,22 @@ def test_l2_hit_rate_per_target_and_kernel(tmp_path):
     assert float(per_kernel["bwd_reduce_kernel"]) == pytest.approx(1 / 6, abs=1e-3)
 
 
+def test_the_occupancy_updates_encoder_is_its_own(tmp_path):
+    """A step's encoder launch and an update of two chunks: the encoder's bytes are the step's
+    alone, and the update is one launch with its chunks' encoders in it."""
+    name = lambda k: f"void ngp::(anonymous namespace)::{k}<2, float>(ngp::HashGridDescriptor)"
+    order = ["hashgrid_fwd_kernel", "mlp_forward_kernel", "ogrid_decay_kernel", "ogrid_prefix_kernel"] + \
+        ["ogrid_points_kernel", "hashgrid_fwd_kernel", "ogrid_density_kernel"] * 2 + ["hashgrid_fwd_kernel"]
+    for d, c in (("f", "FETCH_SIZE"), ("w", "WRITE_SIZE")):
+        _write(tmp_path / d, [(name(k), c, 10.0 if k == "hashgrid_fwd_kernel" else 1.0) for k in order])
+        _write(tmp_path / ("c" + d), [("__amd_rocclr_copyBuffer", c, 1024.0)])
+    out = profiling.traffic(*(str(tmp_path / n) for n in ("f", "w", "cf", "cw")), 1048576.0)
+    (tmp_path / "t.txt").write_text(out)
+    got = profiling.read_traffic(str(tmp_path / "t.txt"))
+    assert got["hashgrid_encode"] == 2 * 10 * 1024.0
+    assert got["occupancy_grid_update"] == 2 * (2 + 2 * (1 + 10 + 1)) * 1024.0
+
+
 def test_read_traffic_of_a_missing_file_is_empty(tmp_path):
     assert profiling.read_traffic(str(tmp_path / "none.txt")) == {}
 
