@@ -208,7 +208,7 @@ __global__ void __launch_bounds__(kBlock)
 
 // [n, L * F] gradients -> [L, n, F], for F = 2: the same the other way.  The level's bucket
 // kernel then reads whole lines; point-major it takes 8 bytes of each of 64 lines, and
-// every level reads the lines again (2^18 ray samples f32: bucket 97 -> 70 us for 15 here).
+// every level reads the lines again (2^18 ray samples f32: bucket 97 -> 68 us for 15 here).
 __global__ void __launch_bounds__(kBlock)
     gradients_to_levels_kernel(uint32_t n_points, uint32_t L, const float2 *__restrict__ pm, float2 *__restrict__ lm) {
     __shared__ float2 tile[kTransposePoints * (NGP_HASHGRID_MAX_LEVELS + 1)];
@@ -313,8 +313,8 @@ inline uint32_t level_last_box_row(const HashGridDescriptor &d, uint32_t l) {
 // 16-bit row within the slice: 10 or 6 bytes instead of 12 or 8.
 constexpr int kBucketThreads = 512;
 // f32 entries: items of 1024 points (two per thread) leave the reducer half as many runs
-// (reduce 64 against 67 us at 2^18 points); the smaller f16 entries gain more from the
-// lighter kernel of one point per thread (bucket 50 against 60 us).
+// (3 us of it at 2^18 points); the smaller f16 entries gain more from the lighter kernel of
+// one point per thread (10 us of the bucket kernel).
 constexpr int bucket_phases(bool half_values) { return half_values ? 1 : 2; }
 constexpr uint32_t bucket_points(bool half_values) { return kBucketThreads * bucket_phases(half_values); }
 constexpr uint32_t bucket_entries(bool half_values) { return bucket_points(half_values) * 8; }  // one item's at most
@@ -805,7 +805,7 @@ __device__ __forceinline__ void sum_runs(float *v, const CellRuns &r) {
 // the entry buffer (bucket_entries), the entries go to run start + rank, and
 // the run's start and length are stored for the reducers.  Within a run, entries are in
 // LDS-atomic order; the reducer's sums do not depend on it beyond f64 rounding.
-// 2^18 ray samples: f32 110 -> 68 us, f16 90 -> 50 us.  It was bound by the run merge
+// 2^18 ray samples: f32 110 -> 68 us, f16 90 -> 55 us.  It was bound by the run merge
 // (each corner found its own runs: 626 vector instructions a wavefront and level) and,
 // once that was cheaper (86 us), by 17 M scattered 12-byte stores.  kSlices: counters for as
 // many slices as a level can reach; the last of them, kMaxSlices, take 32 KiB of LDS.
@@ -1096,10 +1096,11 @@ __global__ void __launch_bounds__(kReduceThreads)
 // it.  Its sums stay f64 until the parts are added, so the result does not depend on the cut.
 // With kAdam, a slice summed in one part is not stored: its rows take the optimizer
 // step in place (params, m, v), and bwd_combine_runs does the same for the others.
-// 2^18 ray samples, f32: 82 -> 65 us, of which the atomics themselves need 27 (34 M f64
+// 2^18 ray samples, f32: 82 -> 67 us, of which the atomics themselves need 27 (34 M f64
 // adds at 1.27 T/s); slices of 64 KiB, two workgroups to a CU, so that one clears or
 // stores its rows while the other adds (128 KiB slices: 80 us); 1,024 points: 29 -> 17.
-// All four parts: f32 190 -> 145 us, f16 176 -> 125; 1,024 points, two parts: 44 -> 25.
+// All four kernels: f32 190 -> 145 us (68 + 5 + 67 + 5), f16 176 -> 130 (55 + 7 + 64 + 5);
+// 1,024 points, two kernels: 44 -> 25.
 struct RunSequence {
     uint32_t *marks;        // 64 words of LDS of the wavefront's own, tags below `tag`
     uint32_t tag;           // of the latest group of 64 places

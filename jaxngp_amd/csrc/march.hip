@@ -351,10 +351,15 @@ __device__ __forceinline__ RayRecord record_of(const RecordStore &st, uint32_t i
 // address per ray, about 10 ns each one after another: 4096 rays took 114 us.)
 // The march is bound by one ray's latency, a chain of windows of about 250
 // instructions: few wavefronts in flight lose little and march few rays past the fill.
-// march_rays of 2^18 camera rays, about 20 samples each, into 2^18 slots: 552 us with
-// launches of growing size, 221 in rounds, 146 with empty stretches crossed at once; 4,096
-// rays into more slots than they fill: 292, 149, 101.  (Rounds of 4,096 rays take 162
-// instead of 152, and beside a training step's MLP backward 21 us of the step.)
+// march_rays of 2^18 camera rays, about 38 samples each, into 2^18 slots, a call: 571 us with
+// launches of growing size, now 161 (0.4 of it in rounds, 0.28 with empty stretches crossed
+// at once).  Rounds of 4,096 rays take 10 us more, and beside a training step's MLP backward
+// 21 us of the step.  Two cascades and growing steps (bound 2, from inside): 713 -> 371, 4,096
+// rays into more slots than they fill 335 -> 182; bounds 4 and 16 5,590 -> 1,145 and 7,490 ->
+// 4,738.  The exception is a grid without an empty cell, where the first round fills the
+// buffer and the workgroups that end early march a block in vain: 2^16 rays, two cascades, 92
+// -> 109 (2^18 rays 93 -> 75).  A watch on the last round's counter between windows mends that
+// at the price of 50 us in the first case, the first round in a launch of its own at 12.
 template <bool kOne>
 __global__ void __launch_bounds__(kBlock)
     march_count_kernel(MarchParams p, bool word_ok, uint32_t n_rays, uint32_t total_samples, uint32_t block_begin,

@@ -367,8 +367,8 @@ __device__ __forceinline__ void forward_only(const float *lds, float dx, float d
 // whose way stood three things: the weights' copy to LDS float by float (10 us a workgroup,
 // two rounds of them), one exponential after the other on a quarter of the lanes, and two
 // wavefronts per SIMD, since the compiler kept the 160 weights of a lane in registers.  Now
-// 16-byte reads from LDS and 88 registers, four wavefronts.  2^18 samples: 70 -> 52 us,
-// 2^20: 230 -> 192, 1,000: 9.9 -> 6.0.
+// 16-byte reads from LDS and 88 registers, four wavefronts.  2^18 samples: 67 -> 47 us,
+// 2^20: 219 -> 175, 1,000: 9.9 -> 6.0.
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
     mlp_forward_kernel(uint32_t n, bool level_major, const float *__restrict__ enc, const float *__restrict__ dirs,
                        const float *__restrict__ params, float *__restrict__ drgbs) {
@@ -444,7 +444,8 @@ __device__ __forceinline__ void dw_part_to_row(float *dst, const v4f *acc, int o
 // Bounded by the f32 matrix unit (464 MFMAs a tile, 103 us for 2^18 samples), with two
 // wavefronts per SIMD between ten barriers a tile to feed it.  A layer's dZ is computed
 // before the barrier that dW's operands wait for, and those are read four samples at a time
-// (scratch_read_at): 2^18 samples 158 -> 150 us, f16 69 -> 67.
+// (scratch_read_at).  2^18 samples, with the sum of the workgroups' rows: 166 -> 146 us, f16
+// 72 -> 62.
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
     mlp_backward_kernel(uint32_t n, bool level_major, const float *__restrict__ enc, const float *__restrict__ dirs,
                         const float *__restrict__ params, const float *__restrict__ dL_ddrgbs,
@@ -1250,8 +1251,9 @@ __global__ void __launch_bounds__(kPrefixThreads)
 // slot chooses its cell and point, hashgrid_encode gathers level by level, and the density
 // MLP runs on its encodings.  The points are random, so the gathers miss: the fused kernel
 // waits for them with two wavefronts per SIMD on all levels' rows at once, and its four
-// lanes of a sample each search the occupied cells.  2^20 cells, T = 2^19: f32 1087 -> 420 us,
-// f16 881 -> 370.
+// lanes of a sample each search the occupied cells.  2^20 random cells of 2^21, T = 2^19, with
+// the decay and the prefix: fused and staged f32 1,112 and 478 us, f16 907 and 399; all 2^21:
+// 1,057 and 631, 861 and 446.
 __global__ void __launch_bounds__(256)
     ogrid_points_kernel(OgridArgs a, uint32_t j0, uint32_t n, const uint32_t *__restrict__ alive,
                         const uint32_t *__restrict__ prefix, const uint64_t *__restrict__ words,

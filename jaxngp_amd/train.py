@@ -97,10 +97,9 @@ class TrainConfig:
     prefetch_march: bool = True
     # FP32: the table's optimizer step taken inside the table gradient's last pass
     # (hashgrid_encode_backward_adam; same results, the gradient never goes through
-    # memory) when the encoder allows it.  Off by default: measured, the step was no
-    # faster (0.784 against 0.780 ms): the separate update streams its 341 MB at
-    # about 6 TB/s, while in the reducer's tail (one workgroup per CU, held by its
-    # 128 KiB of LDS) the same rows move at about 5.5 TB/s, which eats the 98 MB saved
+    # memory) when the encoder allows it.  The step takes 558 us instead of 572 then (it was
+    # no faster with the reducer of 128 KiB slices, one workgroup per CU).  Off by default:
+    # the step then leaves no table gradient in its buffers, which a caller may read.
     fused_table_update: bool = False
 
 
